@@ -903,6 +903,7 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
   b.h_conv.clear();
   b.h_xill.clear();
   b.h_prim.clear();
+  b.h_ang.clear();
   b.h_rrc.clear();
   b.h_nth.clear();
   b.n_nth_sol = 0;
@@ -933,8 +934,6 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
     }
   }
   int64_t o_ener = 0, o_flux = 0, o_pgrid = 0, o_prof = 0, o_xspec = 0, o_dist = 0, o_zone = 0, o_rrc = 0;
-  int64_t o_node = 0;
-  const int64_t node_stride = 2 * (int64_t)g.rel.n_r * g.rel.n_g * 2;
   for (int i = 0; i < n_req; i++) {
     const rx_request &r = req[i];
     if (r.n_flux <= 0 || !r.energy || !r.parameter) {
@@ -1077,11 +1076,7 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
     p.need_cosne = (p.limb != 0 || (p.n_incl > 0 && !xill_model)) ? 1 : 0;
     p.dist_off = o_dist;
     o_dist += (int64_t)p.n_incl * p.n_zones;
-    p.node_off = -1;
-    if (p.n_incl > 0 && !xill_model) {
-      p.node_off = o_node;
-      o_node += node_stride;
-    }
+    if (p.n_incl > 0 && !xill_model) b.h_ang.push_back(i);
     p.pre_status = st;
     b.h_status[i] = st;
   }
@@ -1091,7 +1086,6 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
   b.tot_prof = o_prof;
   b.tot_xspec = o_xspec;
   b.tot_dist = o_dist;
-  b.tot_node = o_node;
   b.tot_zone = o_zone;
   b.tot_rrc = o_rrc;
   b.n_xill1 = (int)b.h_xill.size();
@@ -1174,7 +1168,6 @@ int batch_upload(Batch &b) {
   e |= b.d_flux_in.ensure(sizeof(double) * b.tot_flux);
   e |= b.d_out.ensure(sizeof(double) * b.tot_flux);
   e |= b.d_pgrid.ensure(sizeof(double) * std::max<int64_t>(1, b.tot_pgrid));
-  e |= b.d_node.ensure(sizeof(double) * std::max<int64_t>(1, b.tot_node));
   e |= b.d_rad.ensure(sizeof(RadRec) * nreq * g.nr_fine);
   e |= b.d_rnode.ensure(sizeof(double) * RAD_NODE_ARRAYS * nreq * g.rel.n_r);
   e |= b.d_rnorm.ensure(sizeof(ReqNorm) * nreq);
@@ -1186,6 +1179,7 @@ int batch_upload(Batch &b) {
   e |= b.d_conv.ensure(sizeof(XillWork) * std::max<size_t>(1, b.h_conv.size()));
   e |= b.d_xill.ensure(sizeof(XillWork) * std::max<size_t>(1, b.h_xill.size()));
   e |= b.d_prim.ensure(sizeof(int) * std::max<size_t>(1, b.h_prim.size()));
+  e |= b.d_ang.ensure(sizeof(int) * std::max<size_t>(1, b.h_ang.size()));
   e |= b.d_rrc.ensure(sizeof(XillWork) * std::max<size_t>(1, b.h_rrc.size()));
   e |= b.d_rrcorr.ensure(sizeof(double) * std::max<int64_t>(1, b.tot_rrc));
   e |= b.d_nthw.ensure(sizeof(XillWork) * std::max<size_t>(1, b.h_nth.size()));
@@ -1215,6 +1209,8 @@ int batch_upload(Batch &b) {
                              b.stream);
   if (!b.h_prim.empty())
     e |= (int)hipMemcpyAsync(b.d_prim.p, b.h_prim.data(), sizeof(int) * b.h_prim.size(), hipMemcpyHostToDevice, b.stream);
+  if (!b.h_ang.empty())
+    e |= (int)hipMemcpyAsync(b.d_ang.p, b.h_ang.data(), sizeof(int) * b.h_ang.size(), hipMemcpyHostToDevice, b.stream);
   if (!b.h_xill.empty())
     e |= (int)hipMemcpyAsync(b.d_xill.p, b.h_xill.data(), sizeof(XillWork) * b.h_xill.size(), hipMemcpyHostToDevice,
                              b.stream);
@@ -1232,14 +1228,12 @@ static BatchDev dev_view(Batch &b) {
   bd.n_req = b.n_req;
   bd.nr_fine = g.nr_fine;
   bd.seg_bins = b.seg_bins;
-  bd.node_stride = 2 * g.rel.n_r * g.rel.n_g * 2;
   bd.max_zones = b.max_zones;
   bd.req = b.d_req.as<ReqParams>();
   bd.ener_in = b.d_ener.as<double>();
   bd.flux_in = b.d_flux_in.as<double>();
   bd.out = b.d_out.as<double>();
   bd.pgrid = b.d_pgrid.as<double>();
-  bd.node = b.d_node.as<double>();
   bd.rad = b.d_rad.as<RadRec>();
   bd.rnode = b.d_rnode.as<double>();
   bd.rnorm = b.d_rnorm.as<ReqNorm>();
@@ -1275,6 +1269,7 @@ static int launch_sequence(Batch &b, const RunKey &k, hipStream_t s) {
   e |= launch_nth(bd, static_cast<const XillWork *>(k.d_nth), k.n_nth, s);
   e |= launch_rrad_corr(bd, static_cast<const XillWork *>(k.d_rrc), k.n_rrc, s);
   e |= launch_setup(bd, s);
+  e |= launch_dist(bd, static_cast<const int *>(k.d_ang), k.n_ang, s);
   if (prof) e |= (int)hipEventRecord(b.ev[1], s);
   e |= launch_integrate(bd, k.n_blocks, k.cos_rows != 0, s);
   if (prof) e |= (int)hipEventRecord(b.ev[2], s);
@@ -1351,6 +1346,8 @@ int batch_run(Batch &b, int precision, std::string &err) {
   k.n_rrc = (int)b.h_rrc.size();
   k.d_nth = b.d_nthw.p;
   k.n_nth = (int)b.h_nth.size();
+  k.d_ang = b.d_ang.p;
+  k.n_ang = (int)b.h_ang.size();
   k.prof = g.profile ? 1 : 0;
   k.cos_rows = b.any_limb ? 1 : 0;
   hipStream_t s = b.stream;

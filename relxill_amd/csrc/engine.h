@@ -49,8 +49,8 @@ void rzone_grid(double rmin, double rmax, int nzones, double h, double *rgrid);
 // its padding zeroed, so configurations compare with memcmp.
 struct RunKey {
   BatchDev bd;
-  int n_blocks, n_xill1, n_xill, n_conv, n_prim, n_rrc, n_nth;
-  const void *d_xill, *d_conv, *d_prim, *d_rrc, *d_nth;
+  int n_blocks, n_xill1, n_xill, n_conv, n_prim, n_rrc, n_nth, n_ang;
+  const void *d_xill, *d_conv, *d_prim, *d_rrc, *d_nth, *d_ang;
   int prof, cos_rows;
 };
 
@@ -65,6 +65,7 @@ struct Batch {
   std::vector<int> h_status;  // host-side parse status
   std::vector<double> h_ener, h_flux_in;
   std::vector<int> h_prim;
+  std::vector<int> h_ang;        // requests with an emission-angle distribution (k_dist)
   std::vector<XillWork> h_conv;  // (request, zone) units of k_conv
   std::vector<XillWork> h_xill;  // k_xill units: one-zone requests first, then the others (all zones in one unit)
   int n_xill1 = 0;               // number of one-zone units at the front of h_xill
@@ -72,10 +73,9 @@ struct Batch {
   std::vector<XillWork> h_nth;   // nthcomp solves: (request, 0 source / 1 + zone)
   int n_nth_sol = 0;             // requests with the nthcomp primary (one source solution each)
   int64_t tot_ener = 0, tot_flux = 0, tot_pgrid = 0, tot_prof = 0, tot_xspec = 0, tot_dist = 0, tot_zone = 0;
-  int64_t tot_node = 0;  // node rows of the requests with an angle distribution
   int64_t tot_rrc = 0;
-  DevBuf d_req, d_ener, d_flux_in, d_out, d_pgrid, d_node, d_rad, d_prof, d_dist, d_refl, d_status, d_conv;
-  DevBuf d_xill, d_xspec, d_zone, d_prim, d_rrc, d_rrcorr;
+  DevBuf d_req, d_ener, d_flux_in, d_out, d_pgrid, d_rad, d_prof, d_dist, d_refl, d_status, d_conv;
+  DevBuf d_xill, d_xspec, d_zone, d_prim, d_ang, d_rrc, d_rrcorr;
   DevBuf d_nthw, d_nth, d_nthx, d_nths, d_nthn;
   DevBuf d_items, d_ctr, d_fix, d_reach, d_rnorm, d_rnode;
   int item_cap = 0;

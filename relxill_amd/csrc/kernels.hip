@@ -4,8 +4,10 @@
 //   k_setup      one workgroup per request: (a, mu0) bilinear table
 //                interpolation (interpol_relTable, src/Relprofile.cpp:141-303),
 //                fine radial grid, emissivity (src/Rellp.cpp:518-564), energy
-//                windows, angle distribution (src/Relprofile.cpp:908-938), and
-//                the request's work items (radius chunk x bin segment)
+//                windows and the request's work items (radius chunk x bin
+//                segment)
+//   k_dist       one wavefront per (request, 64 radii): the emission-angle
+//                distribution (src/Relprofile.cpp:908-938)
 //   k_integrate  persistent 64-lane wavefronts over the work items: lane =
 //                fine radius, loop over the segment's bins, fixed-order wave
 //                sum per bin (calc_relline_profile, src/Relprofile.cpp:857-900)
@@ -498,7 +500,7 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
   const ReqParams rq = b.req[req];
   const DevRelTable &T = b.rt;
   const int nr = b.nr_fine;
-  const int n_r = T.n_r, ng = T.n_g;
+  const int n_r = T.n_r;
   if (rq.pre_status != 0) return;  // status already set by the host
   if (rq.model == MOD_XILLVER) {
     // the xillver models (LocalModel::xillver_model, src/LocalModel.cpp:
@@ -537,7 +539,6 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
   __shared__ double s_tre[MAX_NR_TAB], s_tgmin[MAX_NR_TAB], s_tgmax[MAX_NR_TAB];
   __shared__ double s_jr[MAX_LP_R], s_je[MAX_LP_R], s_jd[MAX_LP_R], s_ji[MAX_LP_R];
   __shared__ double s_red[SETUP_THREADS];
-  __shared__ double s_dist[NZ * MAX_INCL];
   __shared__ int s_st, s_ia, s_im, s_rmin;
   __shared__ double s_fa, s_fm, s_rms;
   constexpr int MAX_RC = MAX_NR_FINE / RAD_CHUNK;
@@ -625,19 +626,6 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
                          T.gmin[n01 * n_r + ir], T.gmin[n11 * n_r + ir]);
     s_tgmax[ir] = lerp2f(fa, fm, T.gmax[n00 * n_r + ir], T.gmax[n10 * n_r + ir],
                          T.gmax[n01 * n_r + ir], T.gmax[n11 * n_r + ir]);
-  }
-  if (rq.n_incl > 0) {  // node rows for the angle distribution below
-    double *node = b.node + rq.node_off;
-    const size_t nq = (size_t)n_r * ng;
-    const size_t s00 = n00 * nq, s10 = n10 * nq, s01 = n01 * nq, s11 = n11 * nq;
-    for (size_t q = tid; q < nq; q += SETUP_THREADS) {
-      node[q * 2 + 0] = lerp2f(fa, fm, T.trff1[s00 + q], T.trff1[s10 + q], T.trff1[s01 + q], T.trff1[s11 + q]);
-      node[q * 2 + 1] = lerp2f(fa, fm, T.trff2[s00 + q], T.trff2[s10 + q], T.trff2[s01 + q], T.trff2[s11 + q]);
-      if (rq.need_cosne) {
-        node[nq * 2 + q * 2 + 0] = lerp2f(fa, fm, T.cosne1[s00 + q], T.cosne1[s10 + q], T.cosne1[s01 + q], T.cosne1[s11 + q]);
-        node[nq * 2 + q * 2 + 1] = lerp2f(fa, fm, T.cosne2[s00 + q], T.cosne2[s10 + q], T.cosne2[s01 + q], T.cosne2[s11 + q]);
-      }
-    }
   }
   // lamp-post table node (interpol_lptable, src/Rellp.cpp:219-247)
   const bool lp = (rq.emis_type == EMIS_LP);
@@ -944,80 +932,9 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
     __syncthreads();
   }
 
-  // emission-angle distribution (:908-938).  Lane = fine radius, loop over
-  // the 2 n_g (g*, branch) columns: a radius' record is read once and its
-  // node rows are contiguous.  Neighbouring radii mostly fall into the same
-  // angle bin, so a wavefront whose valid lanes share the bin adds one wave
-  // sum to it; otherwise every lane adds its own term.
-  if (rq.n_incl > 0) {
+  if (rq.n_incl > 0) {  // k_dist adds into the angle distribution
     const int nd = rq.n_incl * nz;  // [zone][angle bin]
-    for (int k = tid; k < nd; k += SETUP_THREADS) s_dist[k] = 0.0;
-    __syncthreads();
-    const double *node = b.node + rq.node_off;
-    const size_t nq2 = (size_t)n_r * ng * 2;
-    const int cols = ng * 2;
-    const double step = (1.0 - 2 * GFAC_H) / (ng - 1);
-    const double gs0 = gstar_node(step, 0), gs1 = gstar_node(step, 1);
-    // per g*: the node value and d_gstar / sqrt(g* (1 - g*)) (s_red is free here)
-    static_assert(2 * MAX_NG <= SETUP_THREADS, "g* factors must fit the reduction buffer");
-    double *s_gs = s_red, *s_gw = s_red + MAX_NG;
-    for (int g = tid; g < ng; g += SETUP_THREADS) {
-      const double gs = gstar_node(step, g);
-      const double dgs = (g == 0 || g == ng - 1) ? 0.5 * (gs1 - gs0) + GFAC_H : gs1 - gs0;
-      s_gs[g] = gs;
-      s_gw[g] = dgs / sqrt(gs - gs * gs);
-    }
-    __syncthreads();
-    const int lane = tid & 63;
-    int derr = 0;
-    for (int i0 = 0; i0 < nr; i0 += SETUP_THREADS) {
-      const int ii = i0 + tid;
-      bool live = ii < nr;
-      RadRec rec = rad_pack(0.0, 0, 0, 1, 0);
-      if (live) {
-        rec = rad[ii];
-        live = rad_ielo(rec) <= rad_iehi(rec);
-      }
-      if (__ballot(live) == 0) continue;
-      const double re = live ? fine_radius(rq.rin, rq.rout, ii, nr) : 0.0;
-      const int K = rad_K(rec), rzone = rad_zone(rec);
-      RadGeo r = {0.0, 0.0, 0.0};
-      if (live) r = rad_geo(s_tre, s_tgmin, s_tgmax, re, K);
-      const double emisw = rec.coef * (r.gmax - r.gmin) * fac;  // emis * weight
-      const double *tlo = node + (size_t)(K + 1) * cols, *thi = node + (size_t)K * cols;
-      for (int q = 0; q < cols; q++) {
-        const int g = q >> 1;
-        const double gs = s_gs[g];
-        double tmp = 0.0;
-        int imu = -1;
-        bool ok = false;
-        if (live) {
-          const double trff = lerp1(r.ifac_r, tlo[q], thi[q]);
-          const double cosne = lerp1(r.ifac_r, tlo[nq2 + q], thi[nq2 + q]);
-          const double gv = gs * (r.gmax - r.gmin) + r.gmin;
-          imu = ((int)(rq.n_incl * (1 - cosne) + 1)) - 1;
-          const double pr = 2 * PI * gv * re;
-          tmp = re * (pr * pr) * trff * emisw * s_gw[g];
-          if (imu < 0 || imu >= rq.n_incl) derr = 40;
-          else if (tmp != tmp) derr = 41;
-          else ok = true;
-          imu += rzone * rq.n_incl;  // the radius' zone
-        }
-        const unsigned long long m_ok = __ballot(ok);
-        if (m_ok == 0) continue;
-        const int first = __ffsll((long long)m_ok) - 1;
-        const int k0 = __builtin_amdgcn_readlane(imu, first);
-        if (__ballot(ok && imu != k0) == 0) {
-          const double sum = wave_sum(ok ? tmp : 0.0);
-          if (lane == first) atomicAdd(&s_dist[k0], sum);
-        } else if (ok) {
-          atomicAdd(&s_dist[imu], tmp);
-        }
-      }
-    }
-    if (derr) atomicMax(&s_st, derr);
-    __syncthreads();
-    for (int k = tid; k < nd; k += SETUP_THREADS) b.dist[rq.dist_off + k] = s_dist[k];
+    for (int k = tid; k < nd; k += SETUP_THREADS) b.dist[rq.dist_off + k] = 0.0;
   }
   __syncthreads();
   if (s_st == 0) {
@@ -1411,6 +1328,124 @@ __device__ inline const double *profile_grid(const BatchDev &b, const ReqParams 
 }
 
 }  // namespace
+
+// Emission-angle distribution of the requests with one (src/Relprofile.cpp:
+// 908-938), one wavefront per (request, chunk of 64 fine radii), after k_setup.
+// Lane = fine radius; the node rows of the chunk's radii (transfer function
+// and cosines) are built in LDS from the table corners, STAGE_MAX values of
+// each at a time, and each lane walks the g* columns, both branches of a
+// column at once (16-byte LDS reads).  Neighbouring columns mostly fall into one angle bin, so a lane sums
+// in a register while its bin stays and adds to the LDS bins when it changes;
+// the wavefront's last bins go as one wave sum when all lanes share the bin.
+// The chunk's sums are added to the request's distribution in HBM (cleared by
+// k_setup, normalised by k_finalize).
+// Bound: FP64 issue, 1000 radii x 2 n_g columns x ~60 operations a request,
+// which one CU takes 16 us for: inside k_setup (one workgroup a request) it
+// was 61 us of a single relxill call (k_setup 87 us) and 165 us of a batch of
+// 1024 (237 us); the 16 wavefronts a request take 12 us and 94 us.
+template <int NZ>
+__global__ __launch_bounds__(64) void k_dist(BatchDev b, const int *__restrict__ reqs, int n_rc) {
+  __shared__ __align__(16) double s_t[STAGE_MAX], s_c[STAGE_MAX];
+  __shared__ double s_dist[NZ * MAX_INCL];
+  __shared__ double2 s_g[MAX_NG];
+  const int req = reqs[blockIdx.x / n_rc], c = blockIdx.x % n_rc;
+  const int lane = threadIdx.x;
+  if (b.status[req] != 0) return;  // uniform over the block
+  const ReqParams &rq = b.req[req];
+  const ReqNorm rn = b.rnorm[req];
+  const int n_incl = rq.n_incl, ng = b.rt.n_g, nr = b.nr_fine, nq = 2 * ng;
+  const int ii = c * RAD_CHUNK + lane;
+  RadRec rec = rad_pack(0.0, 0, 0, 1, 0);
+  if (ii < nr) rec = b.rad[(size_t)req * nr + ii];
+  const bool live = ii < nr && rad_ielo(rec) <= rad_iehi(rec);
+  if (__ballot(live) == 0) return;
+  const int K = rad_K(rec), zone = rad_zone(rec);
+  double amp = 0.0;  // re (2 pi re)^2 emis weight: what a radius' columns share
+  RadGeo r = {0.0, 0.0, 0.0};
+  if (live) {
+    const double *gn = b.rnode + (size_t)req * RAD_NODE_ARRAYS * b.rt.n_r;
+    const double re = fine_radius_at(rn.r1, rn.r2, ii, nr);
+    r = rad_geo(gn, gn + b.rt.n_r, gn + 2 * b.rt.n_r, re, K);
+    const double pr = 2 * PI * re;
+    amp = re * (pr * pr) * (rec.coef * (r.gmax - r.gmin) * rn.fac);
+  }
+  const int zlo = wave_min_i(live ? zone : INT_MAX), zhi = wave_max_i(live ? zone : -1);
+  for (int k = zlo * n_incl + lane; k < (zhi + 1) * n_incl; k += 64) s_dist[k] = 0.0;
+  // per g*: the node value and d_gstar / sqrt(g* (1 - g*))
+  const double step = (1.0 - 2 * GFAC_H) / (ng - 1);
+  const double gs0 = gstar_node(step, 0), gs1 = gstar_node(step, 1);
+  for (int g = lane; g < ng; g += 64) {
+    const double gs = gstar_node(step, g);
+    const double dgs = (g == 0 || g == ng - 1) ? 0.5 * (gs1 - gs0) + GFAC_H : gs1 - gs0;
+    s_g[g] = make_double2(gs, dgs / sqrt(gs - gs * gs));
+  }
+  const int kmin = wave_min_i(live ? K : INT_MAX), kmax = wave_max_i(live ? K : -1);
+  const NodeSrc ts = node_src(b.rt, rn, false), cs = node_src(b.rt, rn, true);
+  const int stage_rows = STAGE_MAX / nq;  // at least 5 (n_g <= MAX_NG)
+  int derr = 0;
+  auto put = [&](int k, double sum) {  // one lane's sum over columns of angle bin k
+    const double v = sum * amp;
+    if (v != v) derr = max(derr, 41);
+    else atomicAdd(&s_dist[zone * n_incl + k], v);
+  };
+  for (int kb = kmin; kb <= kmax; kb += stage_rows - 1) {
+    const int ke = min(kmax, kb + stage_rows - 2);
+    const int tot = (ke - kb + 2) * nq;
+    stage_table_rows<5>(ts, kb, tot, nq, s_t, lane);
+    stage_table_rows<5>(cs, kb, tot, nq, s_c, lane);
+    __syncthreads();
+    const bool mine = live && K >= kb && K <= ke;
+    const int olo = (mine ? K + 1 - kb : 0) * nq, ohi = (mine ? K - kb : 0) * nq;
+    const double2 *tlo = reinterpret_cast<const double2 *>(s_t + olo), *thi = reinterpret_cast<const double2 *>(s_t + ohi);
+    const double2 *clo = reinterpret_cast<const double2 *>(s_c + olo), *chi = reinterpret_cast<const double2 *>(s_c + ohi);
+    int cur[2] = {-1, -1};
+    double acc[2] = {0.0, 0.0};
+    for (int g = 0; g < ng; g++) {
+      const double2 t0 = tlo[g], t1 = thi[g], c0 = clo[g], c1 = chi[g], gg = s_g[g];
+      const double trff[2] = {lerp1(r.ifac_r, t0.x, t1.x), lerp1(r.ifac_r, t0.y, t1.y)};
+      const double cosne[2] = {lerp1(r.ifac_r, c0.x, c1.x), lerp1(r.ifac_r, c0.y, c1.y)};
+      const double gv = gg.x * (r.gmax - r.gmin) + r.gmin;
+      const double gw = gv * gv * gg.y;
+#pragma unroll
+      for (int br = 0; br < 2; br++) {
+        const int imu = ((int)(n_incl * (1 - cosne[br]) + 1)) - 1;
+        if (!mine) continue;
+        if (imu < 0 || imu >= n_incl) {
+          derr = 40;
+          continue;
+        }
+        if (imu != cur[br]) {
+          if (cur[br] >= 0) put(cur[br], acc[br]);
+          cur[br] = imu;
+          acc[br] = 0.0;
+        }
+        acc[br] += gw * trff[br];
+      }
+    }
+#pragma unroll
+    for (int br = 0; br < 2; br++) {
+      const int bin = cur[br] >= 0 ? zone * n_incl + cur[br] : -1;
+      const unsigned long long m_ok = __ballot(bin >= 0);
+      if (m_ok == 0) continue;
+      const int first = __ffsll((long long)m_ok) - 1;
+      const int k0 = __builtin_amdgcn_readlane(bin, first);
+      if (__ballot(bin >= 0 && bin != k0) == 0) {
+        const double v = bin >= 0 ? acc[br] * amp : 0.0;
+        if (v != v) derr = max(derr, 41);
+        const double sum = wave_sum(v);
+        if (lane == first) atomicAdd(&s_dist[k0], sum);
+      } else if (bin >= 0) {
+        put(cur[br], acc[br]);
+      }
+    }
+    __syncthreads();  // the next rows overwrite the staged ones
+  }
+  derr = wave_max_i(derr);
+  if (derr && lane == 0) atomicMax(&b.status[req], derr);
+  __syncthreads();
+  for (int k = zlo * n_incl + lane; k < (zhi + 1) * n_incl; k += 64)
+    if (s_dist[k] != 0.0) unsafeAtomicAdd(&b.dist[rq.dist_off + k], s_dist[k]);
+}
 
 // Byte offset of k_integrate's coefficient slots and bin buffer (FP64 path)
 // behind the lane rows (rows: 64 or 128 of 2 n_g + 1 values).
@@ -2683,6 +2718,16 @@ static size_t integrate_lds(const BatchDev &b, bool cos_rows, size_t elem, int *
   }
   *stage_rows = 2;  // the two rows a radius lerps between (2 nq <= STAGE_MAX: n_g <= MAX_NG)
   return rows + w + std::max(park, (size_t)2 * nq * sizeof(double));
+}
+
+int launch_dist(const BatchDev &b, const int *reqs, int n_reqs, void *stream) {
+  if (n_reqs <= 0) return 0;
+  const int n_rc = (b.nr_fine + RAD_CHUNK - 1) / RAD_CHUNK;
+  if (b.max_zones > LP_ZONES)
+    hipLaunchKernelGGL(k_dist<MAX_ZONES>, dim3(n_reqs * n_rc), dim3(64), 0, (hipStream_t)stream, b, reqs, n_rc);
+  else
+    hipLaunchKernelGGL(k_dist<LP_ZONES>, dim3(n_reqs * n_rc), dim3(64), 0, (hipStream_t)stream, b, reqs, n_rc);
+  return (int)hipGetLastError();
 }
 
 int launch_integrate(const BatchDev &b, int n_blocks, bool cos_rows, void *stream) {

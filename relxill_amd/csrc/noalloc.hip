@@ -130,7 +130,6 @@ int noalloc_eval(int model, const double *parameter, const double *d_energy, con
   p.pgrid_off = conv ? -1 : 0;
   p.prof_off = conv ? 0 : -1;
   p.dist_off = 0;
-  p.node_off = -1;
   p.zone_off = 0;
   p.xspec_off = 0;
   if (st == RX_OK && p.return_rad != 0) {
@@ -166,13 +165,11 @@ int noalloc_eval(int model, const double *parameter, const double *d_energy, con
   bd.n_req = 1;
   bd.nr_fine = g.nr_fine;
   bd.seg_bins = seg;
-  bd.node_stride = 2 * g.rel.n_r * g.rel.n_g * 2;
   bd.req = c.take<ReqParams>(1);
   bd.ener_in = d_energy;
   bd.flux_in = conv ? d_flux_in : nullptr;
   bd.out = d_flux_out;
   bd.pgrid = conv ? nullptr : c.take<double>((size_t)n_flux + 1);
-  bd.node = nullptr;  // line and convolution requests read no node rows
   bd.rad = c.take<RadRec>((size_t)g.nr_fine);
   bd.rnode = c.take<double>((size_t)RAD_NODE_ARRAYS * g.rel.n_r);
   bd.rnorm = c.take<ReqNorm>(1);

@@ -11,8 +11,6 @@
 //   pgrid               profile grids (line models: the caller grid shifted
 //                       to line-energy units; conv models use the shared
 //                       convolution grid instead)
-//   node[n]             (a,mu0)-interpolated table node, FP64:
-//                       trff[n_r][n_g][2] followed by cosne[n_r][n_g][2]
 //   rad[n][nr_fine]     per fine radius record (RadRec, 16 bytes)
 //   rnode[n][3][n_r]    per request: the (a, mu0)-interpolated node radii,
 //                       g_min and g_max that the records' geometry is rebuilt from
@@ -95,9 +93,6 @@ struct ReqParams {
   double xect_src;    // Ecut in the source frame
   int64_t dist_off;
   int64_t zone_off;   // ZoneRec per zone
-  // the request's (a, mu0)-interpolated node rows in node (n_incl > 0 only:
-  // the angle distribution reads them; -1 otherwise)
-  int64_t node_off;
   // primary continuum of the relxill models (PRIM_*; it also selects the
   // xillver table, b.xt[prim]).  nthcomp: n_nth solves (the source's kTe, then
   // the kTe every lamp-post zone sees) with their results at nth[nth_off],
@@ -332,14 +327,12 @@ struct BatchDev {
   int n_req;
   int nr_fine;
   int seg_bins;     // bins per work item (at most)
-  int node_stride;  // doubles per request in node (2 * n_r * n_g * 2)
   int max_zones;    // most zones of a request (k_setup's zone arrays: LP_ZONES or MAX_ZONES)
   ReqParams *req;
   const double *ener_in;
   const double *flux_in;
   double *out;
   double *pgrid;
-  double *node;
   RadRec *rad;
   double *rnode;  // per request: RAD_NODE_ARRAYS * rt.n_r doubles (node radii, g_min, g_max)
   ReqNorm *rnorm;
@@ -373,6 +366,8 @@ struct BatchDev {
 
 // ---- launchers (kernels.hip) ----
 int launch_setup(const BatchDev &b, void *stream);
+// the emission-angle distribution of the n_reqs requests with one
+int launch_dist(const BatchDev &b, const int *reqs, int n_reqs, void *stream);
 int launch_integrate(const BatchDev &b, int n_blocks, bool limb, void *stream);
 int launch_fixup(const BatchDev &b, bool cos_rows, void *stream);
 int launch_finalize(const BatchDev &b, void *stream);
