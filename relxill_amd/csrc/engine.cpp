@@ -604,6 +604,13 @@ int ensure_xilltable_device(int prim, std::string &err) {
   x.ener.resize(t.n_ener + 1);
   for (int i = 0; i < t.n_ener; i++) x.ener[i] = t.elo[i];
   x.ener[t.n_ener] = t.ehi[t.n_ener - 1];
+  x.rr_lo = 1e300;
+  x.rr_hi = -1e300;
+  for (int i = 0; i < t.n_ener; i++) {
+    if (!(x.ener[i] >= 0.15 && x.ener[i + 1] <= 500.0)) continue;
+    x.rr_lo = std::min(x.rr_lo, x.ener[i] / (2. / 3.));
+    x.rr_hi = std::max(x.rr_hi, x.ener[i + 1] / (2. / 3.));
+  }
   int e = upload_vec(x.spec, xilltable_renormed(t)) | upload_vec(x.d_ener, x.ener);
   // the inclination axis (returning-radiation corrections of relxilllp)
   e |= upload_vec(x.incl, t.val[t.n_par - 1]);
@@ -762,6 +769,8 @@ void fill_dev_views(BatchDev &bd) {
     xt.lxi_dim = (k_lxi >= off) ? k_lxi - off : -1;  // (a first axis of six is bracketed on the host)
     xt.n_lxi = k_lxi >= 0 ? t.n_val[k_lxi] : 0;
     xt.lxi_vals = x.lxi.as<float>();
+    xt.rr_lo = x.rr_lo;
+    xt.rr_hi = x.rr_hi;
   }
   bd.rr.n_spin = g.rrad.n_spin;
   bd.rr.n_rad = g.rrad.n_rad;
@@ -904,7 +913,9 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
   b.h_xill.clear();
   b.h_prim.clear();
   b.h_ang.clear();
+  b.h_zone.clear();
   b.h_rrc.clear();
+  b.h_rrad.clear();
   b.h_nth.clear();
   b.n_nth_sol = 0;
   std::vector<XillWork> xill_multi;
@@ -1026,6 +1037,7 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
         o_xspec += (int64_t)xt.n_ener * p.n_zones;
         p.zone_off = o_zone;
         o_zone += p.n_zones;
+        for (int z = 0; lp && z < p.n_zones; z++) b.h_zone.push_back(XillWork{i, z});
         if (p.ion_grad) {
           // zones that differ in logXi as well as in Ecut: one k_xill1 unit each
           for (int z = 0; z < p.n_zones; z++) b.h_xill.push_back(XillWork{i, z});
@@ -1069,9 +1081,11 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
         return RX_ERR_ARG;
       }
       p.rr_corr_off = o_rrc;
-      o_rrc += 2 * (int64_t)p.n_zones;
-      for (int z = 0; z < p.n_zones; z++) b.h_rrc.push_back(XillWork{i, z});
+      o_rrc += (int64_t)p.n_zones * 2 * rrad_chunks(g.xill[p.prim].t.n_ener) * 3;
+      b.h_rrc.push_back(i);
     }
+    p.rr_slot = (int)b.h_rrad.size();
+    if (st == RX_OK && p.return_rad != 0) b.h_rrad.push_back(i);
     const bool xill_model = r.model == MOD_XILLVER;
     p.need_cosne = (p.limb != 0 || (p.n_incl > 0 && !xill_model)) ? 1 : 0;
     p.dist_off = o_dist;
@@ -1179,9 +1193,12 @@ int batch_upload(Batch &b) {
   e |= b.d_conv.ensure(sizeof(XillWork) * std::max<size_t>(1, b.h_conv.size()));
   e |= b.d_xill.ensure(sizeof(XillWork) * std::max<size_t>(1, b.h_xill.size()));
   e |= b.d_prim.ensure(sizeof(int) * std::max<size_t>(1, b.h_prim.size()));
+  e |= b.d_zonew.ensure(sizeof(XillWork) * std::max<size_t>(1, b.h_zone.size()));
   e |= b.d_ang.ensure(sizeof(int) * std::max<size_t>(1, b.h_ang.size()));
-  e |= b.d_rrc.ensure(sizeof(XillWork) * std::max<size_t>(1, b.h_rrc.size()));
-  e |= b.d_rrcorr.ensure(sizeof(double) * std::max<int64_t>(1, b.tot_rrc));
+  e |= b.d_rrc.ensure(sizeof(int) * std::max<size_t>(1, b.h_rrc.size()));
+  e |= b.d_rrad.ensure(sizeof(int) * std::max<size_t>(1, b.h_rrad.size()));
+  e |= b.d_rrpart.ensure(sizeof(double) * std::max<int64_t>(1, b.tot_rrc));
+  e |= b.d_rret.ensure(sizeof(double) * 2 * MAX_RR * std::max<size_t>(1, b.h_rrad.size()));
   e |= b.d_nthw.ensure(sizeof(XillWork) * std::max<size_t>(1, b.h_nth.size()));
   e |= b.d_nth.ensure(sizeof(NthRes) * std::max<size_t>(1, b.h_nth.size()));
   e |= b.d_nthx.ensure(sizeof(double) * (NTH_MAX_POINTS + 1) * std::max(1, b.n_nth_sol));
@@ -1205,10 +1222,14 @@ int batch_upload(Batch &b) {
     e |= (int)hipMemcpyAsync(b.d_conv.p, b.h_conv.data(), sizeof(XillWork) * b.h_conv.size(), hipMemcpyHostToDevice,
                              b.stream);
   if (!b.h_rrc.empty())
-    e |= (int)hipMemcpyAsync(b.d_rrc.p, b.h_rrc.data(), sizeof(XillWork) * b.h_rrc.size(), hipMemcpyHostToDevice,
-                             b.stream);
+    e |= (int)hipMemcpyAsync(b.d_rrc.p, b.h_rrc.data(), sizeof(int) * b.h_rrc.size(), hipMemcpyHostToDevice, b.stream);
+  if (!b.h_rrad.empty())
+    e |= (int)hipMemcpyAsync(b.d_rrad.p, b.h_rrad.data(), sizeof(int) * b.h_rrad.size(), hipMemcpyHostToDevice, b.stream);
   if (!b.h_prim.empty())
     e |= (int)hipMemcpyAsync(b.d_prim.p, b.h_prim.data(), sizeof(int) * b.h_prim.size(), hipMemcpyHostToDevice, b.stream);
+  if (!b.h_zone.empty())
+    e |= (int)hipMemcpyAsync(b.d_zonew.p, b.h_zone.data(), sizeof(XillWork) * b.h_zone.size(), hipMemcpyHostToDevice,
+                             b.stream);
   if (!b.h_ang.empty())
     e |= (int)hipMemcpyAsync(b.d_ang.p, b.h_ang.data(), sizeof(int) * b.h_ang.size(), hipMemcpyHostToDevice, b.stream);
   if (!b.h_xill.empty())
@@ -1252,7 +1273,8 @@ static BatchDev dev_view(Batch &b) {
   fill_dev_views(bd);
   bd.xspec = b.d_xspec.as<double>();
   bd.zone = b.d_zone.as<ZoneRec>();
-  bd.rrcorr = b.d_rrcorr.as<double>();
+  bd.rrpart = b.d_rrpart.as<double>();
+  bd.rret = b.d_rret.as<double>();
   bd.nth = b.d_nth.as<NthRes>();
   bd.nth_x = b.d_nthx.as<double>();
   bd.nth_s = b.d_nths.as<double>();
@@ -1267,7 +1289,8 @@ static int launch_sequence(Batch &b, const RunKey &k, hipStream_t s) {
   int e = 0;
   if (prof) e |= (int)hipEventRecord(b.ev[0], s);
   e |= launch_nth(bd, static_cast<const XillWork *>(k.d_nth), k.n_nth, s);
-  e |= launch_rrad_corr(bd, static_cast<const XillWork *>(k.d_rrc), k.n_rrc, s);
+  e |= launch_zone(bd, static_cast<const XillWork *>(k.d_zone), k.n_zone, s);
+  e |= launch_rrad(bd, static_cast<const int *>(k.d_rrc), k.n_rrc, static_cast<const int *>(k.d_rrad), k.n_rrad, s);
   e |= launch_setup(bd, s);
   e |= launch_dist(bd, static_cast<const int *>(k.d_ang), k.n_ang, s);
   if (prof) e |= (int)hipEventRecord(b.ev[1], s);
@@ -1344,8 +1367,12 @@ int batch_run(Batch &b, int precision, std::string &err) {
   k.d_prim = b.d_prim.p;
   k.d_rrc = b.d_rrc.p;
   k.n_rrc = (int)b.h_rrc.size();
+  k.d_rrad = b.d_rrad.p;
+  k.n_rrad = (int)b.h_rrad.size();
   k.d_nth = b.d_nthw.p;
   k.n_nth = (int)b.h_nth.size();
+  k.d_zone = b.d_zonew.p;
+  k.n_zone = (int)b.h_zone.size();
   k.d_ang = b.d_ang.p;
   k.n_ang = (int)b.h_ang.size();
   k.prof = g.profile ? 1 : 0;

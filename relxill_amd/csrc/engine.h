@@ -49,8 +49,8 @@ void rzone_grid(double rmin, double rmax, int nzones, double h, double *rgrid);
 // its padding zeroed, so configurations compare with memcmp.
 struct RunKey {
   BatchDev bd;
-  int n_blocks, n_xill1, n_xill, n_conv, n_prim, n_rrc, n_nth, n_ang;
-  const void *d_xill, *d_conv, *d_prim, *d_rrc, *d_nth, *d_ang;
+  int n_blocks, n_xill1, n_xill, n_conv, n_prim, n_rrc, n_rrad, n_nth, n_ang, n_zone;
+  const void *d_xill, *d_conv, *d_prim, *d_rrc, *d_rrad, *d_nth, *d_ang, *d_zone;
   int prof, cos_rows;
 };
 
@@ -69,13 +69,15 @@ struct Batch {
   std::vector<XillWork> h_conv;  // (request, zone) units of k_conv
   std::vector<XillWork> h_xill;  // k_xill units: one-zone requests first, then the others (all zones in one unit)
   int n_xill1 = 0;               // number of one-zone units at the front of h_xill
-  std::vector<XillWork> h_rrc;   // (request, zone) units of the returning-radiation corrections
+  std::vector<int> h_rrc;        // requests with returning-radiation corrections (k_rrad_sums)
+  std::vector<int> h_rrad;       // requests with returning radiation (k_rrad)
+  std::vector<XillWork> h_zone;  // (request, zone) units of k_zone (lamp-post relxill models)
   std::vector<XillWork> h_nth;   // nthcomp solves: (request, 0 source / 1 + zone)
   int n_nth_sol = 0;             // requests with the nthcomp primary (one source solution each)
   int64_t tot_ener = 0, tot_flux = 0, tot_pgrid = 0, tot_prof = 0, tot_xspec = 0, tot_dist = 0, tot_zone = 0;
   int64_t tot_rrc = 0;
   DevBuf d_req, d_ener, d_flux_in, d_out, d_pgrid, d_rad, d_prof, d_dist, d_refl, d_status, d_conv;
-  DevBuf d_xill, d_xspec, d_zone, d_prim, d_ang, d_rrc, d_rrcorr;
+  DevBuf d_xill, d_xspec, d_zone, d_prim, d_ang, d_zonew, d_rrc, d_rrad, d_rrpart, d_rret;
   DevBuf d_nthw, d_nth, d_nthx, d_nths, d_nthn;
   DevBuf d_items, d_ctr, d_fix, d_reach, d_rnorm, d_rnode;
   int item_cap = 0;
@@ -123,6 +125,7 @@ struct XillSlot {
   bool loaded = false, dirty = true;
   std::string err;
   std::vector<double> ener;
+  double rr_lo = 1e300, rr_hi = -1e300;  // DevXillTable's
   DevBuf spec, d_ener, ect, q, incl, lxi;
 };
 

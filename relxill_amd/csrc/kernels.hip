@@ -69,9 +69,19 @@ constexpr double NORM_XILLVER_TABLE = 1e15 / 4.0 / 3.14159265358979323846;
 // (src/xilltable.c:478-486): the resident rows are divided by 10^logXi; rows
 // of a table without a density axis are also divided by dens_div =
 // 10^(logN - 15) (rounded to float, as the reference's float array), unless
-// logN is 15 (dens_div 0).
-__device__ __forceinline__ double xval(float v, double dens_div) {
-  return dens_div != 0.0 ? (double)(float)((double)v / dens_div) : (double)v;
+// logN is 15 (dens_div 0).  The quotient by the request's one divisor takes its
+// correctly rounded reciprocal and one correction step (the remainder in one
+// fma), which rounds as the division does, in 3 operations instead of about 10.
+struct DensDiv {
+  double d, r;
+};
+__device__ __forceinline__ DensDiv dens_of(double dens_div) {
+  return DensDiv{dens_div, dens_div != 0.0 ? 1.0 / dens_div : 0.0};
+}
+__device__ __forceinline__ double xval(float v, const DensDiv &dd) {
+  if (dd.d == 0.0) return (double)v;
+  const double q = (double)v * dd.r;
+  return (double)(float)fma(fma(-dd.d, q, (double)v), dd.r, q);
 }
 
 // This thread's part of calcNormWrtXillverTableSpec's sum (src/Xillspec.cpp:179-205)
@@ -145,6 +155,20 @@ __device__ inline double gi_potential_lp(double r, double a, double h, double be
   double beta_fac = sqrt(hh * hh - delta_eq * (q2 + a * a));
   beta_fac = gam * (1.0 + sgn * beta_fac / hh * bet);
   return gi / beta_fac;
+}
+
+// lamp-post emissivity of a fine radius with the flux boost (src/Rellp.cpp:249-253,
+// src/Relphysics.cpp:301-311); *err is set where the table does not reach
+__device__ __forceinline__ double lp_emis_at(const ReqParams &rq, double re, const double *jr, const double *je,
+                                    const double *jd, const double *ji, int ntr, int *err) {
+  LpFine f = lp_on_fine(re, jr, je, jd, ji, ntr);
+  if (f.err) *err = f.err;
+  double boost = pow(gi_potential_lp(re, rq.a, rq.height, rq.beta, f.del_emit), rq.gamma);
+  if (rq.beta > 1e-6) {
+    const double d = sqrt(1.0 - rq.beta * rq.beta) / (1.0 + rq.beta * cos(f.del_emit));
+    boost *= d * d;
+  }
+  return f.emis * boost;
 }
 
 __device__ inline double relat_abberation(double del, double beta) {
@@ -653,107 +677,16 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
   double area = 0.0;
   double cmax = 0.0;  // largest weight of a radius with a window
   int err = 0;
-  // lamp-post emissivity of a fine radius with the flux boost (src/Rellp.cpp:249-253,
-  // src/Relphysics.cpp:301-311)
-  auto lp_emis = [&](double re) {
-    LpFine f = lp_on_fine(re, s_jr, s_je, s_jd, s_ji, ntr);
-    if (f.err) err = f.err;
-    double boost = pow(gi_potential_lp(re, rq.a, rq.height, rq.beta, f.del_emit), rq.gamma);
-    if (rq.beta > 1e-6) {
-      const double d = sqrt(1.0 - rq.beta * rq.beta) / (1.0 + rq.beta * cos(f.del_emit));
-      boost *= d * d;
-    }
-    return f.emis * boost;
-  };
-  // returning radiation (add_returnrad_emis, src/Rellp.cpp:483-507, with
-  // get_rrad_emis_corona, src/Relreturn_Corona.cpp:291-321): the direct
-  // emissivity of every fine radius (parked in the radius records), at the
-  // table zones' centres (inv_rebin_mean), the zones' returning emissivity
-  // sum_re frac_g g^(Gamma-1) tf_r emis(re) (calc_rrad_emis_corona, :119-151),
-  // log-interpolated back onto the fine radii below
-  __shared__ double s_rr_rad[MAX_RR], s_rr_in[MAX_RR], s_rr_ret[MAX_RR], s_rr_corr[2];
-  __shared__ double s_rr_cf[MAX_RR], s_rr_cg[MAX_RR];
-  const bool rrad = lp && rq.return_rad != 0 && s_st == 0;
+  auto lp_emis = [&](double re) { return lp_emis_at(rq, re, s_jr, s_je, s_jd, s_ji, ntr, &err); };
+  // returning radiation: the zones' centres and returning emissivity (k_rrad)
+  __shared__ double s_rr_rad[MAX_RR], s_rr_ret[MAX_RR];
+  const bool rrad = lp && rq.return_rad != 0;
   const int rr_n = rq.rr_n;
   if (rrad) {
-    for (int ii = tid; ii < nr; ii += SETUP_THREADS) rad[ii].coef = lp_emis(fine_radius(rq.rin, rq.rout, ii, nr));
-    const DevRradTable &R = b.rr;
-    const int nt = R.n_rad, k = rq.rr_k, klo = rq.rr_klo;
-    const double *rlo_t = R.rlo + (size_t)k * nt, *rhi_t = R.rhi + (size_t)k * nt;
-    const double rin_f = fine_radius(rq.rin, rq.rout, nr - 1, nr), rout_f = fine_radius(rq.rin, rq.rout, 0, nr);
+    const double *rr = b.rret + (size_t)rq.rr_slot * (2 * MAX_RR);
     for (int i = tid; i < rr_n; i += SETUP_THREADS) {
-      const double lo = (i == 0) ? rin_f : rlo_t[klo + i];
-      const double hi = (i == rr_n - 1) ? rout_f : rhi_t[klo + i];
-      const double rm = 0.5 * (lo + hi);
-      s_rr_rad[i] = rm;
-      // relxilllp above spin 0: the correction factors of the relxill zone
-      // the table zone's centre falls in (rebin_corrfactors_to_rradtable_grid,
-      // src/Relreturn_Corona.cpp:248-289; a centre beyond the last edge takes
-      // the last zone)
-      double cf = 1.0, cg = 1.0;
-      if (rq.rr_corr) {
-        const int n0 = nz;
-        int ind = bsearch_asc(zg, n0 + 1, rm);
-        if (rm < zg[0]) ind = 0;
-        else if (rm > zg[n0] || ind > n0 - 1) ind = n0 - 1;
-        cf = b.rrcorr[rq.rr_corr_off + 2 * ind];
-        cg = b.rrcorr[rq.rr_corr_off + 2 * ind + 1];
-      }
-      s_rr_cf[i] = cf;
-      s_rr_cg[i] = cg;
-    }
-    if (tid < 2) {  // ring-area corrections of the end zones (src/Relreturn_Table.cpp:415-435)
-      const int i = (tid == 0) ? 0 : rr_n - 1;
-      double rl = rlo_t[klo + i];
-      if (klo + i == 0 && rl > rq.rms) rl = rq.rms;
-      const double rh = rhi_t[klo + i];
-      const double lo = (i == 0) ? rin_f : rlo_t[klo + i];
-      const double hi = (i == rr_n - 1) ? rout_f : rhi_t[klo + i];
-      s_rr_corr[tid] = (0.5 * (lo + hi) * (hi - lo)) / (0.5 * (rl + rh) * (rh - rl));
-    }
-    __syncthreads();
-    for (int i = tid; i < rr_n; i += SETUP_THREADS) {
-      // inv_rebin_mean (src/relutility.c:636-663): the fine radii re(ii) > rad >= re(ii+1)
-      const double x = s_rr_rad[i];
-      int lo = 0, hi = nr - 1;
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (fine_radius(rq.rin, rq.rout, mid, nr) > x) lo = mid; else hi = mid;
-      }
-      const double r0 = fine_radius(rq.rin, rq.rout, lo, nr), r1 = fine_radius(rq.rin, rq.rout, lo + 1, nr);
-      s_rr_in[i] = lerp1((x - r1) / (r0 - r1), rad[lo + 1].coef, rad[lo].coef);
-    }
-    __syncthreads();
-    // calc_rrad_emis_corona (src/Relreturn_Corona.cpp:119-151): one wavefront
-    // per incident zone i, lane j its emitting zones (at most 64), summed in a
-    // fixed order; the frac_g weight g^(Gamma-1), or with a g-shift factor off
-    // 1 by more than 1e-3 of the emitting zone its corrected boost over g
-    // (calc_rrad_emis_zone, :87-108); the sum times the incident zone's flux
-    // factor
-    const int ng = R.n_g;
-    const int wv = tid >> 6, lane = tid & 63;
-    for (int i = wv; i < rr_n; i += SETUP_THREADS / 64) {
-      double term = 0.0;
-      const int j = lane;
-      if (j < rr_n) {
-        const size_t t = (size_t)k * nt * nt + (size_t)(klo + i) * nt + (klo + j);
-        const double gmin = R.gmin[t], gmax = R.gmax[t];
-        const double cgj = s_rr_cg[j];
-        double ez = 0.0;
-        for (int jj = 0; jj < ng; jj++) {
-          const double g = (jj + 0.5) / ng * (gmax - gmin) + gmin;  // get_gfac_grid (src/Relreturn_Datastruct.cpp:51-59)
-          double v = R.frac_g[t * ng + jj];
-          if (fabs(cgj - 1) > 1e-3) v *= gshift_boost(cgj, g, rq.gamma) / g;
-          else if (fabs(g - 1) > 1e-3) v *= pow(g, rq.gamma - 1);
-          ez += v;
-        }
-        double tf = R.tf_r[t];
-        if (j == 0 && i < rr_n - 1) tf *= s_rr_corr[0];
-        if (j == rr_n - 1 && i < rr_n - 2) tf *= s_rr_corr[1];
-        term = ez * tf * s_rr_in[j];
-      }
-      const double sum = wave_sum(term);
-      if (lane == 0) s_rr_ret[i] = sum * s_rr_cf[i];
+      s_rr_rad[i] = rr[i];
+      s_rr_ret[i] = rr[MAX_RR + i];
     }
     __syncthreads();
   }
@@ -802,7 +735,8 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
       const int kk = min(max(bsearch_asc(s_rr_rad, rr_n, re), 0), rr_n - 2);
       const double fr = (re - s_rr_rad[kk]) / (s_rr_rad[kk + 1] - s_rr_rad[kk]);
       const double er = exp(fr * log(s_rr_ret[kk + 1]) + (1.0 - fr) * log(s_rr_ret[kk]));
-      emis = (rq.return_rad == 1) ? rad[ii].coef + er : er;
+      const double direct = lp_emis(re);
+      emis = (rq.return_rad == 1) ? direct + er : er;
     }
     // energy window
     double egmin = gmin, egmax = gmax;
@@ -898,40 +832,12 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
     b.refl[req] = o;
   }
 
-  // zones of a relxill request (IonGradient, src/IonGradient.cpp:182-209,
-  // :421-430): the centre radius, its emission angle (inv_rebin_mean of the
-  // fine-grid angles, src/relutility.c:636-663), the source -> disk energy
-  // shift, the Ecut the zone sees with its xillver bracket (float factor,
-  // clamps, ensure_ecut_within_boundarys, src/xilltable.c:1054-1125) and the
-  // normalisation change of the incident spectrum (src/Xillspec.cpp:408-435)
-  const bool relxill_model = (rq.model == MOD_RELXILL || rq.model == MOD_RELXILLLP);
-  if (relxill_model && s_st == 0) {
-    ZoneRec *zr = b.zone + rq.zone_off;
-    const DevXillTable &xt = b.xt[rq.prim];
-    __shared__ double s_zect[NZ];
-    for (int z = tid; z < nz; z += SETUP_THREADS) {
-      double ect;
-      zr[z] = zone_record(xt, b.req[req], z, lp, s_jr, s_je, s_jd, s_ji, ntr, nr, &ect);
-      s_zect[z] = ect;
-    }
-    __syncthreads();
-    if (lp && rq.prim == PRIM_NTHCOMP) {
-      // the nthcomp norms of the source and of every zone's kTe (k_nth)
-      const NthRes *nr = b.nth + rq.nth_off;
-      for (int z = tid; z < nz; z += SETUP_THREADS) zr[z].ncf = nr[1 + z].nf / nr[0].nf;
-    } else if (lp) {
-      const double src = 1. / (block_sum(xill_norm_part(b.cg, rq.xect_src, rq.xgam, tid, SETUP_THREADS),
-                                         s_red) / NORM_XILLVER_TABLE);
-      for (int z = 0; z < nz; z++) {
-        const double ez = s_zect[z];
-        const double disk =
-            1. / (block_sum(xill_norm_part(b.cg, ez, rq.xgam, tid, SETUP_THREADS), s_red) / NORM_XILLVER_TABLE);
-        if (tid == 0) zr[z].ncf = disk / src;
-      }
-    }
-    __syncthreads();
+  // the zone of a broken power-law relxill request (a lamp post's: k_zone)
+  if (rq.model == MOD_RELXILL && tid == 0) {
+    double ect;
+    b.zone[rq.zone_off] =
+        zone_record(b.xt[rq.prim], b.req[req], 0, false, nullptr, nullptr, nullptr, nullptr, 0, nr, &ect);
   }
-
   if (rq.n_incl > 0) {  // k_dist adds into the angle distribution
     const int nd = rq.n_incl * nz;  // [zone][angle bin]
     for (int k = tid; k < nd; k += SETUP_THREADS) b.dist[rq.dist_off + k] = 0.0;
@@ -1010,119 +916,328 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
   if (tid == 0) b.status[req] = s_st;
 }
 
-// relxilllp's returning radiation above spin 0: the xillver correction
-// factors of one zone (calc_rrad_corr_factors, src/Relxill.cpp:164-182, with
-// get_xillver_fluxcorrection_factors, src/Xillspec.cpp:500-526).  The zone's
-// xillver spectra for every inclination (16 table corners with the zone's own
-// Ecut bracket, as k_xill reads them) are averaged with the weights of
-// calc_angle_averaged_xill_spec (:109-126: 0.5 cos(i) / n_incl with the
-// table's inclination, in degrees, read as radians), then
-//   flux factor = energy flux of the average in 0.1-1000 keV over that of the
-//                 normalised cut-off power law on the 500-bin grid (:344-362)
-//   g factor    = photon flux of the average in 0.15-500 keV over that of the
-//                 average shifted 1.5 times lower in energy (rebinned, times
-//                 2/3), over 1.5^Gamma (:454-487).
-// One workgroup per (request, zone); the average sits in dynamic LDS; the
-// sums are fixed-order block sums.  k_setup reads the factors (it runs next).
-constexpr int RRC_THREADS = 256;
-__global__ __launch_bounds__(RRC_THREADS) void k_rrad_corr(BatchDev b, const XillWork *__restrict__ work) {
-  extern __shared__ double s_avg[];
+// Radial zones of the lamp-post relxill requests (IonGradient,
+// src/IonGradient.cpp:182-209, :421-430): the zone record (centre, emission
+// angle, energy shift, the xillver brackets the zone sees) and the
+// normalisation change of the incident spectrum (src/Xillspec.cpp:408-435),
+// one wavefront per (request, zone).  The change is a ratio of two sums over
+// the 500-bin grid (the cut-off power law; 8 exponentials a lane and sum) or
+// of two nthcomp norms (k_nth, which runs before).
+// Bound: the latency of the table rows and the sums, 15 us alone, 20 us for 1280
+// zones (inside k_setup, zone after zone with tree sums: 18 us and 22 us, but
+// after the returning radiation that reads the records).
+__global__ __launch_bounds__(64) void k_zone(BatchDev b, const XillWork *__restrict__ work) {
   __shared__ double s_jr[MAX_LP_R], s_je[MAX_LP_R], s_jd[MAX_LP_R], s_ji[MAX_LP_R];
-  __shared__ double s_red[RRC_THREADS];
   const XillWork wk = work[blockIdx.x];
-  const int req = wk.req, z = wk.zone, tid = threadIdx.x;
+  const int req = wk.req, z = wk.zone, lane = threadIdx.x;
   const ReqParams &rq = b.req[req];
   if (rq.pre_status != 0) return;  // uniform over the block
-  const DevXillTable xt = b.xt[rq.prim];
-  const double dd = rq.xdens_div;
-  lp_rows(b.lp, rq, s_jr, s_je, s_jd, s_ji, tid, RRC_THREADS);
+  const DevXillTable &xt = b.xt[rq.prim];
+  lp_rows(b.lp, rq, s_jr, s_je, s_jd, s_ji, lane, 64);
   double ect;
-  const ZoneRec zr = zone_record(xt, rq, z, true, s_jr, s_je, s_jd, s_ji, b.lp.n_r, b.nr_fine, &ect);
-  int i0[4];
-  double f[4];
-#pragma unroll
-  for (int k = 0; k < 4; k++) {  // the zone's own Ecut and logXi brackets
-    const bool e = (k == xt.ect_dim), l = (k == xt.lxi_dim);
-    i0[k] = e ? zr.ect_ind : (l ? zr.lxi_ind : rq.xind[k]);
-    f[k] = e ? zr.ect_fac : (l ? zr.lxi_fac : rq.xfac[k]);
+  ZoneRec zr = zone_record(xt, rq, z, true, s_jr, s_je, s_jd, s_ji, b.lp.n_r, b.nr_fine, &ect);
+  if (rq.prim == PRIM_NTHCOMP) {
+    const NthRes *n = b.nth + rq.nth_off;
+    zr.ncf = n[1 + z].nf / n[0].nf;
+    zr.pe = n[1 + z].pe;
+  } else {
+    const double gam = rq.xgam;
+    const double src = 1. / (wave_sum(xill_norm_part(b.cg, rq.xect_src, gam, lane, 64)) / NORM_XILLVER_TABLE);
+    const double disk = 1. / (wave_sum(xill_norm_part(b.cg, ect, gam, lane, 64)) / NORM_XILLVER_TABLE);
+    zr.ncf = disk / src;
+    // energy flux of the zone's normalised primary in 0.1-1000 keV
+    // (get_xillver_fluxcorr, src/Xillspec.cpp:344-362)
+    double pe = 0.0;
+    if (rq.rr_corr) {
+      for (int k = lane; k < N_ENER_COARSE; k += 64) {
+        const double e0 = b.cg.coarse[k], e1 = b.cg.coarse[k + 1];
+        if (e0 >= 0.1 && e1 <= 1000.0)
+          pe += cutoffpl_bin(e0, e1, b.cg.coarse_ln[k], ect, gam) * disk * 0.5 * (e0 + e1);
+      }
+    }
+    zr.pe = wave_sum(pe);
   }
-  // the 16 corners in the reference's order (interp_5d_tab_incl, src/xilltable.c:812-876)
-  constexpr unsigned char kCorner[16] = {0x0, 0x8, 0x4, 0x2, 0xC, 0xA, 0x6, 0xE,
-                                         0x1, 0x9, 0x5, 0x3, 0xD, 0xB, 0x7, 0xF};
-  double w[16];
-  unsigned row[16];
+  if (lane == 0) b.zone[rq.zone_off + z] = zr;
+}
+
+// The eight corners of a request's xillver table row on the interpolated axes
+// other than zax (zax index 0), each with its weight, in rows of ni
+// inclinations; one step on zax moves a row by *stride rows.
+__device__ inline void corners8(const DevXillTable &xt, const ReqParams &rq, int zax, double *w8, unsigned *cb,
+                                unsigned *stride) {
+  unsigned st = 1;
 #pragma unroll
-  for (int c = 0; c < 16; c++) {
-    int o[4];
-    double fk[4];
+  for (int k = 0; k < 4; k++)
+    if (k > zax) st *= (unsigned)xt.n_val[k];
+#pragma unroll
+  for (int c = 0; c < 8; c++) {
+    double w = 1.0;
+    unsigned r = 0;
+    int bit = 2;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-      o[k] = (kCorner[c] >> (3 - k)) & 1;
-      fk[k] = o[k] ? f[k] : (1.0 - f[k]);
-    }
-    w[c] = fk[0] * fk[1] * fk[2] * fk[3];
-    const unsigned r = (((unsigned)(i0[0] + o[0]) * xt.n_val[1] + (i0[1] + o[1])) * xt.n_val[2] + (i0[2] + o[2])) *
-                           xt.n_val[3] + (i0[3] + o[3]);
-    row[c] = r * xt.n_incl;
-  }
-  const int ne = xt.n_ener, n_incl = xt.n_incl;
-  const int n_o = xt.n_out > 1 ? 2 : 1;
-  const double *E = xt.ener;
-  for (int e = tid; e < ne; e += RRC_THREADS) {
-    double acc = 0.0;
-    for (int a = 0; a < n_incl; a++) {
-      const double incl_deg = (double)xt.incl_vals[a] * 180 / PI;
-      const double wa = 0.5 * cos(incl_deg * PI / 180) / n_incl;
-      double sv = 0.0;
-      for (int o = 0; o < n_o; o++) {  // (a six-parameter table: both brackets of its first axis)
-        const double wo = n_o == 1 ? 1.0 : (o ? rq.xo_fac : 1.0 - rq.xo_fac);
-        const size_t ob = (size_t)(rq.xo_ind + o) * xt.outer_rows;
-        double so = 0.0;
-#pragma unroll
-        for (int c = 0; c < 16; c++) so += w[c] * xval(xt.spec[(ob + row[c] + a) * ne + e], dd);
-        sv += wo * so;
+      int idx = 0;
+      if (k != zax) {
+        const int o = (c >> bit) & 1;
+        bit--;
+        w *= o ? rq.xfac[k] : (1.0 - rq.xfac[k]);
+        idx = rq.xind[k] + o;
       }
-      acc += wa * sv;
+      r = r * (unsigned)xt.n_val[k] + (unsigned)idx;
     }
-    s_avg[e] = acc;
+    w8[c] = w;
+    cb[c] = r * (unsigned)xt.n_incl;
+  }
+  *stride = st;
+}
+
+// relxilllp's returning radiation above spin 0: the band sums behind the
+// zones' xillver correction factors (calc_rrad_corr_factors,
+// src/Relxill.cpp:164-182, with get_xillver_fluxcorrection_factors,
+// src/Xillspec.cpp:500-526).  A zone's xillver spectra for every inclination
+// are averaged with the weights of calc_angle_averaged_xill_spec (:109-126:
+// 0.5 cos(i) / n_incl with the table's inclination, in degrees, read as
+// radians); of the average this takes
+//   [0] the energy flux in 0.1-1000 keV (:344-362),
+//   [1] the photon flux in 0.15-500 keV,
+//   [2] the photon flux there of the average shifted 1.5 times lower in energy
+//       (rebinned, times 2/3; :454-487): the bins of the band are contiguous,
+//       so their shares of the average add up to its photons in the band's
+//       shifted ends [xt.rr_lo, xt.rr_hi], and no bin is searched for.
+// All three are linear in the average, and the zones differ only in their
+// bracket (i_z, f_z) on the Ecut axis: so the sums are taken once per Ecut
+// node that some zone's bracket touches, and zone z gets those of nodes i_z and
+// i_z + 1 (k_rrad weights them).  An ionisation gradient gives every zone its
+// own logXi bracket too; then each zone takes its own 16 corners.
+// One workgroup per (request, RRA_THREADS table bins), one bin a thread; the
+// partial sums go to rrpart[zone][node][chunk][3].
+// Bound: L2 / HBM reads of 80 rows per Ecut node.  One workgroup per (request,
+// zone) with 160 rows a zone and the shift's rebin took 144 us for one request (362 us with a density
+// division, 696 us for 64 of those); this takes 16 us (16 us, 28 us).
+__global__ __launch_bounds__(RRA_THREADS) void k_rrad_sums(BatchDev b, const int *__restrict__ reqs, int n_chunk) {
+  __shared__ double s_wa[MAX_INCL];
+  __shared__ double s_w[3][RRA_THREADS / 64];
+  __shared__ int s_ind[MAX_ZONES];
+  const int req = reqs[blockIdx.x / n_chunk], chunk = blockIdx.x % n_chunk, tid = threadIdx.x;
+  const ReqParams &rq = b.req[req];
+  const DevXillTable xt = b.xt[rq.prim];
+  const int chunks = rrad_chunks(xt.n_ener);  // of this request's table
+  if (rq.pre_status != 0 || chunk >= chunks) return;  // uniform over the block
+  const DensDiv dd = dens_of(rq.xdens_div);
+  const int nz = rq.n_zones, ni = xt.n_incl, ne = xt.n_ener;
+  const int zax = xt.ect_dim >= 0 ? xt.ect_dim : 3;
+  const bool grad = rq.ion_grad == 1 && xt.lxi_dim >= 0;
+  for (int a = tid; a < ni; a += RRA_THREADS) {
+    const double incl_deg = (double)xt.incl_vals[a] * 180 / PI;
+    s_wa[a] = 0.5 * cos(incl_deg * PI / 180) / ni;
+  }
+  if (tid < nz) s_ind[tid] = xt.ect_dim >= 0 ? b.zone[rq.zone_off + tid].ect_ind : rq.xind[3];
+  __syncthreads();
+  const int e = chunk * RRA_THREADS + tid;
+  const bool in = e < ne;
+  const size_t eb = in ? e : 0;  // a valid address; bins beyond the table weigh nothing
+  const double e0 = xt.ener[eb], e1 = xt.ener[eb + 1];
+  const double we = (in && e0 >= 0.1 && e1 <= 1000.0) ? 0.5 * (e0 + e1) : 0.0;
+  const double wp = (in && e0 >= 0.15 && e1 <= 500.0) ? 1.0 : 0.0;
+  const double zlo = fmax(e0, xt.rr_lo), zhi = fmin(e1, xt.rr_hi);
+  const double wz = (in && zhi > zlo) ? (zhi - zlo) / (e1 - e0) * (2. / 3.) : 0.0;
+  double *part = b.rrpart + rq.rr_corr_off;
+  // the block's sums of a spectrum with value avg in this thread's bin, to nodes
+  // [n0, n1] of zone z
+  double sums[3];
+  auto reduce = [&](double avg) {
+    const double v[3] = {wave_sum(avg * we), wave_sum(avg * wp), wave_sum(avg * wz)};
+    __syncthreads();  // the last sums have been read
+    if ((tid & 63) == 0)
+      for (int k = 0; k < 3; k++) s_w[k][tid >> 6] = v[k];
+    __syncthreads();
+    for (int k = 0; k < 3; k++) {
+      sums[k] = 0.0;
+      for (int w = 0; w < RRA_THREADS / 64; w++) sums[k] += s_w[k][w];
+    }
+  };
+  auto store = [&](int z, int node) {
+    if (tid < 3) part[((size_t)(2 * z + node) * chunks + chunk) * 3 + tid] = sums[tid];
+  };
+  const int n_o = xt.n_out > 1 ? 2 : 1;
+  const size_t nel = (size_t)ne;
+  if (!grad) {
+    int elo = s_ind[0], ehi = s_ind[0];
+    for (int z = 1; z < nz; z++) {
+      elo = min(elo, s_ind[z]);
+      ehi = max(ehi, s_ind[z]);
+    }
+    double w8[8];
+    unsigned cb[8], stride;
+    corners8(xt, rq, zax, w8, cb, &stride);
+    for (int nd = elo; nd <= ehi + 1; nd++) {
+      bool used = false;
+      for (int z = 0; z < nz; z++) used |= nd == s_ind[z] || nd == s_ind[z] + 1;
+      if (!used) continue;  // uniform
+      double avg = 0.0;
+      for (int a = 0; a < ni; a++) {
+        const unsigned po = (unsigned)nd * stride * (unsigned)ni + (unsigned)a;
+        double sv = 0.0;
+        for (int o = 0; o < n_o; o++) {  // (a six-parameter table: both brackets of its first axis)
+          const double wo = n_o == 1 ? 1.0 : (o ? rq.xo_fac : 1.0 - rq.xo_fac);
+          const size_t ob = (size_t)(rq.xo_ind + o) * xt.outer_rows;
+          double so = 0.0;
+#pragma unroll
+          for (int c = 0; c < 8; c++) so += w8[c] * xval(xt.spec[(ob + cb[c] + po) * nel + eb], dd);
+          sv += wo * so;
+        }
+        avg += s_wa[a] * sv;
+      }
+      reduce(avg);
+      for (int z = 0; z < nz; z++) {
+        if (s_ind[z] == nd) store(z, 0);
+        if (s_ind[z] + 1 == nd) store(z, 1);
+      }
+    }
+    return;
+  }
+  for (int z = 0; z < nz; z++) {
+    const ZoneRec &zr = b.zone[rq.zone_off + z];
+    double avg = 0.0;
+    for (int c = 0; c < 16; c++) {  // the zone's own Ecut and logXi brackets
+      double w = 1.0;
+      unsigned r = 0;
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const bool ie = (k == xt.ect_dim), il = (k == xt.lxi_dim);
+        const int o = (c >> (3 - k)) & 1;
+        const double f = ie ? zr.ect_fac : (il ? zr.lxi_fac : rq.xfac[k]);
+        w *= o ? f : (1.0 - f);
+        r = r * (unsigned)xt.n_val[k] + (unsigned)((ie ? zr.ect_ind : (il ? zr.lxi_ind : rq.xind[k])) + o);
+      }
+      for (int o = 0; o < n_o; o++) {
+        const double wo = n_o == 1 ? w : w * (o ? rq.xo_fac : 1.0 - rq.xo_fac);
+        const size_t row = (size_t)(rq.xo_ind + o) * xt.outer_rows + (size_t)r * ni;
+        double sa = 0.0;
+        for (int a = 0; a < ni; a++) sa += s_wa[a] * xval(xt.spec[(row + a) * nel + eb], dd);
+        avg += wo * sa;
+      }
+    }
+    reduce(avg);
+    store(z, 0);
+    store(z, 1);
+  }
+}
+
+// Returning radiation (add_returnrad_emis, src/Rellp.cpp:483-507, with
+// get_rrad_emis_corona, src/Relreturn_Corona.cpp:291-321): the returning
+// emissivity of a request's table zones, sum_re frac_g g^(Gamma-1) tf_r
+// emis(re) (calc_rrad_emis_corona, :119-151), which k_setup log-interpolates
+// onto the fine radii.  One wavefront per incident zone (RR_ZONES to a
+// workgroup), its lanes the emitting zones (at most 64); the direct emissivity
+// at a zone's centre is interpolated between the two fine radii around it
+// (inv_rebin_mean, src/relutility.c:636-663).  The frac_g weight is
+// g^(Gamma-1), or with a g-shift factor off 1 by more than 1e-3 of the emitting
+// zone its corrected boost over g (calc_rrad_emis_zone, :87-108); the sum times
+// the incident zone's flux factor.
+// Bound: FP64 issue of a pow per (incident, emitting zone, energy-shift bin),
+// 50 x 50 x 20 a request: about 180 us on the one CU of the request's k_setup
+// workgroup (239 -> 59 us without it), 30 us over the CUs of its 13 workgroups
+// here; 270 us and 71 us for 64 requests.
+constexpr int RR_ZONES = 4;
+__global__ __launch_bounds__(64 * RR_ZONES) void k_rrad(BatchDev b, const int *__restrict__ reqs) {
+  constexpr int NT = 64 * RR_ZONES, GROUPS = MAX_RR / RR_ZONES;
+  __shared__ double s_jr[MAX_LP_R], s_je[MAX_LP_R], s_jd[MAX_LP_R], s_ji[MAX_LP_R];
+  __shared__ double s_rad[MAX_RR], s_in[MAX_RR], s_cf[MAX_RR], s_cg[MAX_RR], s_corr[2];
+  __shared__ double s_zf[MAX_ZONES], s_zg[MAX_ZONES];
+  const int req = reqs[blockIdx.x / GROUPS], i0 = (blockIdx.x % GROUPS) * RR_ZONES;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const ReqParams &rq = b.req[req];
+  const int rr_n = rq.rr_n, nr = b.nr_fine, nz = rq.n_zones;
+  if (rq.pre_status != 0 || i0 >= rr_n) return;  // uniform over the block
+  const DevLpTable &L = b.lp;
+  lp_rows(L, rq, s_jr, s_je, s_jd, s_ji, tid, NT);
+  const DevRradTable &R = b.rr;
+  const int nt = R.n_rad, k = rq.rr_k, klo = rq.rr_klo;
+  const double *rlo_t = R.rlo + (size_t)k * nt, *rhi_t = R.rhi + (size_t)k * nt;
+  const double rin_f = fine_radius(rq.rin, rq.rout, nr - 1, nr), rout_f = fine_radius(rq.rin, rq.rout, 0, nr);
+  if (rq.rr_corr && tid < nz) {
+    // the correction factors of relxill zone tid from its band sums (k_rrad_sums):
+    //   flux factor = energy flux over that of the zone's normalised primary
+    //   (k_zone); g factor = photon flux over the shifted one's, over 1.5^Gamma
+    const ZoneRec zr = b.zone[rq.zone_off + tid];
+    const DevXillTable &xt = b.xt[rq.prim];
+    const double f = xt.ect_dim >= 0 ? zr.ect_fac : rq.xfac[3];
+    const int chunks = rrad_chunks(xt.n_ener);
+    const double *part = b.rrpart + rq.rr_corr_off + (size_t)(2 * tid) * chunks * 3;
+    double s[3] = {0.0, 0.0, 0.0};
+    for (int c = 0; c < chunks; c++)
+      for (int j = 0; j < 3; j++) s[j] += (1.0 - f) * part[c * 3 + j] + f * part[(chunks + c) * 3 + j];
+    s_zf[tid] = s[0] / zr.pe;
+    s_zg[tid] = s[1] / s[2] / pow(1.5, rq.xgam);
   }
   __syncthreads();
-  // band sums of the average, and of its shifted copy
-  const double gref = 2. / 3.;
-  const GridGuess gx = grid_guess(E, ne);
-  auto ge = [&](int k) { return E[k]; };
-  auto fav = [&](int k) { return s_avg[k]; };
-  double ef = 0.0, pf = 0.0, pz = 0.0;
-  for (int e = tid; e < ne; e += RRC_THREADS) {
-    const double e0 = E[e], e1 = E[e + 1];
-    if (e0 >= 0.1 && e1 <= 1000.0) ef += s_avg[e] * 0.5 * (e0 + e1);
-    if (e0 >= 0.15 && e1 <= 500.0) {
-      pf += s_avg[e];
-      const double lo = e0 / gref, hi = e1 / gref;
-      pz += rebin_bin(lo, hi, count_le(ge, ne, lo, gx), count_le(ge, ne, hi, gx), ge, ne, fav) * gref;
+  int err = 0;  // (k_setup evaluates and flags every fine radius)
+  for (int i = tid; i < rr_n; i += NT) {
+    const double lo = (i == 0) ? rin_f : rlo_t[klo + i];
+    const double hi = (i == rr_n - 1) ? rout_f : rhi_t[klo + i];
+    const double rm = 0.5 * (lo + hi);
+    s_rad[i] = rm;
+    // relxilllp above spin 0: the correction factors of the relxill zone
+    // the table zone's centre falls in (rebin_corrfactors_to_rradtable_grid,
+    // src/Relreturn_Corona.cpp:248-289; a centre beyond the last edge takes
+    // the last zone)
+    double cf = 1.0, cg = 1.0;
+    if (rq.rr_corr) {
+      const double *zg = rq.zgrid;
+      int ind = bsearch_asc(zg, nz + 1, rm);
+      if (rm < zg[0]) ind = 0;
+      else if (rm > zg[nz] || ind > nz - 1) ind = nz - 1;
+      cf = s_zf[ind];
+      cg = s_zg[ind];
     }
-  }
-  const double s_ef = block_sum(ef, s_red), s_pf = block_sum(pf, s_red), s_pz = block_sum(pz, s_red);
-  // the normalised primary of the zone (Ecut / kTe it sees, the source's
-  // Gamma) on the 500-bin grid (calc_normalized_primary_spectrum, :302-332):
-  // the cut-off power law here, nthcomp from its solve (k_nth)
-  double s_pe;
-  if (rq.prim == PRIM_NTHCOMP) {
-    s_pe = b.nth[rq.nth_off + 1 + z].pe;
-  } else {
-    const double nf =
-        1. / (block_sum(xill_norm_part(b.cg, ect, rq.xgam, tid, RRC_THREADS), s_red) / NORM_XILLVER_TABLE);
-    double pe = 0.0;
-    for (int k = tid; k < N_ENER_COARSE; k += RRC_THREADS) {
-      const double e0 = b.cg.coarse[k], e1 = b.cg.coarse[k + 1];
-      if (e0 >= 0.1 && e1 <= 1000.0)
-        pe += cutoffpl_bin(e0, e1, b.cg.coarse_ln[k], ect, rq.xgam) * nf * 0.5 * (e0 + e1);
+    s_cf[i] = cf;
+    s_cg[i] = cg;
+    int a = 0, c = nr - 1;  // the fine radii re(a) > rm >= re(a+1)
+    while (c - a > 1) {
+      const int mid = (a + c) >> 1;
+      if (fine_radius(rq.rin, rq.rout, mid, nr) > rm) a = mid; else c = mid;
     }
-    s_pe = block_sum(pe, s_red);
+    const double r0 = fine_radius(rq.rin, rq.rout, a, nr), r1 = fine_radius(rq.rin, rq.rout, a + 1, nr);
+    const double e0 = lp_emis_at(rq, r0, s_jr, s_je, s_jd, s_ji, L.n_r, &err);
+    const double e1 = lp_emis_at(rq, r1, s_jr, s_je, s_jd, s_ji, L.n_r, &err);
+    s_in[i] = lerp1((rm - r1) / (r0 - r1), e1, e0);
   }
-  if (tid == 0) {
-    b.rrcorr[rq.rr_corr_off + 2 * z] = s_ef / s_pe;
-    b.rrcorr[rq.rr_corr_off + 2 * z + 1] = s_pf / s_pz / pow(1.5, rq.xgam);
+  if (tid >= NT - 2) {  // ring-area corrections of the end zones (src/Relreturn_Table.cpp:415-435)
+    const int w = tid - (NT - 2), i = (w == 0) ? 0 : rr_n - 1;
+    double rl = rlo_t[klo + i];
+    if (klo + i == 0 && rl > rq.rms) rl = rq.rms;
+    const double rh = rhi_t[klo + i];
+    const double lo = (i == 0) ? rin_f : rlo_t[klo + i];
+    const double hi = (i == rr_n - 1) ? rout_f : rhi_t[klo + i];
+    s_corr[w] = (0.5 * (lo + hi) * (hi - lo)) / (0.5 * (rl + rh) * (rh - rl));
+  }
+  __syncthreads();
+  const int i = i0 + (tid >> 6), j = lane, ng = R.n_g;
+  if (i >= rr_n) return;  // (no barrier below)
+  double term = 0.0;
+  if (j < rr_n) {
+    const size_t t = (size_t)k * nt * nt + (size_t)(klo + i) * nt + (klo + j);
+    const double gmin = R.gmin[t], gmax = R.gmax[t];
+    const double cgj = s_cg[j];
+    double ez = 0.0;
+    for (int jj = 0; jj < ng; jj++) {
+      const double g = (jj + 0.5) / ng * (gmax - gmin) + gmin;  // get_gfac_grid (src/Relreturn_Datastruct.cpp:51-59)
+      double v = R.frac_g[t * ng + jj];
+      if (fabs(cgj - 1) > 1e-3) v *= gshift_boost(cgj, g, rq.gamma) / g;
+      else if (fabs(g - 1) > 1e-3) v *= pow(g, rq.gamma - 1);
+      ez += v;
+    }
+    double tf = R.tf_r[t];
+    if (j == 0 && i < rr_n - 1) tf *= s_corr[0];
+    if (j == rr_n - 1 && i < rr_n - 2) tf *= s_corr[1];
+    term = ez * tf * s_in[j];
+  }
+  const double sum = wave_sum(term);
+  if (lane == 0) {
+    double *o = b.rret + (size_t)rq.rr_slot * (2 * MAX_RR);
+    o[i] = s_rad[i];
+    o[MAX_RR + i] = sum * s_cf[i];
   }
 }
 
@@ -2395,7 +2510,7 @@ __global__ __launch_bounds__(XILL_THREADS, 4) void k_xill1(BatchDev b, const Xil
   if (b.status[req] != 0) return;
   const ReqParams &rq = b.req[req];
   const DevXillTable xt = b.xt[rq.prim];
-  const double dd = rq.xdens_div;
+  const DensDiv dd = dens_of(rq.xdens_div);
   // XILL_BINS bins per thread, XILL_THREADS apart: the corner weights and rows
   // are set up once for all of them, and their loads are in flight together
   const int e0 = (blockIdx.x % chunks) * (XILL_THREADS * XILL_BINS) + threadIdx.x;
@@ -2503,7 +2618,7 @@ __global__ __launch_bounds__(XILL_THREADS, 3) void k_xillz(BatchDev b, const Xil
   if (b.status[req] != 0) return;  // uniform over the block
   const ReqParams &rq = b.req[req];
   const DevXillTable xt = b.xt[rq.prim];
-  const double dd = rq.xdens_div;
+  const DensDiv dd = dens_of(rq.xdens_div);
   const int nz = min(rq.n_zones, NZ);
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int zax = xt.ect_dim >= 0 ? xt.ect_dim : 3;
@@ -2521,33 +2636,9 @@ __global__ __launch_bounds__(XILL_THREADS, 3) void k_xillz(BatchDev b, const Xil
   const int ni = xt.n_incl;
   const int n_o = xt.n_out > 1 ? 2 : 1;
   const int n_cand = (ehi - elo + 2) * ni;  // candidate pairs (e, a), e in [elo, ehi + 1]
-  // corner rows of the axes other than zax (zax index 0), in rows of ni
-  // inclinations; one step on zax moves a row by `stride` rows
   double w8[8];
-  unsigned cb[8];
-  unsigned stride = 1;
-#pragma unroll
-  for (int k = 0; k < 4; k++)
-    if (k > zax) stride *= (unsigned)xt.n_val[k];
-#pragma unroll
-  for (int c = 0; c < 8; c++) {
-    double w = 1.0;
-    unsigned r = 0;
-    int bit = 2;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-      int idx = 0;
-      if (k != zax) {
-        const int o = (c >> bit) & 1;
-        bit--;
-        w *= o ? rq.xfac[k] : (1.0 - rq.xfac[k]);
-        idx = rq.xind[k] + o;
-      }
-      r = r * (unsigned)xt.n_val[k] + (unsigned)idx;
-    }
-    w8[c] = w;
-    cb[c] = r * (unsigned)ni;
-  }
+  unsigned cb[8], stride;
+  corners8(xt, rq, zax, w8, cb, &stride);
   const double *dist = b.dist + rq.dist_off;
   const size_t ne = (size_t)xt.n_ener;
   const int e0 = (blockIdx.x % chunks) * (XILL_THREADS * XILL_BINS_Z) + tid;
@@ -2796,11 +2887,21 @@ int launch_xill(const BatchDev &b, const XillWork *work, int n_single, int n_mul
   return (int)hipGetLastError();
 }
 
-int launch_rrad_corr(const BatchDev &b, const XillWork *work, int n_work, void *stream) {
+int launch_rrad(const BatchDev &b, const int *corr_reqs, int n_corr, const int *reqs, int n_reqs, void *stream) {
+  if (n_corr > 0) {
+    const int n_chunk = rrad_chunks(xill_n_ener(b));
+    hipLaunchKernelGGL(k_rrad_sums, dim3(n_corr * n_chunk), dim3(RRA_THREADS), 0, (hipStream_t)stream, b, corr_reqs,
+                       n_chunk);
+  }
+  if (n_reqs > 0)
+    hipLaunchKernelGGL(k_rrad, dim3(n_reqs * (MAX_RR / RR_ZONES)), dim3(64 * RR_ZONES), 0, (hipStream_t)stream, b,
+                       reqs);
+  return (int)hipGetLastError();
+}
+
+int launch_zone(const BatchDev &b, const XillWork *work, int n_work, void *stream) {
   if (n_work <= 0) return 0;
-  const size_t lds = sizeof(double) * (size_t)xill_n_ener(b);
-  (void)hipFuncSetAttribute((const void *)k_rrad_corr, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  hipLaunchKernelGGL(k_rrad_corr, dim3(n_work), dim3(RRC_THREADS), lds, (hipStream_t)stream, b, work);
+  hipLaunchKernelGGL(k_zone, dim3(n_work), dim3(64), 0, (hipStream_t)stream, b, work);
   return (int)hipGetLastError();
 }
 

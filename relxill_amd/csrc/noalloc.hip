@@ -183,6 +183,8 @@ int noalloc_eval(int model, const double *parameter, const double *d_energy, con
   bd.reach = c.take<BinRange>(1);
   bd.fix = c.take<FixEntry>((size_t)fix_cap);
   bd.fix_cap = fix_cap;
+  bd.rret = reinterpret_cast<double *>(bd.fix);  // read by k_setup, before k_integrate queues re-checks
+  static_assert(2 * MAX_RR * sizeof(double) <= 4096 * sizeof(FixEntry), "the returning emissivity fits the queue");
   bd.guard = g.guard;
   bd.xspec = nullptr;
   bd.zone = c.take<ZoneRec>(1);
@@ -206,6 +208,9 @@ int noalloc_eval(int model, const double *parameter, const double *d_energy, con
                          bd.status);
       e |= (int)hipGetLastError();
     }
+    // (the one unit {0, 0} of d_work is the list of request 0)
+    if (p.return_rad != 0 && p.pre_status == 0)
+      e |= launch_rrad(bd, nullptr, 0, reinterpret_cast<const int *>(d_work), 1, s);
     e |= launch_setup(bd, s);
     e |= launch_integrate(bd, n_blocks, cos_rows, s);
     e |= launch_fixup(bd, cos_rows, s);

@@ -21,6 +21,7 @@
 //   xspec               relxill requests: the angle-weighted xillver spectrum
 //                       (n_ener of the xillver table each), written by k_xill
 #pragma once
+#include <hip/hip_runtime.h>
 #include <stdint.h>
 
 namespace rx {
@@ -32,7 +33,11 @@ constexpr int MAX_INCL = 64;      // emission-angle bins
 constexpr int MAX_FFT = 8192;     // convolution grid size limit
 constexpr int LP_ZONES = 10;      // radial zones of relxilllp (N_ZONES, src/common.h:134)
 constexpr int MAX_ZONES = 25;     // with an ionisation gradient (N_ZONES_IONGRAD, src/common.h:135)
-constexpr int MAX_RRC_ENER = 16384;  // xillver bins held in LDS by the returning-radiation corrections
+constexpr int MAX_RRC_ENER = 16384;  // most xillver bins of a request with returning-radiation corrections
+// the returning radiation's band sums: table bins per workgroup, and partial
+// sums (per zone, Ecut node and band) of a table
+constexpr int RRA_THREADS = 256;
+__host__ __device__ constexpr int rrad_chunks(int n_ener) { return (n_ener + RRA_THREADS - 1) / RRA_THREADS; }
 
 enum ModelKind : int {
   MOD_RELLINE = 1,
@@ -119,9 +124,11 @@ struct ReqParams {
   // returning radiation (lamp post): 1 add, -1 or 2 replace the direct
   // emissivity; the table spin, its first zone and the number of zones used
   int return_rad, rr_k, rr_klo, rr_n;
-  // relxilllp above spin 0: the zones' xillver correction factors of the
-  // returning radiation (flux, g shift per zone) at rrcorr[rr_corr_off]
-  int rr_corr;
+  // relxilllp above spin 0: the band sums behind the zones' xillver correction
+  // factors (flux, g shift) of the
+  // returning radiation at rrpart[rr_corr_off] ([zone][2 nodes][chunk][3]);
+  // rr_slot: the request's returning emissivity in rret
+  int rr_corr, rr_slot;
   int64_t rr_corr_off;
 };
 
@@ -131,6 +138,7 @@ struct ReqParams {
 // incident spectrum (src/Xillspec.cpp:408-435).
 struct ZoneRec {
   double rmean, del_emit, shift, ncf, ect_fac, lxi_fac;
+  double pe;  // energy flux of the zone's normalised primary (with rr_corr only)
   int ect_ind, lxi_ind;  // the zone's brackets on the Ecut and logXi axes (with ect_fac, lxi_fac)
 };
 
@@ -249,6 +257,9 @@ struct DevXillTable {
   int lxi_dim;             // inner axis of logXi (-1: none)
   int n_lxi;
   const float *lxi_vals;   // its values (the zones of an ionisation gradient bracket their own)
+  // ends of the bins within 0.15-500 keV, shifted 1.5 times up in energy (the
+  // returning radiation's g factor reads the spectrum there); none: rr_lo > rr_hi
+  double rr_lo, rr_hi;
 };
 
 constexpr int N_ENER_COARSE = 500;  // primary-continuum normalisation grid (src/Xillspec.h:32)
@@ -356,7 +367,9 @@ struct BatchDev {
   double *xspec;
   ZoneRec *zone;
   DevRradTable rr;
-  double *rrcorr;     // relxilllp returning radiation: 2 factors per zone
+  // returning radiation: relxilllp's band sums (per zone 2 Ecut nodes x chunks
+  // x 3), per request the table zones' centres and returning emissivity
+  double *rrpart, *rret;
   // nthcomp primary: per solve its normalisation results, per request the
   // source's solution (x: NTH_MAX_POINTS + 1, E F_E: NTH_MAX_POINTS, jmax)
   NthRes *nth;
@@ -375,9 +388,13 @@ int launch_finalize(const BatchDev &b, void *stream);
 int launch_conv(const BatchDev &b, const XillWork *conv_work, int n_conv_work, void *stream);
 // work: n_single one-zone units, then n_multi units of several zones
 int launch_xill(const BatchDev &b, const XillWork *work, int n_single, int n_multi, void *stream);
-// relxilllp returning radiation above spin 0: the zones' xillver correction
-// factors, one workgroup per (request, zone) of work (before launch_setup)
-int launch_rrad_corr(const BatchDev &b, const XillWork *work, int n_work, void *stream);
+// returning radiation (before launch_setup): the xillver band sums of the
+// n_corr relxilllp requests above spin 0 (after launch_zone), then the returning
+// emissivity of all n_reqs requests with it
+int launch_rrad(const BatchDev &b, const int *corr_reqs, int n_corr, const int *reqs, int n_reqs, void *stream);
+// lamp-post relxill requests: the zone records, one (request, zone) unit each
+// (after launch_nth)
+int launch_zone(const BatchDev &b, const XillWork *work, int n_work, void *stream);
 // relxill requests: the primary continuum added to the output (after launch_conv)
 int launch_primary(const BatchDev &b, const int *reqs, int n_reqs, void *stream);
 int launch_copy(const void *src, void *dst, size_t bytes, void *stream);
