@@ -553,6 +553,11 @@ int ensure_device(std::string &err) {
     e |= upload_vec(g.d_refl_sets, g.refl_sets);
     g.refl_dirty = false;
   }
+  if (!g.nth_grid.p) {
+    e |= g.nth_grid.ensure(nth_grid_bytes());
+    if (!e) e |= launch_nth_grid(g.nth_grid.as<double>(), nullptr);
+    e |= (int)hipDeviceSynchronize();  // read from other streams
+  }
   if (e) {
     err = "device upload failed";
     return RX_ERR_DEVICE;
@@ -772,6 +777,7 @@ void fill_dev_views(BatchDev &bd) {
     xt.rr_lo = x.rr_lo;
     xt.rr_hi = x.rr_hi;
   }
+  bd.nth_tab = g.nth_grid.as<double>();
   bd.rr.n_spin = g.rrad.n_spin;
   bd.rr.n_rad = g.rrad.n_rad;
   bd.rr.n_g = g.rrad.n_g;

@@ -152,6 +152,7 @@ struct Global {
   // returning-radiation table (loaded and uploaded on the first request with it)
   RradTableHost rrad;
   bool rrad_loaded = false, rrad_dirty = true;
+  DevBuf nth_grid;  // what all nthcomp solves share
   DevBuf r_rlo, r_rhi, r_tf, r_gmin, r_gmax, r_fg;
   // convolution grid
   int conv_n = 4096;

@@ -1265,32 +1265,32 @@ __global__ __launch_bounds__(NTH_THREADS_R) void k_nth(BatchDev b, const XillWor
     if (tid == 0) s_kte = rq.xect_src;
   } else {
     // the lamp-post rows in the solve's arrays (the solve overwrites them)
-    lp_rows(b.lp, rq, L.a, L.b, L.c, L.d, tid, NTH_THREADS_R);
+    lp_rows(b.lp, rq, L.t1, L.t2, L.t3, L.d, tid, NTH_THREADS_R);
     if (tid == 0) {
       double ect;
-      (void)zone_record(b.xt[rq.prim], rq, j - 1, true, L.a, L.b, L.c, L.d, b.lp.n_r, b.nr_fine, &ect);
+      (void)zone_record(b.xt[rq.prim], rq, j - 1, true, L.t1, L.t2, L.t3, L.d, b.lp.n_r, b.nr_fine, &ect);
       s_kte = ect;
     }
   }
   __syncthreads();
   const double kte = s_kte;
-  const int nth = nth_solve(L, kte, rq.xgam, 0.05, tid, NTH_THREADS_R);  // kT_bb 0.05 keV (src/relutility.c:625-632)
-  // the spectrum on the 500-bin grid (spec_nthcomp at z = 0), per bin in a
-  const double nfac = nthcomp_normfac(L.x, L.c, nth, 0.0);
+  const int nth = nth_solve(L, nth_grid_tab(b.nth_tab), kte, rq.xgam, tid, NTH_THREADS_R);
+  // the spectrum on the 500-bin grid (spec_nthcomp at z = 0), per bin in t2
+  const double nfac = nthcomp_normfac(L.x, L.t1, nth, 0.0);
   const double *ce = b.cg.coarse;
   double sp = 0.0;
   for (int k = tid; k < N_ENER_COARSE; k += NTH_THREADS_R) {
     const double e0 = ce[k], e1 = ce[k + 1];
-    const double f = nthcomp_bin(e0, e1, nthcomp_edge(L.x, L.c, nth, e0, 0.0), nthcomp_edge(L.x, L.c, nth, e1, 0.0),
+    const double f = nthcomp_bin(e0, e1, nthcomp_edge(L.x, L.t1, nth, e0, 0.0), nthcomp_edge(L.x, L.t1, nth, e1, 0.0),
                                  nfac);
-    L.a[k] = f;
+    L.t2[k] = f;
     if (e0 >= 0.1 && e0 <= 1000.0) sp += f * 0.5 * (e0 + e1) * 1e20 * 1.602177e-09;
   }
   const double nf = 1. / (block_sum(sp, s_red) / NORM_XILLVER_TABLE);
   double pe = 0.0;
   for (int k = tid; k < N_ENER_COARSE; k += NTH_THREADS_R) {
     const double e0 = ce[k], e1 = ce[k + 1];
-    if (e0 >= 0.1 && e1 <= 1000.0) pe += L.a[k] * nf * 0.5 * (e0 + e1);
+    if (e0 >= 0.1 && e1 <= 1000.0) pe += L.t2[k] * nf * 0.5 * (e0 + e1);
   }
   const double s_pe = block_sum(pe, s_red);
   if (tid == 0) b.nth[rq.nth_off + j] = NthRes{nf, s_pe};
@@ -1298,7 +1298,7 @@ __global__ __launch_bounds__(NTH_THREADS_R) void k_nth(BatchDev b, const XillWor
     double *xo = b.nth_x + (size_t)rq.nth_sol * (NTH_N + 1);
     double *so = b.nth_s + (size_t)rq.nth_sol * NTH_N;
     for (int i = tid; i <= nth; i += NTH_THREADS_R) xo[i] = L.x[i];
-    for (int i = tid; i < NTH_N; i += NTH_THREADS_R) so[i] = L.c[i];
+    for (int i = tid; i < NTH_N; i += NTH_THREADS_R) so[i] = L.t1[i];
     if (tid == 0) b.nth_n[rq.nth_sol] = nth;
   }
 }

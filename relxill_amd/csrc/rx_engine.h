@@ -375,6 +375,7 @@ struct BatchDev {
   NthRes *nth;
   double *nth_x, *nth_s;
   int *nth_n;
+  const double *nth_tab;  // the grid all solves share (nth_grid_tab)
 };
 
 // ---- launchers (kernels.hip) ----
@@ -403,11 +404,15 @@ int launch_copy(const void *src, void *dst, size_t bytes, void *stream);
 // photon energies of one Kompaneets solve (the reference's arrays of 900)
 constexpr int NTH_MAX_POINTS = 900;
 struct NthJob {
-  double kte, gam, ktbb;  // keV, photon index, seed temperature (keV)
+  double kte, gam;  // keV, photon index (the seed temperature is 0.05 keV)
 };
 // one solve per job: x (NTH_MAX_POINTS + 1 per job, m_e c^2), E F_E
 // (NTH_MAX_POINTS per job), the number of points
-int launch_nthcomp(const NthJob *jobs, int n_jobs, double *sol_x, double *sol_s, int *sol_n, void *stream);
+int launch_nthcomp(const NthJob *jobs, int n_jobs, const double *tab, double *sol_x, double *sol_s, int *sol_n,
+                   void *stream);
+// the photon grid's factors that every solve shares, once per device
+size_t nth_grid_bytes();
+int launch_nth_grid(double *tab, void *stream);
 // relxill models with the nthcomp primary: one solve per (request, j) of
 // work (j = 0 the source, j = 1 + z zone z of a lamp post), first in a run
 int launch_nth(const BatchDev &b, const XillWork *work, int n_work, void *stream);
