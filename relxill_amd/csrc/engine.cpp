@@ -1005,6 +1005,7 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
       p.zone_off = o_zone;
       o_zone += 1;
       b.h_xill.push_back(XillWork{i, 0});
+      b.h_zone.push_back(XillWork{i, 0});
       b.h_prim.push_back(i);
       if (p.prim == PRIM_NTHCOMP) {
         p.n_nth = 1;
@@ -1043,7 +1044,7 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
         o_xspec += (int64_t)xt.n_ener * p.n_zones;
         p.zone_off = o_zone;
         o_zone += p.n_zones;
-        for (int z = 0; lp && z < p.n_zones; z++) b.h_zone.push_back(XillWork{i, z});
+        for (int z = 0; z < p.n_zones; z++) b.h_zone.push_back(XillWork{i, z});
         if (p.ion_grad) {
           // zones that differ in logXi as well as in Ecut: one k_xill1 unit each
           for (int z = 0; z < p.n_zones; z++) b.h_xill.push_back(XillWork{i, z});
@@ -1100,6 +1101,8 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
     p.pre_status = st;
     b.h_status[i] = st;
   }
+  b.prim_bins = 0;
+  for (int i : b.h_prim) b.prim_bins = std::max(b.prim_bins, b.h_req[i].n_in);
   b.tot_ener = o_ener;
   b.tot_flux = o_flux;
   b.tot_pgrid = o_pgrid;
@@ -1310,7 +1313,7 @@ static int launch_sequence(Batch &b, const RunKey &k, hipStream_t s) {
   if (prof) e |= (int)hipEventRecord(b.ev[5], s);
   e |= launch_conv(bd, static_cast<const XillWork *>(k.d_conv), k.n_conv, s);
   if (prof) e |= (int)hipEventRecord(b.ev[6], s);
-  e |= launch_primary(bd, static_cast<const int *>(k.d_prim), k.n_prim, s);
+  e |= launch_primary(bd, static_cast<const int *>(k.d_prim), k.n_prim, k.prim_bins, s);
   if (prof) e |= (int)hipEventRecord(b.ev[7], s);
   return e;
 }
@@ -1368,6 +1371,7 @@ int batch_run(Batch &b, int precision, std::string &err) {
   k.n_xill = (int)b.h_xill.size();
   k.n_conv = (int)b.h_conv.size();
   k.n_prim = (int)b.h_prim.size();
+  k.prim_bins = b.prim_bins;
   k.d_xill = b.d_xill.p;
   k.d_conv = b.d_conv.p;
   k.d_prim = b.d_prim.p;

@@ -49,7 +49,7 @@ void rzone_grid(double rmin, double rmax, int nzones, double h, double *rgrid);
 // its padding zeroed, so configurations compare with memcmp.
 struct RunKey {
   BatchDev bd;
-  int n_blocks, n_xill1, n_xill, n_conv, n_prim, n_rrc, n_rrad, n_nth, n_ang, n_zone;
+  int n_blocks, n_xill1, n_xill, n_conv, n_prim, n_rrc, n_rrad, n_nth, n_ang, n_zone, prim_bins;
   const void *d_xill, *d_conv, *d_prim, *d_rrc, *d_rrad, *d_nth, *d_ang, *d_zone;
   int prof, cos_rows;
 };
@@ -65,13 +65,14 @@ struct Batch {
   std::vector<int> h_status;  // host-side parse status
   std::vector<double> h_ener, h_flux_in;
   std::vector<int> h_prim;
+  int prim_bins = 0;             // most caller bins of a request in h_prim
   std::vector<int> h_ang;        // requests with an emission-angle distribution (k_dist)
   std::vector<XillWork> h_conv;  // (request, zone) units of k_conv
   std::vector<XillWork> h_xill;  // k_xill units: one-zone requests first, then the others (all zones in one unit)
   int n_xill1 = 0;               // number of one-zone units at the front of h_xill
   std::vector<int> h_rrc;        // requests with returning-radiation corrections (k_rrad_sums)
   std::vector<int> h_rrad;       // requests with returning radiation (k_rrad)
-  std::vector<XillWork> h_zone;  // (request, zone) units of k_zone (lamp-post relxill models)
+  std::vector<XillWork> h_zone;  // (request, zone) units of k_zone (relxill and xillver models)
   std::vector<XillWork> h_nth;   // nthcomp solves: (request, 0 source / 1 + zone)
   int n_nth_sol = 0;             // requests with the nthcomp primary (one source solution each)
   int64_t tot_ener = 0, tot_flux = 0, tot_pgrid = 0, tot_prof = 0, tot_xspec = 0, tot_dist = 0, tot_zone = 0;

@@ -528,27 +528,10 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
   if (rq.pre_status != 0) return;  // status already set by the host
   if (rq.model == MOD_XILLVER) {
     // the xillver models (LocalModel::xillver_model, src/LocalModel.cpp:
-    // 104-128) have no relativistic part: the zone record carries the Ecut
-    // (kTe) bracket, the angle distribution the inclination's bracket, so
-    // that k_xill's sum over angles is the interpolation in the inclination
-    // (interp_5d_tab, src/xilltable.c:878-995); k_primary rebins and adds the
-    // primary
-    if (tid == 0) {
-      // the bracket through the request in global memory: a runtime index
-      // into the local copy rq would move that copy to scratch
-      const ReqParams &gq = b.req[req];
-      const DevXillTable &xt = b.xt[rq.prim];
-      ZoneRec o;
-      o.rmean = 0.0;
-      o.del_emit = 0.0;
-      o.shift = 1.0;
-      o.ncf = 1.0;
-      o.ect_ind = xt.ect_dim >= 0 ? gq.xind[xt.ect_dim] : 0;
-      o.ect_fac = xt.ect_dim >= 0 ? gq.xfac[xt.ect_dim] : 0.0;
-      o.lxi_ind = xt.lxi_dim >= 0 ? gq.xind[xt.lxi_dim] : 0;
-      o.lxi_fac = xt.lxi_dim >= 0 ? gq.xfac[xt.lxi_dim] : 0.0;
-      b.zone[rq.zone_off] = o;
-    }
+    // 104-128) have no relativistic part: the angle distribution carries the
+    // inclination's bracket, so that k_xill's sum over angles is the
+    // interpolation in the inclination (interp_5d_tab, src/xilltable.c:878-995);
+    // k_primary rebins and adds the primary
     double *d = b.dist + rq.dist_off;
     for (int a = tid; a < rq.n_incl; a += SETUP_THREADS)
       d[a] = (a == rq.xinc_ind) ? 1.0 - rq.xinc_fac : ((a == rq.xinc_ind + 1) ? rq.xinc_fac : 0.0);
@@ -832,12 +815,6 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
     b.refl[req] = o;
   }
 
-  // the zone of a broken power-law relxill request (a lamp post's: k_zone)
-  if (rq.model == MOD_RELXILL && tid == 0) {
-    double ect;
-    b.zone[rq.zone_off] =
-        zone_record(b.xt[rq.prim], b.req[req], 0, false, nullptr, nullptr, nullptr, nullptr, 0, nr, &ect);
-  }
   if (rq.n_incl > 0) {  // k_dist adds into the angle distribution
     const int nd = rq.n_incl * nz;  // [zone][angle bin]
     for (int k = tid; k < nd; k += SETUP_THREADS) b.dist[rq.dist_off + k] = 0.0;
@@ -916,13 +893,16 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
   if (tid == 0) b.status[req] = s_st;
 }
 
-// Radial zones of the lamp-post relxill requests (IonGradient,
-// src/IonGradient.cpp:182-209, :421-430): the zone record (centre, emission
-// angle, energy shift, the xillver brackets the zone sees) and the
-// normalisation change of the incident spectrum (src/Xillspec.cpp:408-435),
-// one wavefront per (request, zone).  The change is a ratio of two sums over
-// the 500-bin grid (the cut-off power law; 8 exponentials a lane and sum) or
-// of two nthcomp norms (k_nth, which runs before).
+// Radial zones of the relxill and xillver requests (IonGradient,
+// src/IonGradient.cpp:182-209, :421-430): the zone record (centre, and for the
+// lamp post the emission angle, energy shift and xillver brackets the zone
+// sees) and, for the lamp post, the normalisation change of the incident
+// spectrum (src/Xillspec.cpp:408-435), one wavefront per (request, zone).  The
+// change is a ratio of two sums over the 500-bin grid (the cut-off power law; 8
+// exponentials a lane and sum) or of two nthcomp norms (k_nth, which runs
+// before).  Zone 0's wavefront keeps the norm of the primary at the source
+// (calcNormWrtXillverTableSpec on the 500-bin grid, src/PrimarySource.h:238-292)
+// and its energy boost for k_primary.
 // Bound: the latency of the table rows and the sums, 15 us alone, 20 us for 1280
 // zones (inside k_setup, zone after zone with tree sums: 18 us and 22 us, but
 // after the returning radiation that reads the records).
@@ -933,29 +913,57 @@ __global__ __launch_bounds__(64) void k_zone(BatchDev b, const XillWork *__restr
   const ReqParams &rq = b.req[req];
   if (rq.pre_status != 0) return;  // uniform over the block
   const DevXillTable &xt = b.xt[rq.prim];
-  lp_rows(b.lp, rq, s_jr, s_je, s_jd, s_ji, lane, 64);
-  double ect;
-  ZoneRec zr = zone_record(xt, rq, z, true, s_jr, s_je, s_jd, s_ji, b.lp.n_r, b.nr_fine, &ect);
+  const bool lp = rq.emis_type == EMIS_LP;
+  const double gam = rq.xgam;
+  double ect = rq.xect_src;
+  ZoneRec zr;
+  if (rq.model == MOD_XILLVER) {  // no relativistic part: the request's brackets
+    zr = ZoneRec();
+    zr.shift = 1.0;
+    zr.ect_ind = xt.ect_dim >= 0 ? rq.xind[xt.ect_dim] : 0;
+    zr.ect_fac = xt.ect_dim >= 0 ? rq.xfac[xt.ect_dim] : 0.0;
+    zr.lxi_ind = xt.lxi_dim >= 0 ? rq.xind[xt.lxi_dim] : 0;
+    zr.lxi_fac = xt.lxi_dim >= 0 ? rq.xfac[xt.lxi_dim] : 0.0;
+  } else {
+    if (lp) lp_rows(b.lp, rq, s_jr, s_je, s_jd, s_ji, lane, 64);
+    zr = zone_record(xt, rq, z, lp, s_jr, s_je, s_jd, s_ji, b.lp.n_r, b.nr_fine, &ect);
+  }
+  zr.ncf = 1.0;
+  zr.pe = 0.0;
   if (rq.prim == PRIM_NTHCOMP) {
     const NthRes *n = b.nth + rq.nth_off;
-    zr.ncf = n[1 + z].nf / n[0].nf;
-    zr.pe = n[1 + z].pe;
-  } else {
-    const double gam = rq.xgam;
-    const double src = 1. / (wave_sum(xill_norm_part(b.cg, rq.xect_src, gam, lane, 64)) / NORM_XILLVER_TABLE);
-    const double disk = 1. / (wave_sum(xill_norm_part(b.cg, ect, gam, lane, 64)) / NORM_XILLVER_TABLE);
-    zr.ncf = disk / src;
-    // energy flux of the zone's normalised primary in 0.1-1000 keV
-    // (get_xillver_fluxcorr, src/Xillspec.cpp:344-362)
-    double pe = 0.0;
-    if (rq.rr_corr) {
-      for (int k = lane; k < N_ENER_COARSE; k += 64) {
-        const double e0 = b.cg.coarse[k], e1 = b.cg.coarse[k + 1];
-        if (e0 >= 0.1 && e1 <= 1000.0)
-          pe += cutoffpl_bin(e0, e1, b.cg.coarse_ln[k], ect, gam) * disk * 0.5 * (e0 + e1);
-      }
+    zr.nf = n[0].nf;
+    if (lp) {
+      zr.ncf = n[1 + z].nf / n[0].nf;
+      zr.pe = n[1 + z].pe;
     }
-    zr.pe = wave_sum(pe);
+  } else {
+    const double part = rq.prim == PRIM_BBODY ? bbody_norm_part(b.cg, rq.xktbb, lane, 64)
+                                              : xill_norm_part(b.cg, rq.xect_src, gam, lane, 64);
+    zr.nf = 1. / (wave_sum(part) / NORM_XILLVER_TABLE);
+    if (lp) {
+      const double disk = 1. / (wave_sum(xill_norm_part(b.cg, ect, gam, lane, 64)) / NORM_XILLVER_TABLE);
+      zr.ncf = disk / zr.nf;
+      // energy flux of the zone's normalised primary in 0.1-1000 keV
+      // (get_xillver_fluxcorr, src/Xillspec.cpp:344-362)
+      double pe = 0.0;
+      if (rq.rr_corr) {
+        for (int k = lane; k < N_ENER_COARSE; k += 64) {
+          const double e0 = b.cg.coarse[k], e1 = b.cg.coarse[k + 1];
+          if (e0 >= 0.1 && e1 <= 1000.0)
+            pe += cutoffpl_bin(e0, e1, b.cg.coarse_ln[k], ect, gam) * disk * 0.5 * (e0 + e1);
+        }
+      }
+      zr.pe = wave_sum(pe);
+    }
+  }
+  zr.boost = 1.0;
+  if (lp) {  // flux_boost_source_to_observer, src/PrimarySource.h:84-93
+    zr.boost = pow(rq.g_so, gam);
+    if (rq.beta > 1e-4) {
+      const double dop = sqrt(1.0 - rq.beta * rq.beta) / (1.0 + rq.beta * cos(M_PI - rq.incl));
+      zr.boost *= pow(dop, 2);
+    }
   }
   if (lane == 0) b.zone[rq.zone_off + z] = zr;
 }
@@ -2390,32 +2398,32 @@ __global__ __launch_bounds__(CONV_THREADS_MAX) void k_conv(BatchDev b, const Xil
 // src/PrimarySource.cpp:66-125) for refl_frac >= 0: the cut-off power law with
 // the source's Ecut shifted to the observer (spec_cutoffpl,
 // src/Xillspec.cpp:215-241) on the convolution grid, normalised as the
-// xillver incident spectrum at the source (calcNormWrtXillverTableSpec on the
-// 500-bin grid, src/PrimarySource.h:238-292), times the lamp post's flux boost,
-// rebinned onto the caller grid.  One workgroup per request, after k_conv.
-__global__ __launch_bounds__(PRIM_THREADS) void k_primary(BatchDev b, const int *__restrict__ reqs) {
-  __shared__ double s_w[PRIM_THREADS / 64];
-  const int req = reqs[blockIdx.x];
-  const int tid = threadIdx.x, NT = blockDim.x;
-  const int lane = tid & 63, wave = tid >> 6, nwave = NT >> 6;
+// xillver incident spectrum at the source (k_zone), times the lamp post's flux
+// boost, rebinned onto the caller grid.  After k_conv, one workgroup per
+// (request, PRIM_THREADS * per caller bins); launch_primary chooses per.
+// Bound: the latency of the exponential and the grid reads for few requests,
+// FP64 issue (an exponential and a division a grid bin) for many.  One
+// workgroup a request, with the norm's 500 exponentials and 12 rounds of bins,
+// took 28 us for one request of 3000 bins (47 us with the nthcomp primary) and
+// 57 us for 1024; now 5.5 us (8 us) and 51 us.
+__global__ __launch_bounds__(PRIM_THREADS) void k_primary(BatchDev b, const int *__restrict__ reqs, int chunks, int per) {
+  const int req = reqs[blockIdx.x / chunks];
+  const int j0 = (blockIdx.x % chunks) * (PRIM_THREADS * per) + threadIdx.x;
   const ReqParams &rq = b.req[req];
+  const int j1 = min(rq.n_in, j0 + PRIM_THREADS * per);  // this thread: j0, j0 + PRIM_THREADS, ... below j1
+  if (j0 >= j1) return;
   const bool xill = rq.model == MOD_XILLVER;
   if (xill && b.status[req] != 0) {
-    for (int j = tid; j < rq.n_in; j += NT) b.out[rq.flux_off + j] = 0.0;
+    for (int jb = j0; jb < j1; jb += PRIM_THREADS) b.out[rq.flux_off + jb] = 0.0;
     return;
   }
   if (!xill && (b.status[req] != 0 || !(rq.refl_frac >= 0))) return;
   const DevConvGrid &cg = b.cg;
   const int n = cg.n;
   const double ect = rq.xect_src, gam = rq.xgam;
+  const ZoneRec &z0 = b.zone[rq.zone_off];
   double prim_scale = 1.0;
-  if (rq.emis_type == EMIS_LP) {  // flux_boost_source_to_observer, src/PrimarySource.h:84-93
-    prim_scale = b.refl[req].f_inf_rest / 0.5 * pow(rq.g_so, gam);
-    if (rq.beta > 1e-4) {
-      const double dop = sqrt(1.0 - rq.beta * rq.beta) / (1.0 + rq.beta * cos(M_PI - rq.incl));
-      prim_scale *= pow(dop, 2);
-    }
-  }
+  if (rq.emis_type == EMIS_LP) prim_scale = b.refl[req].f_inf_rest / 0.5 * z0.boost;
   // nthcomp: the source's solve (k_nth) observed at redshift 1/g - 1
   // (spec_nthcomp, src/Xillspec.cpp:243-253) with the norm of its spectrum
   // at the source
@@ -2429,9 +2437,7 @@ __global__ __launch_bounds__(PRIM_THREADS) void k_primary(BatchDev b, const int 
   // the blackbody (relxillNS) takes no energy shift (calc_primary_spectrum,
   // src/Xillspec.cpp:293-295)
   const bool bb = rq.prim == PRIM_BBODY;
-  const double nf = nth  ? b.nth[rq.nth_off].nf
-                    : bb ? 1. / (block_sum4(bbody_norm_part(cg, rq.xktbb, tid, NT), s_w) / NORM_XILLVER_TABLE)
-                         : 1. / (block_sum4(xill_norm_part(cg, ect, gam, tid, NT), s_w) / NORM_XILLVER_TABLE);
+  const double nf = z0.nf;
   // the primary on the convolution grid, evaluated where the rebin reads it
   // (one or two grid bins per output bin on caller grids finer than the
   // convolution grid; every grid bin of the output bin, each with its
@@ -2446,13 +2452,8 @@ __global__ __launch_bounds__(PRIM_THREADS) void k_primary(BatchDev b, const int 
                           : cutoffpl_bin(ce[i], ce[i + 1], cl[i], ect_o, gam);
     return (v * nf) * prim_scale;
   };
-  const GridGuess gc = grid_guess(ce, n);
-  auto ge_c = [&](int k) { return ce[k]; };
   const double *eo = b.ener_in + rq.ener_off;
   double *out = b.out + rq.flux_off;
-  const int n_o = rq.n_in;
-  const int nbo = (n_o + nwave - 1) / nwave;
-  const int jend = min(n_o, (wave + 1) * nbo);
   if (xill) {
     // the xillver models: the table spectrum times 0.5 cos(Incl)
     // (norm_xillver_spec, src/Xillspec.cpp:536-545) rebinned onto the
@@ -2466,33 +2467,29 @@ __global__ __launch_bounds__(PRIM_THREADS) void k_primary(BatchDev b, const int 
     const GridGuess gx = grid_guess(xt.ener, nxt);
     auto ge_x = [&](int k) { return xt.ener[k]; };
     auto refl_at = [&](int k) { return xs[k] * slab; };
-    for (int q = 0; q < nbo; q += 64) {
-      const int jb = wave * nbo + q + lane;
-      if (jb < jend) {
-        const double elo = eo[jb], ehi = eo[jb + 1];
-        const int xlo = count_le(ge_x, nxt, elo, gx);
-        const int xhi = count_le(ge_x, nxt, ehi, gx);
-        double v = rebin_bin(elo, ehi, xlo, xhi, ge_x, nxt, refl_at) * fabs(rf);
-        if (rf >= 0) {
-          const double p = nth  ? nthcomp_bin(elo, ehi, nthcomp_edge(nx, ns, nn, elo, 0.0),
-                                              nthcomp_edge(nx, ns, nn, ehi, 0.0), nfac)
-                           : bb ? bbody_bin(elo, ehi, rq.xktbb)
-                                : cutoffpl_bin(elo, ehi, log(0.5 * (elo + ehi)), ect, gam);
-          v += p * nf;
-        }
-        out[jb] = v;
+    for (int jb = j0; jb < j1; jb += PRIM_THREADS) {
+      const double elo = eo[jb], ehi = eo[jb + 1];
+      const int xlo = count_le(ge_x, nxt, elo, gx);
+      const int xhi = count_le(ge_x, nxt, ehi, gx);
+      double v = rebin_bin(elo, ehi, xlo, xhi, ge_x, nxt, refl_at) * fabs(rf);
+      if (rf >= 0) {
+        const double p = nth  ? nthcomp_bin(elo, ehi, nthcomp_edge(nx, ns, nn, elo, 0.0),
+                                            nthcomp_edge(nx, ns, nn, ehi, 0.0), nfac)
+                         : bb ? bbody_bin(elo, ehi, rq.xktbb)
+                              : cutoffpl_bin(elo, ehi, log(0.5 * (elo + ehi)), ect, gam);
+        v += p * nf;
       }
+      out[jb] = v;
     }
     return;
   }
-  for (int q = 0; q < nbo; q += 64) {
-    const int jb = wave * nbo + q + lane;
-    if (jb < jend) {
-      const double elo = eo[jb], ehi = eo[jb + 1];
-      const int clo = count_le(ge_c, n, elo, gc);
-      const int chi = count_le(ge_c, n, ehi, gc);
-      out[jb] += rebin_bin(elo, ehi, clo, chi, ge_c, n, prim_at);
-    }
+  const GridGuess gc = grid_guess(ce, n);
+  auto ge_c = [&](int k) { return ce[k]; };
+  for (int jb = j0; jb < j1; jb += PRIM_THREADS) {
+    const double elo = eo[jb], ehi = eo[jb + 1];
+    const int clo = count_le(ge_c, n, elo, gc);
+    const int chi = count_le(ge_c, n, ehi, gc);
+    out[jb] += rebin_bin(elo, ehi, clo, chi, ge_c, n, prim_at);
   }
 }
 
@@ -2911,9 +2908,17 @@ int launch_nth(const BatchDev &b, const XillWork *work, int n_work, void *stream
   return (int)hipGetLastError();
 }
 
-int launch_primary(const BatchDev &b, const int *reqs, int n_reqs, void *stream) {
+int launch_primary(const BatchDev &b, const int *reqs, int n_reqs, int max_bins, void *stream) {
   if (n_reqs <= 0) return 0;
-  hipLaunchKernelGGL(k_primary, dim3(n_reqs), dim3(PRIM_THREADS), 0, (hipStream_t)stream, b, reqs);
+  // bins per thread: one until the chip holds no more workgroups at once (1024),
+  // then as many as keep it full: a workgroup's fixed part (parameters, grid
+  // guesses) costs about two bins.  1024 requests of 3000 bins: 72 us with one
+  // bin, 51 us with eleven; 128 requests: 9 us with one, 26 us with twelve.
+  const int rounds = (max_bins + PRIM_THREADS - 1) / PRIM_THREADS;
+  const int per = (int)std::max<int64_t>(1, std::min<int64_t>(rounds, (int64_t)n_reqs * rounds / 1024));
+  const int chunks = (rounds + per - 1) / per;
+  hipLaunchKernelGGL(k_primary, dim3(n_reqs * chunks), dim3(PRIM_THREADS), 0, (hipStream_t)stream, b, reqs, chunks,
+                     per);
   return (int)hipGetLastError();
 }
 

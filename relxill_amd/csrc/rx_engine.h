@@ -139,6 +139,7 @@ struct ReqParams {
 struct ZoneRec {
   double rmean, del_emit, shift, ncf, ect_fac, lxi_fac;
   double pe;  // energy flux of the zone's normalised primary (with rr_corr only)
+  double nf, boost;  // norm and energy boost of the primary at the source
   int ect_ind, lxi_ind;  // the zone's brackets on the Ecut and logXi axes (with ect_fac, lxi_fac)
 };
 
@@ -393,11 +394,12 @@ int launch_xill(const BatchDev &b, const XillWork *work, int n_single, int n_mul
 // n_corr relxilllp requests above spin 0 (after launch_zone), then the returning
 // emissivity of all n_reqs requests with it
 int launch_rrad(const BatchDev &b, const int *corr_reqs, int n_corr, const int *reqs, int n_reqs, void *stream);
-// lamp-post relxill requests: the zone records, one (request, zone) unit each
+// relxill and xillver requests: the zone records, one (request, zone) unit each
 // (after launch_nth)
 int launch_zone(const BatchDev &b, const XillWork *work, int n_work, void *stream);
 // relxill requests: the primary continuum added to the output (after launch_conv)
-int launch_primary(const BatchDev &b, const int *reqs, int n_reqs, void *stream);
+// (max_bins: the most caller bins of a request of the list)
+int launch_primary(const BatchDev &b, const int *reqs, int n_reqs, int max_bins, void *stream);
 int launch_copy(const void *src, void *dst, size_t bytes, void *stream);
 
 // ---- nthcomp primary continuum (nthcomp.hip) ----
