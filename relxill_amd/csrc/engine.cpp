@@ -1163,19 +1163,78 @@ void batch_plan(Batch &b, int seg_bins, int waves_per_cu) {
       }
     }
   }
-  if (seg_bins <= 0) seg_bins = 64;
-  if (waves_per_cu <= 0) waves_per_cu = 8;
+  const int n_rc = (g.nr_fine + RAD_CHUNK - 1) / RAD_CHUNK;
+  int64_t windows = 0;
+  int max_bins = 0;
+  for (int i = 0; i < b.n_req; i++) {
+    if (b.h_status[i] != RX_OK || b.h_req[i].n_e <= 0) continue;
+    windows += n_rc + b.h_req[i].n_zones - 1;
+    max_bins = std::max(max_bins, b.h_req[i].n_e);
+  }
+  const WorkShape ws = work_shape(windows, max_bins);
+  if (seg_bins <= 0) seg_bins = ws.seg_bins;
+  if (waves_per_cu <= 0) waves_per_cu = ws.waves_per_cu;
   b.seg_bins = seg_bins;
   b.waves_per_cu = waves_per_cu;
   // work list bound: every (radius chunk, zone) pair of every request covering
-  // all its bins; the zones are contiguous radius ranges, so a request has at
-  // most n_rc + n_zones - 1 such pairs
-  const int n_rc = (g.nr_fine + RAD_CHUNK - 1) / RAD_CHUNK;
+  // all the bins that a radius of the table can reach; the zones are contiguous
+  // radius ranges, so a request has at most n_rc + n_zones - 1 such pairs
+  const int conv_reach = reach_bins(g.conv_ener.data(), g.conv_n, 1.0);
   int64_t cap = 0;
-  for (int i = 0; i < b.n_req; i++)
-    if (b.h_status[i] == RX_OK)
-      cap += (int64_t)(n_rc + b.h_req[i].n_zones - 1) * ((b.h_req[i].n_e + seg_bins - 1) / seg_bins);
+  for (int i = 0; i < b.n_req; i++) {
+    const ReqParams &p = b.h_req[i];
+    if (b.h_status[i] != RX_OK || p.n_e <= 0) continue;
+    const int bins =
+        p.pgrid_off >= 0 ? reach_bins(&b.h_ener[p.ener_off], p.n_e, p.lineE / (p.z > 0 ? 1 + p.z : 1.0)) : conv_reach;
+    cap += (int64_t)(n_rc + p.n_zones - 1) * ((bins + seg_bins - 1) / seg_bins);
+  }
   b.item_cap = (int)std::min<int64_t>(std::max<int64_t>(cap, 1), INT32_MAX);
+  b.n_blocks = integrate_blocks(b.item_cap, windows, waves_per_cu);
+}
+
+WorkShape work_shape(int64_t windows, int max_bins) {
+  // A window is one chunk of radii (and zone) of one request, 16 a request.
+  // Few windows leave the chip idle: short segments give it more, shorter
+  // items, until an item's set-up (about 10 us of latency) is what it does.
+  // Measured, k_integrate in us, FP32 (FP64), relconv, segments of 4 / 8 / 32 /
+  // 64 / 256 bins: 1 request 15 / 17 / 30 / 43 / - (22 / 25 / 48 / 64 / -), 16
+  // requests 32 / 28 / 44 / 53 / - (52 / 52 / 71 / 78 / -), 64 requests - / - /
+  // 53 / 59 / 140 (- / - / 113 / 105 / 210), 256 requests - / - / 132 / 121 / 150
+  // (- / - / 316 / 299 / 304), 1024 requests - / - / 483 / 387 / 345 (- / - / 1045
+  // / 965 / 924); relline and lamp-post requests order the same way.
+  // Grids beyond 16384 bins keep segments of 64 at least, so that their work
+  // list stays small beside the batch's other buffers.
+  WorkShape w;
+  w.waves_per_cu = 12;
+  if (windows <= 64) w.seg_bins = 4;
+  else if (windows <= 512) w.seg_bins = 8;
+  else if (windows <= 2048) w.seg_bins = 32;
+  else if (windows <= 8192) w.seg_bins = 64;
+  else w.seg_bins = 256;
+  if (max_bins > 16384) w.seg_bins = std::max(w.seg_bins, 64);
+  return w;
+}
+
+int reach_bins(const double *ener, int n, double unit) {
+  // the windows lie between the smallest g_min and the largest g_max of the
+  // table's nodes (1 % to either side for the extrapolation at the ISCO); a bin
+  // more at each end for the bins that hold the ends
+  Global &g = G();
+  const double lo = 0.99 * g.rel_gmin_all * unit, hi = 1.01 * g.rel_gmax_all * unit;
+  if (!(hi > lo)) return n;  // (also a NaN or negative unit)
+  const double *a = std::upper_bound(ener, ener + n + 1, lo), *b = std::upper_bound(ener, ener + n + 1, hi);
+  return std::min<int64_t>(n, std::max<int64_t>(b - a, 0) + 2);
+}
+
+int integrate_blocks(int item_cap, int64_t windows, int waves_per_cu) {
+  // up to 8192 windows (512 requests) a workgroup per possible item and no
+  // hand-out (k_integrate's ONE; 256 relconv requests 121 us, 133 us with
+  // persistent wavefronts), beyond that persistent wavefronts, which keep a
+  // request's items on one XCD and take the long ones first (4096 requests
+  // 1250 us, 1304 us with ONE).  Workgroups without an item cost about 0.2 ns
+  // each: at most 2^18 of them.
+  if (windows <= 8192 && item_cap <= (1 << 18)) return std::max(1, item_cap);
+  return (int)std::min<int64_t>((int64_t)G().n_cu * waves_per_cu, std::max(1, item_cap));
 }
 
 int batch_upload(Batch &b) {
@@ -1363,10 +1422,7 @@ int batch_run(Batch &b, int precision, std::string &err) {
   RunKey k;
   memset(&k, 0, sizeof(k));
   k.bd = dev_view(b);
-  // persistent wavefronts: CUs x waves per CU, but no more than the list can
-  // hold items (a small batch -- the server's -- would start thousands that
-  // find the list empty)
-  k.n_blocks = (int)std::min<int64_t>((int64_t)g.n_cu * b.waves_per_cu, std::max(1, b.item_cap));
+  k.n_blocks = b.n_blocks;
   k.n_xill1 = b.n_xill1;
   k.n_xill = (int)b.h_xill.size();
   k.n_conv = (int)b.h_conv.size();

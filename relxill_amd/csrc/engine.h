@@ -59,7 +59,7 @@ struct Batch {
   int max_zones = 1;          // most zones of a request
   int seg_bins = 64;        // bins per work item
   int seg_forced = 0;       // 0: automatic / autotuned
-  int waves_per_cu = 8;     // persistent integration wavefronts per CU
+  int waves_per_cu = 12;    // persistent integration wavefronts per CU
   int waves_forced = 0;
   std::vector<ReqParams> h_req;
   std::vector<int> h_status;  // host-side parse status
@@ -82,6 +82,7 @@ struct Batch {
   DevBuf d_nthw, d_nth, d_nthx, d_nths, d_nthn;
   DevBuf d_items, d_ctr, d_fix, d_reach, d_rnorm, d_rnode;
   int item_cap = 0;
+  int n_blocks = 1;  // workgroups of k_integrate
   bool any_cosne = false, any_limb = false;
   int fix_cap = 0;
   int last_mode = 1;
@@ -110,6 +111,17 @@ int batch_build(Batch &b, const rx_request *req, int n_req, std::string &err);
 // Chooses the work-item segment length and the persistent wavefronts per CU
 // (0: automatic / autotuned) and sizes the work list.
 void batch_plan(Batch &b, int seg_bins, int waves_per_cu);
+// Bins of an energy grid (n + 1 ascending edges) that the window of some radius of
+// the resident table can reach; unit: the grid's energy of g = 1.
+int reach_bins(const double *ener, int n, double unit);
+// Default work shape of a batch: windows (radius chunk x zone, over all requests)
+// and the most bins of a profile grid.
+struct WorkShape {
+  int seg_bins, waves_per_cu;
+};
+WorkShape work_shape(int64_t windows, int max_bins);
+// Workgroups of k_integrate for a work list of that capacity.
+int integrate_blocks(int item_cap, int64_t windows, int waves_per_cu);
 int batch_upload(Batch &b);
 int batch_run(Batch &b, int precision, std::string &err);
 int batch_sync(Batch &b);

@@ -1450,6 +1450,31 @@ __device__ inline const double *profile_grid(const BatchDev &b, const ReqParams 
   return (off >= 0) ? b.pgrid + off : b.cg.ener;
 }
 
+// The bin edges of a work item in turn: one scalar load a bin ahead, or (ONE) the
+// edges of SUM_BINS bins per load, a group ahead.
+template <int ONE>
+struct EdgeWalk {
+  const double *E;
+  double first, next, grp;
+  __device__ void start(const double *grid, const WorkItem &it, int lane) {
+    E = grid;
+    first = E[it.j0];
+    next = E[min(it.j0 + 1 + (ONE ? lane : 0), it.j1)];
+  }
+  __device__ void group(const WorkItem &it, int jg, int lane) {  // bins [jg, jg + SUM_BINS)
+    if constexpr (ONE) {
+      grp = next;  // lane l: the upper edge of the group's bin l
+      next = E[min(jg + SUM_BINS + 1 + lane, it.j1)];
+    }
+  }
+  __device__ double upper(const WorkItem &it, int j, int jj) {  // of bin j, jj-th of its group
+    if constexpr (ONE) return readlane_d(grp, jj);
+    const double e = next;
+    next = E[min(j + 2, it.j1)];
+    return e;
+  }
+};
+
 }  // namespace
 
 // Emission-angle distribution of the requests with one (src/Relprofile.cpp:
@@ -1602,8 +1627,23 @@ __host__ __device__ inline size_t integrate_rows_bytes(int ng, bool cos_rows, si
 //   between items.
 //   COS: the batch holds emission-angle rows (a request with limb
 //   darkening); COS == 0 compiles the limb factors out.
-template <int MODE, int COS>
-__global__ __launch_bounds__(64, MODE == 0 ? 1 : 3) void k_integrate(BatchDev b, int stage_rows) {
+//   ONE: one workgroup per item of the list's capacity, and no hand-out: for
+//   short lists, where a wavefront takes one item anyway and the walk over the
+//   range counters (one atomic each, 8 when it finds them all empty) would be a
+//   third of the kernel's time.  It also loads an item's edges a group ahead.
+//   A single relconv call (segments of 4 bins): 34 us with the counters, 22 us
+//   without (FP32 36 and 15 us); with the segments of 64 bins that every batch
+//   had by default 64 us (43 us).
+template <int MODE, int COS, int ONE>
+__global__ __launch_bounds__(64, MODE == 0 ? 1 : 3) void k_integrate(BatchDev b_arg, int stage_rows) {
+  // The argument is read through a pointer that every item renews, so that the
+  // compiler reads its fields where an item uses them: kept across the item
+  // loop they took 28 scalar registers more than there are, spilled to vector
+  // lanes and read back for every bin (4096 relconv requests: 1259 us, 1250 us
+  // without the spills, FP64 3700 us and 3535 us).
+  typedef const __attribute__((address_space(4))) BatchDev KArg;
+  KArg *bp = (KArg *)__builtin_amdgcn_kernarg_segment_ptr();
+  const BatchDev &b = *(const BatchDev *)bp;
   constexpr int cos_rows = COS;
   using TV = typename std::conditional<MODE == 0, double, float>::type;
   extern __shared__ double s_dyn[];
@@ -1648,7 +1688,12 @@ __global__ __launch_bounds__(64, MODE == 0 ? 1 : 3) void k_integrate(BatchDev b,
     // the short ones); an empty range sends the wavefront to the next one,
     // and once all N_XQ have been found empty it is done
     int k = -1;
-    while (exhausted < N_XQ) {
+    if constexpr (ONE) {
+      const int kk = blockIdx.x;
+      if (kk >= n_long + n_short) return;
+      k = kk < n_long ? kk : b.item_cap - 1 - (kk - n_long);
+    }
+    while (!ONE && exhausted < N_XQ) {
       const int lo = (int)((int64_t)n_long * xq / N_XQ), hi = (int)((int64_t)n_long * (xq + 1) / N_XQ);
       const int los = (int)((int64_t)n_short * xq / N_XQ), his = (int)((int64_t)n_short * (xq + 1) / N_XQ);
       int kk = 0;
@@ -1666,6 +1711,8 @@ __global__ __launch_bounds__(64, MODE == 0 ? 1 : 3) void k_integrate(BatchDev b,
       xq = (xq + 1) % N_XQ;
     }
     if (k < 0) break;
+    if constexpr (!ONE) asm volatile("" : "+s"(bp));
+    const BatchDev &b = *(const BatchDev *)bp;
     const WorkItem it = b.items[k];
     const ReqParams *rq = b.req + it.req;
     const ReqNorm rn = b.rnorm[it.req];
@@ -1685,6 +1732,8 @@ __global__ __launch_bounds__(64, MODE == 0 ? 1 : 3) void k_integrate(BatchDev b,
       rK = rad_K(pr);
       coef = pr.coef;
     }
+    EdgeWalk<ONE> ew;
+    if constexpr (ONE) ew.start(profile_grid(b, rq), it, lane);
     const bool has_win = ielo <= iehi;
     RadGeo r = {0.0, 0.0, 0.0};
     if (has_win) {
@@ -1755,20 +1804,19 @@ __global__ __launch_bounds__(64, MODE == 0 ? 1 : 3) void k_integrate(BatchDev b,
     const double w32 = has_win ? coef * rn.cmul : 0.0;  // MODE 1 scaled weight
     const float w32f = (float)w32;
     if constexpr (MODE == 0) s_coef[lane] = w64;
-    const double *E = profile_grid(b, rq);
+    if constexpr (!ONE) ew.start(profile_grid(b, rq), it, lane);
     double *acc = profile_acc(b, *rq) + (size_t)zone * rq->n_e;
-    double ehi = E[it.j0];
-    double enext = E[min(it.j0 + 1, it.j1)];
+    double ehi = ew.first;
     double ghi = (ehi - v.gmin) * v.del_g;  // unclamped g* of the bin's upper edge, carried
     EdgePair<TV> cy;  // integrand pair at the next bin's lower edge, when a Romberg bin left it
     cy.ok = false;
     for (int jg = it.j0; jg < it.j1; jg += SUM_BINS) {
       const int jn = min(SUM_BINS, it.j1 - jg);
+      ew.group(it, jg, lane);
       for (int jj = 0; jj < jn; jj++) {
         const int j = jg + jj;
         const double elo = ehi, glo = ghi;
-        ehi = enext;
-        enext = E[min(j + 2, it.j1)];  // next bin's upper edge, loaded a bin ahead
+        ehi = ew.upper(it, j, jj);
         ghi = (ehi - v.gmin) * v.del_g;
         TV val = 0;
         if (j >= ielo && j <= iehi) {
@@ -1818,6 +1866,7 @@ __global__ __launch_bounds__(64, MODE == 0 ? 1 : 3) void k_integrate(BatchDev b,
       if (part == 0 && col < jn) unsafeAtomicAdd(&acc[jg + col], sum);
       __syncthreads();  // the next bins overwrite the parked values
     }
+    if constexpr (ONE) return;
   }
 }
 
@@ -2827,12 +2876,13 @@ int launch_integrate(const BatchDev &b, int n_blocks, bool cos_rows, void *strea
     (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     hipLaunchKernelGGL(kern, dim3(n_blocks), dim3(64), lds, st, b, stage);
   };
+  const bool one = n_blocks >= b.item_cap;  // a workgroup for every item there can be
   if (b.mode == 0) {
-    if (cos_rows) go(k_integrate<0, 1>);
-    else go(k_integrate<0, 0>);
+    if (one) cos_rows ? go(k_integrate<0, 1, 1>) : go(k_integrate<0, 0, 1>);
+    else cos_rows ? go(k_integrate<0, 1, 0>) : go(k_integrate<0, 0, 0>);
   } else {
-    if (cos_rows) go(k_integrate<1, 1>);
-    else go(k_integrate<1, 0>);
+    if (one) cos_rows ? go(k_integrate<1, 1, 1>) : go(k_integrate<1, 0, 1>);
+    else cos_rows ? go(k_integrate<1, 1, 0>) : go(k_integrate<1, 0, 0>);
   }
   return (int)hipGetLastError();
 }

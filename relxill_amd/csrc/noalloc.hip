@@ -152,10 +152,13 @@ int noalloc_eval(int model, const double *parameter, const double *d_energy, con
       seg = t.seg_bins;
       wpc = t.waves_per_cu;
     }
-  if (seg <= 0) seg = 64;
-  if (wpc <= 0) wpc = 8;
   const int n_rc = (g.nr_fine + RAD_CHUNK - 1) / RAD_CHUNK;
-  const int item_cap = n_rc * ((p.n_e + seg - 1) / seg);
+  const WorkShape ws = work_shape(n_rc, p.n_e);
+  if (seg <= 0) seg = ws.seg_bins;
+  if (wpc <= 0) wpc = ws.waves_per_cu;
+  // (a caller's line grid is on the device: all its bins)
+  const int bins = conv ? reach_bins(g.conv_ener.data(), g.conv_n, 1.0) : p.n_e;
+  const int item_cap = n_rc * ((bins + seg - 1) / seg);
   const int fix_cap = std::max(4096, p.n_e * 4);
 
   BatchDev bd;
@@ -199,7 +202,7 @@ int noalloc_eval(int model, const double *parameter, const double *d_energy, con
   e |= (int)hipMemcpyAsync(bd.status, &p.pre_status, sizeof(int), hipMemcpyHostToDevice, s);
   e |= (int)hipMemcpyAsync(d_work, &w0, sizeof(w0), hipMemcpyHostToDevice, s);
   const bool cos_rows = p.limb != 0;
-  const int n_blocks = std::min(g.n_cu * wpc, std::max(1, item_cap));  // no more wavefronts than items
+  const int n_blocks = integrate_blocks(item_cap, n_rc, wpc);
   int out[2] = {0, 0};  // status, FP64 re-check queue overflow
   for (int pass = 0; pass < 2 && e == 0; pass++) {
     bd.mode = (pass == 0 && precision == RX_FP32) ? 1 : 0;

@@ -39,7 +39,8 @@ namespace {
 using Clock = std::chrono::steady_clock;
 
 // work-list sizing bound of the admission estimate (the smallest segment
-// length the autotuner may choose)
+// length the autotuner may choose; the default shape's shorter segments are for
+// batches of at most 32 requests, a few 100 KB a slot)
 constexpr int SERVER_MIN_SEG_BINS = 32;
 
 struct Pending {
