@@ -28,5 +28,7 @@ __all__ = sorted(_LIB_NAMES)
 def __getattr__(name):
     if name in _LIB_NAMES:
         import importlib
-        return getattr(importlib.import_module(".capi", __name__), name)
+        value = getattr(importlib.import_module(".capi", __name__), name)
+        globals()[name] = value  # resolved once: the import system takes 4 us a look-up
+        return value
     raise AttributeError(name)

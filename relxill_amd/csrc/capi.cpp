@@ -50,18 +50,20 @@ int eval_one(int model, const double *parameter, const double *energy, double *f
   r.flux_in = flux;
   r.refl_set = -1;
   Batch &b = plain_batch();
+  b.is_call = b.keep_stage = true;
   st = batch_build(b, &r, 1, err);
   if (st == RX_OK) st = batch_run(b, precision, err);
   if (st == RX_OK) st = batch_sync(b);
   if (st == RX_OK) {
-    if (hipMemcpy(flux, b.d_out.p, sizeof(double) * n_flux, hipMemcpyDeviceToHost) != hipSuccess) {
+    if (b.call_run) {
+      memcpy(flux, result_out(b), sizeof(double) * n_flux);
+    } else if (hipMemcpy(flux, b.dev.out, sizeof(double) * n_flux, hipMemcpyDeviceToHost) != hipSuccess) {
       st = RX_ERR_DEVICE;
       err = "device to host copy failed";
     }
   }
   if (st == RX_OK) {
-    int dst = 0;
-    if (hipMemcpy(&dst, b.d_status.p, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess) dst = RX_ERR_DEVICE;
+    const int dst = result_status(b)[0];
     if (dst != 0) {
       st = public_status(dst);
       err = "model evaluation failed (status " + std::to_string(dst) + ")";
@@ -582,19 +584,27 @@ int rx_batch_sync(rx_batch *b) {
 
 int rx_batch_status(rx_batch *b, int i) {
   if (!b || i < 0 || i >= b->b.n_req) return RX_ERR_ARG;
-  int st = 0;
-  if (hipMemcpy(&st, b->b.d_status.as<int>() + i, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess)
-    return RX_ERR_DEVICE;
-  return public_status(st);
+  Batch &bb = b->b;
+  std::lock_guard<std::mutex> lk(bb.out_mu);
+  if (!bb.synced) {
+    if (hipStreamSynchronize(bb.stream) != hipSuccess) return RX_ERR_DEVICE;
+    bb.synced = true;
+  }
+  return public_status(result_status(bb)[i]);
 }
 
 int rx_batch_output(rx_batch *b, int i, double *flux) {
   if (!b || !flux || i < 0 || i >= b->b.n_req) return RX_ERR_ARG;
-  const ReqParams &p = b->b.h_req[i];
-  if (hipMemcpy(flux, b->b.d_out.as<double>() + p.flux_off, sizeof(double) * p.n_in,
-                hipMemcpyDeviceToHost) != hipSuccess)
-    return RX_ERR_DEVICE;
-  return rx_batch_status(b, i);
+  Batch &bb = b->b;
+  const ReqParams &p = bb.h_req[i];
+  std::lock_guard<std::mutex> lk(bb.out_mu);
+  try {
+    const int st = batch_read(bb, p.flux_off, p.n_in, flux);
+    if (st != RX_OK) return st;
+  } catch (...) {
+    return RX_ERR_NOMEM;
+  }
+  return public_status(result_status(bb)[i]);
 }
 
 int rx_batch_dist(rx_batch *b, int i, double *dist, int n_incl) {
@@ -602,7 +612,7 @@ int rx_batch_dist(rx_batch *b, int i, double *dist, int n_incl) {
   const ReqParams &p = b->b.h_req[i];
   if (n_incl > p.n_incl * p.n_zones) return RX_ERR_ARG;
   if (n_incl == 0) return RX_OK;
-  if (hipMemcpy(dist, b->b.d_dist.as<double>() + p.dist_off, sizeof(double) * n_incl,
+  if (hipMemcpy(dist, b->b.dev.dist + p.dist_off, sizeof(double) * n_incl,
                 hipMemcpyDeviceToHost) != hipSuccess)
     return RX_ERR_DEVICE;
   return RX_OK;
@@ -615,7 +625,7 @@ int rx_batch_zones(rx_batch *b, int i, double *out, int n_zones) {
   if (n_zones > p.n_zones) return RX_ERR_ARG;
   if (n_zones == 0) return RX_OK;
   std::vector<ZoneRec> z(n_zones);
-  if (hipMemcpy(z.data(), b->b.d_zone.as<ZoneRec>() + p.zone_off, sizeof(ZoneRec) * n_zones,
+  if (hipMemcpy(z.data(), b->b.dev.zone + p.zone_off, sizeof(ZoneRec) * n_zones,
                 hipMemcpyDeviceToHost) != hipSuccess)
     return RX_ERR_DEVICE;
   for (int k = 0; k < n_zones; k++) {
@@ -635,7 +645,7 @@ int rx_batch_zones(rx_batch *b, int i, double *out, int n_zones) {
 int rx_batch_reflfrac(rx_batch *b, int i, double *out5) {
   if (!b || !out5 || i < 0 || i >= b->b.n_req) return RX_ERR_ARG;
   LpRefl r;
-  if (hipMemcpy(&r, b->b.d_refl.as<LpRefl>() + i, sizeof(LpRefl), hipMemcpyDeviceToHost) != hipSuccess)
+  if (hipMemcpy(&r, b->b.dev.refl + i, sizeof(LpRefl), hipMemcpyDeviceToHost) != hipSuccess)
     return RX_ERR_DEVICE;
   out5[0] = r.refl_frac;
   out5[1] = r.f_bh;

@@ -38,6 +38,24 @@ DevBuf::~DevBuf() {
   if (p) (void)hipFree(p);
 }
 
+PinnedBuf::~PinnedBuf() {
+  if (p) (void)hipHostFree(p);
+}
+
+bool PinnedBuf::ensure(size_t n) {
+  if (p && bytes >= n) return true;
+  if (p) n = std::max(n, bytes + bytes / 2);  // grows rarely (hipHostFree synchronises)
+  if (p) (void)hipHostFree(p);
+  p = nullptr;
+  bytes = 0;
+  if (hipHostMalloc(&p, n, hipHostMallocDefault) != hipSuccess) {
+    p = nullptr;
+    return false;
+  }
+  bytes = n;
+  return true;
+}
+
 int DevBuf::ensure(size_t n) {
   if (n == 0) n = 8;
   if (p && bytes >= n) return 0;
@@ -884,6 +902,38 @@ static CpRequest remap_cp(int model, const double *par) {
   return c;
 }
 
+// Request blocks up to STAGE_MAX go to the device through pinned memory in one
+// piece (of a server slot, which keeps its pinned memory: up to STAGE_KEEP);
+// larger ones piece by piece from the batch's own arrays, a copy less.
+constexpr size_t STAGE_MAX = 4u << 20, STAGE_KEEP = 32u << 20;
+
+static size_t align_up(size_t n) { return (n + 255) & ~(size_t)255; }
+
+// Offsets of the request block's pieces.
+static void layout_block(Batch &b) {
+  size_t used = 0;
+  auto put = [&](size_t bytes) {
+    const size_t at = used;
+    used += align_up(std::max<size_t>(bytes, 1));
+    return at;
+  };
+  auto list = [&](const auto &v) { return put(sizeof(v[0]) * v.size()); };
+  Batch::BlockOffsets &o = b.off;
+  o.req = list(b.h_req);
+  o.status = list(b.h_status);
+  o.conv = list(b.h_conv);
+  o.xill = list(b.h_xill);
+  o.prim = list(b.h_prim);
+  o.zone = list(b.h_zone);
+  o.ang = list(b.h_ang);
+  o.rrc = list(b.h_rrc);
+  o.rrad = list(b.h_rrad);
+  o.nth = list(b.h_nth);
+  o.ener = put(sizeof(double) * b.tot_ener);
+  o.flux = put(b.any_flux ? sizeof(double) * b.tot_flux : 0);
+  b.block_bytes = used;
+}
+
 int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err) {
   Global &g = G();
   if (n_req <= 0 || !req_in) {
@@ -1122,19 +1172,38 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
   std::stable_sort(b.h_conv.begin(), b.h_conv.end(), [&](const XillWork &x, const XillWork &y) {
     return b.h_req[x.req].n_in > b.h_req[y.req].n_in;
   });
-  b.h_ener.resize(o_ener);
-  b.h_flux_in.assign(o_flux, 0.0);
+  b.any_flux = false;
+  for (int i = 0; i < n_req; i++) b.any_flux |= req[i].flux_in && is_conv(req[i].model) && !is_relxill(req[i].model);
+  // the grids and input spectra: into the request block's pinned memory where the
+  // batch keeps its own (a call, a server slot), else into the batch's arrays
+  const int64_t n_fin = b.any_flux ? o_flux : 0;
+  layout_block(b);
+  b.staged = b.block_bytes <= (b.is_call ? STAGE_MAX : b.keep_stage ? STAGE_KEEP : STAGE_MAX);
+  if (b.keep_stage && b.staged) {
+    if (!b.h_stage.ensure(std::max<size_t>(b.block_bytes, b.one_shot ? STAGE_MAX : 0))) {
+      err = "pinned host allocation failed";
+      return RX_ERR_NOMEM;
+    }
+    b.p_ener = reinterpret_cast<double *>(b.h_stage.as<char>() + b.off.ener);
+    b.p_flux = reinterpret_cast<double *>(b.h_stage.as<char>() + b.off.flux);
+  } else {
+    b.h_ener.resize(o_ener);
+    b.h_flux_in.resize(n_fin);
+    b.p_ener = b.h_ener.data();
+    b.p_flux = b.h_flux_in.data();
+  }
   for (int i = 0; i < n_req; i++) {
     const rx_request &r = req[i];
     const ReqParams &p = b.h_req[i];
-    memcpy(&b.h_ener[p.ener_off], r.energy, sizeof(double) * (r.n_flux + 1));
+    memcpy(b.p_ener + p.ener_off, r.energy, sizeof(double) * (r.n_flux + 1));
     if ((is_relxill(r.model) || r.model == MOD_XILLVER) && p.z > 0) {
       // relxill evaluates on the redshifted grid (shift_energy_grid_redshift,
       // src/XspecSpectrum.h:70-76)
-      for (int k = 0; k <= r.n_flux; k++) b.h_ener[p.ener_off + k] *= (1 + p.z);
+      for (int k = 0; k <= r.n_flux; k++) b.p_ener[p.ener_off + k] *= (1 + p.z);
     }
+    // (k_conv reads the input of requests that have one only)
     if (r.flux_in && is_conv(r.model) && !is_relxill(r.model))
-      memcpy(&b.h_flux_in[p.flux_off], r.flux_in, sizeof(double) * r.n_flux);
+      memcpy(b.p_flux + p.flux_off, r.flux_in, sizeof(double) * r.n_flux);
   }
   b.any_cosne = false;
   b.any_limb = false;
@@ -1185,7 +1254,7 @@ void batch_plan(Batch &b, int seg_bins, int waves_per_cu) {
     const ReqParams &p = b.h_req[i];
     if (b.h_status[i] != RX_OK || p.n_e <= 0) continue;
     const int bins =
-        p.pgrid_off >= 0 ? reach_bins(&b.h_ener[p.ener_off], p.n_e, p.lineE / (p.z > 0 ? 1 + p.z : 1.0)) : conv_reach;
+        p.pgrid_off >= 0 ? reach_bins(b.p_ener + p.ener_off, p.n_e, p.lineE / (p.z > 0 ? 1 + p.z : 1.0)) : conv_reach;
     cap += (int64_t)(n_rc + p.n_zones - 1) * ((bins + seg_bins - 1) / seg_bins);
   }
   b.item_cap = (int)std::min<int64_t>(std::max<int64_t>(cap, 1), INT32_MAX);
@@ -1221,7 +1290,9 @@ int reach_bins(const double *ener, int n, double unit) {
   // more at each end for the bins that hold the ends
   Global &g = G();
   const double lo = 0.99 * g.rel_gmin_all * unit, hi = 1.01 * g.rel_gmax_all * unit;
-  if (!(hi > lo)) return n;  // (also a NaN or negative unit)
+  bool ascending = hi > lo;  // (not with a NaN or negative unit)
+  for (int k = 0; k < n; k++) ascending &= ener[k] < ener[k + 1];
+  if (!ascending) return n;
   const double *a = std::upper_bound(ener, ener + n + 1, lo), *b = std::upper_bound(ener, ener + n + 1, hi);
   return std::min<int64_t>(n, std::max<int64_t>(b - a, 0) + 2);
 }
@@ -1245,67 +1316,119 @@ int batch_upload(Batch &b) {
     for (auto &x : b.ev) e |= (int)hipEventCreate(&x);
   }
   const size_t nreq = b.n_req;
-  e |= b.d_req.ensure(sizeof(ReqParams) * nreq);
-  e |= b.d_ener.ensure(sizeof(double) * b.tot_ener);
-  e |= b.d_flux_in.ensure(sizeof(double) * b.tot_flux);
-  e |= b.d_out.ensure(sizeof(double) * b.tot_flux);
-  e |= b.d_pgrid.ensure(sizeof(double) * std::max<int64_t>(1, b.tot_pgrid));
-  e |= b.d_rad.ensure(sizeof(RadRec) * nreq * g.nr_fine);
-  e |= b.d_rnode.ensure(sizeof(double) * RAD_NODE_ARRAYS * nreq * g.rel.n_r);
-  e |= b.d_rnorm.ensure(sizeof(ReqNorm) * nreq);
-  e |= b.d_prof.ensure(sizeof(double) * std::max<int64_t>(1, b.tot_prof));
-  e |= b.d_dist.ensure(sizeof(double) * std::max<int64_t>(1, b.tot_dist));
-  e |= b.d_zone.ensure(sizeof(ZoneRec) * std::max<int64_t>(1, b.tot_zone));
-  e |= b.d_refl.ensure(sizeof(LpRefl) * nreq);
-  e |= b.d_status.ensure(sizeof(int) * nreq);
-  e |= b.d_conv.ensure(sizeof(XillWork) * std::max<size_t>(1, b.h_conv.size()));
-  e |= b.d_xill.ensure(sizeof(XillWork) * std::max<size_t>(1, b.h_xill.size()));
-  e |= b.d_prim.ensure(sizeof(int) * std::max<size_t>(1, b.h_prim.size()));
-  e |= b.d_zonew.ensure(sizeof(XillWork) * std::max<size_t>(1, b.h_zone.size()));
-  e |= b.d_ang.ensure(sizeof(int) * std::max<size_t>(1, b.h_ang.size()));
-  e |= b.d_rrc.ensure(sizeof(int) * std::max<size_t>(1, b.h_rrc.size()));
-  e |= b.d_rrad.ensure(sizeof(int) * std::max<size_t>(1, b.h_rrad.size()));
-  e |= b.d_rrpart.ensure(sizeof(double) * std::max<int64_t>(1, b.tot_rrc));
-  e |= b.d_rret.ensure(sizeof(double) * 2 * MAX_RR * std::max<size_t>(1, b.h_rrad.size()));
-  e |= b.d_nthw.ensure(sizeof(XillWork) * std::max<size_t>(1, b.h_nth.size()));
-  e |= b.d_nth.ensure(sizeof(NthRes) * std::max<size_t>(1, b.h_nth.size()));
-  e |= b.d_nthx.ensure(sizeof(double) * (NTH_MAX_POINTS + 1) * std::max(1, b.n_nth_sol));
-  e |= b.d_nths.ensure(sizeof(double) * NTH_MAX_POINTS * std::max(1, b.n_nth_sol));
-  e |= b.d_nthn.ensure(sizeof(int) * std::max(1, b.n_nth_sol));
-  e |= b.d_xspec.ensure(sizeof(double) * std::max<int64_t>(1, b.tot_xspec));
-  e |= b.d_items.ensure(sizeof(WorkItem) * (size_t)b.item_cap);
-  e |= b.d_ctr.ensure(sizeof(int) * N_COUNTERS);
-  e |= b.d_reach.ensure(sizeof(BinRange) * nreq);
+  size_t used = b.block_bytes;  // the request block, then what the kernels write
+  auto take = [&](size_t bytes) {
+    const size_t at = used;
+    used += align_up(std::max<size_t>(bytes, 1));
+    return at;
+  };
+  const size_t o_ctr = take(sizeof(int) * N_COUNTERS), o_out = take(sizeof(double) * b.tot_flux),
+               o_pgrid = take(sizeof(double) * b.tot_pgrid), o_rad = take(sizeof(RadRec) * nreq * g.nr_fine),
+               o_rnode = take(sizeof(double) * RAD_NODE_ARRAYS * nreq * g.rel.n_r),
+               o_rnorm = take(sizeof(ReqNorm) * nreq), o_prof = take(sizeof(double) * b.tot_prof),
+               o_dist = take(sizeof(double) * b.tot_dist), o_zone = take(sizeof(ZoneRec) * b.tot_zone),
+               o_refl = take(sizeof(LpRefl) * nreq), o_rrpart = take(sizeof(double) * b.tot_rrc),
+               o_rret = take(sizeof(double) * 2 * MAX_RR * b.h_rrad.size()),
+               o_nth = take(sizeof(NthRes) * b.h_nth.size()),
+               o_nthx = take(sizeof(double) * (NTH_MAX_POINTS + 1) * b.n_nth_sol),
+               o_nths = take(sizeof(double) * NTH_MAX_POINTS * b.n_nth_sol), o_nthn = take(sizeof(int) * b.n_nth_sol),
+               o_xspec = take(sizeof(double) * b.tot_xspec),
+               o_items = take(sizeof(WorkItem) * (size_t)b.item_cap), o_reach = take(sizeof(BinRange) * nreq);
   // FP64 re-check queue: a few percent of the bins (overflow redoes the batch in FP64)
   int64_t bins = 0;
   for (int i = 0; i < b.n_req; i++) bins += b.h_req[i].n_e;
   b.fix_cap = (int)std::min<int64_t>(1 << 22, std::max<int64_t>(1 << 16, bins / 8));
-  e |= b.d_fix.ensure(sizeof(FixEntry) * (size_t)b.fix_cap);
+  const size_t o_fix = take(sizeof(FixEntry) * (size_t)b.fix_cap);
+  e |= b.d_arena.ensure(used);
+  b.call_run = b.is_call && b.staged && sizeof(double) * b.tot_flux <= STAGE_MAX;
+  if (b.call_run) b.deliver_out = b.tot_flux;
+  else if (b.is_call) b.deliver_out = 0;
+  if (!b.h_res.ensure(result_out_offset(b.n_req) + sizeof(double) * b.deliver_out)) e |= 1;
   if (e) return RX_ERR_NOMEM;
-  e |= (int)hipMemcpyAsync(b.d_req.p, b.h_req.data(), sizeof(ReqParams) * nreq, hipMemcpyHostToDevice, b.stream);
-  e |= (int)hipMemcpyAsync(b.d_ener.p, b.h_ener.data(), sizeof(double) * b.tot_ener, hipMemcpyHostToDevice, b.stream);
-  e |= (int)hipMemcpyAsync(b.d_flux_in.p, b.h_flux_in.data(), sizeof(double) * b.tot_flux, hipMemcpyHostToDevice, b.stream);
-  e |= (int)hipMemcpyAsync(b.d_status.p, b.h_status.data(), sizeof(int) * nreq, hipMemcpyHostToDevice, b.stream);
-  if (!b.h_conv.empty())
-    e |= (int)hipMemcpyAsync(b.d_conv.p, b.h_conv.data(), sizeof(XillWork) * b.h_conv.size(), hipMemcpyHostToDevice,
-                             b.stream);
-  if (!b.h_rrc.empty())
-    e |= (int)hipMemcpyAsync(b.d_rrc.p, b.h_rrc.data(), sizeof(int) * b.h_rrc.size(), hipMemcpyHostToDevice, b.stream);
-  if (!b.h_rrad.empty())
-    e |= (int)hipMemcpyAsync(b.d_rrad.p, b.h_rrad.data(), sizeof(int) * b.h_rrad.size(), hipMemcpyHostToDevice, b.stream);
-  if (!b.h_prim.empty())
-    e |= (int)hipMemcpyAsync(b.d_prim.p, b.h_prim.data(), sizeof(int) * b.h_prim.size(), hipMemcpyHostToDevice, b.stream);
-  if (!b.h_zone.empty())
-    e |= (int)hipMemcpyAsync(b.d_zonew.p, b.h_zone.data(), sizeof(XillWork) * b.h_zone.size(), hipMemcpyHostToDevice,
-                             b.stream);
-  if (!b.h_ang.empty())
-    e |= (int)hipMemcpyAsync(b.d_ang.p, b.h_ang.data(), sizeof(int) * b.h_ang.size(), hipMemcpyHostToDevice, b.stream);
-  if (!b.h_xill.empty())
-    e |= (int)hipMemcpyAsync(b.d_xill.p, b.h_xill.data(), sizeof(XillWork) * b.h_xill.size(), hipMemcpyHostToDevice,
-                             b.stream);
-  if (!b.h_nth.empty())
-    e |= (int)hipMemcpyAsync(b.d_nthw.p, b.h_nth.data(), sizeof(XillWork) * b.h_nth.size(), hipMemcpyHostToDevice,
-                             b.stream);
+  char *base = b.d_arena.as<char>();
+  auto at = [&](auto *&ptr, size_t off) { ptr = reinterpret_cast<std::remove_reference_t<decltype(ptr)>>(base + off); };
+  BatchDev &d = b.dev;
+  memset(&d, 0, sizeof(d));
+  d.n_req = b.n_req;
+  d.nr_fine = g.nr_fine;
+  d.seg_bins = b.seg_bins;
+  d.max_zones = b.max_zones;
+  d.item_cap = b.item_cap;
+  d.fix_cap = b.fix_cap;
+  at(d.req, b.off.req);
+  at(d.status, b.off.status);
+  at(d.ener_in, b.off.ener);
+  at(d.flux_in, b.off.flux);
+  at(d.ctr, o_ctr);
+  at(d.out, o_out);
+  at(d.pgrid, o_pgrid);
+  at(d.rad, o_rad);
+  at(d.rnode, o_rnode);
+  at(d.rnorm, o_rnorm);
+  at(d.prof, o_prof);
+  at(d.dist, o_dist);
+  at(d.zone, o_zone);
+  at(d.refl, o_refl);
+  at(d.rrpart, o_rrpart);
+  at(d.rret, o_rret);
+  at(d.nth, o_nth);
+  at(d.nth_x, o_nthx);
+  at(d.nth_s, o_nths);
+  at(d.nth_n, o_nthn);
+  at(d.xspec, o_xspec);
+  at(d.items, o_items);
+  at(d.reach, o_reach);
+  at(d.fix, o_fix);
+  WorkLists &w = b.wl;
+  memset(&w, 0, sizeof(w));
+  at(w.conv, b.off.conv);
+  at(w.xill, b.off.xill);
+  at(w.prim, b.off.prim);
+  at(w.zone, b.off.zone);
+  at(w.ang, b.off.ang);
+  at(w.rrc, b.off.rrc);
+  at(w.rrad, b.off.rrad);
+  at(w.nth, b.off.nth);
+  w.n_conv = (int)b.h_conv.size();
+  w.n_xill = (int)b.h_xill.size();
+  w.n_xill1 = b.n_xill1;
+  w.n_prim = (int)b.h_prim.size();
+  w.n_zone = (int)b.h_zone.size();
+  w.n_ang = (int)b.h_ang.size();
+  w.n_rrc = (int)b.h_rrc.size();
+  w.n_rrad = (int)b.h_rrad.size();
+  w.n_nth = (int)b.h_nth.size();
+  memset(result_ctr(b), 0, sizeof(int) * RES_CTR);
+  memcpy(result_status(b), b.h_status.data(), sizeof(int) * nreq);
+  b.win[0].lo = b.win[0].hi = b.win[1].lo = b.win[1].hi = 0;
+  b.win_next = -1;
+  // the request block to the device: in one piece through pinned memory (a
+  // call's run fetches it from there), or piece by piece where it is large
+  struct Piece {
+    size_t at;
+    const void *src;
+    size_t bytes;
+  };
+  auto piece = [](size_t at, const auto &v) { return Piece{at, v.data(), sizeof(v[0]) * v.size()}; };
+  const Batch::BlockOffsets &o = b.off;
+  const Piece pieces[] = {piece(o.req, b.h_req),   piece(o.status, b.h_status), piece(o.conv, b.h_conv),
+                          piece(o.xill, b.h_xill), piece(o.prim, b.h_prim),     piece(o.zone, b.h_zone),
+                          piece(o.ang, b.h_ang),   piece(o.rrc, b.h_rrc),       piece(o.rrad, b.h_rrad),
+                          piece(o.nth, b.h_nth),   piece(o.ener, b.h_ener),     piece(o.flux, b.h_flux_in)};
+  if (b.staged) {
+    PinnedBuf &stage = b.keep_stage ? b.h_stage : g.stage;
+    if (!b.keep_stage && !stage.ensure(STAGE_MAX)) return RX_ERR_NOMEM;
+    // (a batch that keeps its pinned memory has the grids and inputs there already)
+    const int n = (int)(sizeof pieces / sizeof pieces[0]) - (b.keep_stage ? 2 : 0);
+    for (int k = 0; k < n; k++)
+      if (pieces[k].bytes) memcpy(stage.as<char>() + pieces[k].at, pieces[k].src, pieces[k].bytes);
+    if (b.call_run) return RX_OK;
+    e |= (int)hipMemcpyAsync(base, stage.p, b.block_bytes, hipMemcpyHostToDevice, b.stream);
+    if (b.keep_stage) return e ? RX_ERR_DEVICE : RX_OK;  // (not written again before the run has been waited for)
+  } else {
+    for (const Piece &p : pieces)
+      if (p.bytes) e |= (int)hipMemcpyAsync(base + p.at, p.src, p.bytes, hipMemcpyHostToDevice, b.stream);
+  }
   e |= (int)hipStreamSynchronize(b.stream);
   return e ? RX_ERR_DEVICE : RX_OK;
 }
@@ -1313,41 +1436,67 @@ int batch_upload(Batch &b) {
 static BatchDev dev_view(Batch &b) {
   Global &g = G();
   BatchDev bd;
-  memset(&bd, 0, sizeof(bd));
-  bd.n_req = b.n_req;
-  bd.nr_fine = g.nr_fine;
-  bd.seg_bins = b.seg_bins;
-  bd.max_zones = b.max_zones;
-  bd.req = b.d_req.as<ReqParams>();
-  bd.ener_in = b.d_ener.as<double>();
-  bd.flux_in = b.d_flux_in.as<double>();
-  bd.out = b.d_out.as<double>();
-  bd.pgrid = b.d_pgrid.as<double>();
-  bd.rad = b.d_rad.as<RadRec>();
-  bd.rnode = b.d_rnode.as<double>();
-  bd.rnorm = b.d_rnorm.as<ReqNorm>();
-  bd.prof = b.d_prof.as<double>();
-  bd.dist = b.d_dist.as<double>();
-  bd.refl = b.d_refl.as<LpRefl>();
-  bd.status = b.d_status.as<int>();
-  bd.items = b.d_items.as<WorkItem>();
-  bd.item_cap = b.item_cap;
-  bd.ctr = b.d_ctr.as<int>();
-  bd.reach = b.d_reach.as<BinRange>();
-  bd.fix = b.d_fix.as<FixEntry>();
-  bd.fix_cap = b.fix_cap;
+  memcpy(&bd, &b.dev, sizeof(bd));  // (padding included: run keys compare bytes)
   bd.mode = b.last_mode;
   bd.guard = g.guard;
   fill_dev_views(bd);
-  bd.xspec = b.d_xspec.as<double>();
-  bd.zone = b.d_zone.as<ZoneRec>();
-  bd.rrpart = b.d_rrpart.as<double>();
-  bd.rret = b.d_rret.as<double>();
-  bd.nth = b.d_nth.as<NthRes>();
-  bd.nth_x = b.d_nthx.as<double>();
-  bd.nth_s = b.d_nths.as<double>();
-  bd.nth_n = b.d_nthn.as<int>();
   return bd;
+}
+
+int batch_read(Batch &b, int64_t off, int64_t n, double *to) {
+  // sequential readers (all outputs of a run, one after the other) find theirs in
+  // a window of the output array that one copy brought over, while the next
+  // window is on its way; the first and any stray read take little more than
+  // what they ask for
+  constexpr int64_t FIRST = 1 << 14, MOST = 1 << 18;  // values: 128 KB, 2 MB
+  if (!b.synced) {
+    if (hipStreamSynchronize(b.stream) != hipSuccess) return RX_ERR_DEVICE;
+    b.synced = true;
+  }
+  const int64_t total = b.tot_flux;
+  auto fill = [&](Batch::OutWindow &w, int64_t lo, int64_t len) {
+    len = std::min(len, total - lo);
+    w.lo = w.hi = 0;
+    if (len <= 0) return RX_OK;
+    if (!w.buf.ensure(sizeof(double) * std::min(MOST, total))) return RX_ERR_NOMEM;
+    if (hipMemcpyAsync(w.buf.p, b.dev.out + lo, sizeof(double) * len, hipMemcpyDeviceToHost, b.stream) != hipSuccess)
+      return RX_ERR_DEVICE;
+    w.lo = lo;
+    w.hi = lo + len;
+    w.pending = true;
+    return RX_OK;
+  };
+  const bool seq = off == b.win_next;
+  if (!seq) b.win_len = 0;
+  b.win_next = off + n;
+  while (n > 0) {
+    Batch::OutWindow *w = &b.win[b.win_cur];
+    if (!(off >= w->lo && off < w->hi)) {
+      b.win_cur ^= 1;
+      w = &b.win[b.win_cur];
+    }
+    if (!(off >= w->lo && off < w->hi)) {
+      b.win_len = std::min(MOST, std::max(seq ? FIRST : 0, std::max(n, 2 * b.win_len)));
+      if (const int st = fill(*w, off, b.win_len)) return st;
+    }
+    if (w->pending) {
+      // (the stream holds copies only: the run's kernels were waited for)
+      if (hipStreamSynchronize(b.stream) != hipSuccess) return RX_ERR_DEVICE;
+      b.win[0].pending = b.win[1].pending = false;
+      // a sequential reader's next window
+      Batch::OutWindow &o = b.win[b.win_cur ^ 1];
+      if (seq && w->hi < total) {
+        b.win_len = std::min(MOST, 2 * b.win_len);
+        if (const int st = fill(o, w->hi, b.win_len)) return st;
+      }
+    }
+    const int64_t m = std::min(n, w->hi - off);
+    memcpy(to, w->buf.as<double>() + (off - w->lo), sizeof(double) * m);
+    to += m;
+    off += m;
+    n -= m;
+  }
+  return RX_OK;
 }
 
 // The run's kernels in stream order (events around them when profiling).
@@ -1355,25 +1504,28 @@ static int launch_sequence(Batch &b, const RunKey &k, hipStream_t s) {
   const BatchDev &bd = k.bd;
   const bool prof = k.prof != 0;
   int e = 0;
+  const WorkLists &w = k.wl;
   if (prof) e |= (int)hipEventRecord(b.ev[0], s);
-  e |= launch_nth(bd, static_cast<const XillWork *>(k.d_nth), k.n_nth, s);
-  e |= launch_zone(bd, static_cast<const XillWork *>(k.d_zone), k.n_zone, s);
-  e |= launch_rrad(bd, static_cast<const int *>(k.d_rrc), k.n_rrc, static_cast<const int *>(k.d_rrad), k.n_rrad, s);
+  e |= launch_begin(bd.ctr, k.fetch_src, k.fetch_dst, k.n_fetch, s);
+  e |= launch_nth(bd, w.nth, w.n_nth, s);
+  e |= launch_zone(bd, w.zone, w.n_zone, s);
+  e |= launch_rrad(bd, w.rrc, w.n_rrc, w.rrad, w.n_rrad, s);
   e |= launch_setup(bd, s);
-  e |= launch_dist(bd, static_cast<const int *>(k.d_ang), k.n_ang, s);
+  e |= launch_dist(bd, w.ang, w.n_ang, s);
   if (prof) e |= (int)hipEventRecord(b.ev[1], s);
   e |= launch_integrate(bd, k.n_blocks, k.cos_rows != 0, s);
   if (prof) e |= (int)hipEventRecord(b.ev[2], s);
   e |= launch_fixup(bd, k.cos_rows != 0, s);
   if (prof) e |= (int)hipEventRecord(b.ev[3], s);
-  e |= launch_finalize(bd, s);
+  if (k.finalize) e |= launch_finalize(bd, s);
   if (prof) e |= (int)hipEventRecord(b.ev[4], s);
-  e |= launch_xill(bd, static_cast<const XillWork *>(k.d_xill), k.n_xill1, k.n_xill - k.n_xill1, s);
+  e |= launch_xill(bd, w.xill, w.n_xill1, w.n_xill - w.n_xill1, s);
   if (prof) e |= (int)hipEventRecord(b.ev[5], s);
-  e |= launch_conv(bd, static_cast<const XillWork *>(k.d_conv), k.n_conv, s);
+  e |= launch_conv(bd, w.conv, w.n_conv, s);
   if (prof) e |= (int)hipEventRecord(b.ev[6], s);
-  e |= launch_primary(bd, static_cast<const int *>(k.d_prim), k.n_prim, k.prim_bins, s);
+  e |= launch_primary(bd, w.prim, w.n_prim, k.prim_bins, s);
   if (prof) e |= (int)hipEventRecord(b.ev[7], s);
+  e |= launch_deliver(bd, static_cast<int *>(k.res), static_cast<double *>(k.res_out), k.n_out, s);
   return e;
 }
 
@@ -1423,24 +1575,24 @@ int batch_run(Batch &b, int precision, std::string &err) {
   memset(&k, 0, sizeof(k));
   k.bd = dev_view(b);
   k.n_blocks = b.n_blocks;
-  k.n_xill1 = b.n_xill1;
-  k.n_xill = (int)b.h_xill.size();
-  k.n_conv = (int)b.h_conv.size();
-  k.n_prim = (int)b.h_prim.size();
+  memcpy(&k.wl, &b.wl, sizeof(k.wl));
   k.prim_bins = b.prim_bins;
-  k.d_xill = b.d_xill.p;
-  k.d_conv = b.d_conv.p;
-  k.d_prim = b.d_prim.p;
-  k.d_rrc = b.d_rrc.p;
-  k.n_rrc = (int)b.h_rrc.size();
-  k.d_rrad = b.d_rrad.p;
-  k.n_rrad = (int)b.h_rrad.size();
-  k.d_nth = b.d_nthw.p;
-  k.n_nth = (int)b.h_nth.size();
-  k.d_zone = b.d_zonew.p;
-  k.n_zone = (int)b.h_zone.size();
-  k.d_ang = b.d_ang.p;
-  k.n_ang = (int)b.h_ang.size();
+  // only line profiles and angle distributions are finished by k_finalize
+  k.finalize = b.tot_pgrid > 0 || !b.h_ang.empty();
+  if (b.call_run) {
+    k.fetch_src = b.h_stage.p;
+    k.fetch_dst = b.d_arena.p;
+    k.n_fetch = (int64_t)(b.block_bytes / 16);
+  }
+  k.res = b.h_res.p;
+  k.res_out = result_out(b);
+  k.n_out = b.deliver_out;
+  b.synced = false;
+  {
+    std::lock_guard<std::mutex> lk(b.out_mu);
+    b.win[0].lo = b.win[0].hi = b.win[1].lo = b.win[1].hi = 0;
+    b.win_next = -1;
+  }
   k.prof = g.profile ? 1 : 0;
   k.cos_rows = b.any_limb ? 1 : 0;
   hipStream_t s = b.stream;
@@ -1478,8 +1630,8 @@ int batch_run(Batch &b, int precision, std::string &err) {
 int batch_sync(Batch &b) {
   if (!b.stream) return RX_OK;
   if (hipStreamSynchronize(b.stream) != hipSuccess) return RX_ERR_DEVICE;
-  int ctr[N_COUNTERS] = {};
-  if (hipMemcpy(ctr, b.d_ctr.p, sizeof ctr, hipMemcpyDeviceToHost) != hipSuccess) return RX_ERR_DEVICE;
+  b.synced = true;
+  const int *ctr = result_ctr(b);
   b.fix_overflow = b.last_mode == 1 && ctr[CTR_FIX_OVF] != 0;
   b.counters[0] = std::min(ctr[CTR_ITEMS] + ctr[CTR_ITEMS_S], b.item_cap);
   b.counters[1] = (b.last_mode == 1) ? ctr[CTR_FIX] : 0;
@@ -1489,6 +1641,7 @@ int batch_sync(Batch &b) {
     std::string err;
     if (batch_run(b, RX_FP64, err) != RX_OK) return RX_ERR_DEVICE;
     if (hipStreamSynchronize(b.stream) != hipSuccess) return RX_ERR_DEVICE;
+    b.synced = true;
   }
   if (b.profiled) {
     // events: setup | integrate | fixup | finalize | xill | conv | primary; the

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -18,6 +19,16 @@ struct DevBuf {
   size_t bytes = 0;
   ~DevBuf();
   int ensure(size_t n);  // grows (never shrinks); returns hipError_t
+  template <class T>
+  T *as() const { return reinterpret_cast<T *>(p); }
+};
+
+// Pinned host memory that kernels and copies on a stream read or write.
+struct PinnedBuf {
+  void *p = nullptr;
+  size_t bytes = 0;
+  ~PinnedBuf();
+  bool ensure(size_t n);  // grows (never shrinks)
   template <class T>
   T *as() const { return reinterpret_cast<T *>(p); }
 };
@@ -42,6 +53,13 @@ int n_model_params(int model);
 // Edges of the radial zones (RadialGrid::calculate_radial_grid, src/IonGradient.cpp:457-489).
 void rzone_grid(double rmin, double rmax, int nzones, double h, double *rgrid);
 
+// The work lists of a batch's kernels (device pointers and lengths).
+struct WorkLists {
+  const XillWork *xill, *conv, *zone, *nth;
+  const int *prim, *ang, *rrc, *rrad;
+  int n_xill1, n_xill, n_conv, n_zone, n_nth, n_prim, n_ang, n_rrc, n_rrad;
+};
+
 // Launch configuration of one run: every kernel argument and grid shape.  A
 // run whose configuration equals the previous run's is captured into a
 // hipGraph, which is replayed for as long as the configuration stays equal
@@ -49,9 +67,17 @@ void rzone_grid(double rmin, double rmax, int nzones, double h, double *rgrid);
 // its padding zeroed, so configurations compare with memcmp.
 struct RunKey {
   BatchDev bd;
-  int n_blocks, n_xill1, n_xill, n_conv, n_prim, n_rrc, n_rrad, n_nth, n_ang, n_zone, prim_bins;
-  const void *d_xill, *d_conv, *d_prim, *d_rrc, *d_rrad, *d_nth, *d_ang, *d_zone;
-  int prof, cos_rows;
+  WorkLists wl;
+  int n_blocks, prim_bins;
+  int prof, cos_rows, finalize;
+  // the request block fetched from pinned host memory at the start of the run
+  // (n_fetch 16-byte words; 0: it is on the device) and the results delivered
+  // there at its end (n_out output values; 0: statuses and counters only)
+  const void *fetch_src;
+  void *fetch_dst;
+  int64_t n_fetch;
+  void *res, *res_out;
+  int64_t n_out;
 };
 
 struct Batch {
@@ -77,13 +103,43 @@ struct Batch {
   int n_nth_sol = 0;             // requests with the nthcomp primary (one source solution each)
   int64_t tot_ener = 0, tot_flux = 0, tot_pgrid = 0, tot_prof = 0, tot_xspec = 0, tot_dist = 0, tot_zone = 0;
   int64_t tot_rrc = 0;
-  DevBuf d_req, d_ener, d_flux_in, d_out, d_pgrid, d_rad, d_prof, d_dist, d_refl, d_status, d_conv;
-  DevBuf d_xill, d_xspec, d_zone, d_prim, d_ang, d_zonew, d_rrc, d_rrad, d_rrpart, d_rret;
-  DevBuf d_nthw, d_nth, d_nthx, d_nths, d_nthn;
-  DevBuf d_items, d_ctr, d_fix, d_reach, d_rnorm, d_rnode;
+  // One device allocation holds everything of the batch; it begins with the
+  // request block (what the host writes: parameters, statuses, work lists,
+  // grids, input spectra).
+  DevBuf d_arena;
+  BatchDev dev;   // its pointers (dev_view adds the run's settings and the tables)
+  WorkLists wl;
+  size_t block_bytes = 0;
+  struct BlockOffsets {
+    size_t req, status, conv, xill, prim, zone, ang, rrc, rrad, nth, ener, flux;
+  } off;
+  bool staged = false;  // the block fits the pinned memory
+  double *p_ener = nullptr, *p_flux = nullptr;  // grids and inputs on the host (pinned memory or h_ener, h_flux_in)
+  // The request block in pinned memory (batches that are built again and again
+  // keep their own, others use the library's while they are built), the run's
+  // results (result_*).
+  bool keep_stage = false;
+  PinnedBuf h_stage, h_res;
+  // an evaluation call: the run fetches the request block and delivers the
+  // outputs itself (call_run: this one does)
+  bool is_call = false, call_run = false;
+  int64_t deliver_out = 0;  // output values that a run delivers to h_res
+  // outputs read ahead by rx_batch_output: two pinned windows of the output
+  // array, filled in turn
+  struct OutWindow {
+    int64_t lo = 0, hi = 0;  // values [lo, hi) of the output array
+    bool pending = false;    // its copy is on the stream
+    PinnedBuf buf;
+  };
+  OutWindow win[2];
+  int win_cur = 0;
+  int64_t win_next = -1, win_len = 0;  // end of the last read; length of the last window
+  std::atomic<bool> synced{true};      // the stream was waited for since the last run
+  std::mutex out_mu;                   // readers of one batch in several threads
   int item_cap = 0;
   int n_blocks = 1;  // workgroups of k_integrate
   bool any_cosne = false, any_limb = false;
+  bool any_flux = false;  // some request has an input spectrum
   int fix_cap = 0;
   int last_mode = 1;
   bool fix_overflow = false;
@@ -123,6 +179,16 @@ WorkShape work_shape(int64_t windows, int max_bins);
 // Workgroups of k_integrate for a work list of that capacity.
 int integrate_blocks(int item_cap, int64_t windows, int waves_per_cu);
 int batch_upload(Batch &b);
+// Layout of a run's results in pinned host memory: the first RES_CTR counters,
+// the statuses, the outputs.
+inline int *result_ctr(const Batch &b) { return b.h_res.as<int>(); }
+inline int *result_status(const Batch &b) { return b.h_res.as<int>() + RES_CTR; }
+inline size_t result_out_offset(int n_req) { return (sizeof(int) * (RES_CTR + (size_t)n_req) + 255) & ~(size_t)255; }
+inline double *result_out(const Batch &b) {
+  return reinterpret_cast<double *>(b.h_res.as<char>() + result_out_offset(b.n_req));
+}
+// Copies n output values from off on (after the run's end) to host memory.
+int batch_read(Batch &b, int64_t off, int64_t n, double *to);
 int batch_run(Batch &b, int precision, std::string &err);
 int batch_sync(Batch &b);
 // Public status of a request from its device status.
@@ -165,6 +231,7 @@ struct Global {
   // returning-radiation table (loaded and uploaded on the first request with it)
   RradTableHost rrad;
   bool rrad_loaded = false, rrad_dirty = true;
+  PinnedBuf stage;  // request block of the batch being built (under mu)
   DevBuf nth_grid;  // what all nthcomp solves share
   DevBuf r_rlo, r_rhi, r_tf, r_gmin, r_gmax, r_fg;
   // convolution grid

@@ -1,6 +1,6 @@
 // kernels.hip -- CDNA4 (gfx950) kernels of the relativistic smearing path.
 //
-//   k_reset      clears the run's counters
+//   k_begin      clears the run's counters, fetches a call's request block
 //   k_setup      one workgroup per request: (a, mu0) bilinear table
 //                interpolation (interpol_relTable, src/Relprofile.cpp:141-303),
 //                fine radial grid, emissivity (src/Rellp.cpp:518-564), energy
@@ -19,6 +19,7 @@
 //                1 keV rotation and E/dE weighting, band normalisation, rebin
 //                back and zeroing outside 0.01-1000 keV
 //                (src/Relbase.cpp:93-289)
+//   k_deliver    counters, statuses and a call's outputs to the host
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1311,9 +1312,31 @@ __global__ __launch_bounds__(NTH_THREADS_R) void k_nth(BatchDev b, const XillWor
   }
 }
 
-// Clears the run's counters; launched before k_setup on the batch's stream.
-__global__ __launch_bounds__(64) void k_reset(int *ctr) {
-  for (int i = threadIdx.x; i < N_COUNTERS; i += 64) ctr[i] = 0;
+// First in a run: clears its counters and, for an evaluation call, copies the
+// request block (parameters, work lists, grids, input) from pinned host memory:
+// the launch graph of a call on one grid then holds its transfers too, and a
+// call makes one launch and one wait where it made about nine copies of 5-10 us
+// each before the kernels and three after them.
+constexpr int COPY_THREADS = 256;
+__global__ __launch_bounds__(COPY_THREADS) void k_begin(int *ctr, const uint4 *__restrict__ src,
+                                                        uint4 *__restrict__ dst, int64_t n16) {
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < N_COUNTERS; i += COPY_THREADS) ctr[i] = 0;
+  for (int64_t i = (int64_t)blockIdx.x * COPY_THREADS + threadIdx.x; i < n16; i += (int64_t)gridDim.x * COPY_THREADS)
+    dst[i] = src[i];
+}
+
+// Last in a run: counters, statuses and (calls, server) outputs to pinned host
+// memory, where the host reads them once the stream is done.
+__global__ __launch_bounds__(COPY_THREADS) void k_deliver(BatchDev b, int *__restrict__ res,
+                                                          double *__restrict__ res_out, int64_t n_out) {
+  const int64_t i0 = (int64_t)blockIdx.x * COPY_THREADS + threadIdx.x, step = (int64_t)gridDim.x * COPY_THREADS;
+  if (i0 < RES_CTR) res[i0] = b.ctr[i0];
+  for (int64_t i = i0; i < b.n_req; i += step) res[RES_CTR + i] = b.status[i];
+  const double2 *o2 = reinterpret_cast<const double2 *>(b.out);
+  double2 *r2 = reinterpret_cast<double2 *>(res_out);
+  for (int64_t i = i0; i < n_out / 2; i += step) r2[i] = o2[i];
+  if ((n_out & 1) && i0 == 0) res_out[n_out - 1] = b.out[n_out - 1];
 }
 
 // ---------------------------------------------------------------------------
@@ -2816,9 +2839,24 @@ __global__ __launch_bounds__(256) void k_copy(const double4 *__restrict__ src, d
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
+static int copy_blocks(int64_t words) {
+  return (int)std::max<int64_t>(1, std::min<int64_t>(1024, (words + COPY_THREADS - 1) / COPY_THREADS));
+}
+
+int launch_begin(int *ctr, const void *src, void *dst, int64_t n16, void *stream) {
+  hipLaunchKernelGGL(k_begin, dim3(copy_blocks(n16)), dim3(COPY_THREADS), 0, (hipStream_t)stream, ctr,
+                     (const uint4 *)src, (uint4 *)dst, n16);
+  return (int)hipGetLastError();
+}
+
+int launch_deliver(const BatchDev &b, int *res, double *res_out, int64_t n_out, void *stream) {
+  hipLaunchKernelGGL(k_deliver, dim3(copy_blocks(std::max<int64_t>(b.n_req, n_out / 2))), dim3(COPY_THREADS), 0,
+                     (hipStream_t)stream, b, res, res_out, n_out);
+  return (int)hipGetLastError();
+}
+
 int launch_setup(const BatchDev &b, void *stream) {
   if (b.n_req <= 0) return 0;
-  hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, (hipStream_t)stream, b.ctr);
   if (b.max_zones > LP_ZONES)
     hipLaunchKernelGGL(k_setup<MAX_ZONES>, dim3(b.n_req), dim3(SETUP_THREADS), 0, (hipStream_t)stream, b);
   else

@@ -8,9 +8,11 @@
 // device when the library initialises the device; host code only ever uses
 // that address.  Every call on a GPU shares the array and leaves the last
 // call's contents in it: whatever must start at zero is cleared by the
-// kernels themselves (k_reset clears the counters, k_setup the profile bins
-// that windows reach, k_finalize / k_conv write every output bin), and calls
-// that overlap on one GPU race.
+// kernels themselves (k_noalloc_begin clears the counters, k_setup the profile
+// bins that windows reach, k_finalize / k_conv write every output bin), and
+// calls that overlap on one GPU race.  A call makes no copies: its request goes
+// as a kernel argument, its status comes back in pinned words allocated with
+// the scratch address.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -31,23 +33,35 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 void *g_scratch[kMaxDevices] = {};  // its device address, per device
 
-// relconv's input check (src/LocalModel.cpp:84-86) on device data: an input
-// spectrum whose sum is not positive fails the request with status 50.
-constexpr int CHECK_THREADS = 256;
-__global__ __launch_bounds__(CHECK_THREADS) void k_input_check(const double *flux, int n, ReqParams *req,
-                                                               int *status) {
-  __shared__ double s[CHECK_THREADS];
-  double v = 0.0;
-  for (int i = threadIdx.x; i < n; i += CHECK_THREADS) v += flux[i];
-  s[threadIdx.x] = v;
-  __syncthreads();
-  for (int w = CHECK_THREADS / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
+int *g_res[kMaxDevices] = {};  // pinned words for a call's status and counters, per device
+
+// First kernel of a call: the request record (an argument: no copy), its status,
+// the one-entry work list and the cleared counters, and relconv's input check
+// (src/LocalModel.cpp:84-86) on device data: an input spectrum whose sum is not
+// positive fails the request with status 50 (flux: null to skip it).
+constexpr int BEGIN_THREADS = 256;
+__global__ __launch_bounds__(BEGIN_THREADS) void k_noalloc_begin(ReqParams p, ReqParams *req, int *status,
+                                                                 XillWork *work, int *ctr, const double *flux, int n) {
+  __shared__ double s[BEGIN_THREADS];
+  const int tid = threadIdx.x;
+  for (int i = tid; i < N_COUNTERS; i += BEGIN_THREADS) ctr[i] = 0;
+  int st = p.pre_status;
+  if (flux) {
+    double v = 0.0;
+    for (int i = tid; i < n; i += BEGIN_THREADS) v += flux[i];
+    s[tid] = v;
     __syncthreads();
+    for (int w = BEGIN_THREADS / 2; w > 0; w >>= 1) {
+      if (tid < w) s[tid] += s[tid + w];
+      __syncthreads();
+    }
+    if (!(s[0] > 0.0)) st = RX_ERR_INPUT;
   }
-  if (threadIdx.x == 0 && !(s[0] > 0.0)) {
-    req->pre_status = RX_ERR_INPUT;
-    *status = RX_ERR_INPUT;
+  if (tid == 0) {
+    *req = p;
+    req->pre_status = st;
+    *status = st;
+    *work = XillWork{0, 0};
   }
 }
 
@@ -79,6 +93,14 @@ int noalloc_setup(int device, std::string &err) {
     err = "hipGetSymbolAddress of the scratch array failed";
     return RX_ERR_DEVICE;
   }
+  // (4 KB for the process's life, as the scratch array)
+  void *r = nullptr;
+  if (hipHostMalloc(&r, sizeof(int) * (RES_CTR + 1), hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    err = "pinned host allocation failed";
+    return RX_ERR_NOMEM;
+  }
+  g_res[device] = static_cast<int *>(r);
   g_scratch[device] = p;
   return RX_OK;
 }
@@ -197,42 +219,36 @@ int noalloc_eval(int model, const double *parameter, const double *d_energy, con
           "(RX_NOALLOC_SCRATCH_BYTES): fewer bins or smaller tables";
     return RX_ERR_ARG;
   }
-  const XillWork w0{0, 0};
-  int e = (int)hipMemcpyAsync(bd.req, &p, sizeof(p), hipMemcpyHostToDevice, s);
-  e |= (int)hipMemcpyAsync(bd.status, &p.pre_status, sizeof(int), hipMemcpyHostToDevice, s);
-  e |= (int)hipMemcpyAsync(d_work, &w0, sizeof(w0), hipMemcpyHostToDevice, s);
   const bool cos_rows = p.limb != 0;
   const int n_blocks = integrate_blocks(item_cap, n_rc, wpc);
-  int out[2] = {0, 0};  // status, FP64 re-check queue overflow
+  int *res = g_res[g.device];  // counters, status
+  int e = 0;
   for (int pass = 0; pass < 2 && e == 0; pass++) {
     bd.mode = (pass == 0 && precision == RX_FP32) ? 1 : 0;
-    if (conv && p.pre_status == 0) {
-      hipLaunchKernelGGL(k_input_check, dim3(1), dim3(CHECK_THREADS), 0, s, d_flux_in, n_flux, bd.req,
-                         bd.status);
-      e |= (int)hipGetLastError();
-    }
+    hipLaunchKernelGGL(k_noalloc_begin, dim3(1), dim3(BEGIN_THREADS), 0, s, p, bd.req, bd.status, d_work, bd.ctr,
+                       (conv && p.pre_status == 0) ? d_flux_in : nullptr, n_flux);
+    e |= (int)hipGetLastError();
     // (the one unit {0, 0} of d_work is the list of request 0)
     if (p.return_rad != 0 && p.pre_status == 0)
       e |= launch_rrad(bd, nullptr, 0, reinterpret_cast<const int *>(d_work), 1, s);
     e |= launch_setup(bd, s);
     e |= launch_integrate(bd, n_blocks, cos_rows, s);
     e |= launch_fixup(bd, cos_rows, s);
-    e |= launch_finalize(bd, s);
     if (conv) e |= launch_conv(bd, d_work, 1, s);
-    e |= (int)hipMemcpyAsync(&out[0], bd.status, sizeof(int), hipMemcpyDeviceToHost, s);
-    e |= (int)hipMemcpyAsync(&out[1], bd.ctr + CTR_FIX_OVF, sizeof(int), hipMemcpyDeviceToHost, s);
+    else e |= launch_finalize(bd, s);
+    e |= launch_deliver(bd, res, nullptr, 0, s);
     e |= (int)hipStreamSynchronize(s);
     // an overflowing FP32 re-check queue: the pass is redone in FP64
-    if (!(bd.mode == 1 && out[1] != 0)) break;
+    if (e || !(bd.mode == 1 && res[CTR_FIX_OVF] != 0)) break;
   }
   if (e) {
     (void)hipGetLastError();
     msg = "device error in the allocation-free evaluation";
     return RX_ERR_DEVICE;
   }
-  if (out[0] != 0) {
+  if (res[RES_CTR] != 0) {
     msg = "model evaluation failed";
-    return public_status(out[0]);
+    return public_status(res[RES_CTR]);
   }
   msg = "";
   return RX_OK;

@@ -324,7 +324,7 @@ constexpr int ST_WORKLIST = 60;
 constexpr int N_XQ = 8;
 constexpr int XQ_STRIDE = 32;  // ints between the range counters (one 128-byte line each)
 
-// Device counters of one batch run (cleared by k_reset before k_setup).
+// Device counters of one batch run (cleared by k_begin).
 enum CounterSlot : int {
   CTR_FIX = 0,        // FixEntry entries written
   CTR_FIX_OVF = 1,    // FixEntry queue overflowed
@@ -334,6 +334,8 @@ enum CounterSlot : int {
   CTR_XQ = XQ_STRIDE,  // N_XQ range counters, XQ_STRIDE apart
   N_COUNTERS = CTR_XQ + N_XQ * XQ_STRIDE
 };
+
+constexpr int RES_CTR = 8;  // counters delivered to the host (those before CTR_XQ that are used)
 
 struct BatchDev {
   int n_req;
@@ -380,6 +382,11 @@ struct BatchDev {
 };
 
 // ---- launchers (kernels.hip) ----
+// First in a run: clears the counters and copies the request block (n16 16-byte
+// words of pinned host memory) to the device.
+int launch_begin(int *ctr, const void *src, void *dst, int64_t n16, void *stream);
+// Last in a run: the counters, statuses and n_out outputs to pinned host memory.
+int launch_deliver(const BatchDev &b, int *res, double *res_out, int64_t n_out, void *stream);
 int launch_setup(const BatchDev &b, void *stream);
 // the emission-angle distribution of the n_reqs requests with one
 int launch_dist(const BatchDev &b, const int *reqs, int n_reqs, void *stream);

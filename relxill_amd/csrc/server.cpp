@@ -6,8 +6,8 @@
 // requests in arrival order while their device working set fits the HBM
 // budget (minus what the running batches hold) and the in-flight cap, builds
 // a batch (without holding the queue lock, so submits and polls go on) and
-// launches it, followed on the same stream by the copies of its outputs,
-// statuses and counters into the slot's pinned host buffers.  While every
+// launches it; the run's last kernel writes its outputs, statuses and
+// counters into the slot's pinned host memory.  While every
 // slot is busy, arrivals queue up and the next free slot takes all of them:
 // batches grow with the load.  A finished batch (hipStreamQuery) has its
 // results on the host already; its memory returns to the budget and its
@@ -59,36 +59,11 @@ struct Result {
   std::vector<double> flux;
 };
 
-// Pinned host memory that a batch's outputs are copied into on its stream.
-struct PinnedBuf {
-  void *p = nullptr;
-  size_t bytes = 0;
-  ~PinnedBuf() {
-    if (p) (void)hipHostFree(p);
-  }
-  bool ensure(size_t n) {
-    if (p && bytes >= n) return true;
-    if (p) n = std::max(n, bytes + bytes / 2);  // grows rarely (hipHostFree synchronises)
-    if (p) (void)hipHostFree(p);
-    p = nullptr;
-    bytes = 0;
-    if (hipHostMalloc(&p, n, hipHostMallocDefault) != hipSuccess) {
-      p = nullptr;
-      return false;
-    }
-    bytes = n;
-    return true;
-  }
-  template <class T>
-  T *as() const { return reinterpret_cast<T *>(p); }
-};
-
 struct Slot {
   Batch batch;
   bool busy = false;
   std::vector<Pending> reqs;
   int64_t bytes = 0;
-  PinnedBuf h_out, h_status, h_ctr;
 };
 
 int64_t request_bytes(const Pending &p) {
@@ -144,7 +119,7 @@ struct rx_server {
   bool reap(std::unique_lock<std::mutex> &lk);
 };
 
-// Builds, launches and queues the output copies of one batch on the slot's
+// Builds and launches one batch on the slot's
 // stream (called without the queue lock: only the scheduler thread touches
 // the slots).
 int rx_server::launch(Slot &s, std::vector<Pending> &take, std::string &err) {
@@ -164,24 +139,16 @@ int rx_server::launch(Slot &s, std::vector<Pending> &take, std::string &err) {
   s.batch.seg_forced = 0;
   s.batch.waves_forced = 0;
   s.batch.one_shot = true;
+  s.batch.keep_stage = true;
+  // the run delivers every output to the slot's pinned memory
+  int64_t n_out = 0;
+  for (const Pending &p : take) n_out += (int64_t)p.energy.size() - 1;
+  s.batch.deliver_out = n_out;
   st = batch_build(s.batch, rq.data(), (int)rq.size(), err);
-  if (st != RX_OK) return st;
-  if (!s.h_out.ensure(sizeof(double) * std::max<int64_t>(1, s.batch.tot_flux)) ||
-      !s.h_status.ensure(sizeof(int) * s.batch.n_req) || !s.h_ctr.ensure(sizeof(int) * N_COUNTERS)) {
-    err = "pinned host allocation failed";
-    return RX_ERR_NOMEM;
-  }
-  st = batch_run(s.batch, precision, err);
-  if (st != RX_OK) return st;
-  hipStream_t q = s.batch.stream;
-  int e = (int)hipMemcpyAsync(s.h_out.p, s.batch.d_out.p, sizeof(double) * s.batch.tot_flux, hipMemcpyDeviceToHost, q);
-  e |= (int)hipMemcpyAsync(s.h_status.p, s.batch.d_status.p, sizeof(int) * s.batch.n_req, hipMemcpyDeviceToHost, q);
-  e |= (int)hipMemcpyAsync(s.h_ctr.p, s.batch.d_ctr.p, sizeof(int) * N_COUNTERS, hipMemcpyDeviceToHost, q);
-  if (e) {
-    err = "output copy failed";
-    return RX_ERR_DEVICE;
-  }
-  return RX_OK;
+  if (st == RX_OK) st = batch_run(s.batch, precision, err);
+  // (a batch that is not going to be reaped: its request block may still be on the way)
+  if (st != RX_OK && s.batch.stream) (void)hipStreamSynchronize(s.batch.stream);
+  return st;
 }
 
 void rx_server::launch_ready(std::unique_lock<std::mutex> &lk) {
@@ -241,10 +208,10 @@ bool rx_server::reap(std::unique_lock<std::mutex> &lk) {
     hipError_t q = hipStreamQuery(s.batch.stream);
     if (q == hipErrorNotReady) continue;
     const auto now = Clock::now();
-    const int *st = s.h_status.as<int>();
-    const double *out = s.h_out.as<double>();
+    const int *st = result_status(s.batch);
+    const double *out = result_out(s.batch);
     bool ok = q == hipSuccess;
-    if (ok && precision == RX_FP32 && s.h_ctr.as<int>()[CTR_FIX_OVF] != 0) {
+    if (ok && precision == RX_FP32 && result_ctr(s.batch)[CTR_FIX_OVF] != 0) {
       // the FP64 re-check queue overflowed: redo the batch in FP64 (rare;
       // synchronous, outside the queue lock)
       lk.unlock();
@@ -252,10 +219,6 @@ bool rx_server::reap(std::unique_lock<std::mutex> &lk) {
         std::lock_guard<std::recursive_mutex> g(G().mu);
         std::string err;
         ok = batch_run(s.batch, RX_FP64, err) == RX_OK;
-        ok = ok && hipMemcpyAsync(s.h_out.p, s.batch.d_out.p, sizeof(double) * s.batch.tot_flux,
-                                  hipMemcpyDeviceToHost, s.batch.stream) == hipSuccess;
-        ok = ok && hipMemcpyAsync(s.h_status.p, s.batch.d_status.p, sizeof(int) * s.batch.n_req,
-                                  hipMemcpyDeviceToHost, s.batch.stream) == hipSuccess;
         ok = ok && hipStreamSynchronize(s.batch.stream) == hipSuccess;
       }
       lk.lock();
