@@ -33,19 +33,13 @@ namespace rx {
 
 namespace {
 
-constexpr int SETUP_THREADS = 256;
+constexpr int FINAL_THREADS = 256;
 constexpr int CONV_THREADS = 256;      // smallest convolution workgroup
 constexpr int XILL_THREADS = 256;
 constexpr int XILL_BINS = 4;    // table bins per k_xill thread, one-zone requests
 constexpr int XILL_BINS_Z = 2;  // the same for requests of LP_ZONES zones (ten accumulators per bin)
 constexpr int PRIM_THREADS = 256;
 constexpr int CONV_THREADS_MAX = 1024;  // n/8 threads: 512 for 4096 bins, 1024 for 8192
-
-__device__ inline double lp_ifac(float value, const float *arr, int n, int &ind) {
-  // get_ipol_factor: float search and float quotient (src/relutility.c:419-423)
-  ind = bsearch_asc(arr, n, value);
-  return (double)((value - arr[ind]) / (arr[ind + 1] - arr[ind]));
-}
 
 // spec_cutoffpl (src/Xillspec.cpp:215-241): photons of the cut-off power law
 // exp(1/Ecut) E^-Gamma exp(-E/Ecut) dE in [e0, e1] at E = (e0 + e1) / 2, as
@@ -105,6 +99,20 @@ __device__ inline double bbody_norm_part(const DevConvGrid &cg, double kt, int t
     if (e0 >= 0.1 && e0 <= 1000.0) sp += bbody_bin(e0, e1, kt) * 0.5 * (e0 + e1) * 1e20 * 1.602177e-09;
   }
   return sp;
+}
+
+// bsearch_asc by a whole wavefront: the same bracket of an ascending array from
+// one load a lane (binary search: a dependent load a step, 0.5 us each)
+template <class T, class V>
+__device__ inline int wave_bracket(const T *arr, int n, V val, int lane) {
+  int cnt = 0;  // values that are not above val
+  for (int k = 0; k < n; k += 64) cnt += __popcll(__ballot(k + lane < n && !(arr[min(k + lane, n - 1)] > val)));
+  return min(max(cnt - 1, 0), n - 2);
+}
+
+// get_ipol_factor (src/relutility.c:419-423): float quotient
+__device__ inline double ipol_fac(float value, const float *arr, int ind) {
+  return (double)((value - arr[ind]) / (arr[ind + 1] - arr[ind]));
 }
 
 struct LpFine {
@@ -206,12 +214,13 @@ __device__ inline void lp_rows(const DevLpTable &L, const ReqParams &rq, double 
                                double *ji, int tid, int nt) {
   __shared__ int s_i[3];
   __shared__ double s_f[3];
-  if (tid == 0) {
-    int lia;
-    const double lfa = lp_ifac((float)rq.a, L.a, L.n_a, lia);
-    int h0, h1;
-    const double fh0 = lp_ifac((float)rq.height, L.h + (size_t)lia * L.n_h, L.n_h, h0);
-    const double fh1 = lp_ifac((float)rq.height, L.h + (size_t)(lia + 1) * L.n_h, L.n_h, h1);
+  if (tid < 64) {
+    // the searches are float (src/relutility.c:419-423)
+    const float a = (float)rq.a, h = (float)rq.height;
+    const int lia = wave_bracket(L.a, L.n_a, a, tid);
+    const float *hl = L.h + (size_t)lia * L.n_h, *hu = hl + L.n_h;
+    const int h0 = wave_bracket(hl, L.n_h, h, tid), h1 = wave_bracket(hu, L.n_h, h, tid);
+    const double lfa = ipol_fac(a, L.a, lia), fh0 = ipol_fac(h, hl, h0), fh1 = ipol_fac(h, hu, h1);
     s_i[0] = lia;
     s_i[1] = h0;
     s_i[2] = h1;
@@ -410,6 +419,15 @@ __device__ inline double wave_sum(double v) {
   return (readlane_d(v, 0) + readlane_d(v, 16)) + (readlane_d(v, 32) + readlane_d(v, 48));
 }
 
+// maximum over the 64 lanes; every lane must be active
+__device__ inline double wave_max_d(double v) {
+  v = fmax(v, dpp_d<0xB1>(v));
+  v = fmax(v, dpp_d<0x4E>(v));
+  v = fmax(v, dpp_d<0x141>(v));
+  v = fmax(v, dpp_d<0x140>(v));
+  return fmax(fmax(readlane_d(v, 0), readlane_d(v, 16)), fmax(readlane_d(v, 32), readlane_d(v, 48)));
+}
+
 // min / max over the 64 lanes (quad, half-row and row exchanges, then the rows);
 // every lane must be active
 __device__ inline int wave_min_i(int v) {
@@ -517,12 +535,22 @@ __device__ inline double block_sum(double v, double *red) {
 // setup
 // ---------------------------------------------------------------------------
 // NZ: the most zones of a request in the batch (LP_ZONES, or MAX_ZONES with
-// an ionisation gradient), which sizes the zone arrays in LDS
-template <int NZ>
-__global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
+// an ionisation gradient), which sizes the zone arrays in LDS.  NT: threads.
+// Bound: latency, of the table loads, of a fine radius' chain (a search over
+// the node radii, the emissivity's pow, two bracket searches over the energy
+// grid) and of the barriers between the phases; so what one thread did in turn
+// (table and radius searches, the lamp post's reflection fraction, the list of
+// windows) is done by a wavefront at once, and sums cross the wavefronts in one
+// step.  Batches that leave the chip idle get workgroups of 512 threads, which
+// take the 1000 radii in two rounds instead of four.  Measured before and after:
+// relline call 24 -> 15 us, relline_lp call 43 -> 27 us, relxilllp call 62 -> 31
+// us, 256 relline_lp requests 50 -> 33 us, 4096 relconv requests 176 -> 145 us.
+template <int NZ, int NT>
+__global__ __launch_bounds__(NT, NT == 256 ? 3 : 1) void k_setup(BatchDev b) {
+  constexpr int NW = NT / 64;
   const int req = blockIdx.x;
-  const int tid = threadIdx.x;
-  const ReqParams rq = b.req[req];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const ReqParams &rq = b.req[req];
   const DevRelTable &T = b.rt;
   const int nr = b.nr_fine;
   const int n_r = T.n_r;
@@ -534,40 +562,64 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
     // interpolation in the inclination (interp_5d_tab, src/xilltable.c:878-995);
     // k_primary rebins and adds the primary
     double *d = b.dist + rq.dist_off;
-    for (int a = tid; a < rq.n_incl; a += SETUP_THREADS)
+    for (int a = tid; a < rq.n_incl; a += NT)
       d[a] = (a == rq.xinc_ind) ? 1.0 - rq.xinc_fac : ((a == rq.xinc_ind + 1) ? rq.xinc_fac : 0.0);
     return;
+  }
+  __shared__ double s_tre[MAX_NR_TAB], s_tgmin[MAX_NR_TAB], s_tgmax[MAX_NR_TAB];
+  __shared__ double s_jr[MAX_LP_R], s_je[MAX_LP_R], s_jd[MAX_LP_R], s_ji[MAX_LP_R];
+  __shared__ double s_rr_rad[MAX_RR], s_rr_ret[MAX_RR];
+  __shared__ double s_sum[NW], s_max[NW];
+  __shared__ int s_st, s_ia, s_im, s_rmin;
+  __shared__ double s_fa, s_fm;
+  constexpr int MAX_RC = MAX_NR_FINE / RAD_CHUNK;
+  // energy window of each (radius chunk, zone): bins [s_ulo, s_uhi]
+  __shared__ int s_ulo[MAX_RC * NZ], s_uhi[MAX_RC * NZ];
+  __shared__ int s_pref[MAX_RC * NZ], s_prefs[MAX_RC * NZ];
+  __shared__ int s_base, s_bases, s_jlo, s_jhi;
+  const int n_rc = (nr + RAD_CHUNK - 1) / RAD_CHUNK;
+  const int nz = rq.n_zones;
+  const double *zg = rq.zgrid;
+  const bool lp = (rq.emis_type == EMIS_LP);
+  const DevLpTable &L = b.lp;
+  const int ntr = L.n_r;
+
+  // the (a, mu0) bracket, one wavefront; meanwhile the others begin with the grid
+  if (wave == 0) {
+    const float a = (float)rq.a, mu0 = (float)cos(rq.incl);
+    const int ia = wave_bracket(T.a, T.n_a, a, lane), im = wave_bracket(T.mu0, T.n_mu0, mu0, lane);
+    const float fa = (a - T.a[ia]) / (T.a[ia + 1] - T.a[ia]);
+    const float fm = (mu0 - T.mu0[im]) / (T.mu0[im + 1] - T.mu0[im]);
+    int st = 0;
+    if (!(rq.rout > rq.rin) || !(rq.rin >= rq.rms)) st = 10;
+    if (!(fm >= 0 && fm <= 1 && fa >= 0 && fa <= 1)) st = 11;
+    if (lane == 0) {
+      s_st = st;
+      s_ia = ia;
+      s_im = im;
+      s_fa = fa;
+      s_fm = fm;
+    }
+  }
+  for (int c = tid; c < n_rc * NZ; c += NT) {
+    s_ulo[c] = 0x7fffffff;
+    s_uhi[c] = -1;
   }
   if (rq.model == MOD_RELXILL || rq.model == MOD_RELXILLLP) {
     // the zones' convolutions add into the output (k_conv)
     double *out = b.out + rq.flux_off;
-    for (int j = tid; j < rq.n_in; j += SETUP_THREADS) out[j] = 0.0;
+    for (int j = tid; j < rq.n_in; j += NT) out[j] = 0.0;
   }
-
-  __shared__ double s_tre[MAX_NR_TAB], s_tgmin[MAX_NR_TAB], s_tgmax[MAX_NR_TAB];
-  __shared__ double s_jr[MAX_LP_R], s_je[MAX_LP_R], s_jd[MAX_LP_R], s_ji[MAX_LP_R];
-  __shared__ double s_red[SETUP_THREADS];
-  __shared__ int s_st, s_ia, s_im, s_rmin;
-  __shared__ double s_fa, s_fm, s_rms;
-  constexpr int MAX_RC = MAX_NR_FINE / RAD_CHUNK;
-  // energy window of each (radius chunk, zone): bins [s_ulo, s_uhi]
-  __shared__ int s_ulo[MAX_RC * NZ], s_uhi[MAX_RC * NZ];
-  __shared__ int s_pref[MAX_RC * NZ + 1], s_prefs[MAX_RC * NZ + 1];
-  __shared__ int s_base, s_bases;
-  const int n_rc = (b.nr_fine + RAD_CHUNK - 1) / RAD_CHUNK;
-  const int nz = rq.n_zones;
-  const double *zg = b.req[req].zgrid;
-  for (int c = tid; c < n_rc * NZ; c += SETUP_THREADS) {
-    s_ulo[c] = 0x7fffffff;
-    s_uhi[c] = -1;
+  if (rq.n_incl > 0) {  // k_dist adds into the angle distribution
+    const int nd = rq.n_incl * nz;  // [zone][angle bin]
+    for (int k = tid; k < nd; k += NT) b.dist[rq.dist_off + k] = 0.0;
   }
-
   // profile grid: caller grid shifted to line-energy units (XspecSpectrum.h:61-76)
   const double *E;
   if (rq.pgrid_off >= 0) {
     double *pg = b.pgrid + rq.pgrid_off;
     const double *ein = b.ener_in + rq.ener_off;
-    for (int k = tid; k <= rq.n_in; k += SETUP_THREADS) {
+    for (int k = tid; k <= rq.n_in; k += NT) {
       double e = ein[k];
       if (rq.z > 0) e *= (1 + rq.z);
       pg[k] = e / rq.lineE;
@@ -575,24 +627,6 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
     E = pg;
   } else {
     E = b.cg.ener;
-  }
-
-  if (tid == 0) {
-    int st = 0;
-    const double rms = rq.rms;
-    if (!(rq.rout > rq.rin) || !(rq.rin >= rms)) st = 10;
-    const double mu0 = cos(rq.incl);
-    const int ia = bsearch_asc(T.a, T.n_a, (float)rq.a);
-    const int im = bsearch_asc(T.mu0, T.n_mu0, (float)mu0);
-    const float fa = ((float)rq.a - T.a[ia]) / (T.a[ia + 1] - T.a[ia]);
-    const float fm = ((float)mu0 - T.mu0[im]) / (T.mu0[im + 1] - T.mu0[im]);
-    if (!(fm >= 0 && fm <= 1 && fa >= 0 && fa <= 1)) st = 11;
-    s_st = st;
-    s_ia = ia;
-    s_im = im;
-    s_fa = fa;
-    s_fm = fm;
-    s_rms = rms;
   }
   __syncthreads();
   if (s_st) {
@@ -603,41 +637,54 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
   const double fa = s_fa, fm = s_fm;
   const size_t n00 = (size_t)ia * T.n_mu0 + im, n10 = (size_t)(ia + 1) * T.n_mu0 + im;
   const size_t n01 = (size_t)ia * T.n_mu0 + im + 1, n11 = (size_t)(ia + 1) * T.n_mu0 + im + 1;
-
-  // node radii: lerp in a only (src/Relprofile.cpp:190-193)
-  for (int ir = tid; ir < n_r; ir += SETUP_THREADS) {
+  // node radii: lerp in a only (src/Relprofile.cpp:190-193); node values:
+  // bilinear in (a, mu0) (interpol_a_mu0, :39-80)
+  for (int ir = tid; ir < n_r; ir += NT) {
     s_tre[ir] = lerp1(fa, (double)T.r[n00 * n_r + ir], (double)T.r[n10 * n_r + ir]);
-  }
-  __syncthreads();
-  if (tid == 0) {
-    int st = 0;
-    const double rms = s_rms;
-    // ISCO snap (:195-200)
-    if ((s_tre[n_r - 1] > rms) && ((s_tre[n_r - 1] - rms) / s_tre[n_r - 1] < 1e-3)) {
-      s_tre[n_r - 1] = rms;
-    }
-    const int ind_rmin = bsearch_desc(s_tre, n_r, rq.rin);
-    const int ind_rmax = bsearch_desc(s_tre, n_r, rq.rout);
-    // 1000 rg snap (:235-238)
-    if (s_tre[ind_rmax] < 1000.0 && s_tre[ind_rmax] * 1.01 > 1000.0) s_tre[ind_rmax] = 1000.0;
-    if (!(ind_rmin > 0) || !(s_tre[ind_rmin + 1] <= rq.rin) || !(s_tre[ind_rmin] >= rq.rin) ||
-        !(s_tre[ind_rmax + 1] <= rq.rout) || !(s_tre[ind_rmax] >= rq.rout) ||
-        !(ind_rmax <= ind_rmin) || !(rq.rout <= 1000.0)) {
-      st = 12;
-    }
-    s_rmin = ind_rmin;
-    s_st = st;
-  }
-  // node values: bilinear in (a, mu0) (interpol_a_mu0, :39-80)
-  for (int ir = tid; ir < n_r; ir += SETUP_THREADS) {
     s_tgmin[ir] = lerp2f(fa, fm, T.gmin[n00 * n_r + ir], T.gmin[n10 * n_r + ir],
                          T.gmin[n01 * n_r + ir], T.gmin[n11 * n_r + ir]);
     s_tgmax[ir] = lerp2f(fa, fm, T.gmax[n00 * n_r + ir], T.gmax[n10 * n_r + ir],
                          T.gmax[n01 * n_r + ir], T.gmax[n11 * n_r + ir]);
   }
   // lamp-post table node (interpol_lptable, src/Rellp.cpp:219-247)
-  const bool lp = (rq.emis_type == EMIS_LP);
-  const DevLpTable &L = b.lp;
+  if (lp) lp_rows(L, rq, s_jr, s_je, s_jd, s_ji, tid, NT);
+  // returning radiation: the zones' centres and returning emissivity (k_rrad)
+  const bool rrad = lp && rq.return_rad != 0;
+  const int rr_n = rq.rr_n;
+  if (rrad) {
+    const double *rr = b.rret + (size_t)rq.rr_slot * (2 * MAX_RR);
+    for (int i = tid; i < rr_n; i += NT) {
+      s_rr_rad[i] = rr[i];
+      s_rr_ret[i] = rr[MAX_RR + i];
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    // ISCO snap (src/Relprofile.cpp:195-200)
+    const double rms = rq.rms;
+    if (lane == 0 && (s_tre[n_r - 1] > rms) && ((s_tre[n_r - 1] - rms) / s_tre[n_r - 1] < 1e-3)) s_tre[n_r - 1] = rms;
+    __builtin_amdgcn_wave_barrier();  // (one wavefront: LDS operations are in order)
+    int c_in = 0, c_out = 0;  // nodes not below Rin / Rout (bsearch_desc, src/relutility.c:195-211)
+    for (int k = 0; k < n_r; k += 64) {
+      const bool v = k + lane < n_r;
+      const double t = s_tre[min(k + lane, n_r - 1)];
+      c_in += __popcll(__ballot(v && !(t < rq.rin)));
+      c_out += __popcll(__ballot(v && !(t < rq.rout)));
+    }
+    const int ind_rmin = min(max(c_in - 1, 0), n_r - 2), ind_rmax = min(max(c_out - 1, 0), n_r - 2);
+    if (lane == 0) {
+      int st = 0;
+      // 1000 rg snap (:235-238)
+      if (s_tre[ind_rmax] < 1000.0 && s_tre[ind_rmax] * 1.01 > 1000.0) s_tre[ind_rmax] = 1000.0;
+      if (!(ind_rmin > 0) || !(s_tre[ind_rmin + 1] <= rq.rin) || !(s_tre[ind_rmin] >= rq.rin) ||
+          !(s_tre[ind_rmax + 1] <= rq.rout) || !(s_tre[ind_rmax] >= rq.rout) ||
+          !(ind_rmax <= ind_rmin) || !(rq.rout <= 1000.0)) {
+        st = 12;
+      }
+      s_rmin = ind_rmin;
+      s_st = st;
+    }
+  }
   __syncthreads();
   if (s_st) {
     if (tid == 0) b.status[req] = s_st;
@@ -645,43 +692,63 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
   }
   {  // the node arrays the radius records are rebuilt from (rad_geo)
     double *gn = b.rnode + (size_t)req * RAD_NODE_ARRAYS * n_r;
-    for (int ir = tid; ir < n_r; ir += SETUP_THREADS) {
+    for (int ir = tid; ir < n_r; ir += NT) {
       gn[ir] = s_tre[ir];
       gn[n_r + ir] = s_tgmin[ir];
       gn[2 * n_r + ir] = s_tgmax[ir];
     }
   }
-  const int ntr = L.n_r;
-  if (lp) lp_rows(L, rq, s_jr, s_je, s_jd, s_ji, tid, SETUP_THREADS);
+  const double r1g = fine_radius_r1(rq.rout), r2g = fine_radius_r1(rq.rin);
+  auto fr = [&](int ii) { return fine_radius_at(r1g, r2g, ii, nr); };
+
+  // reflection fractions (calc_refl_frac, src/Rellp.cpp:36-89): lane 0 takes the
+  // inner edge, lane 1 the outer one (the wavefront with the fewest radii)
+  if (lp && wave == NW - 1) {
+    const double edge = lane == 0 ? rq.rin : rq.rout;
+    int klo = lane == 0 ? nr - 2 : 0;  // what the search below finds on a descending grid
+    const bool plain = lane == 0 ? !(fr(klo) < edge) : (fr(1) < edge);
+    if (!plain && lane < 2) {
+      klo = 0;
+      int khi = nr - 1;
+      while (khi - klo > 1) {
+        const int k = (khi + klo) / 2;
+        if (fr(k) < edge) khi = k; else klo = k;
+      }
+    }
+    double del = lp_on_fine(fr(klo), s_jr, s_je, s_jd, s_ji, ntr).del_emit;
+    double dmax = s_jd[ntr - 1];
+    if (dmax < PI / 2.0) dmax = PI / 2.0;
+    if (rq.beta > 1e-6) del = relat_abberation(del, -1. * rq.beta);
+    const double cdel = cos(del);
+    const double cos_bh = readlane_d(cdel, 0), cos_ad = readlane_d(cdel, 1);
+    LpRefl o;
+    o.f_bh = 0.5 * (1.0 - cos_bh);
+    o.f_ad = 0.5 * (cos_bh - cos_ad);
+    o.f_inf_rest = 0.5 * (1.0 + cos(dmax));
+    o.f_inf = (rq.beta > 1e-6) ? 0.5 * (1.0 + cos(relat_abberation(dmax, -1. * rq.beta))) : o.f_inf_rest;
+    o.refl_frac = o.f_ad / o.f_inf;
+    if (lane == 0) {
+      if (!(o.f_inf + o.f_ad < 1.0)) atomicMax(&s_st, 20);
+      b.refl[req] = o;
+    }
+  }
 
   // fine radii: node -> fine map (:249-300), emissivity, energy window (:859-878)
   RadRec *rad = b.rad + (size_t)req * nr;
   const GridGuess gE = grid_guess(E, rq.n_e);
   auto ge = [&](int k) { return E[k]; };
+  const double e_lo = E[0], e_hi = E[rq.n_e];
   double area = 0.0;
   double cmax = 0.0;  // largest weight of a radius with a window
   int err = 0;
-  auto lp_emis = [&](double re) { return lp_emis_at(rq, re, s_jr, s_je, s_jd, s_ji, ntr, &err); };
-  // returning radiation: the zones' centres and returning emissivity (k_rrad)
-  __shared__ double s_rr_rad[MAX_RR], s_rr_ret[MAX_RR];
-  const bool rrad = lp && rq.return_rad != 0;
-  const int rr_n = rq.rr_n;
-  if (rrad) {
-    const double *rr = b.rret + (size_t)rq.rr_slot * (2 * MAX_RR);
-    for (int i = tid; i < rr_n; i += SETUP_THREADS) {
-      s_rr_rad[i] = rr[i];
-      s_rr_ret[i] = rr[MAX_RR + i];
-    }
-    __syncthreads();
-  }
-  for (int ii0 = 0; ii0 < nr; ii0 += SETUP_THREADS) {  // same trip count in every wavefront
+  for (int ii0 = 0; ii0 < nr; ii0 += NT) {  // same trip count in every wavefront
     const int ii = ii0 + tid;
     int wlo = 0x7fffffff, whi = -1;
     int izone = -1;
     if (ii < nr) {
-    const double re = fine_radius(rq.rin, rq.rout, ii, nr);
-    const double rprev = (ii > 0) ? fine_radius(rq.rin, rq.rout, ii - 1, nr) : 0.0;
-    const double rnext = (ii < nr - 1) ? fine_radius(rq.rin, rq.rout, ii + 1, nr) : 0.0;
+    const double re = fr(ii);
+    const double rprev = (ii > 0) ? fr(ii - 1) : 0.0;
+    const double rnext = (ii < nr - 1) ? fr(ii + 1) : 0.0;
     // K = largest k <= ind_rmin with tre[k] > re: the walk of :250-265 starts
     // at the Rin bracket and only moves outwards, so a fine radius rounded
     // just below the innermost node extrapolates that bracket (ifac_r < 0)
@@ -711,23 +778,23 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
       const double alpha = (re > rq.rbr) ? rq.emis2 : rq.emis1;
       emis = pow(re / rq.rbr, -alpha);
       area += emis * (tz * 2);
-    } else if (!rrad) {
-      emis = lp_emis(re);
     } else {
-      // the returning emissivity at this radius (rebin_emisprofile_on_radial_grid,
-      // src/Rellp.cpp:120-175: linear radius factor, log-interpolated values)
-      const int kk = min(max(bsearch_asc(s_rr_rad, rr_n, re), 0), rr_n - 2);
-      const double fr = (re - s_rr_rad[kk]) / (s_rr_rad[kk + 1] - s_rr_rad[kk]);
-      const double er = exp(fr * log(s_rr_ret[kk + 1]) + (1.0 - fr) * log(s_rr_ret[kk]));
-      const double direct = lp_emis(re);
-      emis = (rq.return_rad == 1) ? direct + er : er;
+      emis = lp_emis_at(rq, re, s_jr, s_je, s_jd, s_ji, ntr, &err);
+      if (rrad) {
+        // the returning emissivity at this radius (rebin_emisprofile_on_radial_grid,
+        // src/Rellp.cpp:120-175: linear radius factor, log-interpolated values)
+        const int kk = min(max(bsearch_asc(s_rr_rad, rr_n, re), 0), rr_n - 2);
+        const double f = (re - s_rr_rad[kk]) / (s_rr_rad[kk + 1] - s_rr_rad[kk]);
+        const double er = exp(f * log(s_rr_ret[kk + 1]) + (1.0 - f) * log(s_rr_ret[kk]));
+        emis = (rq.return_rad == 1) ? emis + er : er;
+      }
     }
     // energy window
     double egmin = gmin, egmax = gmax;
     int ielo = 1, iehi = 0;
-    if ((egmax > E[0]) && (egmin < E[rq.n_e])) {
-      if (egmin < E[0]) egmin = E[0];
-      if (egmax > E[rq.n_e]) egmax = E[rq.n_e];
+    if ((egmax > e_lo) && (egmin < e_hi)) {
+      if (egmin < e_lo) egmin = e_lo;
+      if (egmax > e_hi) egmax = e_hi;
       // binary_search (src/relutility.c:155-171) on [E0, E_n]: count - 1, at most n-1
       ielo = min(count_le(ge, rq.n_e, egmin, gE) - 1, rq.n_e - 1);
       iehi = min(count_le(ge, rq.n_e, egmax, gE) - 1, rq.n_e - 1);
@@ -749,7 +816,7 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
     for (int z = zlo; z <= zhi; z++) {
       const int zl = wave_min_i(izone == z ? wlo : 0x7fffffff);
       const int zh = wave_max_i(izone == z ? whi : -1);
-      if ((tid & 63) == 0) {
+      if (lane == 0) {
         s_ulo[(ii / RAD_CHUNK) * NZ + z] = zl;
         s_uhi[(ii / RAD_CHUNK) * NZ + z] = zh;
       }
@@ -758,110 +825,63 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
   if (err) atomicMax(&s_st, err);
   // BKN normalisation: sum emis * 2 pi r dr (norm_emis_profile, src/Rellp.cpp:91-109),
   // applied through ReqNorm instead of a second pass over the records
-  const double total = block_sum(area, s_red);
-  const double cmax_all = block_max(cmax, s_red);
+  const double area_w = wave_sum(area), cmax_w = wave_max_d(cmax);
+  if (lane == 0) {
+    s_sum[wave] = area_w;
+    s_max[wave] = cmax_w;
+  }
+  __syncthreads();
   if (s_st) {
     if (tid == 0) b.status[req] = s_st;
     return;
   }
-  const double fac = lp ? 1.0 : 1.0 / total;
-  if (tid == 0) {
-    ReqNorm n;
-    n.fac = fac;
-    n.fa = fa;
-    n.fm = fm;
-    n.ia = ia;
-    n.im = im;
-    n.r1 = fine_radius_r1(rq.rout);
-    n.r2 = fine_radius_r1(rq.rin);
-    const double m = cmax_all * fac;
-    int k = 0;
-    if (m > 0.0 && m < INFINITY) k = min(1000, max(-1000, -ilogb(m)));
-    n.cmul = ldexp(fac, k);
-    n.cinv = ldexp(1.0, -k);
-    b.rnorm[req] = n;
-  }
-
-  // reflection fractions (calc_refl_frac, src/Rellp.cpp:36-89)
-  if (lp && tid == 0) {
-    auto fr = [&](int ii) { return fine_radius(rq.rin, rq.rout, ii, nr); };
-    int klo = 0, khi = nr - 1;
-    while (khi - klo > 1) {
-      int k = (khi + klo) / 2;
-      if (fr(k) < rq.rin) khi = k; else klo = k;
-    }
-    const int ibh = klo;
-    klo = 0;
-    khi = nr - 1;
-    while (khi - klo > 1) {
-      int k = (khi + klo) / 2;
-      if (fr(k) < rq.rout) khi = k; else klo = k;
-    }
-    const int iad = klo;
-    double del_bh = lp_on_fine(fr(ibh), s_jr, s_je, s_jd, s_ji, ntr).del_emit;
-    double del_ad = lp_on_fine(fr(iad), s_jr, s_je, s_jd, s_ji, ntr).del_emit;
-    double dmax = s_jd[ntr - 1];
-    if (dmax < PI / 2.0) dmax = PI / 2.0;
-    if (rq.beta > 1e-6) {
-      del_bh = relat_abberation(del_bh, -1. * rq.beta);
-      del_ad = relat_abberation(del_ad, -1. * rq.beta);
-    }
-    LpRefl o;
-    o.f_bh = 0.5 * (1.0 - cos(del_bh));
-    o.f_ad = 0.5 * (cos(del_bh) - cos(del_ad));
-    o.f_inf_rest = 0.5 * (1.0 + cos(dmax));
-    o.f_inf = (rq.beta > 1e-6) ? 0.5 * (1.0 + cos(relat_abberation(dmax, -1. * rq.beta))) : o.f_inf_rest;
-    o.refl_frac = o.f_ad / o.f_inf;
-    if (!(o.f_inf + o.f_ad < 1.0)) s_st = 20;
-    b.refl[req] = o;
-  }
-
-  if (rq.n_incl > 0) {  // k_dist adds into the angle distribution
-    const int nd = rq.n_incl * nz;  // [zone][angle bin]
-    for (int k = tid; k < nd; k += SETUP_THREADS) b.dist[rq.dist_off + k] = 0.0;
-  }
-  __syncthreads();
-  if (s_st == 0) {
-    // the profile accumulates with atomic adds: clear the bins any window
-    // reaches (k_finalize writes zeros elsewhere)
-    int jlo = 0x7fffffff, jhi = -1;
-    for (int c = 0; c < n_rc; c++) {
-      for (int z = 0; z < nz; z++) {
-        jlo = min(jlo, s_ulo[c * NZ + z]);
-        jhi = max(jhi, s_uhi[c * NZ + z]);
-      }
-    }
-    if (tid == 0) b.reach[req] = BinRange{jlo, jhi};
-    double *acc = profile_acc(b, rq);
-    // (no window reaches the grid: jlo = INT_MAX > jhi = -1, nothing to clear;
-    // jlo + tid must not be formed then, it would overflow); every zone's
-    // profile over the union of the windows
-    if (jlo <= jhi)
-      for (int z = 0; z < nz; z++)
-        for (int j = jlo + tid; j <= jhi; j += SETUP_THREADS) acc[(size_t)z * rq.n_e + j] = 0.0;
-    // work items: the window of each (radius chunk, zone) cut into segments
-    // of seg_bins; the item's chunk and zone share its rc field.  An item's
-    // time grows with its bins, so segments of at least S / 4 bins go to the
-    // front of the list and the shorter last segments of windows to its back:
-    // k_integrate hands out the long ones first and the wavefronts finish
-    // together on short ones.
-    const int S = b.seg_bins;
-    const int thr = max(1, S / 4);
-    const int n_cz = n_rc * nz;  // pairs q = c nz + z; their windows sit at c NZ + z
-    if (tid == 0) {
-      int tot = 0, tots = 0;
-      for (int q = 0; q < n_cz; q++) {
+  // work items: the window of each (radius chunk, zone) cut into segments
+  // of seg_bins; the item's chunk and zone share its rc field.  An item's
+  // time grows with its bins, so segments of at least S / 4 bins go to the
+  // front of the list and the shorter last segments of windows to its back:
+  // k_integrate hands out the long ones first and the wavefronts finish
+  // together on short ones.  One wavefront lists the windows (64 at a time,
+  // their numbers of segments summed across the lanes) and reserves the
+  // request's places; another one writes the request's norms.
+  const int S = b.seg_bins;
+  const int thr = max(1, S / 4);
+  const int n_cz = n_rc * nz;  // pairs q = c nz + z; their windows sit at c NZ + z
+  if (wave == 0) {
+    int jlo = 0x7fffffff, jhi = -1, tot = 0, tots = 0;
+    for (int q0 = 0; q0 < n_cz; q0 += 64) {
+      const int q = q0 + lane;
+      int nlong = 0, nshort = 0;
+      if (q < n_cz) {
         const int w = (q / nz) * NZ + q % nz;
-        s_pref[q] = tot;
-        s_prefs[q] = tots;
-        if (s_uhi[w] >= s_ulo[w]) {
-          const int len = s_uhi[w] - s_ulo[w] + 1;
+        const int lo = s_ulo[w], hi = s_uhi[w];
+        if (hi >= lo) {
+          jlo = min(jlo, lo);
+          jhi = max(jhi, hi);
+          const int len = hi - lo + 1;
           const int nseg = (len + S - 1) / S;
-          const int nlong = nseg - 1 + (len - (nseg - 1) * S >= thr ? 1 : 0);
-          tot += nlong;
-          tots += nseg - nlong;
+          nlong = nseg - 1 + (len - (nseg - 1) * S >= thr ? 1 : 0);
+          nshort = nseg - nlong;
         }
       }
+      int pl = nlong, ps = nshort;  // inclusive sums over the lanes
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int ul = __shfl_up(pl, d, 64), us = __shfl_up(ps, d, 64);
+        if (lane >= d) {
+          pl += ul;
+          ps += us;
+        }
+      }
+      if (q < n_cz) {
+        s_pref[q] = tot + pl - nlong;
+        s_prefs[q] = tots + ps - nshort;
+      }
+      tot += __builtin_amdgcn_readlane(pl, 63);
+      tots += __builtin_amdgcn_readlane(ps, 63);
+    }
+    jlo = wave_min_i(jlo);
+    jhi = wave_max_i(jhi);
+    if (lane == 0) {
       int base = atomicAdd(&b.ctr[CTR_ITEMS], tot);
       const int bases = atomicAdd(&b.ctr[CTR_ITEMS_S], tots);
       // cannot happen: the host sizes the list for every bin of every request
@@ -872,24 +892,55 @@ __global__ __launch_bounds__(SETUP_THREADS, 3) void k_setup(BatchDev b) {
       }
       s_base = base;
       s_bases = bases;
+      s_jlo = jlo;
+      s_jhi = jhi;
+      b.reach[req] = BinRange{jlo, jhi};
     }
-    __syncthreads();
-    if (s_base >= 0) {
-      for (int q = tid; q < n_cz; q += SETUP_THREADS) {
-        const int c = q / nz, z = q % nz, w = c * NZ + z;
-        int k = s_base + s_pref[q], ks = s_bases + s_prefs[q];
-        for (int j0 = s_ulo[w]; j0 <= s_uhi[w]; j0 += S) {
-          WorkItem it;
-          it.req = req;
-          it.rc = c | (z << 16);
-          it.j0 = j0;
-          it.j1 = min(s_uhi[w] + 1, j0 + S);
-          if (it.j1 - it.j0 >= thr) b.items[k++] = it;
-          else b.items[b.item_cap - 1 - ks++] = it;
-        }
+  } else if (wave == 1 && lane == 0) {
+    double total = s_sum[0], cmax_all = s_max[0];
+    for (int w = 1; w < NW; w++) {
+      total += s_sum[w];
+      cmax_all = fmax(cmax_all, s_max[w]);
+    }
+    ReqNorm n;
+    n.fac = lp ? 1.0 : 1.0 / total;
+    n.fa = fa;
+    n.fm = fm;
+    n.ia = ia;
+    n.im = im;
+    n.r1 = r1g;
+    n.r2 = r2g;
+    const double m = cmax_all * n.fac;
+    int k = 0;
+    if (m > 0.0 && m < INFINITY) k = min(1000, max(-1000, -ilogb(m)));
+    n.cmul = ldexp(n.fac, k);
+    n.cinv = ldexp(1.0, -k);
+    b.rnorm[req] = n;
+  }
+  __syncthreads();
+  // the profile accumulates with atomic adds: clear the bins any window
+  // reaches (k_finalize writes zeros elsewhere); every zone's profile over the
+  // union of the windows.  (No window reaches the grid: jlo = INT_MAX > jhi =
+  // -1, nothing to clear; jlo + tid must not be formed then, it would overflow.)
+  const int jlo = s_jlo, jhi = s_jhi;
+  double *acc = profile_acc(b, rq);
+  if (jlo <= jhi)
+    for (int z = 0; z < nz; z++)
+      for (int j = jlo + tid; j <= jhi; j += NT) acc[(size_t)z * rq.n_e + j] = 0.0;
+  if (s_base >= 0) {
+    for (int q = tid; q < n_cz; q += NT) {
+      const int c = q / nz, z = q % nz, w = c * NZ + z;
+      int k = s_base + s_pref[q], ks = s_bases + s_prefs[q];
+      for (int j0 = s_ulo[w]; j0 <= s_uhi[w]; j0 += S) {
+        WorkItem it;
+        it.req = req;
+        it.rc = c | (z << 16);
+        it.j0 = j0;
+        it.j1 = min(s_uhi[w] + 1, j0 + S);
+        if (it.j1 - it.j0 >= thr) b.items[k++] = it;
+        else b.items[b.item_cap - 1 - ks++] = it;
       }
     }
-    __syncthreads();
   }
   if (tid == 0) b.status[req] = s_st;
 }
@@ -1929,8 +1980,8 @@ __global__ __launch_bounds__(64) void k_fixup(BatchDev b, int cos_rows) {
 // ---------------------------------------------------------------------------
 // finalize: renormalisation (renorm_relline_profile, src/Relprofile.cpp:749-796)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(SETUP_THREADS) void k_finalize(BatchDev b) {
-  __shared__ double s_red[SETUP_THREADS];
+__global__ __launch_bounds__(FINAL_THREADS) void k_finalize(BatchDev b) {
+  __shared__ double s_red[FINAL_THREADS];
   const int req = blockIdx.x;
   const int tid = threadIdx.x;
   const ReqParams rq = b.req[req];
@@ -1939,14 +1990,14 @@ __global__ __launch_bounds__(SETUP_THREADS) void k_finalize(BatchDev b) {
   double *dst = profile_acc(b, rq);
   const int st = b.status[req];
   if (st != 0) {
-    for (int j = tid; j < n_e * rq.n_zones; j += SETUP_THREADS) dst[j] = 0.0;
+    for (int j = tid; j < n_e * rq.n_zones; j += FINAL_THREADS) dst[j] = 0.0;
     return;
   }
   if (rq.prof_off < 0) {  // line models; convolution profiles are finished by k_conv
     const double *E = b.pgrid + rq.pgrid_off;
     const BinRange rc = b.reach[req];
     double loc = 0.0;
-    for (int j = tid; j < n_e; j += SETUP_THREADS) {
+    for (int j = tid; j < n_e; j += FINAL_THREADS) {
       double v = 0.0;
       if (j >= rc.lo && j <= rc.hi) v = dst[j] / (0.5 * (E[j] + E[j + 1]));
       dst[j] = v;
@@ -1955,15 +2006,15 @@ __global__ __launch_bounds__(SETUP_THREADS) void k_finalize(BatchDev b) {
     const double sum = block_sum(loc, s_red);
     if (rq.do_renorm) {
       const double f = rq.norm / sum;
-      for (int j = tid; j < n_e; j += SETUP_THREADS) dst[j] *= f;
+      for (int j = tid; j < n_e; j += FINAL_THREADS) dst[j] *= f;
     }
   }
   for (int z = 0; rq.n_incl > 0 && z < rq.n_zones; z++) {  // each zone's distribution sums to 1
     double *d = b.dist + rq.dist_off + (size_t)z * rq.n_incl;
     double ds = 0.0;
-    for (int k = tid; k < rq.n_incl; k += SETUP_THREADS) ds += d[k];
+    for (int k = tid; k < rq.n_incl; k += FINAL_THREADS) ds += d[k];
     const double dsum = block_sum(ds, s_red);
-    for (int k = tid; k < rq.n_incl; k += SETUP_THREADS) d[k] /= dsum;
+    for (int k = tid; k < rq.n_incl; k += FINAL_THREADS) d[k] /= dsum;
   }
 }
 
@@ -2857,10 +2908,13 @@ int launch_deliver(const BatchDev &b, int *res, double *res_out, int64_t n_out, 
 
 int launch_setup(const BatchDev &b, void *stream) {
   if (b.n_req <= 0) return 0;
-  if (b.max_zones > LP_ZONES)
-    hipLaunchKernelGGL(k_setup<MAX_ZONES>, dim3(b.n_req), dim3(SETUP_THREADS), 0, (hipStream_t)stream, b);
-  else
-    hipLaunchKernelGGL(k_setup<LP_ZONES>, dim3(b.n_req), dim3(SETUP_THREADS), 0, (hipStream_t)stream, b);
+  auto go = [&](auto kern, int nt) { hipLaunchKernelGGL(kern, dim3(b.n_req), dim3(nt), 0, (hipStream_t)stream, b); };
+  // up to one workgroup a CU the wide form (256 requests: 28 us, 31 us with 256
+  // threads); 512 requests: 44 us and 39 us.  1024 threads spill (128 registers)
+  // and are no faster than 512 for one request.
+  const bool wide = b.n_req <= 256;
+  if (b.max_zones > LP_ZONES) wide ? go(k_setup<MAX_ZONES, 512>, 512) : go(k_setup<MAX_ZONES, 256>, 256);
+  else wide ? go(k_setup<LP_ZONES, 512>, 512) : go(k_setup<LP_ZONES, 256>, 256);
   return (int)hipGetLastError();
 }
 
@@ -2935,7 +2989,7 @@ int launch_fixup(const BatchDev &b, bool cos_rows, void *stream) {
 
 int launch_finalize(const BatchDev &b, void *stream) {
   if (b.n_req <= 0) return 0;
-  hipLaunchKernelGGL(k_finalize, dim3(b.n_req), dim3(SETUP_THREADS), 0, (hipStream_t)stream, b);
+  hipLaunchKernelGGL(k_finalize, dim3(b.n_req), dim3(FINAL_THREADS), 0, (hipStream_t)stream, b);
   return (int)hipGetLastError();
 }
 
