@@ -612,9 +612,20 @@ int rx_batch_dist(rx_batch *b, int i, double *dist, int n_incl) {
   const ReqParams &p = b->b.h_req[i];
   if (n_incl > p.n_incl * p.n_zones) return RX_ERR_ARG;
   if (n_incl == 0) return RX_OK;
-  if (hipMemcpy(dist, b->b.dev.dist + p.dist_off, sizeof(double) * n_incl,
-                hipMemcpyDeviceToHost) != hipSuccess)
+  // the device keeps the zones' sums as they are: normalised here
+  double d[MAX_ZONES * MAX_INCL];
+  const size_t nd = (size_t)p.n_incl * p.n_zones;
+  int st = 0;
+  if (nd > sizeof d / sizeof d[0]) return RX_ERR_ARG;  // (a build refuses more)
+  if (hipMemcpy(d, b->b.dev.dist + p.dist_off, sizeof(double) * nd, hipMemcpyDeviceToHost) != hipSuccess ||
+      hipMemcpy(&st, b->b.dev.status + i, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess)
     return RX_ERR_DEVICE;
+  for (int z = 0; st == 0 && p.model != MOD_XILLVER && z < p.n_zones; z++) {
+    double *dz = d + (size_t)z * p.n_incl, sum = 0.0;
+    for (int k = 0; k < p.n_incl; k++) sum += dz[k];
+    for (int k = 0; k < p.n_incl; k++) dz[k] /= sum;
+  }
+  std::copy(d, d + n_incl, dist);
   return RX_OK;
 }
 

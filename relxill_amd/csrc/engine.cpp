@@ -1206,11 +1206,12 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
       memcpy(b.p_flux + p.flux_off, r.flux_in, sizeof(double) * r.n_flux);
   }
   b.any_cosne = false;
-  b.any_limb = false;
+  b.any_limb = b.any_angular = false;
   int64_t bins = 0;
   for (int i = 0; i < n_req; i++) {
     b.any_cosne |= b.h_req[i].need_cosne != 0;
     b.any_limb |= b.h_req[i].limb != 0;
+    b.any_angular |= b.h_req[i].model == MOD_RELXILL_CONV;
     bins += b.h_req[i].n_e;
   }
   // shape class for the autotuner: log2 of the total profile bins, conv flag
@@ -1521,7 +1522,7 @@ static int launch_sequence(Batch &b, const RunKey &k, hipStream_t s) {
   if (prof) e |= (int)hipEventRecord(b.ev[4], s);
   e |= launch_xill(bd, w.xill, w.n_xill1, w.n_xill - w.n_xill1, s);
   if (prof) e |= (int)hipEventRecord(b.ev[5], s);
-  e |= launch_conv(bd, w.conv, w.n_conv, s);
+  e |= launch_conv(bd, w.conv, w.n_conv, k.angular != 0, s);
   if (prof) e |= (int)hipEventRecord(b.ev[6], s);
   e |= launch_primary(bd, w.prim, w.n_prim, k.prim_bins, s);
   if (prof) e |= (int)hipEventRecord(b.ev[7], s);
@@ -1577,8 +1578,7 @@ int batch_run(Batch &b, int precision, std::string &err) {
   k.n_blocks = b.n_blocks;
   memcpy(&k.wl, &b.wl, sizeof(k.wl));
   k.prim_bins = b.prim_bins;
-  // only line profiles and angle distributions are finished by k_finalize
-  k.finalize = b.tot_pgrid > 0 || !b.h_ang.empty();
+  k.finalize = b.tot_pgrid > 0;  // (line profiles)
   if (b.call_run) {
     k.fetch_src = b.h_stage.p;
     k.fetch_dst = b.d_arena.p;
@@ -1595,6 +1595,7 @@ int batch_run(Batch &b, int precision, std::string &err) {
   }
   k.prof = g.profile ? 1 : 0;
   k.cos_rows = b.any_limb ? 1 : 0;
+  k.angular = b.any_angular ? 1 : 0;
   hipStream_t s = b.stream;
   b.profiled = k.prof != 0;
   if (g.use_graphs && !b.graph_failed && !b.one_shot) {

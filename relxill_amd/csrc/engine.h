@@ -69,7 +69,7 @@ struct RunKey {
   BatchDev bd;
   WorkLists wl;
   int n_blocks, prim_bins;
-  int prof, cos_rows, finalize;
+  int prof, cos_rows, finalize, angular;
   // the request block fetched from pinned host memory at the start of the run
   // (n_fetch 16-byte words; 0: it is on the device) and the results delivered
   // there at its end (n_out output values; 0: statuses and counters only)
@@ -138,7 +138,7 @@ struct Batch {
   std::mutex out_mu;                   // readers of one batch in several threads
   int item_cap = 0;
   int n_blocks = 1;  // workgroups of k_integrate
-  bool any_cosne = false, any_limb = false;
+  bool any_cosne = false, any_limb = false, any_angular = false;
   bool any_flux = false;  // some request has an input spectrum
   int fix_cap = 0;
   int last_mode = 1;

@@ -1560,7 +1560,7 @@ struct EdgeWalk {
 // in a register while its bin stays and adds to the LDS bins when it changes;
 // the wavefront's last bins go as one wave sum when all lanes share the bin.
 // The chunk's sums are added to the request's distribution in HBM (cleared by
-// k_setup, normalised by k_finalize).
+// k_setup, left unnormalised: its readers scale by its sum).
 // Bound: FP64 issue, 1000 radii x 2 n_g columns x ~60 operations a request,
 // which one CU takes 16 us for: inside k_setup (one workgroup a request) it
 // was 61 us of a single relxill call (k_setup 87 us) and 165 us of a batch of
@@ -1980,12 +1980,16 @@ __global__ __launch_bounds__(64) void k_fixup(BatchDev b, int cos_rows) {
 // ---------------------------------------------------------------------------
 // finalize: renormalisation (renorm_relline_profile, src/Relprofile.cpp:749-796)
 // ---------------------------------------------------------------------------
+// Line models only: a convolution's profile and angle distribution are sums that
+// their readers (k_conv, k_xill) scale themselves, each by one factor.  While
+// the distributions were normalised here, ten zones' block sums one after the
+// other took 12-14 us of a relxilllp call, one zone's 4.6 us.
 __global__ __launch_bounds__(FINAL_THREADS) void k_finalize(BatchDev b) {
   __shared__ double s_red[FINAL_THREADS];
   const int req = blockIdx.x;
   const int tid = threadIdx.x;
-  const ReqParams rq = b.req[req];
-  if (rq.model == MOD_XILLVER) return;  // no profile; k_primary writes the output
+  const ReqParams &rq = b.req[req];
+  if (rq.prof_off >= 0 || rq.model == MOD_XILLVER) return;
   const int n_e = rq.n_e;
   double *dst = profile_acc(b, rq);
   const int st = b.status[req];
@@ -1993,28 +1997,19 @@ __global__ __launch_bounds__(FINAL_THREADS) void k_finalize(BatchDev b) {
     for (int j = tid; j < n_e * rq.n_zones; j += FINAL_THREADS) dst[j] = 0.0;
     return;
   }
-  if (rq.prof_off < 0) {  // line models; convolution profiles are finished by k_conv
-    const double *E = b.pgrid + rq.pgrid_off;
-    const BinRange rc = b.reach[req];
-    double loc = 0.0;
-    for (int j = tid; j < n_e; j += FINAL_THREADS) {
-      double v = 0.0;
-      if (j >= rc.lo && j <= rc.hi) v = dst[j] / (0.5 * (E[j] + E[j + 1]));
-      dst[j] = v;
-      loc += v;
-    }
-    const double sum = block_sum(loc, s_red);
-    if (rq.do_renorm) {
-      const double f = rq.norm / sum;
-      for (int j = tid; j < n_e; j += FINAL_THREADS) dst[j] *= f;
-    }
+  const double *E = b.pgrid + rq.pgrid_off;
+  const BinRange rc = b.reach[req];
+  double loc = 0.0;
+  for (int j = tid; j < n_e; j += FINAL_THREADS) {
+    double v = 0.0;
+    if (j >= rc.lo && j <= rc.hi) v = dst[j] / (0.5 * (E[j] + E[j + 1]));
+    dst[j] = v;
+    loc += v;
   }
-  for (int z = 0; rq.n_incl > 0 && z < rq.n_zones; z++) {  // each zone's distribution sums to 1
-    double *d = b.dist + rq.dist_off + (size_t)z * rq.n_incl;
-    double ds = 0.0;
-    for (int k = tid; k < rq.n_incl; k += FINAL_THREADS) ds += d[k];
-    const double dsum = block_sum(ds, s_red);
-    for (int k = tid; k < rq.n_incl; k += FINAL_THREADS) d[k] /= dsum;
+  const double sum = block_sum(loc, s_red);
+  if (rq.do_renorm) {
+    const double f = rq.norm / sum;
+    for (int j = tid; j < n_e; j += FINAL_THREADS) dst[j] *= f;
   }
 }
 
@@ -2211,23 +2206,34 @@ __device__ inline double block_sum4(double v, double *s_w) {
   return t;
 }
 
-// Two block sums at once (one pair of barriers).
-__device__ inline void block_sum2(double a, double c, double *out, double (*s_w)[CONV_THREADS_MAX / 64]) {
-  const double wa = wave_sum(a), wc = wave_sum(c);
+// N block sums at once (one pair of barriers).
+template <int N>
+__device__ inline void block_sums(const double *v, double *out, double (*s_w)[CONV_THREADS_MAX / 64]) {
   const int wave = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    s_w[0][wave] = wa;
-    s_w[1][wave] = wc;
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    const double w = wave_sum(v[i]);
+    if ((threadIdx.x & 63) == 0) s_w[i][wave] = w;
+    out[i] = 0.0;
   }
   __syncthreads();
-  double ta = 0.0, tc = 0.0;
-  for (int k = 0; k < (int)(blockDim.x >> 6); k++) {
-    ta += s_w[0][k];
-    tc += s_w[1][k];
-  }
+  for (int k = 0; k < (int)(blockDim.x >> 6); k++)
+#pragma unroll
+    for (int i = 0; i < N; i++) out[i] += s_w[i][k];
   __syncthreads();
-  out[0] = ta;
-  out[1] = tc;
+}
+
+// The power of two at or below a normal v > 0; 0 for every other v.
+__device__ inline double pow2_of(double v) {
+  const long long e = __double_as_longlong(v) & 0x7ff0000000000000ll;
+  return v > 0 && e != 0x7ff0000000000000ll ? __longlong_as_double(e) : 0.0;
+}
+
+// Sum of one zone's angle distribution as k_dist leaves it.
+__device__ inline double dist_sum(const double *d, int n) {
+  double s = 0.0;
+  for (int k = 0; k < n; k++) s += d[k];
+  return s;
 }
 
 // calcFFTNormFactor band (src/Relbase.cpp:205): bins with E_lo >= 0.01 and
@@ -2244,9 +2250,16 @@ __device__ inline bool in_band(const DevConvGrid &cg, int i) { return i >= cg.ba
 // and inverted with a half-length complex FFT.  Grid-walking phases give each
 // wavefront a contiguous run of bins, one bin per lane, so that neighbouring
 // lanes read neighbouring addresses.
+// WIDE: launch_conv's form for few units.  ANG: relxill_conv requests (resident
+// reflection spectra weighted by the angle distribution) are among the units;
+// ANG == 0 compiles them out, which frees the scalar registers that were spilled
+// (4096 relconv units 356 us and 350 us).
+// Bound: the latency of the phases between the barriers for few units, LDS
+// traffic and FP64 issue for many (two workgroups a CU: 70 KB of LDS each).
+template <int WIDE, int ANG>
 __global__ __launch_bounds__(CONV_THREADS_MAX) void k_conv(BatchDev b, const XillWork *__restrict__ work) {
   extern __shared__ double2 s_buf[];  // P(n) complex
-  __shared__ double s_w[2][CONV_THREADS_MAX / 64];
+  __shared__ double s_w[3][CONV_THREADS_MAX / 64];
   const int NT = blockDim.x;
   const int req = work[blockIdx.x].req;
   const int zone = work[blockIdx.x].zone;
@@ -2267,7 +2280,7 @@ __global__ __launch_bounds__(CONV_THREADS_MAX) void k_conv(BatchDev b, const Xil
   const double *Ec = cg.ener;
   const double *cf = cg.cfac;
   const double2 *tw = reinterpret_cast<const double2 *>(cg.tw);
-  const bool angular = (rq.model == MOD_RELXILL_CONV);
+  const bool angular = ANG && rq.model == MOD_RELXILL_CONV;
   const bool relxill = (rq.model == MOD_RELXILL || rq.model == MOD_RELXILLLP);
   // input: the caller's spectrum, or for relxill each zone's angle-weighted
   // xillver spectrum on the table grid (k_xill)
@@ -2302,7 +2315,7 @@ __global__ __launch_bounds__(CONV_THREADS_MAX) void k_conv(BatchDev b, const Xil
   const double *fin = relxill ? b.xspec + rq.xspec_off + (size_t)zone * n_in : b.flux_in + rq.flux_off;
   const double *dist = b.dist + rq.dist_off + (size_t)zone * rq.n_incl;
   // 1. x = rebinned input * E/dE (real part), y = rotated profile * E/dE (imag part)
-  double sx = 0.0;
+  double sx = 0.0, sxa = 0.0;  // band sum, sum of the magnitudes
   const int nb = n / nwave;  // bins per wavefront (a multiple of 64)
   if (!angular) {
     // _rebin_spectrum of the input, 4 conv bins per lane at a time: the edges
@@ -2377,6 +2390,7 @@ __global__ __launch_bounds__(CONV_THREADS_MAX) void k_conv(BatchDev b, const Xil
         }
         const int i = i4[u];
         if (elo[u] >= 0.01 && ehi[u] < 1000.0) sx += xr;  // calcFFTNormFactor band (src/Relbase.cpp:205)
+        if constexpr (WIDE) sxa += fabs(xr);
         s_buf[P(i)].x = xr * cf[i];
       }
     }
@@ -2394,10 +2408,24 @@ __global__ __launch_bounds__(CONV_THREADS_MAX) void k_conv(BatchDev b, const Xil
     ph[q] = (q < per && i >= rc.lo && i <= rc.hi) ? prof[i] * cg.inv_emid[i] : 0.0;
     sph += ph[q];
   }
-  double s2[2];
-  block_sum2(sx, sph, s2, s_w);
+  const double p2[3] = {sx, sph, sxa};
+  double s2[3];
+  block_sums<WIDE ? 3 : 2>(p2, s2, s_w);
   double sum_xill = s2[0];
-  const double f = rq.do_renorm ? rq.norm / s2[1] : 1.0;
+  // The profile's renormalisation.  WIDE: as a power of two, which is exact in
+  // every bin and brings the profile to the input's scale (the two inputs of one
+  // complex transform, whose rounding errors reach both), times a rest that only
+  // the profile's sums carry (the result is normalised by them): against FP64
+  // sums in another order 4e-13 in bins 1e-4 below the maximum, 4e-12 without.
+  double f = rq.do_renorm ? rq.norm / s2[1] : 1.0, f_rest = 1.0;
+  if constexpr (WIDE) {
+    double f2 = pow2_of(f);
+    if (!angular && s2[2] > 0) f2 = pow2_of(s2[2] / s2[1]);
+    if (f2 > 0) {
+      f_rest = f / f2;
+      f = f2;
+    }
+  }
   double sr = 0.0, sa = 0.0;
 #pragma unroll
   for (int q = 0; q < 8; q++) {
@@ -2413,12 +2441,13 @@ __global__ __launch_bounds__(CONV_THREADS_MAX) void k_conv(BatchDev b, const Xil
   // (barrier inside: the buffer is complete)
   double sum_rel, sum_prof = 1.0;
   if (angular || relxill) {
+    const double p3[2] = {sr, sa};
     double s3[2];
-    block_sum2(sr, sa, s3, s_w);
-    sum_rel = s3[0];
-    sum_prof = s3[1];
+    block_sums<2>(p3, s3, s_w);
+    sum_rel = s3[0] * f_rest;
+    sum_prof = s3[1] * f_rest;
   } else {
-    sum_rel = block_sum4(sr, s_w[0]);
+    sum_rel = block_sum4(sr, s_w[0]) * f_rest;
   }
   if (angular) {
     sum_xill = 0.0;
@@ -2488,6 +2517,9 @@ __global__ __launch_bounds__(CONV_THREADS_MAX) void k_conv(BatchDev b, const Xil
   // values below (the rebin is linear), which saves a pass over the buffer
   double fnorm = sum_rel * sum_xill / sum_conv;
   if (angular && !zone_used) fnorm = 0.0;
+  // the distribution's own sum: a normalised one scales the spectrum and its band
+  // sum, whose ratio to the convolution's sum fnorm holds, once each
+  if (angular) fnorm /= dist_sum(dist, rs->n_incl);
   if (relxill) fnorm *= refl_scale;
   // the conv grid edges go to the upper part of the buffer, free after the
   // half-length FFT (its values occupy slots below P(m))
@@ -2704,10 +2736,12 @@ __global__ __launch_bounds__(XILL_THREADS, 4) void k_xill1(BatchDev b, const Xil
 #pragma unroll
     for (int u = 0; u < XILL_BINS; u++) acc[u] += d * s[u];
   }
+  // (the xillver models' weights are no distribution: an inclination bracket)
+  const double scale = rq.model == MOD_XILLVER ? zr.ncf : zr.ncf * dist_sum(dist, xt.n_incl);
   double *dst = b.xspec + rq.xspec_off + (size_t)wk.zone * xt.n_ener;
 #pragma unroll
   for (int u = 0; u < XILL_BINS; u++)
-    if (in[u]) dst[eb[u]] = acc[u] / zr.ncf;
+    if (in[u]) dst[eb[u]] = acc[u] / scale;
 }
 
 // relxilllp: the same for the zones of a lamp-post request (src/Relxill.cpp:
@@ -2729,7 +2763,7 @@ template <int NZ>
 __global__ __launch_bounds__(XILL_THREADS, 3) void k_xillz(BatchDev b, const XillWork *__restrict__ work, int chunks) {
   constexpr int NW = XILL_THREADS / 64;
   __shared__ int s_ind[NZ];
-  __shared__ double s_fac[NZ];
+  __shared__ double s_fac[NZ], s_scale[NZ];
   __shared__ unsigned s_off[XILL_THREADS];
   __shared__ double s_k[XILL_THREADS][NZ];
   __shared__ int s_wn[NW];
@@ -2746,6 +2780,7 @@ __global__ __launch_bounds__(XILL_THREADS, 3) void k_xillz(BatchDev b, const Xil
     const ZoneRec &zr = b.zone[rq.zone_off + tid];
     s_ind[tid] = xt.ect_dim >= 0 ? zr.ect_ind : rq.xind[3];
     s_fac[tid] = xt.ect_dim >= 0 ? zr.ect_fac : rq.xfac[3];
+    s_scale[tid] = zr.ncf * dist_sum(b.dist + rq.dist_off + tid * xt.n_incl, xt.n_incl);
   }
   __syncthreads();
   int elo = s_ind[0], ehi = s_ind[0];
@@ -2836,11 +2871,11 @@ __global__ __launch_bounds__(XILL_THREADS, 3) void k_xillz(BatchDev b, const Xil
 #pragma unroll
   for (int z = 0; z < NZ; z++) {
     if (z < nz) {
-      const double ncf = b.zone[rq.zone_off + z].ncf;
+      const double scale = s_scale[z];
       double *dst = b.xspec + rq.xspec_off + (size_t)z * ne;
 #pragma unroll
       for (int u = 0; u < XILL_BINS_Z; u++)
-        if (in[u]) dst[eb[u]] = acc[z][u] / ncf;
+        if (in[u]) dst[eb[u]] = acc[z][u] / scale;
     }
   }
 }
@@ -2994,13 +3029,27 @@ int launch_finalize(const BatchDev &b, void *stream) {
 }
 
 static size_t conv_lds(int n) { return (size_t)(n + n / 16) * sizeof(double2); }
+// n/8 threads fill a pass of the transforms.
 static int conv_threads(int n) { return std::max(CONV_THREADS, n / 8); }
 
-int launch_conv(const BatchDev &b, const XillWork *conv_work, int n_conv_work, void *stream) {
+int launch_conv(const BatchDev &b, const XillWork *conv_work, int n_conv_work, bool angular, void *stream) {
   if (n_conv_work <= 0) return 0;
   const size_t lds = conv_lds(b.cg.n);
-  (void)hipFuncSetAttribute((const void *)k_conv, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  hipLaunchKernelGGL(k_conv, dim3(n_conv_work), dim3(conv_threads(b.cg.n)), lds, (hipStream_t)stream, b, conv_work);
+  auto go = [&](auto kern, int nt) {
+    (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL(kern, dim3(n_conv_work), dim3(nt), lds, (hipStream_t)stream, b, conv_work);
+  };
+  // where every unit has a CU of its own the most threads (but not more than
+  // bins, which a wavefront takes by the 64), so that the phases over the grid
+  // take half the rounds: 1 relxill unit of 4096 bins 36 us and 33 us, 256 relconv
+  // units 50 us and 45 us; 1024 units 110 us and 127 us
+  if (n_conv_work <= 256) {
+    const int nt = std::min(CONV_THREADS_MAX, b.cg.n);
+    angular ? go(k_conv<1, 1>, nt) : go(k_conv<1, 0>, nt);
+  } else {
+    const int nt = conv_threads(b.cg.n);
+    angular ? go(k_conv<0, 1>, nt) : go(k_conv<0, 0>, nt);
+  }
   return (int)hipGetLastError();
 }
 

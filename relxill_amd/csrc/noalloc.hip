@@ -234,7 +234,7 @@ int noalloc_eval(int model, const double *parameter, const double *d_energy, con
     e |= launch_setup(bd, s);
     e |= launch_integrate(bd, n_blocks, cos_rows, s);
     e |= launch_fixup(bd, cos_rows, s);
-    if (conv) e |= launch_conv(bd, d_work, 1, s);
+    if (conv) e |= launch_conv(bd, d_work, 1, false, s);
     else e |= launch_finalize(bd, s);
     e |= launch_deliver(bd, res, nullptr, 0, s);
     e |= (int)hipStreamSynchronize(s);

@@ -394,7 +394,8 @@ int launch_integrate(const BatchDev &b, int n_blocks, bool limb, void *stream);
 int launch_fixup(const BatchDev &b, bool cos_rows, void *stream);
 int launch_finalize(const BatchDev &b, void *stream);
 // conv_work: (request, zone) pairs; relxill requests have one per zone
-int launch_conv(const BatchDev &b, const XillWork *conv_work, int n_conv_work, void *stream);
+// (angular: a relxill_conv request is among them)
+int launch_conv(const BatchDev &b, const XillWork *conv_work, int n_conv_work, bool angular, void *stream);
 // work: n_single one-zone units, then n_multi units of several zones
 int launch_xill(const BatchDev &b, const XillWork *work, int n_single, int n_multi, void *stream);
 // returning radiation (before launch_setup): the xillver band sums of the
