@@ -1151,6 +1151,9 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
     p.pre_status = st;
     b.h_status[i] = st;
   }
+  b.n_prim_rel = (int)(std::stable_partition(b.h_prim.begin(), b.h_prim.end(),
+                                             [&](int i) { return b.h_req[i].model != MOD_XILLVER; }) -
+                       b.h_prim.begin());
   b.prim_bins = 0;
   for (int i : b.h_prim) b.prim_bins = std::max(b.prim_bins, b.h_req[i].n_in);
   b.tot_ener = o_ener;
@@ -1394,6 +1397,7 @@ int batch_upload(Batch &b) {
   w.n_xill = (int)b.h_xill.size();
   w.n_xill1 = b.n_xill1;
   w.n_prim = (int)b.h_prim.size();
+  w.n_prim_rel = b.n_prim_rel;
   w.n_zone = (int)b.h_zone.size();
   w.n_ang = (int)b.h_ang.size();
   w.n_rrc = (int)b.h_rrc.size();
@@ -1509,22 +1513,27 @@ static int launch_sequence(Batch &b, const RunKey &k, hipStream_t s) {
   if (prof) e |= (int)hipEventRecord(b.ev[0], s);
   e |= launch_begin(bd.ctr, k.fetch_src, k.fetch_dst, k.n_fetch, s);
   e |= launch_nth(bd, w.nth, w.n_nth, s);
-  e |= launch_zone(bd, w.zone, w.n_zone, s);
+  // the angle distributions and the zone records go with k_integrate where it
+  // can take them; the records come first where the returning radiation reads them
+  const bool side = integrate_takes_side(bd, k.n_blocks), zone_side = side && w.n_rrc == 0;
+  SideWork sw = {w.ang, w.zone, side ? w.n_ang : 0, 0, zone_side ? w.n_zone : 0};
+  if (!zone_side) e |= launch_zone(bd, w.zone, w.n_zone, s);
   e |= launch_rrad(bd, w.rrc, w.n_rrc, w.rrad, w.n_rrad, s);
   e |= launch_setup(bd, s);
-  e |= launch_dist(bd, w.ang, w.n_ang, s);
+  if (!side) e |= launch_dist(bd, w.ang, w.n_ang, s);
   if (prof) e |= (int)hipEventRecord(b.ev[1], s);
-  e |= launch_integrate(bd, k.n_blocks, k.cos_rows != 0, s);
+  e |= launch_integrate(bd, k.n_blocks, k.cos_rows != 0, &sw, s);
   if (prof) e |= (int)hipEventRecord(b.ev[2], s);
   e |= launch_fixup(bd, k.cos_rows != 0, s);
   if (prof) e |= (int)hipEventRecord(b.ev[3], s);
   if (k.finalize) e |= launch_finalize(bd, s);
   if (prof) e |= (int)hipEventRecord(b.ev[4], s);
-  e |= launch_xill(bd, w.xill, w.n_xill1, w.n_xill - w.n_xill1, s);
+  const int with_xill = xill_takes_primary(w.n_xill, w.n_prim_rel);
+  e |= launch_xill(bd, w.xill, w.n_xill1, w.n_xill - w.n_xill1, w.prim, with_xill, k.prim_bins, s);
   if (prof) e |= (int)hipEventRecord(b.ev[5], s);
   e |= launch_conv(bd, w.conv, w.n_conv, k.angular != 0, s);
   if (prof) e |= (int)hipEventRecord(b.ev[6], s);
-  e |= launch_primary(bd, w.prim, w.n_prim, k.prim_bins, s);
+  e |= launch_primary(bd, w.prim + with_xill, w.n_prim - with_xill, k.prim_bins, s);
   if (prof) e |= (int)hipEventRecord(b.ev[7], s);
   e |= launch_deliver(bd, static_cast<int *>(k.res), static_cast<double *>(k.res_out), k.n_out, s);
   return e;

@@ -57,7 +57,7 @@ void rzone_grid(double rmin, double rmax, int nzones, double h, double *rgrid);
 struct WorkLists {
   const XillWork *xill, *conv, *zone, *nth;
   const int *prim, *ang, *rrc, *rrad;
-  int n_xill1, n_xill, n_conv, n_zone, n_nth, n_prim, n_ang, n_rrc, n_rrad;
+  int n_xill1, n_xill, n_conv, n_zone, n_nth, n_prim, n_prim_rel, n_ang, n_rrc, n_rrad;
 };
 
 // Launch configuration of one run: every kernel argument and grid shape.  A
@@ -90,7 +90,8 @@ struct Batch {
   std::vector<ReqParams> h_req;
   std::vector<int> h_status;  // host-side parse status
   std::vector<double> h_ener, h_flux_in;
-  std::vector<int> h_prim;
+  std::vector<int> h_prim;       // requests with a primary: n_prim_rel relxill ones, then the xillver models
+  int n_prim_rel = 0;
   int prim_bins = 0;             // most caller bins of a request in h_prim
   std::vector<int> h_ang;        // requests with an emission-angle distribution (k_dist)
   std::vector<XillWork> h_conv;  // (request, zone) units of k_conv

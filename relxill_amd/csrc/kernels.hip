@@ -958,10 +958,10 @@ __global__ __launch_bounds__(NT, NT == 256 ? 3 : 1) void k_setup(BatchDev b) {
 // Bound: the latency of the table rows and the sums, 15 us alone, 20 us for 1280
 // zones (inside k_setup, zone after zone with tree sums: 18 us and 22 us, but
 // after the returning radiation that reads the records).
-__global__ __launch_bounds__(64) void k_zone(BatchDev b, const XillWork *__restrict__ work) {
-  __shared__ double s_jr[MAX_LP_R], s_je[MAX_LP_R], s_jd[MAX_LP_R], s_ji[MAX_LP_R];
-  const XillWork wk = work[blockIdx.x];
-  const int req = wk.req, z = wk.zone, lane = threadIdx.x;
+constexpr int ZONE_LDS = 4 * MAX_LP_R;  // doubles
+__device__ __forceinline__ void zone_unit(const BatchDev &b, const XillWork wk, int lane, double *lds) {
+  double *s_jr = lds, *s_je = lds + MAX_LP_R, *s_jd = lds + 2 * MAX_LP_R, *s_ji = lds + 3 * MAX_LP_R;
+  const int req = wk.req, z = wk.zone;
   const ReqParams &rq = b.req[req];
   if (rq.pre_status != 0) return;  // uniform over the block
   const DevXillTable &xt = b.xt[rq.prim];
@@ -1018,6 +1018,11 @@ __global__ __launch_bounds__(64) void k_zone(BatchDev b, const XillWork *__restr
     }
   }
   if (lane == 0) b.zone[rq.zone_off + z] = zr;
+}
+
+__global__ __launch_bounds__(64) void k_zone(BatchDev b, const XillWork *__restrict__ work) {
+  __shared__ double s_lds[ZONE_LDS];
+  zone_unit(b, work[blockIdx.x], threadIdx.x, s_lds);
 }
 
 // The eight corners of a request's xillver table row on the interpolated axes
@@ -1554,24 +1559,28 @@ struct EdgeWalk {
 // Emission-angle distribution of the requests with one (src/Relprofile.cpp:
 // 908-938), one wavefront per (request, chunk of 64 fine radii), after k_setup.
 // Lane = fine radius; the node rows of the chunk's radii (transfer function
-// and cosines) are built in LDS from the table corners, STAGE_MAX values of
+// and cosines) are built in LDS from the table corners, DIST_STAGE values of
 // each at a time, and each lane walks the g* columns, both branches of a
-// column at once (16-byte LDS reads).  Neighbouring columns mostly fall into one angle bin, so a lane sums
-// in a register while its bin stays and adds to the LDS bins when it changes;
-// the wavefront's last bins go as one wave sum when all lanes share the bin.
+// column at once (16-byte LDS reads).  Neighbouring columns mostly fall into
+// one angle bin, so a lane sums in a register while its bin stays and adds to
+// the LDS bins when it changes; the wavefront's last bins go as one wave sum
+// when all lanes share the bin.  By itself (k_dist) or as workgroups of
+// k_integrate.
 // The chunk's sums are added to the request's distribution in HBM (cleared by
 // k_setup, left unnormalised: its readers scale by its sum).
 // Bound: FP64 issue, 1000 radii x 2 n_g columns x ~60 operations a request,
 // which one CU takes 16 us for: inside k_setup (one workgroup a request) it
 // was 61 us of a single relxill call (k_setup 87 us) and 165 us of a batch of
-// 1024 (237 us); the 16 wavefronts a request take 12 us and 94 us.
-template <int NZ>
-__global__ __launch_bounds__(64) void k_dist(BatchDev b, const int *__restrict__ reqs, int n_rc) {
-  __shared__ __align__(16) double s_t[STAGE_MAX], s_c[STAGE_MAX];
-  __shared__ double s_dist[NZ * MAX_INCL];
-  __shared__ double2 s_g[MAX_NG];
-  const int req = reqs[blockIdx.x / n_rc], c = blockIdx.x % n_rc;
-  const int lane = threadIdx.x;
+// 1024 (237 us); the 16 wavefronts a request take 12 us and 70 us (92 us with
+// staging areas of 640 values, which halved the wavefronts per CU).
+constexpr int DIST_STAGE = 320;  // staged values of each of the two arrays (2 rows of 2 MAX_NG at least)
+__host__ __device__ constexpr int dist_lds(int n_zones) {  // doubles
+  return 2 * DIST_STAGE + 2 * MAX_NG + n_zones * MAX_INCL;
+}
+__device__ __forceinline__ void dist_chunk(const BatchDev &b, int req, int c, int lane, double *lds) {
+  double *s_t = lds, *s_c = lds + DIST_STAGE;
+  double2 *s_g = reinterpret_cast<double2 *>(lds + 2 * DIST_STAGE);
+  double *s_dist = lds + 2 * DIST_STAGE + 2 * MAX_NG;  // [zone][angle bin]
   if (b.status[req] != 0) return;  // uniform over the block
   const ReqParams &rq = b.req[req];
   const ReqNorm rn = b.rnorm[req];
@@ -1603,7 +1612,7 @@ __global__ __launch_bounds__(64) void k_dist(BatchDev b, const int *__restrict__
   }
   const int kmin = wave_min_i(live ? K : INT_MAX), kmax = wave_max_i(live ? K : -1);
   const NodeSrc ts = node_src(b.rt, rn, false), cs = node_src(b.rt, rn, true);
-  const int stage_rows = STAGE_MAX / nq;  // at least 5 (n_g <= MAX_NG)
+  const int stage_rows = DIST_STAGE / nq;  // at least 2 (n_g <= MAX_NG)
   int derr = 0;
   auto put = [&](int k, double sum) {  // one lane's sum over columns of angle bin k
     const double v = sum * amp;
@@ -1669,6 +1678,11 @@ __global__ __launch_bounds__(64) void k_dist(BatchDev b, const int *__restrict__
     if (s_dist[k] != 0.0) unsafeAtomicAdd(&b.dist[rq.dist_off + k], s_dist[k]);
 }
 
+__global__ __launch_bounds__(64) void k_dist(BatchDev b, const int *__restrict__ reqs, int n_rc) {
+  extern __shared__ __align__(16) double s_lds[];
+  dist_chunk(b, reqs[blockIdx.x / n_rc], blockIdx.x % n_rc, threadIdx.x, s_lds);
+}
+
 // Byte offset of k_integrate's coefficient slots and bin buffer (FP64 path)
 // behind the lane rows (rows: 64 or 128 of 2 n_g + 1 values).
 __host__ __device__ inline size_t integrate_rows_bytes(int ng, bool cos_rows, size_t elem) {
@@ -1708,8 +1722,13 @@ __host__ __device__ inline size_t integrate_rows_bytes(int ng, bool cos_rows, si
 //   A single relconv call (segments of 4 bins): 34 us with the counters, 22 us
 //   without (FP32 36 and 15 us); with the segments of 64 bins that every batch
 //   had by default 64 us (43 us).
+//   ONE also takes the angle distribution's chunks and, where nothing before
+//   reads them, the zone records along as its first workgroups (side): they and
+//   the items need nothing of each other and leave the chip idle between them.
+//   As launches of their own they were 12 us and 5-17 us of every relxill call
+//   (relxill 120 us, 109 us with them here; 128 relxilllp requests 566 us, 554 us).
 template <int MODE, int COS, int ONE>
-__global__ __launch_bounds__(64, MODE == 0 ? 1 : 3) void k_integrate(BatchDev b_arg, int stage_rows) {
+__global__ __launch_bounds__(64, MODE == 0 ? 1 : 3) void k_integrate(BatchDev b_arg, int stage_rows, SideWork side) {
   // The argument is read through a pointer that every item renews, so that the
   // compiler reads its fields where an item uses them: kept across the item
   // loop they took 28 scalar registers more than there are, spilled to vector
@@ -1720,8 +1739,22 @@ __global__ __launch_bounds__(64, MODE == 0 ? 1 : 3) void k_integrate(BatchDev b_
   const BatchDev &b = *(const BatchDev *)bp;
   constexpr int cos_rows = COS;
   using TV = typename std::conditional<MODE == 0, double, float>::type;
-  extern __shared__ double s_dyn[];
+  extern __shared__ __align__(16) double s_dyn[];
   const int lane = threadIdx.x;
+  int one_item = blockIdx.x;
+  if constexpr (ONE) {
+    const int n_chunk = side.n_ang * side.n_rc;
+    if (one_item < n_chunk) {
+      dist_chunk(b, side.ang[one_item / side.n_rc], one_item % side.n_rc, lane, s_dyn);
+      return;
+    }
+    one_item -= n_chunk;
+    if (one_item < side.n_zone) {
+      zone_unit(b, side.zone[one_item], lane, s_dyn);
+      return;
+    }
+    one_item -= side.n_zone;
+  }
   const int ng = b.rt.n_g;
   const int RS = 2 * ng + 1;  // odd row stride: lanes' rows start in distinct banks
   TV *rows = reinterpret_cast<TV *>(s_dyn);
@@ -1763,7 +1796,7 @@ __global__ __launch_bounds__(64, MODE == 0 ? 1 : 3) void k_integrate(BatchDev b_
     // and once all N_XQ have been found empty it is done
     int k = -1;
     if constexpr (ONE) {
-      const int kk = blockIdx.x;
+      const int kk = one_item;
       if (kk >= n_long + n_short) return;
       k = kk < n_long ? kk : b.item_cap - 1 - (kk - n_long);
     }
@@ -1946,7 +1979,7 @@ __global__ __launch_bounds__(64, MODE == 0 ? 1 : 3) void k_integrate(BatchDev b_
 
 // FP64 re-check of guarded FP32 bins, one entry per lane.
 __global__ __launch_bounds__(64) void k_fixup(BatchDev b, int cos_rows) {
-  extern __shared__ double s_dyn[];
+  extern __shared__ __align__(16) double s_dyn[];
   const int lane = threadIdx.x;
   const int ng = b.rt.n_g;
   const int RS = 2 * ng + 1;
@@ -2554,16 +2587,19 @@ __global__ __launch_bounds__(CONV_THREADS_MAX) void k_conv(BatchDev b, const Xil
 // the source's Ecut shifted to the observer (spec_cutoffpl,
 // src/Xillspec.cpp:215-241) on the convolution grid, normalised as the
 // xillver incident spectrum at the source (k_zone), times the lamp post's flux
-// boost, rebinned onto the caller grid.  After k_conv, one workgroup per
-// (request, PRIM_THREADS * per caller bins); launch_primary chooses per.
+// boost, rebinned onto the caller grid.  One workgroup per
+// (request, PRIM_THREADS * per caller bins); prim_work chooses per.  Few relxill
+// requests: with k_xill, before k_conv adds to the output; many, and the xillver
+// models, which read k_xill's spectra: after k_conv.
 // Bound: the latency of the exponential and the grid reads for few requests,
 // FP64 issue (an exponential and a division a grid bin) for many.  One
 // workgroup a request, with the norm's 500 exponentials and 12 rounds of bins,
 // took 28 us for one request of 3000 bins (47 us with the nthcomp primary) and
 // 57 us for 1024; now 5.5 us (8 us) and 51 us.
-__global__ __launch_bounds__(PRIM_THREADS) void k_primary(BatchDev b, const int *__restrict__ reqs, int chunks, int per) {
-  const int req = reqs[blockIdx.x / chunks];
-  const int j0 = (blockIdx.x % chunks) * (PRIM_THREADS * per) + threadIdx.x;
+__device__ __forceinline__ void primary_bins(const BatchDev &b, const PrimWork &pw, int block) {
+  const int per = pw.per;
+  const int req = pw.reqs[block / pw.chunks];
+  const int j0 = (block % pw.chunks) * (PRIM_THREADS * per) + threadIdx.x;
   const ReqParams &rq = b.req[req];
   const int j1 = min(rq.n_in, j0 + PRIM_THREADS * per);  // this thread: j0, j0 + PRIM_THREADS, ... below j1
   if (j0 >= j1) return;
@@ -2648,6 +2684,8 @@ __global__ __launch_bounds__(PRIM_THREADS) void k_primary(BatchDev b, const int 
   }
 }
 
+__global__ __launch_bounds__(PRIM_THREADS) void k_primary(BatchDev b, PrimWork pw) { primary_bins(b, pw, blockIdx.x); }
+
 // relxill: the xillver spectrum of the request's parameters for every
 // emission angle (interp_5d_tab_incl, src/xilltable.c:812-876: 16 corners of
 // the four interpolated parameters, in the reference's order and with its
@@ -2656,8 +2694,17 @@ __global__ __launch_bounds__(PRIM_THREADS) void k_primary(BatchDev b, const int 
 // thread; every table read is coalesced across the block.  Angles with zero
 // weight are skipped (they add exactly 0).  The zone's Ecut bracket, angle
 // distribution and normalisation change come from its zone record.
-__global__ __launch_bounds__(XILL_THREADS, 4) void k_xill1(BatchDev b, const XillWork *__restrict__ work, int chunks) {
-  const XillWork wk = work[blockIdx.x / chunks];
+// PRIM: the first workgroups are k_primary's (it needs nothing of this kernel's:
+// the convolutions add to what it leaves in the output).
+template <int PRIM>
+__global__ __launch_bounds__(XILL_THREADS, 4) void k_xill1(BatchDev b, const XillWork *__restrict__ work, int chunks,
+                                                           PrimWork pw) {
+  if (PRIM && (int)blockIdx.x < pw.blocks) {
+    primary_bins(b, pw, blockIdx.x);
+    return;
+  }
+  const int block = PRIM ? blockIdx.x - pw.blocks : blockIdx.x;
+  const XillWork wk = work[block / chunks];
   const int req = wk.req;
   if (b.status[req] != 0) return;
   const ReqParams &rq = b.req[req];
@@ -2665,7 +2712,7 @@ __global__ __launch_bounds__(XILL_THREADS, 4) void k_xill1(BatchDev b, const Xil
   const DensDiv dd = dens_of(rq.xdens_div);
   // XILL_BINS bins per thread, XILL_THREADS apart: the corner weights and rows
   // are set up once for all of them, and their loads are in flight together
-  const int e0 = (blockIdx.x % chunks) * (XILL_THREADS * XILL_BINS) + threadIdx.x;
+  const int e0 = (block % chunks) * (XILL_THREADS * XILL_BINS) + threadIdx.x;
   if (e0 >= xt.n_ener) return;
   const ZoneRec zr = b.zone[rq.zone_off + wk.zone];
   int i0[4];
@@ -2759,15 +2806,22 @@ __global__ __launch_bounds__(XILL_THREADS, 4) void k_xill1(BatchDev b, const Xil
 // candidates, in a fixed order), then streams the 8 rows of each listed pair.
 // Tables without an Ecut axis use the request's bracket on the fourth axis
 // for every zone.
-template <int NZ>
-__global__ __launch_bounds__(XILL_THREADS, 3) void k_xillz(BatchDev b, const XillWork *__restrict__ work, int chunks) {
+// PRIM: as k_xill1's.
+template <int NZ, int PRIM>
+__global__ __launch_bounds__(XILL_THREADS, 3) void k_xillz(BatchDev b, const XillWork *__restrict__ work, int chunks,
+                                                           PrimWork pw) {
+  if (PRIM && (int)blockIdx.x < pw.blocks) {
+    primary_bins(b, pw, blockIdx.x);
+    return;
+  }
+  const int block = PRIM ? blockIdx.x - pw.blocks : blockIdx.x;
   constexpr int NW = XILL_THREADS / 64;
   __shared__ int s_ind[NZ];
   __shared__ double s_fac[NZ], s_scale[NZ];
   __shared__ unsigned s_off[XILL_THREADS];
   __shared__ double s_k[XILL_THREADS][NZ];
   __shared__ int s_wn[NW];
-  const XillWork wk = work[blockIdx.x / chunks];
+  const XillWork wk = work[block / chunks];
   const int req = wk.req;
   if (b.status[req] != 0) return;  // uniform over the block
   const ReqParams &rq = b.req[req];
@@ -2796,7 +2850,7 @@ __global__ __launch_bounds__(XILL_THREADS, 3) void k_xillz(BatchDev b, const Xil
   corners8(xt, rq, zax, w8, cb, &stride);
   const double *dist = b.dist + rq.dist_off;
   const size_t ne = (size_t)xt.n_ener;
-  const int e0 = (blockIdx.x % chunks) * (XILL_THREADS * XILL_BINS_Z) + tid;
+  const int e0 = (block % chunks) * (XILL_THREADS * XILL_BINS_Z) + tid;
   int eb[XILL_BINS_Z];
   bool in[XILL_BINS_Z];
 #pragma unroll
@@ -2984,26 +3038,36 @@ static size_t integrate_lds(const BatchDev &b, bool cos_rows, size_t elem, int *
   return rows + w + std::max(park, (size_t)2 * nq * sizeof(double));
 }
 
+static int fine_chunks(const BatchDev &b) { return (b.nr_fine + RAD_CHUNK - 1) / RAD_CHUNK; }
+
 int launch_dist(const BatchDev &b, const int *reqs, int n_reqs, void *stream) {
   if (n_reqs <= 0) return 0;
-  const int n_rc = (b.nr_fine + RAD_CHUNK - 1) / RAD_CHUNK;
-  if (b.max_zones > LP_ZONES)
-    hipLaunchKernelGGL(k_dist<MAX_ZONES>, dim3(n_reqs * n_rc), dim3(64), 0, (hipStream_t)stream, b, reqs, n_rc);
-  else
-    hipLaunchKernelGGL(k_dist<LP_ZONES>, dim3(n_reqs * n_rc), dim3(64), 0, (hipStream_t)stream, b, reqs, n_rc);
+  hipLaunchKernelGGL(k_dist, dim3(n_reqs * fine_chunks(b)), dim3(64), sizeof(double) * dist_lds(b.max_zones),
+                     (hipStream_t)stream, b, reqs, fine_chunks(b));
   return (int)hipGetLastError();
 }
 
-int launch_integrate(const BatchDev &b, int n_blocks, bool cos_rows, void *stream) {
+bool integrate_takes_side(const BatchDev &b, int n_blocks) { return n_blocks >= b.item_cap; }
+
+int launch_integrate(const BatchDev &b, int n_blocks, bool cos_rows, const SideWork *side_in, void *stream) {
   if (b.n_req <= 0 || n_blocks <= 0) return 0;
   hipStream_t st = (hipStream_t)stream;
   int stage = 0;
-  const size_t lds = integrate_lds(b, cos_rows, b.mode == 0 ? sizeof(double) : sizeof(float), &stage);
+  size_t lds = integrate_lds(b, cos_rows, b.mode == 0 ? sizeof(double) : sizeof(float), &stage);
+  SideWork side = SideWork();
+  if (side_in) {
+    side = *side_in;
+    side.n_rc = fine_chunks(b);
+    if (side.n_ang > 0) lds = std::max(lds, sizeof(double) * dist_lds(b.max_zones));
+    if (side.n_zone > 0) lds = std::max(lds, sizeof(double) * ZONE_LDS);
+  }
+  const bool one = integrate_takes_side(b, n_blocks);  // a workgroup for every item there can be
+  const int n_side = side.n_ang * side.n_rc + side.n_zone;
+  if (n_side > 0 && !one) return (int)hipErrorInvalidValue;
   auto go = [&](auto kern) {
     (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL(kern, dim3(n_blocks), dim3(64), lds, st, b, stage);
+    hipLaunchKernelGGL(kern, dim3(n_side + n_blocks), dim3(64), lds, st, b, stage, side);
   };
-  const bool one = n_blocks >= b.item_cap;  // a workgroup for every item there can be
   if (b.mode == 0) {
     if (one) cos_rows ? go(k_integrate<0, 1, 1>) : go(k_integrate<0, 0, 1>);
     else cos_rows ? go(k_integrate<0, 1, 0>) : go(k_integrate<0, 0, 0>);
@@ -3061,16 +3125,46 @@ static int xill_n_ener(const BatchDev &b) {
   return n;
 }
 
-int launch_xill(const BatchDev &b, const XillWork *work, int n_single, int n_multi, void *stream) {
+// k_primary's split of n_reqs requests of up to max_bins caller bins.
+static PrimWork prim_work(const int *reqs, int n_reqs, int max_bins) {
+  // bins per thread: one until the chip holds no more workgroups at once (1024),
+  // then as many as keep it full: a workgroup's fixed part (parameters, grid
+  // guesses) costs about two bins.  1024 requests of 3000 bins: 72 us with one
+  // bin, 51 us with eleven; 128 requests: 9 us with one, 26 us with twelve.
+  PrimWork pw;
+  pw.reqs = reqs;
+  const int rounds = (max_bins + PRIM_THREADS - 1) / PRIM_THREADS;
+  pw.per = (int)std::max<int64_t>(1, std::min<int64_t>(rounds, (int64_t)n_reqs * rounds / 1024));
+  pw.chunks = (rounds + pw.per - 1) / pw.per;
+  pw.blocks = n_reqs * pw.chunks;
+  return pw;
+}
+
+// up to 256 requests: one relxill request 109 us and 100 us a call, 128
+// relxilllp 554 us and 550 us; with 1024, whose launches fill the chip, 2.09 ms
+// and 2.15 ms (k_xill1 loses a wavefront per SIMD to the primary's registers)
+int xill_takes_primary(int n_xill, int n_prim) { return n_xill > 0 && n_prim <= 256 ? n_prim : 0; }
+
+int launch_xill(const BatchDev &b, const XillWork *work, int n_single, int n_multi, const int *prim, int n_prim,
+                int max_bins, void *stream) {
+  static_assert(XILL_THREADS == PRIM_THREADS, "k_primary's workgroups run in k_xill's launches");
+  PrimWork pw = prim_work(prim, n_prim, max_bins);
   if (n_single > 0) {
     const int chunks = (xill_n_ener(b) + XILL_THREADS * XILL_BINS - 1) / (XILL_THREADS * XILL_BINS);
-    hipLaunchKernelGGL(k_xill1, dim3(n_single * chunks), dim3(XILL_THREADS), 0, (hipStream_t)stream, b,
-                       work, chunks);
+    const int grid = pw.blocks + n_single * chunks;
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(grid), dim3(XILL_THREADS), 0, (hipStream_t)stream, b, work, chunks, pw);
+    };
+    pw.blocks > 0 ? go(k_xill1<1>) : go(k_xill1<0>);
+    pw.blocks = 0;  // (taken)
   }
   if (n_multi > 0) {
     const int chunks = (xill_n_ener(b) + XILL_THREADS * XILL_BINS_Z - 1) / (XILL_THREADS * XILL_BINS_Z);
-    hipLaunchKernelGGL(k_xillz<LP_ZONES>, dim3(n_multi * chunks), dim3(XILL_THREADS), 0,
-                       (hipStream_t)stream, b, work + n_single, chunks);
+    const int grid = pw.blocks + n_multi * chunks;
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(grid), dim3(XILL_THREADS), 0, (hipStream_t)stream, b, work + n_single, chunks, pw);
+    };
+    pw.blocks > 0 ? go(k_xillz<LP_ZONES, 1>) : go(k_xillz<LP_ZONES, 0>);
   }
   return (int)hipGetLastError();
 }
@@ -3101,15 +3195,8 @@ int launch_nth(const BatchDev &b, const XillWork *work, int n_work, void *stream
 
 int launch_primary(const BatchDev &b, const int *reqs, int n_reqs, int max_bins, void *stream) {
   if (n_reqs <= 0) return 0;
-  // bins per thread: one until the chip holds no more workgroups at once (1024),
-  // then as many as keep it full: a workgroup's fixed part (parameters, grid
-  // guesses) costs about two bins.  1024 requests of 3000 bins: 72 us with one
-  // bin, 51 us with eleven; 128 requests: 9 us with one, 26 us with twelve.
-  const int rounds = (max_bins + PRIM_THREADS - 1) / PRIM_THREADS;
-  const int per = (int)std::max<int64_t>(1, std::min<int64_t>(rounds, (int64_t)n_reqs * rounds / 1024));
-  const int chunks = (rounds + per - 1) / per;
-  hipLaunchKernelGGL(k_primary, dim3(n_reqs * chunks), dim3(PRIM_THREADS), 0, (hipStream_t)stream, b, reqs, chunks,
-                     per);
+  const PrimWork pw = prim_work(reqs, n_reqs, max_bins);
+  hipLaunchKernelGGL(k_primary, dim3(pw.blocks), dim3(PRIM_THREADS), 0, (hipStream_t)stream, b, pw);
   return (int)hipGetLastError();
 }
 

@@ -232,7 +232,7 @@ int noalloc_eval(int model, const double *parameter, const double *d_energy, con
     if (p.return_rad != 0 && p.pre_status == 0)
       e |= launch_rrad(bd, nullptr, 0, reinterpret_cast<const int *>(d_work), 1, s);
     e |= launch_setup(bd, s);
-    e |= launch_integrate(bd, n_blocks, cos_rows, s);
+    e |= launch_integrate(bd, n_blocks, cos_rows, nullptr, s);
     e |= launch_fixup(bd, cos_rows, s);
     if (conv) e |= launch_conv(bd, d_work, 1, false, s);
     else e |= launch_finalize(bd, s);

@@ -382,6 +382,19 @@ struct BatchDev {
 };
 
 // ---- launchers (kernels.hip) ----
+// Work that k_integrate takes along: angle distributions (requests, chunks of
+// fine radii each) and zone records.
+struct SideWork {
+  const int *ang;
+  const XillWork *zone;
+  int n_ang, n_rc, n_zone;
+};
+// k_primary's workgroups: chunks a request, per bins a thread.
+struct PrimWork {
+  const int *reqs;
+  int blocks, chunks, per;
+};
+
 // First in a run: clears the counters and copies the request block (n16 16-byte
 // words of pinned host memory) to the device.
 int launch_begin(int *ctr, const void *src, void *dst, int64_t n16, void *stream);
@@ -390,14 +403,20 @@ int launch_deliver(const BatchDev &b, int *res, double *res_out, int64_t n_out, 
 int launch_setup(const BatchDev &b, void *stream);
 // the emission-angle distribution of the n_reqs requests with one
 int launch_dist(const BatchDev &b, const int *reqs, int n_reqs, void *stream);
-int launch_integrate(const BatchDev &b, int n_blocks, bool limb, void *stream);
+// (side: the distributions and zone records it takes along, of a launch that
+// integrate_takes_side allows; may be null)
+bool integrate_takes_side(const BatchDev &b, int n_blocks);
+int launch_integrate(const BatchDev &b, int n_blocks, bool limb, const SideWork *side, void *stream);
 int launch_fixup(const BatchDev &b, bool cos_rows, void *stream);
 int launch_finalize(const BatchDev &b, void *stream);
 // conv_work: (request, zone) pairs; relxill requests have one per zone
 // (angular: a relxill_conv request is among them)
 int launch_conv(const BatchDev &b, const XillWork *conv_work, int n_conv_work, bool angular, void *stream);
 // work: n_single one-zone units, then n_multi units of several zones
-int launch_xill(const BatchDev &b, const XillWork *work, int n_single, int n_multi, void *stream);
+// (and the primaries of n_prim relxill requests: xill_takes_primary of them)
+int xill_takes_primary(int n_xill, int n_prim);
+int launch_xill(const BatchDev &b, const XillWork *work, int n_single, int n_multi, const int *prim, int n_prim,
+                int max_bins, void *stream);
 // returning radiation (before launch_setup): the xillver band sums of the
 // n_corr relxilllp requests above spin 0 (after launch_zone), then the returning
 // emissivity of all n_reqs requests with it
