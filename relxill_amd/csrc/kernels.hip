@@ -1491,13 +1491,15 @@ __device__ inline void stage_table_rows(const NodeSrc &s, int kb, int tot, int n
   }
 }
 
-// k_fixup: one lane's FP64 row values, straight from the table, for the g*
+// k_fixup: an entry's FP64 row values, straight from the table, for the g*
 // brackets that the FP64 integral of the bin [e0, e1] reads (its points lie
 // between the bin's clamped ends, whose brackets bound theirs; one bracket of
 // margin either side) and for the brackets of the two edge norms; the other
-// columns of the row are not read.
+// columns of the row are not read.  Lane l of the entry's FIX_LANES takes every
+// FIX_LANES-th column.
+constexpr int FIX_LANES = 8;
 __device__ inline void load_radius_table(const BatchDev &b, const ReqNorm &rn, const RadGeo &r, int K, int limb,
-                                         double e0, double e1, double *myT, double *myC, RadiusView &v) {
+                                         double e0, double e1, double *myT, double *myC, RadiusView &v, int l) {
   v.gmin = r.gmin;
   v.gmax = r.gmax;
   v.del_g = 1. / (r.gmax - r.gmin);  // set_str_relbf, src/Relprofile.cpp:733
@@ -1509,19 +1511,16 @@ __device__ inline void load_radius_table(const BatchDev &b, const ReqNorm &rn, c
   };
   const NodeSrc ts = node_src(b.rt, rn, false);
   const NodeSrc cs = node_src(b.rt, rn, true);
-  auto fill = [&](int ia, int ib) {  // columns of brackets ia .. ib
-#pragma unroll 4
-    for (int c = 2 * ia; c <= 2 * ib + 3; c++) {
-      myT[c] = lerp1_(r.ifac_r, node_value(ts, K + 1, c), node_value(ts, K, c));
-      if (limb) myC[c] = lerp1_(r.ifac_r, node_value(cs, K + 1, c), node_value(cs, K, c));
-    }
+  auto put = [&](int c) {
+    myT[c] = lerp1_(r.ifac_r, node_value(ts, K + 1, c), node_value(ts, K, c));
+    if (limb) myC[c] = lerp1_(r.ifac_r, node_value(cs, K + 1, c), node_value(cs, K, c));
   };
-  fill(max(0, bracket(e0) - 1), min(ng - 2, bracket(e1) + 1));
-  const EdgePt pL = edge_point(false, v), pU = edge_point(true, v);
-  fill(pL.ind, pL.ind);
-  fill(pU.ind, pU.ind);
-  v.normL = edge_norm64(false, v);
-  v.normU = edge_norm64(true, v);
+  const int ia = max(0, bracket(e0) - 1), ib = min(ng - 2, bracket(e1) + 1);
+#pragma unroll 4
+  for (int c = 2 * ia + l; c <= 2 * ib + 3; c += FIX_LANES) put(c);
+  // four columns of each edge bracket
+  static_assert(FIX_LANES == 8, "a lane per column of the two edge brackets");
+  put(2 * edge_point(l >= 4, v).ind + (l & 3));
 }
 
 __device__ inline const double *profile_grid(const BatchDev &b, const ReqParams *rq) {
@@ -1977,14 +1976,21 @@ __global__ __launch_bounds__(64, MODE == 0 ? 1 : 3) void k_integrate(BatchDev b_
   }
 }
 
-// FP64 re-check of guarded FP32 bins, one entry per lane.
+// FP64 re-check of guarded FP32 bins, FIX_LANES lanes an entry, the entries
+// spread over the workgroups.  Bound: latency, of the entry's records, its table
+// columns and its integral.  One lane an entry read up to 2 n_g columns in turn,
+// 8 corner loads each, in wavefronts of 64 neighbouring entries: 1 entry 6.5 us,
+// 577 entries 19 us, 3017 wide bins of convolutions 30 us, 12354 30 us; with the
+// columns over the lanes 3.5 us, 8.5 us, 17 us and 20 us (26 us with 1024
+// workgroups).
 __global__ __launch_bounds__(64) void k_fixup(BatchDev b, int cos_rows) {
   extern __shared__ __align__(16) double s_dyn[];
-  const int lane = threadIdx.x;
+  constexpr int PER = 64 / FIX_LANES;  // entries per wavefront
+  const int sub = threadIdx.x / FIX_LANES, l = threadIdx.x % FIX_LANES;
   const int ng = b.rt.n_g;
   const int RS = 2 * ng + 1;
-  double *myT = s_dyn + lane * RS;
-  double *myC = cos_rows ? s_dyn + (64 + lane) * RS : myT;
+  double *myT = s_dyn + sub * RS;
+  double *myC = cos_rows ? s_dyn + (PER + sub) * RS : myT;
   const int n = min(b.ctr[CTR_FIX], b.fix_cap);
   RadiusView v;
   v.ng = ng;
@@ -1995,18 +2001,26 @@ __global__ __launch_bounds__(64) void k_fixup(BatchDev b, int cos_rows) {
   v.C64 = myC;
   v.T32 = nullptr;
   v.C32 = nullptr;
-  for (int e = blockIdx.x * 64 + lane; e < n; e += gridDim.x * 64) {
-    const FixEntry fe = b.fix[e];
+  for (int e0 = blockIdx.x; e0 < n; e0 += gridDim.x * PER) {  // (uniform: the barriers are met by all)
+    const int e = e0 + sub * gridDim.x;
+    const bool live = e < n;
+    const FixEntry fe = b.fix[live ? e : e0];
     const ReqParams *rq = b.req + fe.req;
     const RadRec pr = b.rad[(size_t)fe.req * b.nr_fine + fe.rad];
     const double *gn = b.rnode + (size_t)fe.req * RAD_NODE_ARRAYS * b.rt.n_r;
     const ReqNorm &rn = b.rnorm[fe.req];
+    const double *E = profile_grid(b, rq);
+    const double elo = E[fe.bin], ehi = E[fe.bin + 1];
     const RadGeo r = rad_geo(gn, gn + b.rt.n_r, gn + 2 * b.rt.n_r, fine_radius_at(rn.r1, rn.r2, fe.rad, b.nr_fine),
                              rad_K(pr));
-    const double *E = profile_grid(b, rq);
-    load_radius_table(b, b.rnorm[fe.req], r, rad_K(pr), rq->limb, E[fe.bin], E[fe.bin + 1], myT, myC, v);
-    const double val = integ_bin<0>(E[fe.bin], E[fe.bin + 1], v) * (pr.coef * b.rnorm[fe.req].fac);
-    unsafeAtomicAdd(&profile_acc(b, *rq)[(size_t)rad_zone(pr) * rq->n_e + fe.bin], val - fe.v32);
+    load_radius_table(b, rn, r, rad_K(pr), rq->limb, elo, ehi, myT, myC, v, l);
+    __syncthreads();  // one wavefront: the entry's columns before its lanes read them
+    v.normL = edge_norm64(false, v);
+    v.normU = edge_norm64(true, v);
+    const double val = integ_bin<0>(elo, ehi, v) * (pr.coef * rn.fac);
+    if (live && l == 0)
+      unsafeAtomicAdd(&profile_acc(b, *rq)[(size_t)rad_zone(pr) * rq->n_e + fe.bin], val - fe.v32);
+    __syncthreads();  // the next entry's columns overwrite them
   }
 }
 
@@ -3007,10 +3021,6 @@ int launch_setup(const BatchDev &b, void *stream) {
   return (int)hipGetLastError();
 }
 
-static size_t row_lds(const BatchDev &b, bool cos_rows, size_t elem) {
-  return (size_t)(cos_rows ? 2 : 1) * 64 * (2 * b.rt.n_g + 1) * elem;
-}
-
 // LDS of one k_integrate wavefront: lane rows, then (FP64 path) 64 weight
 // slots, then the SUM_BINS x SUM_STRIDE parked values, which double as the
 // node-row staging area.  *stage_rows: node rows the staging area takes, as
@@ -3080,9 +3090,9 @@ int launch_integrate(const BatchDev &b, int n_blocks, bool cos_rows, const SideW
 
 int launch_fixup(const BatchDev &b, bool cos_rows, void *stream) {
   if (b.mode != 1 || b.n_req <= 0) return 0;
-  const size_t lds = row_lds(b, cos_rows, sizeof(double));
+  const size_t lds = (size_t)(cos_rows ? 2 : 1) * (64 / FIX_LANES) * (2 * b.rt.n_g + 1) * sizeof(double);
   (void)hipFuncSetAttribute((const void *)k_fixup, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  hipLaunchKernelGGL(k_fixup, dim3(1024), dim3(64), lds, (hipStream_t)stream, b, (int)cos_rows);
+  hipLaunchKernelGGL(k_fixup, dim3(2048), dim3(64), lds, (hipStream_t)stream, b, (int)cos_rows);
   return (int)hipGetLastError();
 }
 
