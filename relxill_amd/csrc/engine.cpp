@@ -1210,6 +1210,8 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
   }
   b.any_cosne = false;
   b.any_limb = b.any_angular = false;
+  b.one_unit = (int)b.h_conv.size() == n_req;  // (and no second zone: one each)
+  for (const XillWork &u : b.h_conv) b.one_unit &= u.zone == 0;
   int64_t bins = 0;
   for (int i = 0; i < n_req; i++) {
     b.any_cosne |= b.h_req[i].need_cosne != 0;
@@ -1526,16 +1528,21 @@ static int launch_sequence(Batch &b, const RunKey &k, hipStream_t s) {
   if (prof) e |= (int)hipEventRecord(b.ev[2], s);
   e |= launch_fixup(bd, k.cos_rows != 0, s);
   if (prof) e |= (int)hipEventRecord(b.ev[3], s);
-  if (k.finalize) e |= launch_finalize(bd, s);
-  if (prof) e |= (int)hipEventRecord(b.ev[4], s);
+  // results by the last kernel where it has one workgroup a request
   const int with_xill = xill_takes_primary(w.n_xill, w.n_prim_rel);
+  const Deliver none = {nullptr, nullptr};
+  const Deliver to_host = {static_cast<int *>(k.res), k.n_out > 0 ? static_cast<double *>(k.res_out) : nullptr};
+  const bool by_line = k.finalize && w.n_conv == 0 && w.n_prim == 0;
+  const bool by_conv = k.one_unit && conv_delivers(w.n_conv) && w.n_prim == with_xill;
+  if (k.finalize) e |= launch_finalize(bd, by_line ? to_host : none, s);
+  if (prof) e |= (int)hipEventRecord(b.ev[4], s);
   e |= launch_xill(bd, w.xill, w.n_xill1, w.n_xill - w.n_xill1, w.prim, with_xill, k.prim_bins, s);
   if (prof) e |= (int)hipEventRecord(b.ev[5], s);
-  e |= launch_conv(bd, w.conv, w.n_conv, k.angular != 0, s);
+  e |= launch_conv(bd, w.conv, w.n_conv, k.angular != 0, by_conv ? to_host : none, s);
   if (prof) e |= (int)hipEventRecord(b.ev[6], s);
   e |= launch_primary(bd, w.prim + with_xill, w.n_prim - with_xill, k.prim_bins, s);
   if (prof) e |= (int)hipEventRecord(b.ev[7], s);
-  e |= launch_deliver(bd, static_cast<int *>(k.res), static_cast<double *>(k.res_out), k.n_out, s);
+  if (!by_line && !by_conv) e |= launch_deliver(bd, to_host.res, to_host.out, k.n_out, s);
   return e;
 }
 
@@ -1605,6 +1612,7 @@ int batch_run(Batch &b, int precision, std::string &err) {
   k.prof = g.profile ? 1 : 0;
   k.cos_rows = b.any_limb ? 1 : 0;
   k.angular = b.any_angular ? 1 : 0;
+  k.one_unit = b.one_unit ? 1 : 0;
   hipStream_t s = b.stream;
   b.profiled = k.prof != 0;
   if (g.use_graphs && !b.graph_failed && !b.one_shot) {

@@ -69,7 +69,7 @@ struct RunKey {
   BatchDev bd;
   WorkLists wl;
   int n_blocks, prim_bins;
-  int prof, cos_rows, finalize, angular;
+  int prof, cos_rows, finalize, angular, one_unit;
   // the request block fetched from pinned host memory at the start of the run
   // (n_fetch 16-byte words; 0: it is on the device) and the results delivered
   // there at its end (n_out output values; 0: statuses and counters only)
@@ -140,6 +140,7 @@ struct Batch {
   int item_cap = 0;
   int n_blocks = 1;  // workgroups of k_integrate
   bool any_cosne = false, any_limb = false, any_angular = false;
+  bool one_unit = false;  // every request has one unit of k_conv
   bool any_flux = false;  // some request has an input spectrum
   int fix_cap = 0;
   int last_mode = 1;

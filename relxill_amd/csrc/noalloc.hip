@@ -234,9 +234,9 @@ int noalloc_eval(int model, const double *parameter, const double *d_energy, con
     e |= launch_setup(bd, s);
     e |= launch_integrate(bd, n_blocks, cos_rows, nullptr, s);
     e |= launch_fixup(bd, cos_rows, s);
-    if (conv) e |= launch_conv(bd, d_work, 1, false, s);
-    else e |= launch_finalize(bd, s);
-    e |= launch_deliver(bd, res, nullptr, 0, s);
+    const Deliver dl = {res, nullptr};
+    if (conv) e |= launch_conv(bd, d_work, 1, false, dl, s);
+    else e |= launch_finalize(bd, dl, s);
     e |= (int)hipStreamSynchronize(s);
     // an overflowing FP32 re-check queue: the pass is redone in FP64
     if (e || !(bd.mode == 1 && res[CTR_FIX_OVF] != 0)) break;

@@ -382,6 +382,14 @@ struct BatchDev {
 };
 
 // ---- launchers (kernels.hip) ----
+// Pinned host memory that a run's last kernel with one workgroup a request
+// writes the results to, in place of k_deliver (null: nothing; out null:
+// counters and statuses only).
+struct Deliver {
+  int *res;
+  double *out;
+};
+
 // Work that k_integrate takes along: angle distributions (requests, chunks of
 // fine radii each) and zone records.
 struct SideWork {
@@ -408,10 +416,12 @@ int launch_dist(const BatchDev &b, const int *reqs, int n_reqs, void *stream);
 bool integrate_takes_side(const BatchDev &b, int n_blocks);
 int launch_integrate(const BatchDev &b, int n_blocks, bool limb, const SideWork *side, void *stream);
 int launch_fixup(const BatchDev &b, bool cos_rows, void *stream);
-int launch_finalize(const BatchDev &b, void *stream);
+int launch_finalize(const BatchDev &b, const Deliver &dl, void *stream);
 // conv_work: (request, zone) pairs; relxill requests have one per zone
 // (angular: a relxill_conv request is among them)
-int launch_conv(const BatchDev &b, const XillWork *conv_work, int n_conv_work, bool angular, void *stream);
+int launch_conv(const BatchDev &b, const XillWork *conv_work, int n_conv_work, bool angular, const Deliver &dl,
+                void *stream);
+bool conv_delivers(int n_conv_work);  // (launch_conv takes a Deliver)
 // work: n_single one-zone units, then n_multi units of several zones
 // (and the primaries of n_prim relxill requests: xill_takes_primary of them)
 int xill_takes_primary(int n_xill, int n_prim);
