@@ -245,6 +245,17 @@ __device__ inline void lp_rows(const DevLpTable &L, const ReqParams &rq, double 
   __syncthreads();
 }
 
+// The fine radii around r: the largest i in 0 .. nr - 2 with re(i) > r, or 0
+// (the radii descend; r1, r2: fine_radius_r1 of rout and rin).  The grid's own
+// formula gives the index to the rounding; the comparisons decide.
+__device__ inline int fine_above(double r1, double r2, double r, int nr) {
+  int i = (int)((1.0 / sqrt(r) - r1) / (r2 - r1) * (nr - 1));
+  i = min(max(i, 0), nr - 2);
+  while (i > 0 && !(fine_radius_at(r1, r2, i, nr) > r)) i--;
+  while (i < nr - 2 && fine_radius_at(r1, r2, i + 1, nr) > r) i++;
+  return i;
+}
+
 // One radial zone of a relxill request (IonGradient, src/IonGradient.cpp:
 // 182-209, :421-430): its centre, for the lamp post the emission angle there
 // (inv_rebin_mean of the fine grid's angles, src/relutility.c:636-663), the
@@ -290,12 +301,9 @@ __device__ inline ZoneRec zone_record(const DevXillTable &xt, const ReqParams &r
     o.lxi_fac = (float)(num / den);
   }
   if (lp) {
-    int lo = 0, hi = nr - 1;  // re(lo) > rmean >= re(hi)
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (fine_radius(rq.rin, rq.rout, mid, nr) > o.rmean) lo = mid; else hi = mid;
-    }
-    const double r0 = fine_radius(rq.rin, rq.rout, lo, nr), r1 = fine_radius(rq.rin, rq.rout, lo + 1, nr);
+    const double q1 = fine_radius_r1(rq.rout), q2 = fine_radius_r1(rq.rin);
+    const int lo = fine_above(q1, q2, o.rmean, nr);
+    const double r0 = fine_radius_at(q1, q2, lo, nr), r1 = fine_radius_at(q1, q2, lo + 1, nr);
     const LpFine f0 = lp_on_fine(r0, jr, je, jd, ji, ntr);
     const LpFine f1 = lp_on_fine(r1, jr, je, jd, ji, ntr);
     o.del_emit = lerp1((o.rmean - r1) / (r0 - r1), f1.del_emit, f0.del_emit);
@@ -1201,17 +1209,23 @@ __global__ __launch_bounds__(RRA_THREADS) void k_rrad_sums(BatchDev b, const int
 // zone its corrected boost over g (calc_rrad_emis_zone, :87-108); the sum times
 // the incident zone's flux factor.
 // Bound: FP64 issue of a pow per (incident, emitting zone, energy-shift bin),
-// 50 x 50 x 20 a request: about 180 us on the one CU of the request's k_setup
-// workgroup (239 -> 59 us without it), 30 us over the CUs of its 13 workgroups
-// here; 270 us and 71 us for 64 requests.
+// 50 x 50 x 20 a request, and before it the latency of the emissivity's chain:
+// about 180 us on the one CU of the request's k_setup workgroup (239 -> 59 us
+// without it), 24 us over the CUs of its 13 workgroups here (29 us with both
+// emissivities of a zone and the search for its radii on one thread); 270 us
+// and 57 us for 64 requests.
+// SPLIT: a workgroup's wavefronts share one incident zone's energy-shift bins,
+// for few requests, which leave the chip idle (1 request 14 us).
 constexpr int RR_ZONES = 4;
+template <int SPLIT>
 __global__ __launch_bounds__(64 * RR_ZONES) void k_rrad(BatchDev b, const int *__restrict__ reqs) {
-  constexpr int NT = 64 * RR_ZONES, GROUPS = MAX_RR / RR_ZONES;
+  constexpr int NT = 64 * RR_ZONES, PER = SPLIT ? 1 : RR_ZONES, GROUPS = MAX_RR / PER;
   __shared__ double s_jr[MAX_LP_R], s_je[MAX_LP_R], s_jd[MAX_LP_R], s_ji[MAX_LP_R];
   __shared__ double s_rad[MAX_RR], s_in[MAX_RR], s_cf[MAX_RR], s_cg[MAX_RR], s_corr[2];
-  __shared__ double s_zf[MAX_ZONES], s_zg[MAX_ZONES];
-  const int req = reqs[blockIdx.x / GROUPS], i0 = (blockIdx.x % GROUPS) * RR_ZONES;
-  const int tid = threadIdx.x, lane = tid & 63;
+  __shared__ double s_zf[MAX_ZONES], s_zg[MAX_ZONES], s_e[2][MAX_RR], s_r[2][MAX_RR];
+  __shared__ double s_term[RR_ZONES][64];
+  const int req = reqs[blockIdx.x / GROUPS], i0 = (blockIdx.x % GROUPS) * PER;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const ReqParams &rq = b.req[req];
   const int rr_n = rq.rr_n, nr = b.nr_fine, nz = rq.n_zones;
   if (rq.pre_status != 0 || i0 >= rr_n) return;  // uniform over the block
@@ -1221,28 +1235,52 @@ __global__ __launch_bounds__(64 * RR_ZONES) void k_rrad(BatchDev b, const int *_
   const int nt = R.n_rad, k = rq.rr_k, klo = rq.rr_klo;
   const double *rlo_t = R.rlo + (size_t)k * nt, *rhi_t = R.rhi + (size_t)k * nt;
   const double rin_f = fine_radius(rq.rin, rq.rout, nr - 1, nr), rout_f = fine_radius(rq.rin, rq.rout, 0, nr);
-  if (rq.rr_corr && tid < nz) {
-    // the correction factors of relxill zone tid from its band sums (k_rrad_sums):
+  // wavefronts 0 and 1: the emissivity at the fine radius outside and inside
+  // each table zone's centre; 2: the end zones; 3: the relxill zones' factors
+  auto centre = [&](int i) {
+    const double lo = (i == 0) ? rin_f : rlo_t[klo + i];
+    const double hi = (i == rr_n - 1) ? rout_f : rhi_t[klo + i];
+    return 0.5 * (lo + hi);
+  };
+  if (wave < 2) {
+    if (lane < rr_n) {
+      int err = 0;  // (k_setup evaluates and flags every fine radius)
+      const double q1 = fine_radius_r1(rq.rout), q2 = fine_radius_r1(rq.rin);
+      const int a = fine_above(q1, q2, centre(lane), nr) + wave;
+      const double r = fine_radius_at(q1, q2, a, nr);
+      s_r[wave][lane] = r;
+      s_e[wave][lane] = lp_emis_at(rq, r, s_jr, s_je, s_jd, s_ji, L.n_r, &err);
+    }
+  } else if (wave == 2) {  // ring-area corrections of the end zones (src/Relreturn_Table.cpp:415-435)
+    if (lane < 2) {
+      const int i = (lane == 0) ? 0 : rr_n - 1;
+      double rl = rlo_t[klo + i];
+      if (klo + i == 0 && rl > rq.rms) rl = rq.rms;
+      const double rh = rhi_t[klo + i];
+      const double lo = (i == 0) ? rin_f : rlo_t[klo + i];
+      const double hi = (i == rr_n - 1) ? rout_f : rhi_t[klo + i];
+      s_corr[lane] = (0.5 * (lo + hi) * (hi - lo)) / (0.5 * (rl + rh) * (rh - rl));
+    }
+  } else if (rq.rr_corr && lane < nz) {
+    // the correction factors of relxill zone lane from its band sums (k_rrad_sums):
     //   flux factor = energy flux over that of the zone's normalised primary
     //   (k_zone); g factor = photon flux over the shifted one's, over 1.5^Gamma
-    const ZoneRec zr = b.zone[rq.zone_off + tid];
+    const ZoneRec zr = b.zone[rq.zone_off + lane];
     const DevXillTable &xt = b.xt[rq.prim];
     const double f = xt.ect_dim >= 0 ? zr.ect_fac : rq.xfac[3];
     const int chunks = rrad_chunks(xt.n_ener);
-    const double *part = b.rrpart + rq.rr_corr_off + (size_t)(2 * tid) * chunks * 3;
+    const double *part = b.rrpart + rq.rr_corr_off + (size_t)(2 * lane) * chunks * 3;
     double s[3] = {0.0, 0.0, 0.0};
+#pragma unroll 4
     for (int c = 0; c < chunks; c++)
       for (int j = 0; j < 3; j++) s[j] += (1.0 - f) * part[c * 3 + j] + f * part[(chunks + c) * 3 + j];
-    s_zf[tid] = s[0] / zr.pe;
-    s_zg[tid] = s[1] / s[2] / pow(1.5, rq.xgam);
+    s_zf[lane] = s[0] / zr.pe;
+    s_zg[lane] = s[1] / s[2] / pow(1.5, rq.xgam);
   }
   __syncthreads();
-  int err = 0;  // (k_setup evaluates and flags every fine radius)
-  for (int i = tid; i < rr_n; i += NT) {
-    const double lo = (i == 0) ? rin_f : rlo_t[klo + i];
-    const double hi = (i == rr_n - 1) ? rout_f : rhi_t[klo + i];
-    const double rm = 0.5 * (lo + hi);
-    s_rad[i] = rm;
+  if (tid < rr_n) {
+    const double rm = centre(tid);
+    s_rad[tid] = rm;
     // relxilllp above spin 0: the correction factors of the relxill zone
     // the table zone's centre falls in (rebin_corrfactors_to_rradtable_grid,
     // src/Relreturn_Corona.cpp:248-289; a centre beyond the last edge takes
@@ -1256,37 +1294,21 @@ __global__ __launch_bounds__(64 * RR_ZONES) void k_rrad(BatchDev b, const int *_
       cf = s_zf[ind];
       cg = s_zg[ind];
     }
-    s_cf[i] = cf;
-    s_cg[i] = cg;
-    int a = 0, c = nr - 1;  // the fine radii re(a) > rm >= re(a+1)
-    while (c - a > 1) {
-      const int mid = (a + c) >> 1;
-      if (fine_radius(rq.rin, rq.rout, mid, nr) > rm) a = mid; else c = mid;
-    }
-    const double r0 = fine_radius(rq.rin, rq.rout, a, nr), r1 = fine_radius(rq.rin, rq.rout, a + 1, nr);
-    const double e0 = lp_emis_at(rq, r0, s_jr, s_je, s_jd, s_ji, L.n_r, &err);
-    const double e1 = lp_emis_at(rq, r1, s_jr, s_je, s_jd, s_ji, L.n_r, &err);
-    s_in[i] = lerp1((rm - r1) / (r0 - r1), e1, e0);
-  }
-  if (tid >= NT - 2) {  // ring-area corrections of the end zones (src/Relreturn_Table.cpp:415-435)
-    const int w = tid - (NT - 2), i = (w == 0) ? 0 : rr_n - 1;
-    double rl = rlo_t[klo + i];
-    if (klo + i == 0 && rl > rq.rms) rl = rq.rms;
-    const double rh = rhi_t[klo + i];
-    const double lo = (i == 0) ? rin_f : rlo_t[klo + i];
-    const double hi = (i == rr_n - 1) ? rout_f : rhi_t[klo + i];
-    s_corr[w] = (0.5 * (lo + hi) * (hi - lo)) / (0.5 * (rl + rh) * (rh - rl));
+    s_cf[tid] = cf;
+    s_cg[tid] = cg;
+    const double r0 = s_r[0][tid], r1 = s_r[1][tid];
+    s_in[tid] = lerp1((rm - r1) / (r0 - r1), s_e[1][tid], s_e[0][tid]);
   }
   __syncthreads();
-  const int i = i0 + (tid >> 6), j = lane, ng = R.n_g;
-  if (i >= rr_n) return;  // (no barrier below)
+  const int i = SPLIT ? i0 : i0 + wave, j = lane, ng = R.n_g;
+  if (i >= rr_n) return;  // (SPLIT: not reached; else no barrier below)
   double term = 0.0;
   if (j < rr_n) {
     const size_t t = (size_t)k * nt * nt + (size_t)(klo + i) * nt + (klo + j);
     const double gmin = R.gmin[t], gmax = R.gmax[t];
     const double cgj = s_cg[j];
     double ez = 0.0;
-    for (int jj = 0; jj < ng; jj++) {
+    for (int jj = SPLIT ? wave : 0; jj < ng; jj += SPLIT ? RR_ZONES : 1) {
       const double g = (jj + 0.5) / ng * (gmax - gmin) + gmin;  // get_gfac_grid (src/Relreturn_Datastruct.cpp:51-59)
       double v = R.frac_g[t * ng + jj];
       if (fabs(cgj - 1) > 1e-3) v *= gshift_boost(cgj, g, rq.gamma) / g;
@@ -1297,6 +1319,13 @@ __global__ __launch_bounds__(64 * RR_ZONES) void k_rrad(BatchDev b, const int *_
     if (j == 0 && i < rr_n - 1) tf *= s_corr[0];
     if (j == rr_n - 1 && i < rr_n - 2) tf *= s_corr[1];
     term = ez * tf * s_in[j];
+  }
+  if constexpr (SPLIT) {
+    s_term[wave][lane] = term;
+    __syncthreads();
+    if (wave > 0) return;
+    term = 0.0;
+    for (int w = 0; w < RR_ZONES; w++) term += s_term[w][lane];
   }
   const double sum = wave_sum(term);
   if (lane == 0) {
@@ -3228,9 +3257,15 @@ int launch_rrad(const BatchDev &b, const int *corr_reqs, int n_corr, const int *
     hipLaunchKernelGGL(k_rrad_sums, dim3(n_corr * n_chunk), dim3(RRA_THREADS), 0, (hipStream_t)stream, b, corr_reqs,
                        n_chunk);
   }
-  if (n_reqs > 0)
-    hipLaunchKernelGGL(k_rrad, dim3(n_reqs * (MAX_RR / RR_ZONES)), dim3(64 * RR_ZONES), 0, (hipStream_t)stream, b,
-                       reqs);
+  if (n_reqs > 0) {
+    auto go = [&](auto kern, int groups) {
+      hipLaunchKernelGGL(kern, dim3(n_reqs * groups), dim3(64 * RR_ZONES), 0, (hipStream_t)stream, b, reqs);
+    };
+    // a workgroup per incident zone repeats the emissivities of all zones, which
+    // costs nothing while CUs are idle: 8 requests' set-up 95 us and 102 us, 24
+    // requests 117 us and 121 us; 32 requests 127 us and 122 us
+    n_reqs <= 24 ? go(k_rrad<1>, MAX_RR) : go(k_rrad<0>, MAX_RR / RR_ZONES);
+  }
   return (int)hipGetLastError();
 }
 
