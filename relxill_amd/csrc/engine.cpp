@@ -1514,13 +1514,16 @@ static int launch_sequence(Batch &b, const RunKey &k, hipStream_t s) {
   const WorkLists &w = k.wl;
   if (prof) e |= (int)hipEventRecord(b.ev[0], s);
   e |= launch_begin(bd.ctr, k.fetch_src, k.fetch_dst, k.n_fetch, s);
-  e |= launch_nth(bd, w.nth, w.n_nth, s);
   // the angle distributions and the zone records go with k_integrate where it
   // can take them; the records come first where the returning radiation reads them
   const bool side = integrate_takes_side(bd, k.n_blocks), zone_side = side && w.n_rrc == 0;
   SideWork sw = {w.ang, w.zone, side ? w.n_ang : 0, 0, zone_side ? w.n_zone : 0};
-  if (!zone_side) e |= launch_zone(bd, w.zone, w.n_zone, s);
-  e |= launch_rrad(bd, w.rrc, w.n_rrc, w.rrad, w.n_rrad, s);
+  // (beside the sums it needs, or after the solves that they need)
+  const bool nth_side = w.n_rrc > 0 && w.n_nth > 0 && rrad_takes_nth(w.n_rrc);
+  if (!nth_side) e |= launch_nth(bd, w.nth, w.n_nth, s);
+  e |= launch_before_rrad(bd, w.rrc, w.n_rrc, nth_side ? w.nth : w.zone, nth_side ? w.n_nth : w.n_zone, nth_side, s);
+  if (!zone_side && (nth_side || w.n_rrc == 0)) e |= launch_zone(bd, w.zone, w.n_zone, s);
+  e |= launch_rrad(bd, w.rrad, w.n_rrad, s);
   e |= launch_setup(bd, s);
   if (!side) e |= launch_dist(bd, w.ang, w.n_ang, s);
   if (prof) e |= (int)hipEventRecord(b.ev[1], s);

@@ -97,7 +97,7 @@ struct Batch {
   std::vector<XillWork> h_conv;  // (request, zone) units of k_conv
   std::vector<XillWork> h_xill;  // k_xill units: one-zone requests first, then the others (all zones in one unit)
   int n_xill1 = 0;               // number of one-zone units at the front of h_xill
-  std::vector<int> h_rrc;        // requests with returning-radiation corrections (k_rrad_sums)
+  std::vector<int> h_rrc;        // requests with returning-radiation corrections (k_before_rrad)
   std::vector<int> h_rrad;       // requests with returning radiation (k_rrad)
   std::vector<XillWork> h_zone;  // (request, zone) units of k_zone (relxill and xillver models)
   std::vector<XillWork> h_nth;   // nthcomp solves: (request, 0 source / 1 + zone)

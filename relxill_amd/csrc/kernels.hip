@@ -967,7 +967,8 @@ __global__ __launch_bounds__(NT, NT == 256 ? 3 : 1) void k_setup(BatchDev b) {
 // zones (inside k_setup, zone after zone with tree sums: 18 us and 22 us, but
 // after the returning radiation that reads the records).
 constexpr int ZONE_LDS = 4 * MAX_LP_R;  // doubles
-__device__ __forceinline__ void zone_unit(const BatchDev &b, const XillWork wk, int lane, double *lds) {
+// (nt threads; the first wavefront's do the work behind the lamp post's rows)
+__device__ __forceinline__ void zone_unit(const BatchDev &b, const XillWork wk, int lane, int nt, double *lds) {
   double *s_jr = lds, *s_je = lds + MAX_LP_R, *s_jd = lds + 2 * MAX_LP_R, *s_ji = lds + 3 * MAX_LP_R;
   const int req = wk.req, z = wk.zone;
   const ReqParams &rq = b.req[req];
@@ -985,9 +986,11 @@ __device__ __forceinline__ void zone_unit(const BatchDev &b, const XillWork wk, 
     zr.lxi_ind = xt.lxi_dim >= 0 ? rq.xind[xt.lxi_dim] : 0;
     zr.lxi_fac = xt.lxi_dim >= 0 ? rq.xfac[xt.lxi_dim] : 0.0;
   } else {
-    if (lp) lp_rows(b.lp, rq, s_jr, s_je, s_jd, s_ji, lane, 64);
+    if (lp) lp_rows(b.lp, rq, s_jr, s_je, s_jd, s_ji, lane, nt);
+    if (lane >= 64) return;
     zr = zone_record(xt, rq, z, lp, s_jr, s_je, s_jd, s_ji, b.lp.n_r, b.nr_fine, &ect);
   }
+  if (lane >= 64) return;
   zr.ncf = 1.0;
   zr.pe = 0.0;
   if (rq.prim == PRIM_NTHCOMP) {
@@ -1030,7 +1033,7 @@ __device__ __forceinline__ void zone_unit(const BatchDev &b, const XillWork wk, 
 
 __global__ __launch_bounds__(64) void k_zone(BatchDev b, const XillWork *__restrict__ work) {
   __shared__ double s_lds[ZONE_LDS];
-  zone_unit(b, work[blockIdx.x], threadIdx.x, s_lds);
+  zone_unit(b, work[blockIdx.x], threadIdx.x, 64, s_lds);
 }
 
 // The eight corners of a request's xillver table row on the interpolated axes
@@ -1086,12 +1089,20 @@ __device__ inline void corners8(const DevXillTable &xt, const ReqParams &rq, int
 // partial sums go to rrpart[zone][node][chunk][3].
 // Bound: L2 / HBM reads of 80 rows per Ecut node.  One workgroup per (request,
 // zone) with 160 rows a zone and the shift's rebin took 144 us for one request (362 us with a density
-// division, 696 us for 64 of those); this takes 16 us (16 us, 28 us).
-__global__ __launch_bounds__(RRA_THREADS) void k_rrad_sums(BatchDev b, const int *__restrict__ reqs, int n_chunk) {
-  __shared__ double s_wa[MAX_INCL];
-  __shared__ double s_w[3][RRA_THREADS / 64];
-  __shared__ int s_ind[MAX_ZONES];
-  const int req = reqs[blockIdx.x / n_chunk], chunk = blockIdx.x % n_chunk, tid = threadIdx.x;
+// division, 696 us for 64 of those); this takes 16 us (16 us, 28 us), with the brackets from
+// the lamp post's rows 24 us, but beside the zone records.
+// The brackets are taken from the lamp post's rows here too, so that the sums
+// need nothing of k_zone or k_nth and run beside them (k_before_rrad).
+struct RradLds {
+  double rows[ZONE_LDS];
+  double wa[MAX_INCL];
+  double w[3][RRA_THREADS / 64];
+  double ect_fac[MAX_ZONES], lxi_fac[MAX_ZONES];
+  int ect_ind[MAX_ZONES], lxi_ind[MAX_ZONES];
+};
+__device__ __forceinline__ void rrad_sums(const BatchDev &b, int req, int chunk, int tid, RradLds &S) {
+  double *s_wa = S.wa, (*s_w)[RRA_THREADS / 64] = S.w;
+  int *s_ind = S.ect_ind;
   const ReqParams &rq = b.req[req];
   const DevXillTable xt = b.xt[rq.prim];
   const int chunks = rrad_chunks(xt.n_ener);  // of this request's table
@@ -1104,7 +1115,20 @@ __global__ __launch_bounds__(RRA_THREADS) void k_rrad_sums(BatchDev b, const int
     const double incl_deg = (double)xt.incl_vals[a] * 180 / PI;
     s_wa[a] = 0.5 * cos(incl_deg * PI / 180) / ni;
   }
-  if (tid < nz) s_ind[tid] = xt.ect_dim >= 0 ? b.zone[rq.zone_off + tid].ect_ind : rq.xind[3];
+  if (xt.ect_dim >= 0 || grad) {
+    double *jr = S.rows, *je = jr + MAX_LP_R, *jd = je + MAX_LP_R, *ji = jd + MAX_LP_R;
+    lp_rows(b.lp, rq, jr, je, jd, ji, tid, RRA_THREADS);
+    if (tid < nz) {
+      double ect;
+      const ZoneRec zr = zone_record(xt, rq, tid, true, jr, je, jd, ji, b.lp.n_r, b.nr_fine, &ect);
+      s_ind[tid] = xt.ect_dim >= 0 ? zr.ect_ind : rq.xind[3];
+      S.ect_fac[tid] = zr.ect_fac;
+      S.lxi_ind[tid] = zr.lxi_ind;
+      S.lxi_fac[tid] = zr.lxi_fac;
+    }
+  } else if (tid < nz) {
+    s_ind[tid] = rq.xind[3];
+  }
   __syncthreads();
   const int e = chunk * RRA_THREADS + tid;
   const bool in = e < ne;
@@ -1170,7 +1194,8 @@ __global__ __launch_bounds__(RRA_THREADS) void k_rrad_sums(BatchDev b, const int
     return;
   }
   for (int z = 0; z < nz; z++) {
-    const ZoneRec &zr = b.zone[rq.zone_off + z];
+    const double zef = S.ect_fac[z], zlf = S.lxi_fac[z];
+    const int zei = S.ect_ind[z], zli = S.lxi_ind[z];
     double avg = 0.0;
     for (int c = 0; c < 16; c++) {  // the zone's own Ecut and logXi brackets
       double w = 1.0;
@@ -1179,9 +1204,9 @@ __global__ __launch_bounds__(RRA_THREADS) void k_rrad_sums(BatchDev b, const int
       for (int k = 0; k < 4; k++) {
         const bool ie = (k == xt.ect_dim), il = (k == xt.lxi_dim);
         const int o = (c >> (3 - k)) & 1;
-        const double f = ie ? zr.ect_fac : (il ? zr.lxi_fac : rq.xfac[k]);
+        const double f = ie ? zef : (il ? zlf : rq.xfac[k]);
         w *= o ? f : (1.0 - f);
-        r = r * (unsigned)xt.n_val[k] + (unsigned)((ie ? zr.ect_ind : (il ? zr.lxi_ind : rq.xind[k])) + o);
+        r = r * (unsigned)xt.n_val[k] + (unsigned)((ie ? zei : (il ? zli : rq.xind[k])) + o);
       }
       for (int o = 0; o < n_o; o++) {
         const double wo = n_o == 1 ? w : w * (o ? rq.xo_fac : 1.0 - rq.xo_fac);
@@ -1262,7 +1287,7 @@ __global__ __launch_bounds__(64 * RR_ZONES) void k_rrad(BatchDev b, const int *_
       s_corr[lane] = (0.5 * (lo + hi) * (hi - lo)) / (0.5 * (rl + rh) * (rh - rl));
     }
   } else if (rq.rr_corr && lane < nz) {
-    // the correction factors of relxill zone lane from its band sums (k_rrad_sums):
+    // the correction factors of relxill zone lane from its band sums (rrad_sums):
     //   flux factor = energy flux over that of the zone's normalised primary
     //   (k_zone); g factor = photon flux over the shifted one's, over 1.5^Gamma
     const ZoneRec zr = b.zone[rq.zone_off + lane];
@@ -1344,30 +1369,33 @@ __global__ __launch_bounds__(64 * RR_ZONES) void k_rrad(BatchDev b, const int *_
 // 500-bin grid and the energy flux of the normalised spectrum in 0.1-1000 keV
 // (calc_xillver_normalization_change_source_to_disk, src/Xillspec.cpp:408-435;
 // get_xillver_fluxcorr, :344-362); the source's also keeps its solution for
-// k_primary.  First in a run: k_rrad_corr and k_setup read the results.
+// k_primary.  First in a run: k_zone reads the results.
 constexpr int NTH_THREADS_R = 256;
 
-__global__ __launch_bounds__(NTH_THREADS_R) void k_nth(BatchDev b, const XillWork *__restrict__ work) {
-  __shared__ NthLds L;
-  __shared__ double s_red[NTH_THREADS_R];
-  __shared__ double s_kte;
-  const XillWork wk = work[blockIdx.x];
-  const int req = wk.req, j = wk.zone, tid = threadIdx.x;
+struct NthJobLds {
+  NthLds L;
+  double red[NTH_THREADS_R];
+  double kte;
+};
+__device__ __forceinline__ void nth_job(const BatchDev &b, const XillWork wk, int tid, NthJobLds &S) {
+  NthLds &L = S.L;
+  double *s_red = S.red;
+  const int req = wk.req, j = wk.zone;
   const ReqParams &rq = b.req[req];
   if (rq.pre_status != 0) return;  // uniform over the block
   if (j == 0) {
-    if (tid == 0) s_kte = rq.xect_src;
+    if (tid == 0) S.kte = rq.xect_src;
   } else {
     // the lamp-post rows in the solve's arrays (the solve overwrites them)
     lp_rows(b.lp, rq, L.t1, L.t2, L.t3, L.d, tid, NTH_THREADS_R);
     if (tid == 0) {
       double ect;
       (void)zone_record(b.xt[rq.prim], rq, j - 1, true, L.t1, L.t2, L.t3, L.d, b.lp.n_r, b.nr_fine, &ect);
-      s_kte = ect;
+      S.kte = ect;
     }
   }
   __syncthreads();
-  const double kte = s_kte;
+  const double kte = S.kte;
   const int nth = nth_solve(L, nth_grid_tab(b.nth_tab), kte, rq.xgam, tid, NTH_THREADS_R);
   // the spectrum on the 500-bin grid (spec_nthcomp at z = 0), per bin in t2
   const double nfac = nthcomp_normfac(L.x, L.t1, nth, 0.0);
@@ -1395,6 +1423,32 @@ __global__ __launch_bounds__(NTH_THREADS_R) void k_nth(BatchDev b, const XillWor
     for (int i = tid; i < NTH_N; i += NTH_THREADS_R) so[i] = L.t1[i];
     if (tid == 0) b.nth_n[rq.nth_sol] = nth;
   }
+}
+
+__global__ __launch_bounds__(NTH_THREADS_R) void k_nth(BatchDev b, const XillWork *__restrict__ work) {
+  __shared__ NthJobLds s_job;
+  nth_job(b, work[blockIdx.x], threadIdx.x, s_job);
+}
+
+// Before k_rrad, side by side: the xillver band sums, and the nthcomp solves
+// (NTH) or the zone records.  One after the other zones and sums were 17 us and
+// 16 us of a relxilllp call, solves, zones and sums 23 us, 10 us and 16 us of a
+// relxilllpCp call; 24 us, and 24 us and 10 us, here.
+template <int NTH>
+__global__ __launch_bounds__(RRA_THREADS) void k_before_rrad(BatchDev b, const XillWork *__restrict__ work, int n_work,
+                                                             const int *__restrict__ reqs, int n_chunk) {
+  static_assert(RRA_THREADS == NTH_THREADS_R, "one workgroup size");
+  constexpr size_t LDS = NTH ? (sizeof(NthJobLds) > sizeof(RradLds) ? sizeof(NthJobLds) : sizeof(RradLds))
+                             : sizeof(RradLds);
+  __shared__ __align__(16) char s_raw[LDS];
+  const int tid = threadIdx.x;
+  if ((int)blockIdx.x < n_work) {
+    if constexpr (NTH) nth_job(b, work[blockIdx.x], tid, *reinterpret_cast<NthJobLds *>(s_raw));
+    else zone_unit(b, work[blockIdx.x], tid, RRA_THREADS, reinterpret_cast<double *>(s_raw));
+    return;
+  }
+  const int k = blockIdx.x - n_work;
+  rrad_sums(b, reqs[k / n_chunk], k % n_chunk, tid, *reinterpret_cast<RradLds *>(s_raw));
 }
 
 // First in a run: clears its counters and, for an evaluation call, copies the
@@ -1789,7 +1843,7 @@ __global__ __launch_bounds__(64, MODE == 0 ? 1 : 3) void k_integrate(BatchDev b_
     }
     one_item -= n_chunk;
     if (one_item < side.n_zone) {
-      zone_unit(b, side.zone[one_item], lane, s_dyn);
+      zone_unit(b, side.zone[one_item], lane, 64, s_dyn);
       return;
     }
     one_item -= side.n_zone;
@@ -3251,12 +3305,24 @@ int launch_xill(const BatchDev &b, const XillWork *work, int n_single, int n_mul
   return (int)hipGetLastError();
 }
 
-int launch_rrad(const BatchDev &b, const int *corr_reqs, int n_corr, const int *reqs, int n_reqs, void *stream) {
-  if (n_corr > 0) {
-    const int n_chunk = rrad_chunks(xill_n_ener(b));
-    hipLaunchKernelGGL(k_rrad_sums, dim3(n_corr * n_chunk), dim3(RRA_THREADS), 0, (hipStream_t)stream, b, corr_reqs,
-                       n_chunk);
-  }
+// the solves' LDS (45 KB) leaves three workgroups a CU: 8 requests' set-up 101 us,
+// 111 us with the solves in a launch of their own, 32 requests 121 us and 130 us;
+// 64 requests (72 us and 61 us for solves, zones and sums) keep them apart
+bool rrad_takes_nth(int n_corr) { return n_corr <= 32; }
+
+int launch_before_rrad(const BatchDev &b, const int *corr_reqs, int n_corr, const XillWork *work, int n_work, bool nth,
+                       void *stream) {
+  if (n_corr <= 0) return 0;
+  const int n_chunk = rrad_chunks(xill_n_ener(b));
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(n_work + n_corr * n_chunk), dim3(RRA_THREADS), 0, (hipStream_t)stream, b, work,
+                       n_work, corr_reqs, n_chunk);
+  };
+  nth ? go(k_before_rrad<1>) : go(k_before_rrad<0>);
+  return (int)hipGetLastError();
+}
+
+int launch_rrad(const BatchDev &b, const int *reqs, int n_reqs, void *stream) {
   if (n_reqs > 0) {
     auto go = [&](auto kern, int groups) {
       hipLaunchKernelGGL(kern, dim3(n_reqs * groups), dim3(64 * RR_ZONES), 0, (hipStream_t)stream, b, reqs);

@@ -230,7 +230,7 @@ int noalloc_eval(int model, const double *parameter, const double *d_energy, con
     e |= (int)hipGetLastError();
     // (the one unit {0, 0} of d_work is the list of request 0)
     if (p.return_rad != 0 && p.pre_status == 0)
-      e |= launch_rrad(bd, nullptr, 0, reinterpret_cast<const int *>(d_work), 1, s);
+      e |= launch_rrad(bd, reinterpret_cast<const int *>(d_work), 1, s);
     e |= launch_setup(bd, s);
     e |= launch_integrate(bd, n_blocks, cos_rows, nullptr, s);
     e |= launch_fixup(bd, cos_rows, s);

@@ -428,9 +428,14 @@ int xill_takes_primary(int n_xill, int n_prim);
 int launch_xill(const BatchDev &b, const XillWork *work, int n_single, int n_multi, const int *prim, int n_prim,
                 int max_bins, void *stream);
 // returning radiation (before launch_setup): the xillver band sums of the
-// n_corr relxilllp requests above spin 0 (after launch_zone), then the returning
-// emissivity of all n_reqs requests with it
-int launch_rrad(const BatchDev &b, const int *corr_reqs, int n_corr, const int *reqs, int n_reqs, void *stream);
+// n_corr relxilllp requests above spin 0, with the zone records or (nth, where
+// rrad_takes_nth) the nthcomp solves of work beside them
+bool rrad_takes_nth(int n_corr);
+int launch_before_rrad(const BatchDev &b, const int *corr_reqs, int n_corr, const XillWork *work, int n_work, bool nth,
+                       void *stream);
+// the returning emissivity of all n_reqs requests with it (after the sums and
+// the zone records)
+int launch_rrad(const BatchDev &b, const int *reqs, int n_reqs, void *stream);
 // relxill and xillver requests: the zone records, one (request, zone) unit each
 // (after launch_nth)
 int launch_zone(const BatchDev &b, const XillWork *work, int n_work, void *stream);
