@@ -2267,13 +2267,29 @@ __device__ __forceinline__ void dft(double2 *v) {
   }
 }
 
+// The twiddles of this thread's first value in a radix-R pass (at most 7).
+__device__ __forceinline__ void load_twiddles(double2 *w, int R, int N, int Ns, const double2 *twp) {
+  const int j = threadIdx.x;
+  if (j >= N / R) return;
+  const int k = j & (Ns - 1);
+#pragma unroll
+  for (int r = 1; r < 8; r++)
+    if (r < R) w[r - 1] = twp[r * Ns + k];
+}
+
+// Radix of the pass with N / Ns left.
+__device__ __forceinline__ int fft_radix(int left) { return left % 8 == 0 ? 8 : left % 4 == 0 ? 4 : 2; }
+
 // One Stockham radix-R pass over N complex values in LDS (padded layout):
 // thread j loads x[j + r N/R] r = 0..R-1, twiddles by w^(r (j mod Ns)),
 // w = exp(S 2 pi i / (Ns R)) (table twp[r Ns + k], forward sign, conjugated
 // for S = +1), transforms, and stores at (j / Ns) Ns R + j mod Ns + r Ns.
-// PER j values per thread; reads finish before any write.
+// PER j values per thread; reads finish before any write.  w holds the first
+// j's twiddles, and receives the next pass' before the barriers, so that their
+// reads (L2) are in flight meanwhile (1 unit 30.8 us and 29.6 us, 256 units 46 us
+// and 41 us, 4096 units 350 us and 342 us).
 template <int R, int S, int PER>
-__device__ __forceinline__ void fft_pass(double2 *buf, int N, int Ns, const double2 *twp) {
+__device__ __forceinline__ void fft_pass(double2 *buf, int N, int Ns, const double2 *twp, double2 *w) {
   const int J = N / R;
   double2 v[PER][R];
   const int lgNs = __ffs(Ns) - 1;  // Ns is a power of two
@@ -2286,15 +2302,16 @@ __device__ __forceinline__ void fft_pass(double2 *buf, int N, int Ns, const doub
       for (int r = 0; r < R; r++) {
         double2 x = buf[P(j + r * J)];
         if (r > 0) {
-          double2 w = twp[r * Ns + k];
-          if (S > 0) w.y = -w.y;
-          x = cmul(x, w);
+          double2 t = u == 0 ? w[r - 1] : twp[r * Ns + k];
+          if (S > 0) t.y = -t.y;
+          x = cmul(x, t);
         }
         v[u][r] = x;
       }
       dft<R, S>(v[u]);
     }
   }
+  if (Ns * R < N) load_twiddles(w, fft_radix(N / (Ns * R)), N, Ns * R, twp + R * Ns);
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < PER; u++) {
@@ -2310,38 +2327,33 @@ __device__ __forceinline__ void fft_pass(double2 *buf, int N, int Ns, const doub
 }
 
 // The block has at least N/8 threads, so a pass holds at most 8 values per
-// thread: PER = 1 (R = 8), <= 2 (R = 4), <= 4 (R = 2); radix 16 keeps PER = 1.
+// thread: PER = 1 (R = 8), <= 2 (R = 4), <= 4 (R = 2).
 template <int R, int S>
-__device__ __forceinline__ void fft_pass_any(double2 *buf, int N, int Ns, const double2 *twp) {
+__device__ __forceinline__ void fft_pass_any(double2 *buf, int N, int Ns, const double2 *twp, double2 *w) {
   const int per = (N / R + blockDim.x - 1) / blockDim.x;
-  if (per <= 1) fft_pass<R, S, 1>(buf, N, Ns, twp);
-  else if (R <= 8 && per <= 2) fft_pass<R, S, (R <= 8 ? 2 : 1)>(buf, N, Ns, twp);
-  else if (R <= 4 && per <= 4) fft_pass<R, S, (R <= 4 ? 4 : 1)>(buf, N, Ns, twp);
-  else fft_pass<R, S, (R <= 2 ? 8 : 1)>(buf, N, Ns, twp);
+  if (per <= 1) fft_pass<R, S, 1>(buf, N, Ns, twp, w);
+  else if (R <= 4 && per <= 2) fft_pass<R, S, (R <= 4 ? 2 : 1)>(buf, N, Ns, twp, w);
+  else fft_pass<R, S, (R <= 2 ? 4 : 1)>(buf, N, Ns, twp, w);
 }
 
 // Unnormalised complex FFT of N (power of two, 2..8192) values in LDS,
 // natural order in and out; radix-8 passes, then one of radix 4 or 2 (the
 // block has at least N/8 threads).  twp holds the passes' tables one after
-// the other (R Ns entries each), in the same plan as the host builds them.
+// the other (R Ns entries each), in the same plan as the host builds them (the
+// first pass' twiddles are all 1).
 template <int S>
 __device__ __forceinline__ void lds_fft(double2 *buf, int N, const double2 *twp) {
+  double2 w[7];
+#pragma unroll
+  for (int r = 0; r < 7; r++) w[r] = make_double2(1.0, 0.0);
   int Ns = 1;
   while (Ns < N) {
-    const int left = N / Ns;
-    if (left % 8 == 0) {
-      fft_pass_any<8, S>(buf, N, Ns, twp);
-      twp += 8 * Ns;
-      Ns *= 8;
-    } else if (left % 4 == 0) {
-      fft_pass_any<4, S>(buf, N, Ns, twp);
-      twp += 4 * Ns;
-      Ns *= 4;
-    } else {
-      fft_pass_any<2, S>(buf, N, Ns, twp);
-      twp += 2 * Ns;
-      Ns *= 2;
-    }
+    const int R = fft_radix(N / Ns);
+    if (R == 8) fft_pass_any<8, S>(buf, N, Ns, twp, w);
+    else if (R == 4) fft_pass_any<4, S>(buf, N, Ns, twp, w);
+    else fft_pass_any<2, S>(buf, N, Ns, twp, w);
+    twp += R * Ns;
+    Ns *= R;
   }
 }
 
@@ -3242,7 +3254,8 @@ int launch_conv(const BatchDev &b, const XillWork *conv_work, int n_conv_work, b
   // where every unit has a CU of its own the most threads (but not more than
   // bins, which a wavefront takes by the 64), so that the phases over the grid
   // take half the rounds: 1 relxill unit of 4096 bins 36 us and 33 us, 256 relconv
-  // units 50 us and 45 us; 1024 units 110 us and 127 us
+  // units 50 us and 45 us; 1024 units 110 us and 127 us (1.2 to 5 us less all of
+  // them with the twiddles read ahead)
   if (conv_delivers(n_conv_work)) {
     const int nt = std::min(CONV_THREADS_MAX, b.cg.n);
     angular ? go(k_conv<1, 1>, nt) : go(k_conv<1, 0>, nt);
