@@ -180,7 +180,7 @@ int noalloc_eval(int model, const double *parameter, const double *d_energy, con
   if (wpc <= 0) wpc = ws.waves_per_cu;
   // (a caller's line grid is on the device: all its bins)
   const int bins = conv ? reach_bins(g.conv_ener.data(), g.conv_n, 1.0) : p.n_e;
-  const int item_cap = n_rc * ((bins + seg - 1) / seg);
+  auto items = [&](int s) { return n_rc * ((bins + s - 1) / s); };
   const int fix_cap = std::max(4096, p.n_e * 4);
 
   BatchDev bd;
@@ -189,7 +189,6 @@ int noalloc_eval(int model, const double *parameter, const double *d_energy, con
   Carve c{static_cast<char *>(g_scratch[g.device])};
   bd.n_req = 1;
   bd.nr_fine = g.nr_fine;
-  bd.seg_bins = seg;
   bd.req = c.take<ReqParams>(1);
   bd.ener_in = d_energy;
   bd.flux_in = conv ? d_flux_in : nullptr;
@@ -202,8 +201,6 @@ int noalloc_eval(int model, const double *parameter, const double *d_energy, con
   bd.dist = c.take<double>(1);
   bd.refl = c.take<LpRefl>(1);
   bd.status = c.take<int>(1);
-  bd.items = c.take<WorkItem>((size_t)item_cap);
-  bd.item_cap = item_cap;
   bd.ctr = c.take<int>(N_COUNTERS);
   bd.reach = c.take<BinRange>(1);
   bd.fix = c.take<FixEntry>((size_t)fix_cap);
@@ -214,6 +211,12 @@ int noalloc_eval(int model, const double *parameter, const double *d_energy, con
   bd.xspec = nullptr;
   bd.zone = c.take<ZoneRec>(1);
   XillWork *d_work = c.take<XillWork>(1);
+  // the work list last: where short segments' does not fit, that of longer ones
+  while (seg < 64 && c.used + 256 + sizeof(WorkItem) * (size_t)items(seg) > kScratchBytes) seg *= 2;
+  const int item_cap = items(seg);
+  bd.seg_bins = seg;
+  bd.items = c.take<WorkItem>((size_t)item_cap);
+  bd.item_cap = item_cap;
   if (c.used > kScratchBytes) {
     msg = "request needs more work memory than the allocation-free entry point holds "
           "(RX_NOALLOC_SCRATCH_BYTES): fewer bins or smaller tables";
