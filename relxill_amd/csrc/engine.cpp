@@ -1182,6 +1182,12 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
   const int64_t n_fin = b.any_flux ? o_flux : 0;
   layout_block(b);
   b.staged = b.block_bytes <= (b.is_call ? STAGE_MAX : b.keep_stage ? STAGE_KEEP : STAGE_MAX);
+  // (a server slot takes pinned memory from its second large batch on: allocating
+  // it costs a new server's first batches more than their copies)
+  if (b.one_shot && b.h_stage.bytes < b.block_bytes && !b.stage_wanted) {
+    b.stage_wanted = true;
+    b.staged = false;
+  }
   if (b.keep_stage && b.staged) {
     if (!b.h_stage.ensure(std::max<size_t>(b.block_bytes, b.one_shot ? STAGE_MAX : 0))) {
       err = "pinned host allocation failed";

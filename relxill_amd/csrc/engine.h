@@ -120,6 +120,7 @@ struct Batch {
   // keep their own, others use the library's while they are built), the run's
   // results (result_*).
   bool keep_stage = false;
+  bool stage_wanted = false;  // a server slot's pinned request block has been missed once
   PinnedBuf h_stage, h_res;
   // an evaluation call: the run fetches the request block and delivers the
   // outputs itself (call_run: this one does)
