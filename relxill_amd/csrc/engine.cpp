@@ -902,11 +902,6 @@ static CpRequest remap_cp(int model, const double *par) {
   return c;
 }
 
-// Request blocks up to STAGE_MAX go to the device through pinned memory in one
-// piece (of a server slot, which keeps its pinned memory: up to STAGE_KEEP);
-// larger ones piece by piece from the batch's own arrays, a copy less.
-constexpr size_t STAGE_MAX = 4u << 20, STAGE_KEEP = 32u << 20;
-
 static size_t align_up(size_t n) { return (n + 255) & ~(size_t)255; }
 
 // Offsets of the request block's pieces.
@@ -1181,7 +1176,7 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
   // batch keeps its own (a call, a server slot), else into the batch's arrays
   const int64_t n_fin = b.any_flux ? o_flux : 0;
   layout_block(b);
-  b.staged = b.block_bytes <= (b.is_call ? STAGE_MAX : b.keep_stage ? STAGE_KEEP : STAGE_MAX);
+  b.staged = b.block_bytes <= STAGE_MAX;
   // (a server slot takes pinned memory from its second large batch on: allocating
   // it costs a new server's first batches more than their copies)
   if (b.one_shot && b.h_stage.bytes < b.block_bytes && !b.stage_wanted) {

@@ -80,6 +80,10 @@ struct RunKey {
   int64_t n_out;
 };
 
+// Request blocks up to STAGE_MAX go to the device through pinned memory in one
+// piece; larger ones piece by piece from the batch's own arrays, a copy less.
+constexpr size_t STAGE_MAX = 4u << 20;
+
 struct Batch {
   int n_req = 0;
   int max_zones = 1;          // most zones of a request
