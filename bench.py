@@ -612,7 +612,7 @@ def main():
     tpath = os.path.join(ROOT, "profiles", "hbm_traffic_relconv_batch4096.json")
     if os.path.exists(tpath):
         tj = json.load(open(tpath))
-        ki = tj.get("kernels", {}).get("k_integrate<1, 0>")
+        ki = tj.get("kernels", {}).get("k_integrate<1, 0, 0>")
         if ki and len(reqs) == 4096:
             traffic = round(ki["read_bytes"] + ki["write_bytes"])
             traffic_src = tj.get("source")
@@ -622,7 +622,7 @@ def main():
                     frac=achieved / HBM_PEAK_GBS, traffic=traffic, traffic_source=traffic_src,
                     traffic_shape=traffic_shape, valu_busy=valu_busy,
                     algorithmic_bytes=round(alg_bytes),
-                    kernel="k_integrate<1, 0>", kernel_ms=round(kms32[1], 4),
+                    kernel="k_integrate<1, 0, 0>", kernel_ms=round(kms32[1], 4),
                     kernel_ms_all={k: round(v, 4) for k, v in zip(KERNELS, kms32)})
 
     cpu = None

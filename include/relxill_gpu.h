@@ -365,7 +365,8 @@ int rx_batch_zones(rx_batch *b, int i, double *out, int n_zones);
 int rx_batch_reflfrac(rx_batch *b, int i, double *out5);
 /* Integration work shape: bins per work item (segment of one chunk of 64
  * fine radii; 0: automatic / autotuned) and persistent wavefronts per CU
- * (0: automatic / autotuned). */
+ * (0: automatic / autotuned; batches of up to 8192 windows run one workgroup per
+ * item instead). */
 int rx_batch_set_shape(rx_batch *b, int seg_bins, int waves_per_cu);
 void rx_batch_destroy(rx_batch *b);
 
@@ -378,9 +379,11 @@ int rx_reflset_create(const double *refl_energy, int n_refl, const double *refl,
 int rx_reflsets_clear(void);
 
 /* Kernel timing of the last rx_batch_run with profiling enabled: per kernel
- * (0 k_setup (with k_reset), 1 k_integrate, 2 k_fixup, 3 k_finalize, 4 k_conv,
- * 5 k_xill, 6 k_primary) the duration in ms measured with HIP events on the
- * batch's stream. */
+ * (0 everything up to k_setup and, in launches of their own, the angle
+ * distributions; 1 k_integrate, with the distributions and zone records it takes
+ * along; 2 k_fixup, 3 k_finalize, 4 k_conv, 5 k_xill with the primaries it takes
+ * along, 6 k_primary otherwise) the duration in ms measured with HIP events on
+ * the batch's stream. */
 #define RX_N_TIMED 7
 int rx_profile_enable(int on);
 /* Streams `bytes` through a plain device copy kernel `reps` times (after one

@@ -1,4 +1,4 @@
-"""The zones' returning-radiation correction factors (k_zone, k_rrad_sums,
+"""The zones' returning-radiation correction factors (k_zone, k_before_rrad,
 k_rrad) at the edges of their tiles against the oracle: xillver tables of one
 workgroup's bins, one less, one more and several workgroups, 4 and 10
 inclinations (those of 2, 3 or 5 give the synthetic tables a negative average and status 41), a table whose band 0.15-500 keV reaches beyond its last edge when
