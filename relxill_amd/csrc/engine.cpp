@@ -1247,7 +1247,16 @@ void batch_plan(Batch &b, int seg_bins, int waves_per_cu) {
     windows += n_rc + b.h_req[i].n_zones - 1;
     max_bins = std::max(max_bins, b.h_req[i].n_e);
   }
-  const WorkShape ws = work_shape(windows, max_bins);
+  const int conv_reach = reach_bins(g.conv_ener.data(), g.conv_n, 1.0);
+  auto reach = [&](const ReqParams &p) {  // the profile bins that the table's g range reaches
+    return p.pgrid_off >= 0 ? reach_bins(b.p_ener + p.ener_off, p.n_e, p.lineE / (p.z > 0 ? 1 + p.z : 1.0))
+                            : conv_reach;
+  };
+  int64_t window_bins = 0;
+  for (int i = 0; windows <= 64 && i < b.n_req; i++)
+    if (b.h_status[i] == RX_OK && b.h_req[i].n_e > 0)
+      window_bins += (int64_t)(n_rc + b.h_req[i].n_zones - 1) * reach(b.h_req[i]);
+  const WorkShape ws = work_shape(windows, max_bins, window_bins);
   if (seg_bins <= 0) seg_bins = ws.seg_bins;
   if (waves_per_cu <= 0) waves_per_cu = ws.waves_per_cu;
   b.seg_bins = seg_bins;
@@ -1255,20 +1264,17 @@ void batch_plan(Batch &b, int seg_bins, int waves_per_cu) {
   // work list bound: every (radius chunk, zone) pair of every request covering
   // all the bins that a radius of the table can reach; the zones are contiguous
   // radius ranges, so a request has at most n_rc + n_zones - 1 such pairs
-  const int conv_reach = reach_bins(g.conv_ener.data(), g.conv_n, 1.0);
   int64_t cap = 0;
   for (int i = 0; i < b.n_req; i++) {
     const ReqParams &p = b.h_req[i];
     if (b.h_status[i] != RX_OK || p.n_e <= 0) continue;
-    const int bins =
-        p.pgrid_off >= 0 ? reach_bins(b.p_ener + p.ener_off, p.n_e, p.lineE / (p.z > 0 ? 1 + p.z : 1.0)) : conv_reach;
-    cap += (int64_t)(n_rc + p.n_zones - 1) * ((bins + seg_bins - 1) / seg_bins);
+    cap += (int64_t)(n_rc + p.n_zones - 1) * ((reach(p) + seg_bins - 1) / seg_bins);
   }
   b.item_cap = (int)std::min<int64_t>(std::max<int64_t>(cap, 1), INT32_MAX);
   b.n_blocks = integrate_blocks(b.item_cap, windows, waves_per_cu);
 }
 
-WorkShape work_shape(int64_t windows, int max_bins) {
+WorkShape work_shape(int64_t windows, int max_bins, int64_t window_bins) {
   // A window is one chunk of radii (and zone) of one request, 16 a request.
   // Few windows leave the chip idle: short segments give it more, shorter
   // items, until an item's set-up (about 10 us of latency) is what it does.
@@ -1278,11 +1284,17 @@ WorkShape work_shape(int64_t windows, int max_bins) {
   // 53 / 59 / 140 (- / - / 113 / 105 / 210), 256 requests - / - / 132 / 121 / 150
   // (- / - / 316 / 299 / 304), 1024 requests - / - / 483 / 387 / 345 (- / - / 1045
   // / 965 / 924); relline and lamp-post requests order the same way.
+  // Up to 64 windows (four requests) the segments follow window_bins, the bins
+  // that all windows together can reach (a window takes about 1/20 of them): as
+  // short as leaves the chip no second round of items.  Segments of 1 / 2 / 4
+  // bins: relline 299 bins (5 k) 14 / 17 / 18, relconv (15 k) 12.6 / 14 / 16,
+  // relline 1500 bins (14 k) 12 / 13 / 16, 3000 bins (29 k) 18 / 14 / 16, three
+  // relconv requests (44 k) 20 / 14 / 17, relline 8000 bins (77 k) 40 / 22 / 15.
   // Grids beyond 16384 bins keep segments of 64 at least, so that their work
   // list stays small beside the batch's other buffers.
   WorkShape w;
   w.waves_per_cu = 12;
-  if (windows <= 64) w.seg_bins = 4;
+  if (windows <= 64) w.seg_bins = window_bins <= 18000 ? 1 : window_bins <= 45000 ? 2 : 4;
   else if (windows <= 512) w.seg_bins = 8;
   else if (windows <= 2048) w.seg_bins = 32;
   else if (windows <= 8192) w.seg_bins = 64;

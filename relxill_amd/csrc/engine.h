@@ -182,7 +182,7 @@ int reach_bins(const double *ener, int n, double unit);
 struct WorkShape {
   int seg_bins, waves_per_cu;
 };
-WorkShape work_shape(int64_t windows, int max_bins);
+WorkShape work_shape(int64_t windows, int max_bins, int64_t window_bins);
 // Workgroups of k_integrate for a work list of that capacity.
 int integrate_blocks(int item_cap, int64_t windows, int waves_per_cu);
 int batch_upload(Batch &b);

@@ -936,17 +936,22 @@ __global__ __launch_bounds__(NT, NT == 256 ? 3 : 1) void k_setup(BatchDev b) {
     for (int z = 0; z < nz; z++)
       for (int j = jlo + tid; j <= jhi; j += NT) acc[(size_t)z * rq.n_e + j] = 0.0;
   if (s_base >= 0) {
-    for (int q = tid; q < n_cz; q += NT) {
+    // SEG_LANES lanes a window, a lane per segment (all but the last are S bins
+    // long): one lane a window took 2-9 us for segments of one bin
+    constexpr int SEG_LANES = 16;
+    for (int q = tid / SEG_LANES; q < n_cz; q += NT / SEG_LANES) {
       const int c = q / nz, z = q % nz, w = c * NZ + z;
-      int k = s_base + s_pref[q], ks = s_bases + s_prefs[q];
-      for (int j0 = s_ulo[w]; j0 <= s_uhi[w]; j0 += S) {
+      const int k = s_base + s_pref[q], ks = s_bases + s_prefs[q];
+      const int uhi = s_uhi[w];
+      int i = tid % SEG_LANES;
+      for (int64_t j0 = s_ulo[w] + (int64_t)i * S; j0 <= uhi; j0 += SEG_LANES * (int64_t)S, i += SEG_LANES) {
         WorkItem it;
         it.req = req;
         it.rc = c | (z << 16);
-        it.j0 = j0;
-        it.j1 = min(s_uhi[w] + 1, j0 + S);
-        if (it.j1 - it.j0 >= thr) b.items[k++] = it;
-        else b.items[b.item_cap - 1 - ks++] = it;
+        it.j0 = (int)j0;
+        it.j1 = (int)min((int64_t)uhi + 1, j0 + S);
+        if (it.j1 - it.j0 >= thr) b.items[k + i] = it;
+        else b.items[b.item_cap - 1 - ks] = it;
       }
     }
   }

@@ -175,11 +175,11 @@ int noalloc_eval(int model, const double *parameter, const double *d_energy, con
       wpc = t.waves_per_cu;
     }
   const int n_rc = (g.nr_fine + RAD_CHUNK - 1) / RAD_CHUNK;
-  const WorkShape ws = work_shape(n_rc, p.n_e);
-  if (seg <= 0) seg = ws.seg_bins;
-  if (wpc <= 0) wpc = ws.waves_per_cu;
   // (a caller's line grid is on the device: all its bins)
   const int bins = conv ? reach_bins(g.conv_ener.data(), g.conv_n, 1.0) : p.n_e;
+  const WorkShape ws = work_shape(n_rc, p.n_e, (int64_t)n_rc * bins);
+  if (seg <= 0) seg = ws.seg_bins;
+  if (wpc <= 0) wpc = ws.waves_per_cu;
   auto items = [&](int s) { return n_rc * ((bins + s - 1) / s); };
   const int fix_cap = std::max(4096, p.n_e * 4);
 

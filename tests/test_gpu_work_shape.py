@@ -26,7 +26,7 @@ def tabs():
 
 
 @pytest.mark.parametrize("band", [(0.1, 10.0), (5.0, 7.0), (6.0, 40.0), (0.05, 0.9)])
-@pytest.mark.parametrize("n_bins", [1, 3, 4, 5, 7, 9, 31, 33, 65, 700])
+@pytest.mark.parametrize("n_bins", [1, 3, 4, 5, 7, 9, 31, 33, 65, 700, 2000, 9000])
 def test_single_calls(tabs, n_bins, band):
     e = log_grid(n_bins, *band)
     for z in (0.0, 0.4):
