@@ -673,7 +673,7 @@ int rx_batch_set_shape(rx_batch *b, int seg_bins, int waves_per_cu) {
   b->b.seg_forced = seg_bins;
   b->b.waves_forced = waves_per_cu;
   batch_plan(b->b, seg_bins, waves_per_cu);
-  return batch_upload(b->b);
+  return batch_place_items(b->b);
 }
 
 void rx_batch_destroy(rx_batch *b) {
@@ -790,7 +790,7 @@ int rx_batch_autotune(rx_batch *b, int precision) {
   // the fastest of `trials` timings of `reps` runs each of one shape
   auto time_shape = [&](int sg, int w, int trials, int reps, double &dt) {
     batch_plan(b->b, sg, w);
-    if (batch_upload(b->b) != RX_OK) return false;
+    if (batch_place_items(b->b) != RX_OK) return false;
     if (batch_run(b->b, precision, err) != RX_OK || batch_sync(b->b) != RX_OK) return false;
     for (int trial = 0; trial < trials; trial++) {
       auto t0 = std::chrono::steady_clock::now();
@@ -830,7 +830,7 @@ int rx_batch_autotune(rx_batch *b, int precision) {
   b->b.seg_forced = best_s;
   b->b.waves_forced = best_w;
   batch_plan(b->b, best_s, best_w);
-  if (batch_upload(b->b) != RX_OK) return -RX_ERR_DEVICE;
+  if (batch_place_items(b->b) != RX_OK) return -RX_ERR_DEVICE;
   return best_s * 256 + best_w;
 }
 

@@ -1327,9 +1327,20 @@ int integrate_blocks(int item_cap, int64_t windows, int waves_per_cu) {
   return (int)std::min<int64_t>((int64_t)G().n_cu * waves_per_cu, std::max(1, item_cap));
 }
 
+int batch_place_items(Batch &b) {
+  b.ready = false;
+  if (b.d_items.ensure(sizeof(WorkItem) * (size_t)b.item_cap)) return RX_ERR_NOMEM;
+  b.dev.items = b.d_items.as<WorkItem>();
+  b.dev.item_cap = b.item_cap;
+  b.dev.seg_bins = b.seg_bins;
+  b.ready = true;
+  return RX_OK;
+}
+
 int batch_upload(Batch &b) {
   Global &g = G();
   int e = 0;
+  b.ready = false;
   if (!b.stream) {
     e |= (int)hipStreamCreateWithFlags(&b.stream, hipStreamNonBlocking);
     for (auto &x : b.ev) e |= (int)hipEventCreate(&x);
@@ -1351,8 +1362,7 @@ int batch_upload(Batch &b) {
                o_nth = take(sizeof(NthRes) * b.h_nth.size()),
                o_nthx = take(sizeof(double) * (NTH_MAX_POINTS + 1) * b.n_nth_sol),
                o_nths = take(sizeof(double) * NTH_MAX_POINTS * b.n_nth_sol), o_nthn = take(sizeof(int) * b.n_nth_sol),
-               o_xspec = take(sizeof(double) * b.tot_xspec),
-               o_items = take(sizeof(WorkItem) * (size_t)b.item_cap), o_reach = take(sizeof(BinRange) * nreq);
+               o_xspec = take(sizeof(double) * b.tot_xspec), o_reach = take(sizeof(BinRange) * nreq);
   // FP64 re-check queue: a few percent of the bins (overflow redoes the batch in FP64)
   int64_t bins = 0;
   for (int i = 0; i < b.n_req; i++) bins += b.h_req[i].n_e;
@@ -1370,9 +1380,7 @@ int batch_upload(Batch &b) {
   memset(&d, 0, sizeof(d));
   d.n_req = b.n_req;
   d.nr_fine = g.nr_fine;
-  d.seg_bins = b.seg_bins;
   d.max_zones = b.max_zones;
-  d.item_cap = b.item_cap;
   d.fix_cap = b.fix_cap;
   at(d.req, b.off.req);
   at(d.status, b.off.status);
@@ -1395,7 +1403,6 @@ int batch_upload(Batch &b) {
   at(d.nth_s, o_nths);
   at(d.nth_n, o_nthn);
   at(d.xspec, o_xspec);
-  at(d.items, o_items);
   at(d.reach, o_reach);
   at(d.fix, o_fix);
   WorkLists &w = b.wl;
@@ -1418,6 +1425,7 @@ int batch_upload(Batch &b) {
   w.n_rrc = (int)b.h_rrc.size();
   w.n_rrad = (int)b.h_rrad.size();
   w.n_nth = (int)b.h_nth.size();
+  if (const int st = batch_place_items(b)) return st;
   memset(result_ctr(b), 0, sizeof(int) * RES_CTR);
   memcpy(result_status(b), b.h_status.data(), sizeof(int) * nreq);
   b.win[0].lo = b.win[0].hi = b.win[1].lo = b.win[1].hi = 0;
@@ -1602,6 +1610,10 @@ int batch_run(Batch &b, int precision, std::string &err) {
   if (b.config_gen != g.config_gen) {
     err = "tables, convolution grid, fine-grid size or reflection sets changed since the batch was built";
     return RX_ERR_ARG;
+  }
+  if (!b.ready) {
+    err = "the batch's device memory could not be allocated";
+    return RX_ERR_NOMEM;
   }
   b.last_mode = (precision == RX_FP32) ? 1 : 0;
   RunKey k;

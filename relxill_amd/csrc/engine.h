@@ -108,10 +108,13 @@ struct Batch {
   int n_nth_sol = 0;             // requests with the nthcomp primary (one source solution each)
   int64_t tot_ener = 0, tot_flux = 0, tot_pgrid = 0, tot_prof = 0, tot_xspec = 0, tot_dist = 0, tot_zone = 0;
   int64_t tot_rrc = 0;
-  // One device allocation holds everything of the batch; it begins with the
-  // request block (what the host writes: parameters, statuses, work lists,
-  // grids, input spectra).
-  DevBuf d_arena;
+  // One device allocation holds everything of the batch but k_integrate's work
+  // list; it begins with the request block (what the host writes: parameters,
+  // statuses, work lists, grids, input spectra).  The work list, whose length
+  // follows the work shape, has its own: a new shape leaves the last run's
+  // outputs, distributions, zones and statuses where they are.
+  DevBuf d_arena, d_items;
+  bool ready = false;  // both are there and laid out
   BatchDev dev;   // its pointers (dev_view adds the run's settings and the tables)
   WorkLists wl;
   size_t block_bytes = 0;
@@ -186,6 +189,8 @@ WorkShape work_shape(int64_t windows, int max_bins, int64_t window_bins);
 // Workgroups of k_integrate for a work list of that capacity.
 int integrate_blocks(int item_cap, int64_t windows, int waves_per_cu);
 int batch_upload(Batch &b);
+// Sizes the work list for the batch's work shape (batch_plan).
+int batch_place_items(Batch &b);
 // Layout of a run's results in pinned host memory: the first RES_CTR counters,
 // the statuses, the outputs.
 inline int *result_ctr(const Batch &b) { return b.h_res.as<int>(); }
