@@ -2593,11 +2593,18 @@ __global__ __launch_bounds__(CONV_THREADS_MAX) void k_conv(BatchDev b, const Xil
   // complex transform, whose rounding errors reach both), times a rest that only
   // the profile's sums carry (the result is normalised by them): against FP64
   // sums in another order 4e-13 in bins 1e-4 below the maximum, 4e-12 without.
-  double f = rq.do_renorm ? rq.norm / s2[1] : 1.0, f_rest = 1.0;
+  // The product of the transforms is brought back by p_scale, so that it does not
+  // go with the input's square (an input of 1e-165 a bin underflowed).
+  double f = rq.do_renorm ? rq.norm / s2[1] : 1.0, f_rest = 1.0, p_scale = 1.0;
   if constexpr (WIDE) {
-    double f2 = pow2_of(f);
-    if (!angular && s2[2] > 0) f2 = pow2_of(s2[2] / s2[1]);
-    if (f2 > 0) {
+    const double f1 = pow2_of(f);
+    double f2 = f1;
+    if (!angular && s2[2] > 0) {
+      const double r = pow2_of(s2[2] / s2[1]);
+      if (r > 0) f2 = r;
+    }
+    if (f1 > 0 && f2 > 0) {
+      p_scale = f1 / f2;
       f_rest = f / f2;
       f = f2;
     }
@@ -2662,6 +2669,10 @@ __global__ __launch_bounds__(CONV_THREADS_MAX) void k_conv(BatchDev b, const Xil
         }
       } else {
         X = make_double2(0.5 * (wk.x + wn.x), 0.5 * (wk.y - wn.y));
+        if constexpr (WIDE) {
+          X.x *= p_scale;
+          X.y *= p_scale;
+        }
       }
       Pk[u] = cmul(X, Y);
     }
