@@ -2566,7 +2566,7 @@ __global__ __launch_bounds__(CONV_THREADS_MAX) void k_conv(BatchDev b, const Xil
         }
         const int i = i4[u];
         if (elo[u] >= 0.01 && ehi[u] < 1000.0) sx += xr;  // calcFFTNormFactor band (src/Relbase.cpp:205)
-        if constexpr (WIDE) sxa += fabs(xr);
+        sxa += fabs(xr);
         s_buf[P(i)].x = xr * cf[i];
       }
     }
@@ -2586,28 +2586,28 @@ __global__ __launch_bounds__(CONV_THREADS_MAX) void k_conv(BatchDev b, const Xil
   }
   const double p2[3] = {sx, sph, sxa};
   double s2[3];
-  block_sums<WIDE ? 3 : 2>(p2, s2, s_w);
-  double sum_xill = s2[0];
-  // The profile's renormalisation.  WIDE: as a power of two, which is exact in
-  // every bin and brings the profile to the input's scale (the two inputs of one
-  // complex transform, whose rounding errors reach both), times a rest that only
-  // the profile's sums carry (the result is normalised by them): against FP64
-  // sums in another order 4e-13 in bins 1e-4 below the maximum, 4e-12 without.
-  // The product of the transforms is brought back by p_scale, so that it does not
-  // go with the input's square (an input of 1e-165 a bin underflowed).
+  block_sums<3>(p2, s2, s_w);
+  double sum_xill = readlane_d(s2[0], 0);
+  // The profile's renormalisation: as a power of two, which is exact in every bin
+  // and brings the profile to the input's scale (the two inputs of one complex
+  // transform, whose rounding errors reach both: an input of 1e-12 a bin beside a
+  // profile of 1 came out 1.6e-5 of the maximum off), times a rest that only the
+  // profile's sums carry (the result is normalised by them): against FP64 sums in
+  // another order 4e-13 in bins 1e-4 below the maximum, 4e-12 without.  The
+  // product of the transforms is brought back by p_scale, so that it does not go
+  // with the input's square (an input of 1e-165 a bin underflowed).  4096 units
+  // 343 us and 345 us without and with it.
   double f = rq.do_renorm ? rq.norm / s2[1] : 1.0, f_rest = 1.0, p_scale = 1.0;
-  if constexpr (WIDE) {
-    const double f1 = pow2_of(f);
-    double f2 = f1;
-    if (!angular && s2[2] > 0) {
-      const double r = pow2_of(s2[2] / s2[1]);
-      if (r > 0) f2 = r;
-    }
-    if (f1 > 0 && f2 > 0) {
-      p_scale = f1 / f2;
-      f_rest = f / f2;
-      f = f2;
-    }
+  const double f1 = pow2_of(f);
+  double f2 = f1;
+  if (!angular && s2[2] > 0) {
+    const double r = pow2_of(s2[2] / s2[1]);
+    if (r > 0) f2 = r;
+  }
+  if (f1 > 0 && f2 > 0) {  // (the same in every lane: kept in scalar registers)
+    p_scale = readlane_d(f1 / f2, 0);
+    f_rest = readlane_d(f / f2, 0);
+    f = f2;
   }
   double sr = 0.0, sa = 0.0;
 #pragma unroll
@@ -2669,10 +2669,8 @@ __global__ __launch_bounds__(CONV_THREADS_MAX) void k_conv(BatchDev b, const Xil
         }
       } else {
         X = make_double2(0.5 * (wk.x + wn.x), 0.5 * (wk.y - wn.y));
-        if constexpr (WIDE) {
-          X.x *= p_scale;
-          X.y *= p_scale;
-        }
+        X.x *= p_scale;
+        X.y *= p_scale;
       }
       Pk[u] = cmul(X, Y);
     }

@@ -35,3 +35,21 @@ def test_few_units(dev, model, prec):
     for k in EXPONENTS:
         y, st = rx.eval_model(model, par, e, np.ldexp(f, k), precision=prec)
         assert st == 0 and conv_err(np.ldexp(y, -k), ref) < 1e-8, k
+
+
+@pytest.mark.parametrize("model", [rx.MODEL_RELCONV, 12])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_many_units(dev, model, prec):
+    e = log_grid(301, 0.2, 80.0)
+    f, par = _input(e), list(rx.DEFAULTS[model])
+    ref, st = rx.eval_model(model, par, e, f, precision=prec)
+    assert st == 0
+    reqs = [dict(model=model, energy=e, params=par, flux_in=np.ldexp(f, EXPONENTS[i % len(EXPONENTS)]))
+            for i in range(257)]
+    b = rx.Batch(reqs)
+    b.run(prec)
+    b.sync()
+    for i, k in enumerate(EXPONENTS):
+        y, st = b.output(i)
+        assert st == 0 and conv_err(np.ldexp(y, -k), ref) < 1e-8, k
+    b.close()
