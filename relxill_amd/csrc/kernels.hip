@@ -890,12 +890,15 @@ __global__ __launch_bounds__(NT, NT == 256 ? 3 : 1) void k_setup(BatchDev b) {
     jlo = wave_min_i(jlo);
     jhi = wave_max_i(jhi);
     if (lane == 0) {
-      int base = atomicAdd(&b.ctr[CTR_ITEMS], tot);
-      const int bases = atomicAdd(&b.ctr[CTR_ITEMS_S], tots);
-      // cannot happen: the host sizes the list for every bin of every request
-      if (base + tot > b.item_cap || bases + tots > b.item_cap) {
+      static_assert(CTR_ITEMS % 2 == 0 && CTR_ITEMS_S == CTR_ITEMS + 1, "one aligned 64-bit word");
+      unsigned long long *ctr = reinterpret_cast<unsigned long long *>(&b.ctr[CTR_ITEMS]);
+      int base, bases;
+      // the host sizes the list for the bins that the table's radii reach
+      // (reach_bins); a request that it does not hold all the same fails, and its
+      // neighbours' items stay whole
+      if (!reserve_items([&](uint64_t v) { return (uint64_t)atomicAdd(ctr, (unsigned long long)v); }, tot, tots,
+                         b.item_cap, base, bases)) {
         atomicOr(&b.ctr[CTR_ITEMS_OVF], 1);
-        s_st = ST_WORKLIST;
         base = -1;
       }
       s_base = base;
@@ -955,7 +958,7 @@ __global__ __launch_bounds__(NT, NT == 256 ? 3 : 1) void k_setup(BatchDev b) {
       }
     }
   }
-  if (tid == 0) b.status[req] = s_st;
+  if (tid == 0) b.status[req] = s_base >= 0 ? 0 : ST_WORKLIST;
 }
 
 // Radial zones of the relxill and xillver requests (IonGradient,
