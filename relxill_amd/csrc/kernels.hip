@@ -436,6 +436,15 @@ __device__ inline double wave_max_d(double v) {
   return fmax(fmax(readlane_d(v, 0), readlane_d(v, 16)), fmax(readlane_d(v, 32), readlane_d(v, 48)));
 }
 
+// What one lane wrote to LDS is there for the other lanes of its wavefront behind
+// this (the hardware keeps a wavefront's LDS operations in order; the fence keeps
+// the compiler from moving them across).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // min / max over the 64 lanes (quad, half-row and row exchanges, then the rows);
 // every lane must be active
 __device__ inline int wave_min_i(int v) {
@@ -578,7 +587,10 @@ __global__ __launch_bounds__(NT, NT == 256 ? 3 : 1) void k_setup(BatchDev b) {
   __shared__ double s_jr[MAX_LP_R], s_je[MAX_LP_R], s_jd[MAX_LP_R], s_ji[MAX_LP_R];
   __shared__ double s_rr_rad[MAX_RR], s_rr_ret[MAX_RR];
   __shared__ double s_sum[NW], s_max[NW];
-  __shared__ int s_st, s_ia, s_im, s_rmin;
+  // statuses of the three stages, each tested behind a barrier of its own and not
+  // written after it (a wavefront may still be at the test of the one before)
+  __shared__ int s_st, s_st_edge, s_st_rad, s_st_refl;
+  __shared__ int s_ia, s_im, s_rmin;
   __shared__ double s_fa, s_fm;
   constexpr int MAX_RC = MAX_NR_FINE / RAD_CHUNK;
   // energy window of each (radius chunk, zone): bins [s_ulo, s_uhi]
@@ -603,6 +615,7 @@ __global__ __launch_bounds__(NT, NT == 256 ? 3 : 1) void k_setup(BatchDev b) {
     if (!(fm >= 0 && fm <= 1 && fa >= 0 && fa <= 1)) st = 11;
     if (lane == 0) {
       s_st = st;
+      s_st_rad = s_st_refl = 0;
       s_ia = ia;
       s_im = im;
       s_fa = fa;
@@ -671,7 +684,7 @@ __global__ __launch_bounds__(NT, NT == 256 ? 3 : 1) void k_setup(BatchDev b) {
     // ISCO snap (src/Relprofile.cpp:195-200)
     const double rms = rq.rms;
     if (lane == 0 && (s_tre[n_r - 1] > rms) && ((s_tre[n_r - 1] - rms) / s_tre[n_r - 1] < 1e-3)) s_tre[n_r - 1] = rms;
-    __builtin_amdgcn_wave_barrier();  // (one wavefront: LDS operations are in order)
+    wave_lds_fence();  // (the other lanes read the node)
     int c_in = 0, c_out = 0;  // nodes not below Rin / Rout (bsearch_desc, src/relutility.c:195-211)
     for (int k = 0; k < n_r; k += 64) {
       const bool v = k + lane < n_r;
@@ -690,12 +703,12 @@ __global__ __launch_bounds__(NT, NT == 256 ? 3 : 1) void k_setup(BatchDev b) {
         st = 12;
       }
       s_rmin = ind_rmin;
-      s_st = st;
+      s_st_edge = st;
     }
   }
   __syncthreads();
-  if (s_st) {
-    if (tid == 0) b.status[req] = s_st;
+  if (s_st_edge) {
+    if (tid == 0) b.status[req] = s_st_edge;
     return;
   }
   {  // the node arrays the radius records are rebuilt from (rad_geo)
@@ -736,7 +749,7 @@ __global__ __launch_bounds__(NT, NT == 256 ? 3 : 1) void k_setup(BatchDev b) {
     o.f_inf = (rq.beta > 1e-6) ? 0.5 * (1.0 + cos(relat_abberation(dmax, -1. * rq.beta))) : o.f_inf_rest;
     o.refl_frac = o.f_ad / o.f_inf;
     if (lane == 0) {
-      if (!(o.f_inf + o.f_ad < 1.0)) atomicMax(&s_st, 20);
+      if (!(o.f_inf + o.f_ad < 1.0)) s_st_refl = 20;
       b.refl[req] = o;
     }
   }
@@ -830,7 +843,7 @@ __global__ __launch_bounds__(NT, NT == 256 ? 3 : 1) void k_setup(BatchDev b) {
       }
     }
   }
-  if (err) atomicMax(&s_st, err);
+  if (err) atomicMax(&s_st_rad, err);
   // BKN normalisation: sum emis * 2 pi r dr (norm_emis_profile, src/Rellp.cpp:91-109),
   // applied through ReqNorm instead of a second pass over the records
   const double area_w = wave_sum(area), cmax_w = wave_max_d(cmax);
@@ -839,8 +852,8 @@ __global__ __launch_bounds__(NT, NT == 256 ? 3 : 1) void k_setup(BatchDev b) {
     s_max[wave] = cmax_w;
   }
   __syncthreads();
-  if (s_st) {
-    if (tid == 0) b.status[req] = s_st;
+  if (const int st = s_st_rad ? s_st_rad : s_st_refl) {
+    if (tid == 0) b.status[req] = st;
     return;
   }
   // work items: the window of each (radius chunk, zone) cut into segments
