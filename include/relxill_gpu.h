@@ -413,11 +413,14 @@ int rx_batch_counters(rx_batch *b, int64_t *out);
 /* Launch graphs (default on): a batch run whose kernel arguments and grid
  * shapes equal the previous run's is captured into a hipGraph and replayed
  * while they stay equal (the XSPEC entry points reuse one batch, so repeated
- * calls on one grid replay a graph).  rx_set_graphs(0) launches every kernel
- * directly.  rx_batch_graph_replays: runs of the batch served by a graph.
+ * calls on one grid replay a graph, whatever their parameters).
+ * rx_set_graphs(0) launches every kernel directly.  rx_batch_graph_replays: runs
+ * of the batch served by a graph; rx_call_graph_replays: calls of rx_eval_model
+ * and the lmod* entry points.
  * No counterpart in the reference (launch mechanics of the device path). */
 int rx_set_graphs(int on);
 int64_t rx_batch_graph_replays(rx_batch *b);
+int64_t rx_call_graph_replays(void);
 
 /* Autotuner: times candidate work shapes (segment bins x waves per CU) for
  * this batch on the device and keeps the fastest for batches of the same

@@ -174,6 +174,7 @@ _EXPORTS = {
                                              ctypes.c_int, ctypes.c_int, ctypes.c_void_p]),
     "rx_set_graphs": (ctypes.c_int, [ctypes.c_int]),
     "rx_batch_graph_replays": (ctypes.c_int64, [ctypes.c_void_p]),
+    "rx_call_graph_replays": (ctypes.c_int64, []),
     "rx_server_start": (ctypes.c_void_p, [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int]),
     "rx_server_submit": (ctypes.c_int64, [ctypes.c_void_p, ctypes.POINTER(_Request)]),
     "rx_server_poll": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int64, _D,

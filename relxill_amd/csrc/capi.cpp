@@ -766,6 +766,12 @@ int64_t rx_batch_graph_replays(rx_batch *b) {
   return b->b.graph_replays;
 }
 
+int64_t rx_call_graph_replays(void) {
+  Global &g = G();
+  std::lock_guard<std::recursive_mutex> lk(g.mu);
+  return plain_batch().graph_replays;
+}
+
 int rx_batch_counters(rx_batch *b, int64_t *out) {
   if (!b || !out) return RX_ERR_ARG;
   for (int k = 0; k < 3; k++) out[k] = b->b.counters[k];

@@ -1257,6 +1257,16 @@ void batch_plan(Batch &b, int seg_bins, int waves_per_cu) {
     if (b.h_status[i] == RX_OK && b.h_req[i].n_e > 0)
       window_bins += (int64_t)(n_rc + b.h_req[i].n_zones - 1) * reach(b.h_req[i]);
   const WorkShape ws = work_shape(windows, max_bins, window_bins);
+  // calls on one grid keep their segments and their list's length while the reach
+  // stays near what they were chosen for: it moves with the line's energy and
+  // redshift, and every change of either is another launch configuration
+  Batch::CallShape &k = b.call_shape;
+  if (b.is_call) {
+    const bool near = k.windows == windows && k.max_bins == max_bins && 2 * window_bins <= 3 * k.window_bins &&
+                      2 * k.window_bins <= 3 * window_bins;
+    if (!near) k = {windows, max_bins, window_bins, 0, 0};
+    if (seg_bins <= 0) seg_bins = k.seg_bins;
+  }
   if (seg_bins <= 0) seg_bins = ws.seg_bins;
   if (waves_per_cu <= 0) waves_per_cu = ws.waves_per_cu;
   b.seg_bins = seg_bins;
@@ -1269,6 +1279,13 @@ void batch_plan(Batch &b, int seg_bins, int waves_per_cu) {
     const ReqParams &p = b.h_req[i];
     if (b.h_status[i] != RX_OK || p.n_e <= 0) continue;
     cap += (int64_t)(n_rc + p.n_zones - 1) * ((reach(p) + seg_bins - 1) / seg_bins);
+  }
+  if (b.is_call) {
+    if (k.seg_bins != seg_bins || cap > k.item_cap) {
+      k.seg_bins = seg_bins;
+      k.item_cap = cap > ONE_ITEMS || cap + cap / 8 <= ONE_ITEMS ? cap + cap / 8 : ONE_ITEMS;
+    }
+    cap = k.item_cap;
   }
   b.item_cap = (int)std::min<int64_t>(std::max<int64_t>(cap, 1), INT32_MAX);
   b.n_blocks = integrate_blocks(b.item_cap, windows, waves_per_cu);
@@ -1323,7 +1340,7 @@ int integrate_blocks(int item_cap, int64_t windows, int waves_per_cu) {
   // request's items on one XCD and take the long ones first (4096 requests
   // 1250 us, 1304 us with ONE).  Workgroups without an item cost about 0.2 ns
   // each: at most 2^18 of them.
-  if (windows <= 8192 && item_cap <= (1 << 18)) return std::max(1, item_cap);
+  if (windows <= 8192 && item_cap <= ONE_ITEMS) return std::max(1, item_cap);
   return (int)std::min<int64_t>((int64_t)G().n_cu * waves_per_cu, std::max(1, item_cap));
 }
 

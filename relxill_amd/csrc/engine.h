@@ -146,6 +146,12 @@ struct Batch {
   std::atomic<bool> synced{true};      // the stream was waited for since the last run
   std::mutex out_mu;                   // readers of one batch in several threads
   int item_cap = 0;
+  // the work shape of the last evaluation call and what it was chosen for
+  struct CallShape {
+    int64_t windows, max_bins, window_bins;
+    int seg_bins;
+    int64_t item_cap;
+  } call_shape = {};
   int n_blocks = 1;  // workgroups of k_integrate
   bool any_cosne = false, any_limb = false, any_angular = false;
   bool one_unit = false;  // every request has one unit of k_conv
@@ -186,7 +192,9 @@ struct WorkShape {
   int seg_bins, waves_per_cu;
 };
 WorkShape work_shape(int64_t windows, int max_bins, int64_t window_bins);
-// Workgroups of k_integrate for a work list of that capacity.
+// Workgroups of k_integrate for a work list of that capacity: one an item for
+// lists of up to ONE_ITEMS.
+constexpr int ONE_ITEMS = 1 << 18;
 int integrate_blocks(int item_cap, int64_t windows, int waves_per_cu);
 int batch_upload(Batch &b);
 // Sizes the work list for the batch's work shape (batch_plan).
