@@ -1240,22 +1240,19 @@ void batch_plan(Batch &b, int seg_bins, int waves_per_cu) {
     }
   }
   const int n_rc = (g.nr_fine + RAD_CHUNK - 1) / RAD_CHUNK;
-  int64_t windows = 0;
-  int max_bins = 0;
-  for (int i = 0; i < b.n_req; i++) {
-    if (b.h_status[i] != RX_OK || b.h_req[i].n_e <= 0) continue;
-    windows += n_rc + b.h_req[i].n_zones - 1;
-    max_bins = std::max(max_bins, b.h_req[i].n_e);
-  }
   const int conv_reach = reach_bins(g.conv_ener.data(), g.conv_n, 1.0);
-  auto reach = [&](const ReqParams &p) {  // the profile bins that the table's g range reaches
-    return p.pgrid_off >= 0 ? reach_bins(b.p_ener + p.ener_off, p.n_e, p.lineE / (p.z > 0 ? 1 + p.z : 1.0))
-                            : conv_reach;
-  };
-  int64_t window_bins = 0;
-  for (int i = 0; windows <= 64 && i < b.n_req; i++)
-    if (b.h_status[i] == RX_OK && b.h_req[i].n_e > 0)
-      window_bins += (int64_t)(n_rc + b.h_req[i].n_zones - 1) * reach(b.h_req[i]);
+  int64_t windows = 0, window_bins = 0;
+  int max_bins = 0;
+  std::vector<int> reach(b.n_req, 0);  // the profile bins that the table's g range reaches
+  for (int i = 0; i < b.n_req; i++) {
+    const ReqParams &p = b.h_req[i];
+    if (b.h_status[i] != RX_OK || p.n_e <= 0) continue;
+    reach[i] = p.pgrid_off < 0 ? conv_reach
+                               : reach_bins(b.p_ener + p.ener_off, p.n_e, p.lineE / (p.z > 0 ? 1 + p.z : 1.0));
+    windows += n_rc + p.n_zones - 1;
+    window_bins += (int64_t)(n_rc + p.n_zones - 1) * reach[i];
+    max_bins = std::max(max_bins, p.n_e);
+  }
   const WorkShape ws = work_shape(windows, max_bins, window_bins);
   // calls on one grid keep their segments and their list's length while the reach
   // stays near what they were chosen for: it moves with the line's energy and
@@ -1275,11 +1272,8 @@ void batch_plan(Batch &b, int seg_bins, int waves_per_cu) {
   // all the bins that a radius of the table can reach; the zones are contiguous
   // radius ranges, so a request has at most n_rc + n_zones - 1 such pairs
   int64_t cap = 0;
-  for (int i = 0; i < b.n_req; i++) {
-    const ReqParams &p = b.h_req[i];
-    if (b.h_status[i] != RX_OK || p.n_e <= 0) continue;
-    cap += (int64_t)(n_rc + p.n_zones - 1) * ((reach(p) + seg_bins - 1) / seg_bins);
-  }
+  for (int i = 0; i < b.n_req; i++)
+    cap += (int64_t)(n_rc + b.h_req[i].n_zones - 1) * ((reach[i] + seg_bins - 1) / seg_bins);
   if (b.is_call) {
     if (k.seg_bins != seg_bins || cap > k.item_cap) {
       k.seg_bins = seg_bins;
@@ -1292,28 +1286,37 @@ void batch_plan(Batch &b, int seg_bins, int waves_per_cu) {
 }
 
 WorkShape work_shape(int64_t windows, int max_bins, int64_t window_bins) {
-  // A window is one chunk of radii (and zone) of one request, 16 a request.
-  // Few windows leave the chip idle: short segments give it more, shorter
-  // items, until an item's set-up (about 10 us of latency) is what it does.
-  // Measured, k_integrate in us, FP32 (FP64), relconv, segments of 4 / 8 / 32 /
-  // 64 / 256 bins: 1 request 15 / 17 / 30 / 43 / - (22 / 25 / 48 / 64 / -), 16
-  // requests 32 / 28 / 44 / 53 / - (52 / 52 / 71 / 78 / -), 64 requests - / - /
-  // 53 / 59 / 140 (- / - / 113 / 105 / 210), 256 requests - / - / 132 / 121 / 150
-  // (- / - / 316 / 299 / 304), 1024 requests - / - / 483 / 387 / 345 (- / - / 1045
-  // / 965 / 924); relline and lamp-post requests order the same way.
-  // Up to 64 windows (four requests) the segments follow window_bins, the bins
-  // that all windows together can reach (a window takes about 1/20 of them): as
-  // short as leaves the chip no second round of items.  Segments of 1 / 2 / 4
-  // bins: relline 299 bins (5 k) 14 / 17 / 18, relconv (15 k) 12.6 / 14 / 16,
+  // A window is one chunk of radii (and zone) of one request, 16 a request;
+  // window_bins: the bins that all windows together can reach (a window takes
+  // about 1/20 of them).  Few windows leave the chip idle: short segments give it
+  // more, shorter items, until an item's set-up (about 10 us of latency) is what
+  // it does.  Up to 64 windows (four requests) the segments are as short as leaves
+  // the chip no second round of items: k_integrate in us, segments of 1 / 2 / 4
+  // bins, relline 299 bins (5 k) 14 / 17 / 18, relconv (15 k) 12.6 / 14 / 16,
   // relline 1500 bins (14 k) 12 / 13 / 16, 3000 bins (29 k) 18 / 14 / 16, three
   // relconv requests (44 k) 20 / 14 / 17, relline 8000 bins (77 k) 40 / 22 / 15.
+  // Up to 2048 windows (128 requests) they grow with the reach, so that the items
+  // stay below about 10^5: a run in us, FP32 (FP64), segments of 8 / 16 / 32 / 64
+  // bins, 16 relconv requests (216 k) 96 / 98 / 113 / 121 (90 / 87 / 102 / 111), 32
+  // (432 k) 110 / 102 / 117 / 128 (110 / 103 / 108 / 118), 5 relline requests of 8000
+  // bins (444 k) 82 / 85 / 100 / 120 (83 / 82 / 94 / 115), of 3000 bins 8
+  // requests (266 k) 71 / 77 / 85 / 107 (73 / 73 / 80 / 101), 16 (532 k) 84 / 82 /
+  // 88 / 108 (93 / 86 / 86 / 102), of 8000 bins 8 requests (710 k) 106 / 99 / 110 /
+  // 122 (123 / 108 / 115 / 121), 16 (1.4 M) 156 / 121 / 125 / 129 (188 / 144 / 142 /
+  // 148), 32 (2.8 M) 238 / 189 / 163 / 174 (311 / 254 / 216 / 216), 64 (5.7 M) 369 /
+  // 283 / 245 / 239 (517 / 404 / 359 / 333).  From 513 windows on there are enough
+  // items without segments below 32 bins, even of short reach: 64 relline requests
+  // of 300 bins 80 / 80 / 79 / 91 (76 / 73 / 66 / 78).
+  // 256 requests, k_integrate, segments of 32 / 64 / 256 bins 132 / 121 / 150 (316 /
+  // 299 / 304), 1024 requests 483 / 387 / 345 (1045 / 965 / 924).
   // Grids beyond 16384 bins keep segments of 64 at least, so that their work
   // list stays small beside the batch's other buffers.
   WorkShape w;
   w.waves_per_cu = 12;
+  const int by_reach = window_bins <= 450000 ? 8 : window_bins <= 1000000 ? 16 : window_bins <= 4000000 ? 32 : 64;
   if (windows <= 64) w.seg_bins = window_bins <= 18000 ? 1 : window_bins <= 45000 ? 2 : 4;
-  else if (windows <= 512) w.seg_bins = 8;
-  else if (windows <= 2048) w.seg_bins = 32;
+  else if (windows <= 512) w.seg_bins = by_reach;
+  else if (windows <= 2048) w.seg_bins = std::max(32, by_reach);
   else if (windows <= 8192) w.seg_bins = 64;
   else w.seg_bins = 256;
   if (max_bins > 16384) w.seg_bins = std::max(w.seg_bins, 64);

@@ -186,8 +186,9 @@ void batch_plan(Batch &b, int seg_bins, int waves_per_cu);
 // Bins of an energy grid (n + 1 ascending edges) that the window of some radius of
 // the resident table can reach; unit: the grid's energy of g = 1.
 int reach_bins(const double *ener, int n, double unit);
-// Default work shape of a batch: windows (radius chunk x zone, over all requests)
-// and the most bins of a profile grid.
+// Default work shape of a batch: windows (radius chunk x zone, over all requests),
+// the most bins of a profile grid, and the bins that the windows together can
+// reach (reach_bins of a request times its windows).
 struct WorkShape {
   int seg_bins, waves_per_cu;
 };
