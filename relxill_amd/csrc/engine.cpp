@@ -1177,14 +1177,9 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
   const int64_t n_fin = b.any_flux ? o_flux : 0;
   layout_block(b);
   b.staged = b.block_bytes <= STAGE_MAX;
-  // (a server slot takes pinned memory from its second large batch on: allocating
-  // it costs a new server's first batches more than their copies)
-  if (b.one_shot && b.h_stage.bytes < b.block_bytes && !b.stage_wanted) {
-    b.stage_wanted = true;
-    b.staged = false;
-  }
   if (b.keep_stage && b.staged) {
-    if (!b.h_stage.ensure(std::max<size_t>(b.block_bytes, b.one_shot ? STAGE_MAX : 0))) {
+    const size_t least = !b.reserve ? 0 : b.block_bytes <= SLOT_SMALL ? SLOT_SMALL : STAGE_MAX;
+    if (!b.h_stage.ensure(std::max(b.block_bytes, least))) {
       err = "pinned host allocation failed";
       return RX_ERR_NOMEM;
     }
@@ -1349,7 +1344,7 @@ int integrate_blocks(int item_cap, int64_t windows, int waves_per_cu) {
 
 int batch_place_items(Batch &b) {
   b.ready = false;
-  if (b.d_items.ensure(sizeof(WorkItem) * (size_t)b.item_cap)) return RX_ERR_NOMEM;
+  if (b.d_items.ensure(std::max(sizeof(WorkItem) * (size_t)b.item_cap, b.reserve ? SLOT_SMALL : 0))) return RX_ERR_NOMEM;
   b.dev.items = b.d_items.as<WorkItem>();
   b.dev.item_cap = b.item_cap;
   b.dev.seg_bins = b.seg_bins;
@@ -1388,11 +1383,12 @@ int batch_upload(Batch &b) {
   for (int i = 0; i < b.n_req; i++) bins += b.h_req[i].n_e;
   b.fix_cap = (int)std::min<int64_t>(1 << 22, std::max<int64_t>(1 << 16, bins / 8));
   const size_t o_fix = take(sizeof(FixEntry) * (size_t)b.fix_cap);
-  e |= b.d_arena.ensure(used);
+  e |= b.d_arena.ensure(std::max(used, b.reserve));
   b.call_run = b.is_call && b.staged && sizeof(double) * b.tot_flux <= STAGE_MAX;
   if (b.call_run) b.deliver_out = b.tot_flux;
   else if (b.is_call) b.deliver_out = 0;
-  if (!b.h_res.ensure(result_out_offset(b.n_req) + sizeof(double) * b.deliver_out)) e |= 1;
+  const size_t res_bytes = result_out_offset(b.n_req) + sizeof(double) * b.deliver_out;
+  if (!b.h_res.ensure(std::max(res_bytes, b.reserve ? SLOT_SMALL : 0))) e |= 1;
   if (e) return RX_ERR_NOMEM;
   char *base = b.d_arena.as<char>();
   auto at = [&](auto *&ptr, size_t off) { ptr = reinterpret_cast<std::remove_reference_t<decltype(ptr)>>(base + off); };

@@ -83,6 +83,16 @@ struct RunKey {
 // Request blocks up to STAGE_MAX go to the device through pinned memory in one
 // piece; larger ones piece by piece from the batch's own arrays, a copy less.
 constexpr size_t STAGE_MAX = 4u << 20;
+// What a server slot's batch takes at least.  Growing frees memory, which waits for
+// the other slots' batches, and allocates anew: 250 us for 2 MB and more, device or
+// pinned, 1-60 us below that.  So its device allocation is SLOT_RESERVE at once (a
+// slot's share of the server's budget at most: Batch::reserve), its other pieces are
+// just below 2 MB, and its pinned request block is that or, for larger requests,
+// STAGE_MAX.  Bursts of 8 / 32 / 64 / 128 requests at a new server, the first / second
+// / third of them in ms: 0.7 0.3 0.3 / 1.0 0.7 0.7 / 1.5 1.2 1.2 / 3.8 2.3 2.0; with
+// every piece grown to what the batch at hand takes 1.3 0.9 0.5 / 2.0 1.5 0.7 / 2.8 2.8
+// 2.2 / 6.2 6.5 4.7.
+constexpr size_t SLOT_RESERVE = 16u << 20, SLOT_SMALL = 1900u << 10;
 
 struct Batch {
   int n_req = 0;
@@ -115,6 +125,7 @@ struct Batch {
   // outputs, distributions, zones and statuses where they are.
   DevBuf d_arena, d_items;
   bool ready = false;  // both are there and laid out
+  size_t reserve = 0;  // a server slot: least bytes of d_arena (SLOT_RESERVE)
   BatchDev dev;   // its pointers (dev_view adds the run's settings and the tables)
   WorkLists wl;
   size_t block_bytes = 0;
@@ -127,7 +138,6 @@ struct Batch {
   // keep their own, others use the library's while they are built), the run's
   // results (result_*).
   bool keep_stage = false;
-  bool stage_wanted = false;  // a server slot's pinned request block has been missed once
   PinnedBuf h_stage, h_res;
   // an evaluation call: the run fetches the request block and delivers the
   // outputs itself (call_run: this one does)

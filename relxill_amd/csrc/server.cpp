@@ -140,6 +140,7 @@ int rx_server::launch(Slot &s, std::vector<Pending> &take, std::string &err) {
   s.batch.waves_forced = 0;
   s.batch.one_shot = true;
   s.batch.keep_stage = true;
+  s.batch.reserve = (size_t)std::min<int64_t>(SLOT_RESERVE, budget / n_streams);
   // the run delivers every output to the slot's pinned memory
   int64_t n_out = 0;
   for (const Pending &p : take) n_out += (int64_t)p.energy.size() - 1;
