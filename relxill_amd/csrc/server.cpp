@@ -38,9 +38,7 @@ namespace {
 
 using Clock = std::chrono::steady_clock;
 
-// work-list sizing bound of the admission estimate (the smallest segment
-// length the autotuner may choose; the default shape's shorter segments are for
-// batches of at most 32 requests, a few 100 KB a slot)
+// the smallest segment length the autotuner may choose
 constexpr int SERVER_MIN_SEG_BINS = 32;
 
 struct Pending {
@@ -49,7 +47,8 @@ struct Pending {
   int refl_set;
   std::vector<double> energy, params, flux_in;
   Clock::time_point t_submit;
-  int64_t bytes;
+  int64_t bytes;          // of the device working set, without the work list
+  int64_t windows, bins;  // of its profile: (radius chunk, zone) pairs, bins a pair
 };
 
 struct Result {
@@ -66,7 +65,8 @@ struct Slot {
   int64_t bytes = 0;
 };
 
-int64_t request_bytes(const Pending &p) {
+// Sets the request's share of the admission estimate.
+void estimate(Pending &p) {
   Global &g = G();
   const bool lpx = (p.model == MOD_RELXILLLP || p.model == MOD_RELXILLLPCP);
   const bool xill = (p.model == MOD_XILLVER || p.model == MOD_XILLVERCP || p.model == MOD_XILLVERNS);
@@ -81,7 +81,6 @@ int64_t request_bytes(const Pending &p) {
   const int64_t n_rc = (g.nr_fine + RAD_CHUNK - 1) / RAD_CHUNK;
   int64_t b = sizeof(ReqParams) + 8 * (2 * (n_in + 1) + 2 * n_in);
   b += 8 * (n_e + 1) + 8 * n_e * nz;
-  b += (int64_t)sizeof(WorkItem) * (n_rc + nz - 1) * ((n_e + SERVER_MIN_SEG_BINS - 1) / SERVER_MIN_SEG_BINS);
   b += (int64_t)sizeof(FixEntry) * (n_e / 8 + 1);
   b += (int64_t)sizeof(RadRec) * g.nr_fine + 8 * RAD_NODE_ARRAYS * (int64_t)g.rel.n_r;
   b += 8 * MAX_INCL * nz + sizeof(LpRefl) + sizeof(ReqNorm) + 64;
@@ -89,11 +88,30 @@ int64_t request_bytes(const Pending &p) {
     int64_t ne = 0;
     for (int pr = 0; pr < N_PRIM; pr++) ne = std::max<int64_t>(ne, g.xill[pr].t.n_ener);
     b += (8 * ne + (int64_t)(2 * sizeof(XillWork) + sizeof(ZoneRec)) + 16) * nz;
+    if (lpx) b += 8 * 3 * 2 * (int64_t)rrad_chunks((int)ne) * nz;  // (the returning radiation's band sums)
   }
+  if (lpx || p.model == MOD_RELLINELP || p.model == MOD_RELCONVLP) b += 8 * 2 * MAX_RR + 4;
   if (p.model == MOD_RELXILLCP || p.model == MOD_RELXILLLPCP || p.model == MOD_XILLVERCP)  // nthcomp solves
     b += (int64_t)(sizeof(XillWork) + sizeof(NthRes)) * (nz + 1) + 8 * (2 * NTH_MAX_POINTS + 1) + 4;
-  return b;
+  p.bytes = b;
+  p.windows = xill ? 0 : n_rc + nz - 1;
+  p.bins = xill ? 0 : n_e;
 }
+
+// The work list of a batch, whose segments follow the whole batch.
+struct ListSize {
+  int64_t windows = 0, window_bins = 0;
+  int max_bins = 0;
+  void add(const Pending &p) {
+    windows += p.windows;
+    window_bins += p.windows * p.bins;
+    max_bins = (int)std::max<int64_t>(max_bins, p.bins);
+  }
+  int64_t bytes() const {
+    const int seg = std::min(SERVER_MIN_SEG_BINS, work_shape(windows, max_bins, window_bins).seg_bins);
+    return (int64_t)sizeof(WorkItem) * (window_bins / seg + windows);
+  }
+};
 
 }  // namespace
 
@@ -159,6 +177,7 @@ void rx_server::launch_ready(std::unique_lock<std::mutex> &lk) {
     if (s.busy || pending.empty()) continue;
     std::vector<Pending> take;
     int64_t bytes = 0;
+    ListSize list;
     // as many as one pinned request block holds (grids, inputs, parameters): a
     // backlog then goes over the slots, and neither the build of a batch nor the
     // hand-out of its results, under the lock, grows with it.  100 k requests a
@@ -169,12 +188,16 @@ void rx_server::launch_ready(std::unique_lock<std::mutex> &lk) {
       block += 2 * sizeof(double) * p.energy.size() + 1024;
       if (!take.empty() && block > STAGE_MAX) break;
       if (inflight_reqs + (int)take.size() >= max_inflight) break;
-      if (inflight_bytes + bytes + p.bytes > budget && !(take.empty() && inflight_reqs == 0)) break;
+      ListSize with = list;
+      with.add(p);
+      if (inflight_bytes + bytes + p.bytes + with.bytes() > budget && !(take.empty() && inflight_reqs == 0)) break;
       bytes += p.bytes;
+      list = with;
       take.push_back(std::move(p));
       pending.pop_front();
     }
     if (take.empty()) break;
+    bytes += list.bytes();
     s.busy = true;  // reserved: its budget share is counted below
     inflight_bytes += bytes;
     inflight_reqs += (int)take.size();
@@ -315,7 +338,7 @@ int64_t rx_server_submit(rx_server *s, const rx_request *req) {
   if (req->flux_in) p.flux_in.assign(req->flux_in, req->flux_in + req->n_flux);
   p.t_submit = Clock::now();
   std::lock_guard<std::mutex> lk(s->mu);
-  p.bytes = request_bytes(p);
+  estimate(p);
   p.ticket = s->next_ticket++;
   s->results[p.ticket] = Result();
   s->submitted++;
