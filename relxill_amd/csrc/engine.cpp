@@ -49,6 +49,7 @@ bool PinnedBuf::ensure(size_t n) {
   p = nullptr;
   bytes = 0;
   if (hipHostMalloc(&p, n, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();  // (as below)
     p = nullptr;
     return false;
   }
@@ -68,6 +69,7 @@ int DevBuf::ensure(size_t n) {
   bytes = 0;
   hipError_t e = hipMalloc(&p, n);
   if (e != hipSuccess) {
+    (void)hipGetLastError();  // reported here: the next launch's check must not find it
     p = nullptr;
     return (int)e;
   }
