@@ -530,7 +530,7 @@ int ensure_device(std::string &err) {
   } else {
     (void)hipSetDevice(g.device);
   }
-  int e = 0;
+  int e = 0;  // (what could not be uploaded stays to be uploaded)
   const bool lp_dirty = g.lp_dirty && g.lp_loaded;
   if (g.rel_dirty || lp_dirty || g.conv_dirty || g.refl_dirty) {
     // resident buffers are about to be overwritten or reallocated: no kernel
@@ -549,7 +549,7 @@ int ensure_device(std::string &err) {
     e |= upload_vec(g.t_a, t.a) | upload_vec(g.t_mu0, t.mu0) | upload_vec(g.t_r, t.r) |
          upload_vec(g.t_gmin, t.gmin) | upload_vec(g.t_gmax, t.gmax) | upload_vec(g.t_trff1, t.trff1) |
          upload_vec(g.t_trff2, t.trff2) | upload_vec(g.t_cosne1, t.cosne1) | upload_vec(g.t_cosne2, t.cosne2);
-    g.rel_dirty = false;
+    if (!e) g.rel_dirty = false;
   }
   if (lp_dirty) {
     const LpTableHost &t = g.lp;
@@ -559,7 +559,7 @@ int ensure_device(std::string &err) {
     }
     e |= upload_vec(g.l_a, t.a) | upload_vec(g.l_h, t.h) | upload_vec(g.l_rad, t.rad) |
          upload_vec(g.l_int, t.intens) | upload_vec(g.l_del, t.del) | upload_vec(g.l_inc, t.del_inc);
-    g.lp_dirty = false;
+    if (!e) g.lp_dirty = false;
   }
   if (g.conv_dirty) {
     e |= upload_vec(g.c_coarse, g.coarse_ener) | upload_vec(g.c_coarse_ln, g.coarse_ln);
@@ -567,16 +567,18 @@ int ensure_device(std::string &err) {
     e |= upload_vec(g.c_ener, g.conv_ener) | upload_vec(g.c_cfac, g.conv_cfac) | upload_vec(g.c_tw, g.conv_tw);
     e |= upload_vec(g.c_cfinv, g.conv_cfinv) | upload_vec(g.c_inv_emid, g.conv_inv_emid);
     e |= upload_vec(g.c_twp_fwd, g.conv_twp_fwd) | upload_vec(g.c_twp_inv, g.conv_twp_inv);
-    g.conv_dirty = false;
+    if (!e) g.conv_dirty = false;
   }
   if (g.refl_dirty) {
     e |= upload_vec(g.d_refl_sets, g.refl_sets);
-    g.refl_dirty = false;
+    if (!e) g.refl_dirty = false;
   }
-  if (!g.nth_grid.p) {
-    e |= g.nth_grid.ensure(nth_grid_bytes());
-    if (!e) e |= launch_nth_grid(g.nth_grid.as<double>(), nullptr);
-    e |= (int)hipDeviceSynchronize();  // read from other streams
+  if (!g.nth_grid_ready) {
+    int n = g.nth_grid.ensure(nth_grid_bytes());
+    if (!n) n |= launch_nth_grid(g.nth_grid.as<double>(), nullptr);
+    n |= (int)hipDeviceSynchronize();  // read from other streams
+    g.nth_grid_ready = n == 0;
+    e |= n;
   }
   if (e) {
     err = "device upload failed";

@@ -264,6 +264,7 @@ struct Global {
   bool rrad_loaded = false, rrad_dirty = true;
   PinnedBuf stage;  // request block of the batch being built (under mu)
   DevBuf nth_grid;  // what all nthcomp solves share
+  bool nth_grid_ready = false;
   DevBuf r_rlo, r_rhi, r_tf, r_gmin, r_gmax, r_fg;
   // convolution grid
   int conv_n = 4096;
