@@ -465,20 +465,6 @@ __device__ inline int wave_max_i(int v) {
              max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
 }
 
-// block-wide maximum
-__device__ inline double block_max(double v, double *red) {
-  const int tid = threadIdx.x;
-  red[tid] = v;
-  __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if (tid < s) red[tid] = fmax(red[tid], red[tid + s]);
-    __syncthreads();
-  }
-  double r = red[0];
-  __syncthreads();
-  return r;
-}
-
 // 1/x to within an ulp or two: hardware estimate and two Newton steps
 // (cheaper than the IEEE division sequence; the rebin weights need ~1e-15).
 __device__ __forceinline__ double rcp64(double x) {
@@ -2191,7 +2177,7 @@ __global__ __launch_bounds__(FINAL_THREADS) void k_finalize(BatchDev b, Deliver 
 namespace {
 
 // LDS index of complex element i: one pad slot every 16 elements, so that the
-// stride-16 writes of a radix-16 pass fall into distinct banks.
+// strided writes of the passes spread over the banks.
 __device__ inline int P(int i) { return i + (i >> 4); }
 
 __device__ inline double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
@@ -2230,7 +2216,7 @@ __device__ inline void tw16(double2 &x) {
   if (N2 * K1 != 0) x = cmul(x, w16<S, N2 * K1>());
 }
 
-// In-register DFT of length R (2, 4, 8 or 16), natural order in and out.
+// In-register DFT of length R (2, 4 or 8), natural order in and out.
 template <int R, int S>
 __device__ __forceinline__ void dft(double2 *v) {
   if (R == 2) {
@@ -2239,7 +2225,8 @@ __device__ __forceinline__ void dft(double2 *v) {
     v[1] = csub(t, v[1]);
   } else if (R == 4) {
     dft4<S>(v[0], v[1], v[2], v[3]);
-  } else if (R == 8) {
+  } else {
+    static_assert(R == 2 || R == 4 || R == 8, "the passes' radices");
     // n = 2 n1 + n2, k = k1 + 4 k2: two DFT4 (even, odd), twiddle, butterflies
     dft4<S>(v[0], v[2], v[4], v[6]);
     dft4<S>(v[1], v[3], v[5], v[7]);
@@ -2256,35 +2243,6 @@ __device__ __forceinline__ void dft(double2 *v) {
     v[6] = csub(e2, o2);
     v[3] = cadd(e3, o3);
     v[7] = csub(e3, o3);
-  } else {
-    // n = 4 n1 + n2, k = k1 + 4 k2: DFT4 over n1 for each n2 (result k1 in
-    // slot n2 + 4 k1), twiddle w16^(n2 k1), DFT4 over n2 for each k1 (result
-    // k2 in slot n2 = k2 of row k1), then the transpose to natural order.
-    dft4<S>(v[0], v[4], v[8], v[12]);
-    dft4<S>(v[1], v[5], v[9], v[13]);
-    dft4<S>(v[2], v[6], v[10], v[14]);
-    dft4<S>(v[3], v[7], v[11], v[15]);
-    tw16<S, 1, 1>(v[5]);
-    tw16<S, 1, 2>(v[9]);
-    tw16<S, 1, 3>(v[13]);
-    tw16<S, 2, 1>(v[6]);
-    tw16<S, 2, 2>(v[10]);
-    tw16<S, 2, 3>(v[14]);
-    tw16<S, 3, 1>(v[7]);
-    tw16<S, 3, 2>(v[11]);
-    tw16<S, 3, 3>(v[15]);
-    dft4<S>(v[0], v[1], v[2], v[3]);
-    dft4<S>(v[4], v[5], v[6], v[7]);
-    dft4<S>(v[8], v[9], v[10], v[11]);
-    dft4<S>(v[12], v[13], v[14], v[15]);
-    // slot 4 k1 + k2 holds X[k1 + 4 k2]
-    double2 t[16];
-#pragma unroll
-    for (int k1 = 0; k1 < 4; k1++)
-#pragma unroll
-      for (int k2 = 0; k2 < 4; k2++) t[k1 + 4 * k2] = v[4 * k1 + k2];
-#pragma unroll
-    for (int k = 0; k < 16; k++) v[k] = t[k];
   }
 }
 

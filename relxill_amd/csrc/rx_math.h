@@ -721,18 +721,6 @@ RX_HD inline int bsearch_asc(const T *arr, int n, V val) {
   return klo;
 }
 
-// descending search (src/relutility.c:195-211)
-template <class T, class V>
-RX_HD inline int bsearch_desc(const T *arr, int n, V val) {
-  if (n <= 1) return -1;
-  int klo = 0, khi = n - 1;
-  while ((khi - klo) > 1) {
-    int k = (khi + klo) / 2;
-    if (arr[k] < val) khi = k; else klo = k;
-  }
-  return klo;
-}
-
 // Places for a request's tot long work items (from the front of the list) and
 // tots short ones (from its back).  Both counts are in one 64-bit counter (long
 // ones in the low half), so that one add decides whether all of them fit between
