@@ -1348,8 +1348,12 @@ int integrate_blocks(int item_cap, int64_t windows, int waves_per_cu) {
 
 int batch_place_items(Batch &b) {
   b.ready = false;
-  if (b.d_items.ensure(std::max(sizeof(WorkItem) * (size_t)b.item_cap, b.reserve ? SLOT_SMALL : 0))) return RX_ERR_NOMEM;
-  b.dev.items = b.d_items.as<WorkItem>();
+  if (b.item_cap <= b.arena_items) {
+    b.dev.items = reinterpret_cast<WorkItem *>(b.d_arena.as<char>() + b.arena_items_at);
+  } else {
+    if (b.d_items.ensure(sizeof(WorkItem) * (size_t)b.item_cap)) return RX_ERR_NOMEM;
+    b.dev.items = b.d_items.as<WorkItem>();
+  }
   b.dev.item_cap = b.item_cap;
   b.dev.seg_bins = b.seg_bins;
   b.ready = true;
@@ -1387,6 +1391,8 @@ int batch_upload(Batch &b) {
   for (int i = 0; i < b.n_req; i++) bins += b.h_req[i].n_e;
   b.fix_cap = (int)std::min<int64_t>(1 << 22, std::max<int64_t>(1 << 16, bins / 8));
   const size_t o_fix = take(sizeof(FixEntry) * (size_t)b.fix_cap);
+  b.arena_items_at = take(sizeof(WorkItem) * (size_t)b.item_cap);
+  b.arena_items = b.item_cap;
   e |= b.d_arena.ensure(std::max(used, b.reserve));
   b.call_run = b.is_call && b.staged && sizeof(double) * b.tot_flux <= STAGE_MAX;
   if (b.call_run) b.deliver_out = b.tot_flux;

@@ -118,13 +118,16 @@ struct Batch {
   int n_nth_sol = 0;             // requests with the nthcomp primary (one source solution each)
   int64_t tot_ener = 0, tot_flux = 0, tot_pgrid = 0, tot_prof = 0, tot_xspec = 0, tot_dist = 0, tot_zone = 0;
   int64_t tot_rrc = 0;
-  // One device allocation holds everything of the batch but k_integrate's work
-  // list; it begins with the request block (what the host writes: parameters,
-  // statuses, work lists, grids, input spectra).  The work list, whose length
-  // follows the work shape, has its own: a new shape leaves the last run's
-  // outputs, distributions, zones and statuses where they are.
+  // One device allocation holds everything of the batch; it begins with the
+  // request block (what the host writes: parameters, statuses, work lists, grids,
+  // input spectra) and ends with k_integrate's work list as the batch was built.  A
+  // work shape set later whose list is longer has it in an allocation of its own, so
+  // that the last run's outputs, distributions, zones and statuses stay where they
+  // are.
   DevBuf d_arena, d_items;
-  bool ready = false;  // both are there and laid out
+  int arena_items = 0;        // items that the first one's list takes
+  size_t arena_items_at = 0;  // its offset
+  bool ready = false;  // what the batch needs is there and laid out
   size_t reserve = 0;  // a server slot: least bytes of d_arena (SLOT_RESERVE)
   BatchDev dev;   // its pointers (dev_view adds the run's settings and the tables)
   WorkLists wl;
