@@ -547,7 +547,7 @@ __device__ inline double block_sum(double v, double *red) {
 // step.  Batches that leave the chip idle get workgroups of 512 threads, which
 // take the 1000 radii in two rounds instead of four.  Measured before and after:
 // relline call 24 -> 15 us, relline_lp call 43 -> 27 us, relxilllp call 62 -> 31
-// us, 256 relline_lp requests 50 -> 33 us, 4096 relconv requests 176 -> 145 us.
+// us, 256 relline_lp requests 50 -> 33 us, 4096 relconv requests 176 -> 131 us.
 template <int NZ, int NT>
 __global__ __launch_bounds__(NT, NT == 256 ? 3 : 1) void k_setup(BatchDev b) {
   constexpr int NW = NT / 64;
@@ -1371,8 +1371,7 @@ __global__ __launch_bounds__(64 * RR_ZONES) void k_rrad(BatchDev b, const int *_
 // Kompaneets solve per (request, j) of work, j = 0 for the source's kTe (the
 // nthcomp models keep kTe in the source frame, src/Relxill.cpp:197-200),
 // j = 1 + z for the kTe lamp-post zone z sees (kTe times the zone's source ->
-// disk energy shift, src/IonGradient.cpp:196-209, from the zone record as
-// k_setup computes it).  Each solve writes its normalisation nf on the
+// disk energy shift, src/IonGradient.cpp:196-209, from zone_record).  Each solve writes its normalisation nf on the
 // 500-bin grid and the energy flux of the normalised spectrum in 0.1-1000 keV
 // (calc_xillver_normalization_change_source_to_disk, src/Xillspec.cpp:408-435;
 // get_xillver_fluxcorr, :344-362); the source's also keeps its solution for
@@ -1501,8 +1500,6 @@ __global__ __launch_bounds__(COPY_THREADS) void k_deliver(BatchDev b, int *__res
 // ---------------------------------------------------------------------------
 namespace {
 
-// The transfer function (and cosines) of one fine radius, lerped from its two
-// table-node rows into a lane-private LDS row, and the FP64 edge norms.
 // One row of a fine radius (2 n_g values), lerped from its two node rows into
 // LDS; 8 values per round, so that a round's 16 loads are in flight together.
 template <class TV>
@@ -1524,8 +1521,8 @@ __device__ inline void lerp_row(double ifac, const double *lo, const double *hi,
 // A request's (a, mu0)-interpolated node rows (interpol_a_mu0,
 // src/Relprofile.cpp:39-80), read from the table's four corners: row ir,
 // column c (g* column c >> 1, branch c & 1) of the transfer function or of
-// the emission-angle cosines.  k_setup computes the same lerp2f for the rows
-// of the angle distribution, so every consumer sees the same bits.
+// the emission-angle cosines.  k_integrate, k_fixup and the angle distributions
+// all build their rows from it, so every consumer sees the same bits.
 struct NodeSrc {
   const float *a1, *a2;  // branch 0 and 1 arrays
   size_t s00, s10, s01, s11;

@@ -93,7 +93,7 @@ int noalloc_setup(int device, std::string &err) {
     err = "hipGetSymbolAddress of the scratch array failed";
     return RX_ERR_DEVICE;
   }
-  // (4 KB for the process's life, as the scratch array)
+  // (a few words for the process's life, as the scratch array)
   void *r = nullptr;
   if (hipHostMalloc(&r, sizeof(int) * (RES_CTR + 1), hipHostMallocDefault) != hipSuccess) {
     (void)hipGetLastError();
