@@ -892,12 +892,17 @@ __global__ __launch_bounds__(NT, NT == 256 ? 3 : 1) void k_setup(BatchDev b) {
       static_assert(CTR_ITEMS % 2 == 0 && CTR_ITEMS_S == CTR_ITEMS + 1, "one aligned 64-bit word");
       unsigned long long *ctr = reinterpret_cast<unsigned long long *>(&b.ctr[CTR_ITEMS]);
       int base, bases;
+      bool first_out;
       // the host sizes the list for the bins that the table's radii reach
       // (reach_bins); a request that it does not hold all the same fails, and its
       // neighbours' items stay whole
       if (!reserve_items([&](uint64_t v) { return (uint64_t)atomicAdd(ctr, (unsigned long long)v); }, tot, tots,
-                         b.item_cap, base, bases)) {
+                         b.item_cap, base, bases, first_out)) {
         atomicOr(&b.ctr[CTR_ITEMS_OVF], 1);
+        if (first_out) {
+          b.ctr[CTR_FIT] = base;
+          b.ctr[CTR_FIT_S] = bases;
+        }
         base = -1;
       }
       s_base = base;
@@ -1862,8 +1867,9 @@ __global__ __launch_bounds__(64, MODE == 0 ? 1 : 3) void k_integrate(BatchDev b_
                                               integrate_rows_bytes(ng, cos_rows != 0, sizeof(TV)));
   TV *s_bins = (MODE == 0) ? reinterpret_cast<TV *>(s_coef + 64) : reinterpret_cast<TV *>(s_coef);
   // long items at [0, n_long), short ones at the back of the list
-  const int n_long = min(b.ctr[CTR_ITEMS], b.item_cap);
-  const int n_short = min(b.ctr[CTR_ITEMS_S], b.item_cap - n_long);
+  const int asked = b.ctr[CTR_ITEMS], asked_s = b.ctr[CTR_ITEMS_S], fit = b.ctr[CTR_FIT], fit_s = b.ctr[CTR_FIT_S];
+  const bool ovf = b.ctr[CTR_ITEMS_OVF] != 0;
+  const int n_long = ovf ? fit : asked, n_short = ovf ? fit_s : asked_s;
   const int nr = b.nr_fine;
   // turn-round roles: SUM_LANES lanes per bin; lane (col, part) sums radii
   // SUM_BINS part .. SUM_BINS part + SUM_BINS - 1 of bin col

@@ -328,9 +328,11 @@ constexpr int XQ_STRIDE = 32;  // ints between the range counters (one 128-byte 
 enum CounterSlot : int {
   CTR_FIX = 0,        // FixEntry entries written
   CTR_FIX_OVF = 1,    // FixEntry queue overflowed
-  CTR_ITEMS = 2,      // long work items written (from the front of the list)
-  CTR_ITEMS_S = 3,    // short work items written (from the back of the list); one 64-bit word with CTR_ITEMS
-  CTR_ITEMS_OVF = 4,  // work list overflowed
+  CTR_ITEMS = 2,      // long work items asked for (from the front of the list)
+  CTR_ITEMS_S = 3,    // short work items asked for (from the back of the list); one 64-bit word with CTR_ITEMS
+  CTR_ITEMS_OVF = 4,  // work list overflowed: the items written are CTR_FIT and CTR_FIT_S
+  CTR_FIT = 5,
+  CTR_FIT_S = 6,
   CTR_XQ = XQ_STRIDE,  // N_XQ range counters, XQ_STRIDE apart
   N_COUNTERS = CTR_XQ + N_XQ * XQ_STRIDE
 };

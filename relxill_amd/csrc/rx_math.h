@@ -724,18 +724,19 @@ RX_HD inline int bsearch_asc(const T *arr, int n, V val) {
 // Places for a request's tot long work items (from the front of the list) and
 // tots short ones (from its back).  Both counts are in one 64-bit counter (long
 // ones in the low half), so that one add decides whether all of them fit between
-// the two ends; an add that does not fit is taken back.  While it stands no other
-// one fits either, so the places given out leave no gaps.  add: atomic, returns
-// the value before.
+// the two ends.  The first add that does not fit stays, so that none behind it
+// fits either: the places given out are those of the adds before it, without a
+// gap, and first_out tells that request to keep their counts (base, bases).  add:
+// atomic, returns the value before.
 template <class Add>
-RX_HD inline bool reserve_items(Add add, int tot, int tots, int cap, int &base, int &bases) {
-  const uint64_t n = (uint64_t)(uint32_t)tot | (uint64_t)(uint32_t)tots << 32;
-  const uint64_t was = add(n);
+RX_HD inline bool reserve_items(Add add, int tot, int tots, int cap, int &base, int &bases, bool &first_out) {
+  const uint64_t was = add((uint64_t)(uint32_t)tot | (uint64_t)(uint32_t)tots << 32);
+  const uint64_t used = (was & 0xffffffffull) + (was >> 32);
   base = (int)(uint32_t)was;
   bases = (int)(was >> 32);
-  if ((was & 0xffffffffull) + (was >> 32) + (uint64_t)tot + (uint64_t)tots <= (uint64_t)cap) return true;
-  (void)add(0 - n);
-  return false;
+  const bool fits = used + (uint64_t)tot + (uint64_t)tots <= (uint64_t)cap;
+  first_out = !fits && used <= (uint64_t)cap;
+  return fits;
 }
 
 // fine radial grid point ii (src/relutility.c:666-677), from r1 = 1/sqrt(Rout)

@@ -1,7 +1,8 @@
 """Places in k_integrate's work list (reserve_items), compiled for the host and
 asked for by several threads at once: lists that hold every request and lists
-that do not.  Long items grow from the front and short ones from the back, and
-no place may be given out twice, nor any left out before the last."""
+that do not.  Long items grow from the front and short ones from the back, no
+place may be given out twice, and the places up to the counts that the first
+refused request keeps are all given out, none beyond."""
 import os
 import subprocess
 
@@ -25,8 +26,8 @@ int main(int argc, char **argv) {
     std::atomic<uint64_t> ctr{0};
     std::vector<std::atomic<int>> slot(cap);
     for (auto &s : slot) s = 0;
-    std::atomic<int> bad{0}, refused{0};
-    std::atomic<long> given{0};
+    std::atomic<int> bad{0}, refused{0}, first{0};
+    std::atomic<long> fit{0}, fit_s{0};
     std::vector<std::thread> th;
     for (int t = 0; t < 8; t++)
       th.emplace_back([&, t] {
@@ -35,11 +36,16 @@ int main(int argc, char **argv) {
           r = r * 1664525u + 1013904223u;
           const int tot = (r >> 8) % (most + 1), tots = (r >> 20) % 17;
           int base = -1, bases = -1;
-          if (!rx::reserve_items([&](uint64_t v) { return ctr.fetch_add(v); }, tot, tots, cap, base, bases)) {
+          bool first_out = false;
+          if (!rx::reserve_items([&](uint64_t v) { return ctr.fetch_add(v); }, tot, tots, cap, base, bases, first_out)) {
             refused++;
+            if (first_out) {
+              first++;
+              fit = base;
+              fit_s = bases;
+            }
             continue;
           }
-          given += tot + tots;
           for (int k = 0; k < tot + tots; k++) {
             const int at = k < tot ? base + k : cap - 1 - (bases + (k - tot));
             if (at < 0 || at >= cap || slot[at].fetch_add(1) != 0) bad++;
@@ -47,8 +53,9 @@ int main(int argc, char **argv) {
         }
       });
     for (auto &x : th) x.join();
-    const long n_long = (uint32_t)ctr.load(), n_short = ctr.load() >> 32;
-    if (n_long + n_short != given) bad++;  // (what was refused is out of the counts)
+    if (first != (refused ? 1 : 0)) bad++;
+    const long n_long = refused ? (long)fit : (long)(uint32_t)ctr.load();
+    const long n_short = refused ? (long)fit_s : (long)(ctr.load() >> 32);
     for (long k = 0; k < cap; k++)
       if ((slot[k] == 1) != (k < n_long || k >= cap - n_short)) bad++;
     printf("%d %d\n", (int)bad, (int)refused);
