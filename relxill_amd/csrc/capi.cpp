@@ -778,7 +778,7 @@ int rx_batch_counters(rx_batch *b, int64_t *out) {
   return RX_OK;
 }
 
-// Times every (segment bins, waves per CU) candidate on this batch and keeps
+// Times the default and every (segment bins, waves per CU) candidate on this batch and keeps
 // the fastest for batches of the same shape class (log2 of the profile bins
 // and whether convolutions are present).
 int rx_batch_autotune(rx_batch *b, int precision) {
@@ -808,13 +808,14 @@ int rx_batch_autotune(rx_batch *b, int precision) {
     }
     return true;
   };
-  for (int w : wpcs) {
-    for (int sg : segs) {
-      double dt = 1e30;
-      if (!time_shape(sg, w, 3, 2, dt)) return -RX_ERR_DEVICE;
-      cands.push_back({sg, w, dt});
-    }
-  }
+  // the default shape too: small batches' has shorter segments than these
+  const WorkShape def = batch_default_shape(b->b);
+  cands.push_back({def.seg_bins, def.waves_per_cu, 1e30});
+  for (int w : wpcs)
+    for (int sg : segs)
+      if (sg != def.seg_bins || w != def.waves_per_cu) cands.push_back({sg, w, 1e30});
+  for (auto &c : cands)
+    if (!time_shape(c.seg, c.wpc, 3, 2, c.dt)) return -RX_ERR_DEVICE;
   // the three fastest timed again, in turns, with more runs: shapes within a
   // few percent of each other are told apart despite the host timer's noise
   std::sort(cands.begin(), cands.end(), [](const Cand &x, const Cand &y) { return x.dt < y.dt; });

@@ -1228,6 +1228,39 @@ int batch_build(Batch &b, const rx_request *req_in, int n_req, std::string &err)
   return batch_upload(b);
 }
 
+// What the default work shape and the work list's length follow: the batch's
+// windows and, per request, the profile bins that the table's g range reaches.
+struct Reach {
+  std::vector<int> bins;  // 0: a request that does not run
+  int64_t windows = 0, window_bins = 0;
+  int max_bins = 0;
+};
+
+static int radius_chunks() { return (G().nr_fine + RAD_CHUNK - 1) / RAD_CHUNK; }
+
+static Reach batch_reach(const Batch &b) {
+  Global &g = G();
+  Reach r;
+  r.bins.assign(b.n_req, 0);
+  const int conv_reach = reach_bins(g.conv_ener.data(), g.conv_n, 1.0);
+  for (int i = 0; i < b.n_req; i++) {
+    const ReqParams &p = b.h_req[i];
+    if (b.h_status[i] != RX_OK || p.n_e <= 0) continue;
+    r.bins[i] = p.pgrid_off < 0 ? conv_reach
+                                : reach_bins(b.p_ener + p.ener_off, p.n_e, p.lineE / (p.z > 0 ? 1 + p.z : 1.0));
+    const int64_t w = radius_chunks() + p.n_zones - 1;
+    r.windows += w;
+    r.window_bins += w * r.bins[i];
+    r.max_bins = std::max(r.max_bins, p.n_e);
+  }
+  return r;
+}
+
+WorkShape batch_default_shape(const Batch &b) {
+  const Reach r = batch_reach(b);
+  return work_shape(r.windows, r.max_bins, r.window_bins);
+}
+
 void batch_plan(Batch &b, int seg_bins, int waves_per_cu) {
   Global &g = G();
   if (seg_bins <= 0 || waves_per_cu <= 0) {
@@ -1238,29 +1271,16 @@ void batch_plan(Batch &b, int seg_bins, int waves_per_cu) {
       }
     }
   }
-  const int n_rc = (g.nr_fine + RAD_CHUNK - 1) / RAD_CHUNK;
-  const int conv_reach = reach_bins(g.conv_ener.data(), g.conv_n, 1.0);
-  int64_t windows = 0, window_bins = 0;
-  int max_bins = 0;
-  std::vector<int> reach(b.n_req, 0);  // the profile bins that the table's g range reaches
-  for (int i = 0; i < b.n_req; i++) {
-    const ReqParams &p = b.h_req[i];
-    if (b.h_status[i] != RX_OK || p.n_e <= 0) continue;
-    reach[i] = p.pgrid_off < 0 ? conv_reach
-                               : reach_bins(b.p_ener + p.ener_off, p.n_e, p.lineE / (p.z > 0 ? 1 + p.z : 1.0));
-    windows += n_rc + p.n_zones - 1;
-    window_bins += (int64_t)(n_rc + p.n_zones - 1) * reach[i];
-    max_bins = std::max(max_bins, p.n_e);
-  }
-  const WorkShape ws = work_shape(windows, max_bins, window_bins);
+  const Reach r = batch_reach(b);
+  const WorkShape ws = work_shape(r.windows, r.max_bins, r.window_bins);
   // calls on one grid keep their segments and their list's length while the reach
   // stays near what they were chosen for: it moves with the line's energy and
   // redshift, and every change of either is another launch configuration
   Batch::CallShape &k = b.call_shape;
   if (b.is_call) {
-    const bool near = k.windows == windows && k.max_bins == max_bins && 2 * window_bins <= 3 * k.window_bins &&
-                      2 * k.window_bins <= 3 * window_bins;
-    if (!near) k = {windows, max_bins, window_bins, 0, 0};
+    const bool near = k.windows == r.windows && k.max_bins == r.max_bins && 2 * r.window_bins <= 3 * k.window_bins &&
+                      2 * k.window_bins <= 3 * r.window_bins;
+    if (!near) k = {r.windows, r.max_bins, r.window_bins, 0, 0};
     if (seg_bins <= 0) seg_bins = k.seg_bins;
   }
   if (seg_bins <= 0) seg_bins = ws.seg_bins;
@@ -1272,7 +1292,7 @@ void batch_plan(Batch &b, int seg_bins, int waves_per_cu) {
   // radius ranges, so a request has at most n_rc + n_zones - 1 such pairs
   int64_t cap = 0;
   for (int i = 0; i < b.n_req; i++)
-    cap += (int64_t)(n_rc + b.h_req[i].n_zones - 1) * ((reach[i] + seg_bins - 1) / seg_bins);
+    cap += (int64_t)(radius_chunks() + b.h_req[i].n_zones - 1) * ((r.bins[i] + seg_bins - 1) / seg_bins);
   if (b.is_call) {
     if (k.seg_bins != seg_bins || cap > k.item_cap) {
       k.seg_bins = seg_bins;
@@ -1281,7 +1301,7 @@ void batch_plan(Batch &b, int seg_bins, int waves_per_cu) {
     cap = k.item_cap;
   }
   b.item_cap = (int)std::min<int64_t>(std::max<int64_t>(cap, 1), INT32_MAX);
-  b.n_blocks = integrate_blocks(b.item_cap, windows, waves_per_cu);
+  b.n_blocks = integrate_blocks(b.item_cap, r.windows, waves_per_cu);
 }
 
 WorkShape work_shape(int64_t windows, int max_bins, int64_t window_bins) {

@@ -206,6 +206,7 @@ struct WorkShape {
   int seg_bins, waves_per_cu;
 };
 WorkShape work_shape(int64_t windows, int max_bins, int64_t window_bins);
+WorkShape batch_default_shape(const Batch &b);  // of a built batch
 // Workgroups of k_integrate for a work list of that capacity: one an item for
 // lists of up to ONE_ITEMS.
 constexpr int ONE_ITEMS = 1 << 18;
