@@ -413,10 +413,10 @@ int rx_batch_counters(rx_batch *b, int64_t *out);
 /* Launch graphs (default on): a batch run whose kernel arguments and grid
  * shapes equal the previous run's is captured into a hipGraph and replayed
  * while they stay equal (the XSPEC entry points reuse one batch, so repeated
- * calls on one grid replay a graph, whatever their parameters).
- * rx_set_graphs(0) launches every kernel directly.  rx_batch_graph_replays: runs
- * of the batch served by a graph; rx_call_graph_replays: calls of rx_eval_model
- * and the lmod* entry points.
+ * calls of one model on one grid replay a graph, also while the line's energy and
+ * the redshift vary).  rx_set_graphs(0) launches every kernel directly.
+ * rx_batch_graph_replays: runs of the batch served by a graph;
+ * rx_call_graph_replays: calls of rx_eval_model and the lmod* entry points.
  * No counterpart in the reference (launch mechanics of the device path). */
 int rx_set_graphs(int on);
 int64_t rx_batch_graph_replays(rx_batch *b);

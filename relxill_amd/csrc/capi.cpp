@@ -672,7 +672,11 @@ int rx_batch_set_shape(rx_batch *b, int seg_bins, int waves_per_cu) {
   std::lock_guard<std::recursive_mutex> lk(g.mu);
   b->b.seg_forced = seg_bins;
   b->b.waves_forced = waves_per_cu;
-  batch_plan(b->b, seg_bins, waves_per_cu);
+  try {
+    batch_plan(b->b, seg_bins, waves_per_cu);
+  } catch (...) {
+    return RX_ERR_NOMEM;
+  }
   return batch_place_items(b->b);
 }
 
@@ -781,7 +785,7 @@ int rx_batch_counters(rx_batch *b, int64_t *out) {
 // Times the default and every (segment bins, waves per CU) candidate on this batch and keeps
 // the fastest for batches of the same shape class (log2 of the profile bins
 // and whether convolutions are present).
-int rx_batch_autotune(rx_batch *b, int precision) {
+int rx_batch_autotune(rx_batch *b, int precision) try {
   if (!b) return RX_ERR_ARG;
   Global &g = G();
   std::lock_guard<std::recursive_mutex> lk(g.mu);
@@ -839,6 +843,8 @@ int rx_batch_autotune(rx_batch *b, int precision) {
   batch_plan(b->b, best_s, best_w);
   if (batch_place_items(b->b) != RX_OK) return -RX_ERR_DEVICE;
   return best_s * 256 + best_w;
+} catch (...) {
+  return -RX_ERR_NOMEM;
 }
 
 /* ---- reflection sets ---- */
